@@ -74,7 +74,7 @@ struct SolveDev {
     int cur;             // blocked path: ping-pong buffer holding the current correction
     unsigned int maxupd_bits[16];  // per-sweep max |delta| (float bits) for the max-update rule
     unsigned int seq;    // host mirror: written last by a check (the host waits for it)
-    unsigned int pad_;
+    int stop_lid;        // max-update rule: the launch that found the stop (INT_MAX: none)
 };
 
 // An event pair recorded around a group of launches; resolved (elapsed time
@@ -230,9 +230,9 @@ int cd_fill_i32(cd_context* ctx, int* p, size_t n, int v);
 
 // Device buffers of one plain Poisson solve, supplied by the caller instead
 // of the context's grow-only workspace (the allocation-free entry point).
-// Sizes for a w x h grid: partials 4*nred doubles (nred = ceil(w/64)*ceil(h/4)),
+// Sizes for a w x h grid: partials cd_partials_bytes(nred) (nred = ceil(w/64)*ceil(h/4)),
 // e32/e32b 2*plane floats each in the bricked layout (mixed precision without
-// holes; e32 n floats with holes), r BF16 2*plane (no holes), FP32 2*plane
+// holes; n floats each with holes), phi2 n doubles (FP64 sweeps), r BF16 2*plane (no holes), FP32 2*plane
 // (no holes, max-update rule) or FP32 n (holes).
 struct SolveWork {
     double* partials = nullptr;
@@ -240,7 +240,12 @@ struct SolveWork {
     float* e32 = nullptr;
     float* e32b = nullptr;
     void* r = nullptr;
+    double* phi2 = nullptr;
 };
+
+// Bytes of the reduction partials: four doubles for each of nred workgroups,
+// and room for the per-tile maxima of the max-update rule on small grids.
+constexpr size_t cd_partials_bytes(size_t nred) { return sizeof(double) * 4 * nred + 32768; }
 
 // Poisson solve on device-resident data.  b is the right-hand side (not
 // modified), phi the warm start/result (FP64).  mask: optional per-cell
@@ -252,7 +257,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                              cd_solve_stats* st, const SolveWork* work = nullptr);
 
 // Sizes of the solve buffers of a w x h grid: nred reduction blocks (the
-// partials hold 4*nred doubles) and npk elements of the bricked layout.
+// partials hold cd_partials_bytes(nred)) and npk elements of the bricked layout.
 void cd_solve_work_sizes(int w, int h, size_t* nred, size_t* npk);
 
 // Hole mask of a right-hand side (per-cell neighbour-validity bits, NaN

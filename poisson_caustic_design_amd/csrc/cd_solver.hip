@@ -30,11 +30,10 @@
 #include <type_traits>
 
 #include "cd_internal.h"
+#include "cd_sweeps.h"
 
 namespace {
 
-constexpr int SWEEP_BX = 64;   // x-pairs per block (128 columns)
-constexpr int SWEEP_BY = 4;    // rows per block
 constexpr int RED_BX = 64;
 constexpr int RED_BY = 4;
 
@@ -106,6 +105,7 @@ __global__ void k_rhs_finish(const double* __restrict__ partials, int nblocks, S
             st->last_max_update = INFINITY;
             st->rmean32 = 0.f;
             st->cur = 0;
+            st->stop_lid = INT_MAX;
             for (int k = 0; k < 16; ++k) st->maxupd_bits[k] = 0u;
         } else {
             st->bnorm = sqrt(s);
@@ -114,16 +114,19 @@ __global__ void k_rhs_finish(const double* __restrict__ partials, int nblocks, S
 }
 
 // ---------------------------------------------------------------------------
-// defect correction: phi64 += e32, e32 = 0 (elementwise)
+// defect correction, natural layout: phi64 += the current correction of the
+// ping-pong pair; the next batch of sweeps starts from ea = 0
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_flush(double* __restrict__ phi, float* __restrict__ e,
-                                               size_t n) {
+__global__ __launch_bounds__(256) void k_flush(double* __restrict__ phi, float* __restrict__ ea,
+                                               const float* __restrict__ eb,
+                                               const SolveDev* __restrict__ st, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
+    const bool second = st->cur != 0;
     for (; i < n; i += stride) {
-        float ev = e[i];
+        const float ev = second ? eb[i] : ea[i];
         phi[i] += (double)ev;
-        e[i] = 0.f;
+        ea[i] = 0.f;
     }
 }
 
@@ -288,7 +291,8 @@ __device__ __forceinline__ void residual_rows(const double* __restrict__ phi,
     }
 }
 template <int OUT, int ROWS>
-__global__ __launch_bounds__(256) void k_residual(const double* __restrict__ phi,
+__global__ __launch_bounds__(256) void k_residual(const double* __restrict__ phi0,
+                                                  const double* __restrict__ phi1,
                                                   const double* __restrict__ b,
                                                   const uint8_t* __restrict__ mask,
                                                   const SolveDev* __restrict__ st,
@@ -296,6 +300,8 @@ __global__ __launch_bounds__(256) void k_residual(const double* __restrict__ phi
                                                   unsigned short* __restrict__ r16, Brick bk,
                                                   int w, int h, double* __restrict__ partials) {
     __shared__ double smem[32];
+    // FP64 sweeps: the iterate is in either buffer of the pair (phi0, phi1)
+    const double* __restrict__ phi = phi1 && st->cur ? phi1 : phi0;
     const double bmean = st->bmean;
     double rs = 0.0, rq = 0.0;
     if (mask)
@@ -314,13 +320,13 @@ __global__ __launch_bounds__(256) void k_residual(const double* __restrict__ phi
 // launch of k_residual<OUT, rows> for rows in {1, 2, 4, 8}
 template <int OUT>
 void launch_residual(int rows, dim3 grid, dim3 blk, hipStream_t s, const double* phi,
-                     const double* b, const uint8_t* mask, const SolveDev* st, float* r32,
+                     const double* phi1, const double* b, const uint8_t* mask, const SolveDev* st, float* r32,
                      unsigned short* r16, const Brick& bk, int w, int h, double* partials) {
     switch (rows) {
-    case 8: hipLaunchKernelGGL((k_residual<OUT, 8>), grid, blk, 0, s, phi, b, mask, st, r32, r16, bk, w, h, partials); break;
-    case 4: hipLaunchKernelGGL((k_residual<OUT, 4>), grid, blk, 0, s, phi, b, mask, st, r32, r16, bk, w, h, partials); break;
-    case 2: hipLaunchKernelGGL((k_residual<OUT, 2>), grid, blk, 0, s, phi, b, mask, st, r32, r16, bk, w, h, partials); break;
-    default: hipLaunchKernelGGL((k_residual<OUT, 1>), grid, blk, 0, s, phi, b, mask, st, r32, r16, bk, w, h, partials); break;
+    case 8: hipLaunchKernelGGL((k_residual<OUT, 8>), grid, blk, 0, s, phi, phi1, b, mask, st, r32, r16, bk, w, h, partials); break;
+    case 4: hipLaunchKernelGGL((k_residual<OUT, 4>), grid, blk, 0, s, phi, phi1, b, mask, st, r32, r16, bk, w, h, partials); break;
+    case 2: hipLaunchKernelGGL((k_residual<OUT, 2>), grid, blk, 0, s, phi, phi1, b, mask, st, r32, r16, bk, w, h, partials); break;
+    default: hipLaunchKernelGGL((k_residual<OUT, 1>), grid, blk, 0, s, phi, phi1, b, mask, st, r32, r16, bk, w, h, partials); break;
     }
 }
 
@@ -378,59 +384,206 @@ __global__ void k_check(const double* __restrict__ partials, int nblocks, SolveD
 }
 
 // ---------------------------------------------------------------------------
-// red-black SOR half-sweep.  `color` 0 updates cells with (x+y) even.
-// e: iterate (FP32 correction or FP64 phi); r: right-hand side with its mean
-// *rmean projected out; the update is the reference's
+// Temporally blocked red-black SOR in the natural row-major layout: FP64 sweeps
+// (T = double, e the iterate, r = b) and FP32 sweeps with holes or on grids the
+// bricked layout cannot address (T = float, e the correction).  Regions and
+// stores as described in cd_sweeps.h.  The update is the reference's
 //   delta = omega / cnt * (sum - cnt * val - rhs)   (solver.cpp:47, 56)
+// with the operations, and hence the bits, of one half-sweep over the whole
+// grid per launch; colour 0 is x+y even.  A neighbour outside the grid or on a
+// hole holds zero in the region, so it drops out of the sum; such a cell is
+// never updated (a select, not a zero factor: an isolated cell's value may be
+// infinite).  oc = omega / cnt and cnt come per cell on tiles at the grid border
+// and with a mask, and are constants elsewhere.
+//
+// A half-sweep per launch was bound by its launches: two of 3.8 us (plus gaps)
+// per sweep on a 512 x 512 grid, where 8 sweeps in one launch take about 11 us.
 // ---------------------------------------------------------------------------
+constexpr int NAT_R = 4;    // rows per wave
+constexpr int NAT_NW = 16;  // waves per workgroup
+constexpr int NAT_RY = NAT_R * NAT_NW;
+
+// Per-cell constants of a tile at the grid border or with a mask.
 template <typename T>
-__global__ __launch_bounds__(256) void k_rb_sweep(T* __restrict__ e, const T* __restrict__ r,
-                                                  const uint8_t* __restrict__ mask, int w, int h,
-                                                  int color, T omega,
-                                                  const T* __restrict__ rmean, SolveDev* st,
-                                                  int track_max, int sweep) {
-    if (st->done) return;
-    __shared__ float smax[SWEEP_BX * SWEEP_BY / CD_WAVE];
-    const int y = blockIdx.y * SWEEP_BY + threadIdx.y;
-    const int x = 2 * (blockIdx.x * SWEEP_BX + threadIdx.x) + ((y + color) & 1);
-    float m = 0.f;
-    if (y < h && x < w) {
-        const size_t i = (size_t)y * w + x;
-        const T c = e[i];
-        T s = 0, cnt = 0;
-        bool hole = false;
-        if (mask) {
-            const uint8_t mk = mask[i];
-            hole = (mk & M_HOLE) != 0;
-            if (mk & M_L) { cnt += 1; s += e[i - 1]; }
-            if (mk & M_U) { cnt += 1; s += e[i - w]; }
-            if (mk & M_R) { cnt += 1; s += e[i + 1]; }
-            if (mk & M_D) { cnt += 1; s += e[i + w]; }
+struct NatCells {
+    T oc[2][NAT_R], cnt[2][NAT_R];
+    unsigned live;  // bit c * NAT_R + k: the cell is in the grid and no hole
+};
+
+__device__ __forceinline__ float nat_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double nat_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Rows K0 <= k < K1 of a half-sweep of colour C; mx[p] takes the largest
+// |update| of the lane's cells of column parity p.
+template <typename T, int C, bool GENERAL, bool TRACK, int K0, int K1>
+__device__ __forceinline__ void nat_half(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
+                                         const NatCells<T>& cl, T oc4, T up_row, T down_row,
+                                         T (&mx)[2]) {
+#pragma unroll
+    for (int k = K0; k < K1; ++k) {
+        const int p = (k + C) & 1;  // column parity of colour-C cells in row k
+        const T o = ev[1 - C][k];
+        const T up = k > 0 ? ev[1 - C][k - 1] : up_row;
+        const T down = k < NAT_R - 1 ? ev[1 - C][k + 1] : down_row;
+        const T left = p ? o : lane_prev(o);
+        const T right = p ? lane_next(o) : o;
+        const T s = left + up + right + down;
+        const T v = ev[C][k];
+        // (4 v is exact: the fused form has the unfused one's bits)
+        const T res = GENERAL ? s - cl.cnt[C][k] * v : nat_fma((T)-4, v, s);
+        const T d = (GENERAL ? cl.oc[C][k] : oc4) * (res - rv[C][k]);
+        if (GENERAL) {
+            const bool live = (cl.live >> (C * NAT_R + k)) & 1u;
+            ev[C][k] = live ? v + d : (T)0;
+            if (TRACK && live) mx[p] = fmax(mx[p], fabs(d));
         } else {
-            if (x > 0) { cnt += 1; s += e[i - 1]; }
-            if (y > 0) { cnt += 1; s += e[i - w]; }
-            if (x < w - 1) { cnt += 1; s += e[i + 1]; }
-            if (y < h - 1) { cnt += 1; s += e[i + w]; }
-        }
-        if (!hole) {
-            const T rv = r[i] - *rmean;
-            const T d = omega / cnt * (s - cnt * c - rv);
-            e[i] = c + d;
-            m = (float)fabs(d);
+            ev[C][k] = v + d;
+            if (TRACK) mx[p] = fmax(mx[p], fabs(d));
         }
     }
-    if (track_max) {
-        const int tid = threadIdx.y * SWEEP_BX + threadIdx.x;
-        m = cd_wave_max(m);
-        if ((tid & (CD_WAVE - 1)) == 0) smax[tid / CD_WAVE] = m;
+}
+
+// Everything between the loads and the stores of a region: nsweeps sweeps.
+// edge_up / edge_down: the wave's first / last row has no row beyond it.
+template <typename T, bool GENERAL, bool TRACK>
+__device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
+                                        const NatCells<T>& cl, T (*xch)[NAT_NW][2][64], T oc4,
+                                        bool edge_up, bool edge_down, int wave, int lane,
+                                        int nsweeps, unsigned (*smax)[64], bool track0,
+                                        bool track1) {
+    const int wu = max(wave - 1, 0), wd = min(wave + 1, NAT_NW - 1);
+    auto publish = [&](int c) {
+        xch[c][wave][0][lane] = ev[c][0];
+        xch[c][wave][1][lane] = ev[c][NAT_R - 1];
+    };
+    for (int j = 0; j < nsweeps; ++j) {
+        T mx[2] = {(T)0, (T)0};
+        T up, down;
+        publish(1);
+        nat_half<T, 0, GENERAL, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
         __syncthreads();
-        if (tid == 0) {
-            float t = smax[0];
-            for (int k = 1; k < SWEEP_BX * SWEEP_BY / CD_WAVE; ++k) t = fmaxf(t, smax[k]);
+        up = xch[1][wu][1][lane];
+        down = xch[1][wd][0][lane];
+        if (GENERAL && edge_up) up = (T)0;
+        if (GENERAL && edge_down) down = (T)0;
+        nat_half<T, 0, GENERAL, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
+        nat_half<T, 0, GENERAL, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
+        publish(0);
+        nat_half<T, 1, GENERAL, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
+        __syncthreads();
+        up = xch[0][wu][1][lane];
+        down = xch[0][wd][0][lane];
+        if (GENERAL && edge_up) up = (T)0;
+        if (GENERAL && edge_down) down = (T)0;
+        nat_half<T, 1, GENERAL, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
+        nat_half<T, 1, GENERAL, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
+        if (TRACK) {
             // non-negative floats order like their bit patterns
-            atomicMax(&st->maxupd_bits[sweep & 1], __float_as_uint(t));
+            const float m = fmaxf(track0 ? (float)mx[0] : 0.f, track1 ? (float)mx[1] : 0.f);
+            atomicMax(&smax[j][lane], __float_as_uint(m));
         }
     }
+}
+
+template <typename T, bool TRACK>
+__global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
+    const T* ein, T* eout, const T* __restrict__ r, const uint8_t* __restrict__ mask,
+    SweepTiles tiles, int nsweeps, T omega, const T* __restrict__ rmean, SolveDev* st,
+    int out_index, float* __restrict__ tmax, TrackArgs track) {
+    __shared__ T xch[2][NAT_NW][2][64];
+    __shared__ unsigned smax[TRACK ? kTrackSweeps : 1][64];
+    __shared__ float red[TRACK ? NAT_NW * kTrackSweeps : 1];
+    const int tile = tile_of_block();
+    if (tile >= tiles.ntiles) return;
+    if (TRACK) {
+        if (st->stop_lid < track.lid) return;
+        const TrackPlan plan = track_decide<NAT_NW>(track, st, tiles.ntiles, nsweeps, red);
+        if (plan.nsweeps == 0) return;
+        nsweeps = plan.nsweeps;
+        if (plan.redo) {
+            const T* in = eout;
+            eout = const_cast<T*>(ein);
+            ein = in;
+            out_index ^= 1;
+        }
+        for (int i = threadIdx.x; i < kTrackSweeps * 64; i += 64 * NAT_NW) (&smax[0][0])[i] = 0u;
+        __syncthreads();
+    }
+    const Region g = region_of(tiles, tile);
+    const int w = tiles.w, h = tiles.h;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x0 = g.X0 + 2 * lane, Yw = g.Y0 + wave * NAT_R;
+    const T rm = *rmean;
+    T ev[2][NAT_R], rv[2][NAT_R];
+    NatCells<T> cl;
+    uint8_t mk[2][NAT_R];
+    // branch-free loads from clamped addresses: all in flight together
+#pragma unroll
+    for (int k = 0; k < NAT_R; ++k)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const size_t i = (size_t)min(Yw + k, h - 1) * w + min(x0 + ((k + c) & 1), w - 1);
+            ev[c][k] = ein[i];
+            rv[c][k] = r[i];
+            mk[c][k] = mask ? mask[i] : (uint8_t)0;
+        }
+    const bool general = mask || g.left || g.right || g.top || g.bottom;
+    const T oc4 = omega / (T)4;
+    if (general) {
+        cl.live = 0u;
+#pragma unroll
+        for (int k = 0; k < NAT_R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int x = x0 + ((k + c) & 1), y = Yw + k;
+                const uint8_t m = mk[c][k];
+                int n = (int)(x > 0) + (int)(y > 0) + (int)(x < w - 1) + (int)(y < h - 1);
+                if (mask) n = __popc(m & (M_L | M_U | M_R | M_D));
+                const bool live = x < w && y < h && !(m & M_HOLE);
+                if (live) cl.live |= 1u << (c * NAT_R + k);
+                else ev[c][k] = (T)0;
+                cl.cnt[c][k] = (T)n;
+                cl.oc[c][k] = omega / (T)n;
+                rv[c][k] = rv[c][k] - rm;
+            }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NAT_R; ++k) {
+            rv[0][k] = rv[0][k] - rm;
+            rv[1][k] = rv[1][k] - rm;
+        }
+    }
+    // the cells whose updates count for the stop rule: those at distance >= halo
+    // from the region's inner borders (all exact; two tiles may count one)
+    const int dy0 = wave * NAT_R, hl = tiles.halo;
+    const bool rows_ok = (g.top || dy0 >= hl) && (g.bottom || dy0 + NAT_R <= NAT_RY - hl);
+    auto col_ok = [&](int dx) { return rows_ok && (g.left || dx >= hl) && (g.right || dx < SW_RX - hl); };
+    const bool t0 = TRACK && col_ok(2 * lane), t1 = TRACK && col_ok(2 * lane + 1);
+    if (general)
+        nat_run<T, true, TRACK>(ev, rv, cl, xch, oc4, g.top && wave == 0,
+                                g.bottom && wave == NAT_NW - 1, wave, lane, nsweeps, smax, t0, t1);
+    else
+        nat_run<T, false, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, smax, t0,
+                                 t1);
+#pragma unroll
+    for (int k = 0; k < NAT_R; ++k) {
+        const int y = Yw + k;
+        if (y < g.ys0 || y >= g.ys1) continue;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int x = x0 + ((k + c) & 1);
+            if (x >= g.xs0 && x < g.xs1) eout[(size_t)y * w + x] = ev[c][k];
+        }
+    }
+    if (TRACK) {
+        __syncthreads();
+        for (int j = wave; j < nsweeps; j += NAT_NW) {
+            const float m = cd_wave_max(__uint_as_float(smax[j][lane]));
+            if (lane == 0) tmax[(size_t)tile * kTrackSweeps + j] = m;
+        }
+    }
+    if (threadIdx.x == 0) st->cur = out_index;  // same value from every workgroup
 }
 
 // ---------------------------------------------------------------------------
@@ -502,14 +655,6 @@ struct RhsRegsT {
     __device__ __forceinline__ void set(int c, int k, int, int, float x) { v[c][k] = x; }
 };
 using RhsRegs = RhsRegsT<BK_R>;
-
-// value of lane l-1 (0 in lane 0) / lane l+1 (0 in lane 63): DPP wave shifts
-__device__ __forceinline__ float lane_prev(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_next(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
 
 // Per-lane facts of a region for the sweep helpers: packed column `lane`
 // holds cells x0 = X0 + 2 lane and x0 + 1 of rows Yw .. Yw + R - 1.
@@ -933,22 +1078,9 @@ __global__ void k_maxcheck_blocked(SolveDev* st, int first_sweep, int nsweeps, d
 __global__ void k_reopen(SolveDev* st) {
     if (threadIdx.x != 0) return;
     st->done = 0;
+    st->stop_lid = INT_MAX;
     st->sweeps_at_done = -1;
     for (int j = 0; j < 16; ++j) st->maxupd_bits[j] = 0u;
-}
-
-// max-update stop rule after the black half of sweep `sweep` (solver.cpp:142)
-__global__ void k_maxcheck(SolveDev* st, int sweep, double tol) {
-    if (threadIdx.x != 0) return;
-    if (!st->done) {
-        float mu = __uint_as_float(st->maxupd_bits[sweep & 1]);
-        st->last_max_update = (double)mu;
-        if ((double)mu < tol) {
-            st->done = 1;
-            st->sweeps_at_done = sweep + 1;
-        }
-    }
-    st->maxupd_bits[(sweep + 1) & 1] = 0u;
 }
 
 __global__ void k_set_holes_nan(double* __restrict__ phi, const uint8_t* __restrict__ mask,
@@ -958,6 +1090,28 @@ __global__ void k_set_holes_nan(double* __restrict__ phi, const uint8_t* __restr
 }
 
 inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
+
+// Tiles of the natural-layout sweeps: the halo (twice the sweeps of a launch)
+// that the cost model finds cheapest per sweep.  A launch costs NAT_FIXED_US
+// (dispatch, loads, stores) plus, per half-sweep, the time of a workgroup,
+// times the workgroups per CU past one.  tmax_bytes: room for a tracking
+// launch's two arrays of per-tile maxima.
+SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t tmax_bytes) {
+    const double half_us = fp64 ? 0.36 : 0.30, fixed_us = 5.5;
+    SweepTiles best = sweep_tiles(w, h, NAT_RY, 4);
+    double best_cost = INFINITY;
+    for (int halo = 4; halo <= 28; halo += 4) {
+        const SweepTiles t = sweep_tiles(w, h, NAT_RY, halo);
+        if (track && 2 * sizeof(float) * kTrackSweeps * (size_t)t.ntiles > tmax_bytes) continue;
+        const int sweeps = std::min(halo / 2, std::max(batch, 1));
+        const double cost = (fixed_us + 2 * sweeps * half_us * std::max(1.0, t.ntiles / 256.0)) / sweeps;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = t;
+        }
+    }
+    return best;
+}
 
 // Over-relaxation factor.  > 0: as given.  < 0: the reference's
 // 2/(1+3.14159265/width) (solver.cpp:71).  == 0: the optimum for this
@@ -1593,8 +1747,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         ws = *work;
     } else {
         // (sum, sum^2) per block for checks, four dot products per block for FCG
-        CD_TRY(ctx->ensure(ctx->partials, sizeof(double) * 4 * (size_t)nred));
+        CD_TRY(ctx->ensure(ctx->partials, cd_partials_bytes(nred)));
         CD_TRY(ctx->ensure(ctx->solve_dev, sizeof(SolveDev)));
+        if (!mixed) CD_TRY(ctx->ensure(ctx->e64w, sizeof(double) * n));
         if (mixed) {
             CD_TRY(ctx->ensure(ctx->e32, sizeof(float) * (blocked ? npk : n)));
             // FP32 rhs (natural layout), BF16 rhs (bricked layout) or, under
@@ -1602,18 +1757,20 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             const size_t rb = blocked ? (o->stop == CD_STOP_MAX_UPDATE ? sizeof(float) : sizeof(unsigned short)) * npk
                                       : sizeof(float) * n;
             CD_TRY(ctx->ensure(ctx->r32, rb));
-            if (blocked) CD_TRY(ctx->ensure(ctx->e32b, sizeof(float) * npk));
+            CD_TRY(ctx->ensure(ctx->e32b, sizeof(float) * (blocked ? npk : n)));
         }
         ws.partials = ctx->partials.as<double>();
         ws.sd = ctx->solve_dev.as<SolveDev>();
         ws.e32 = mixed ? ctx->e32.as<float>() : nullptr;
-        ws.e32b = blocked ? ctx->e32b.as<float>() : nullptr;
+        ws.e32b = mixed ? ctx->e32b.as<float>() : nullptr;
         ws.r = mixed ? ctx->r32.ptr : nullptr;
+        ws.phi2 = mixed ? nullptr : ctx->e64w.as<double>();
     }
     double* partials = ws.partials;
     SolveDev* sd = ws.sd;
     float* e32 = mixed ? ws.e32 : nullptr;
-    float* e32b = blocked ? ws.e32b : nullptr;
+    float* e32b = mixed ? ws.e32b : nullptr;
+    double* phi2 = mixed ? nullptr : ws.phi2;  // FP64 sweeps: second buffer of the iterate
     float* r32 = mixed ? static_cast<float*>(ws.r) : nullptr;
     unsigned short* r16 = blocked ? static_cast<unsigned short*>(ws.r) : nullptr;
     const int track = o->stop == CD_STOP_MAX_UPDATE;
@@ -1670,17 +1827,17 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             if (flush)
                 hipLaunchKernelGGL(k_flush_packed, rgrid, rblk, 0, s, phi, e32, e32b, sd, w, h, bk);
             if (track)
-                launch_residual<3>(kResidualRows, cgrid, rblk, s, phi, b, mask, sd, r32, r16, bk,
+                launch_residual<3>(kResidualRows, cgrid, rblk, s, phi, nullptr, b, mask, sd, r32, r16, bk,
                                    w, h, partials);
             else
-                launch_residual<2>(kResidualRows, cgrid, rblk, s, phi, b, mask, sd, r32, r16, bk,
+                launch_residual<2>(kResidualRows, cgrid, rblk, s, phi, nullptr, b, mask, sd, r32, r16, bk,
                                    w, h, partials);
         } else if (mixed) {
-            hipLaunchKernelGGL(k_flush, dim3(fblocks), dim3(CD_BLOCK), 0, s, phi, e32, n);
-            launch_residual<1>(kResidualRows, cgrid, rblk, s, phi, b, mask, sd, r32, r16, bk, w, h,
+            hipLaunchKernelGGL(k_flush, dim3(fblocks), dim3(CD_BLOCK), 0, s, phi, e32, e32b, sd, n);
+            launch_residual<1>(kResidualRows, cgrid, rblk, s, phi, nullptr, b, mask, sd, r32, r16, bk, w, h,
                                partials);
         } else {
-            launch_residual<0>(kResidualRows, cgrid, rblk, s, phi, b, mask, sd, r32, r16, bk, w, h,
+            launch_residual<0>(kResidualRows, cgrid, rblk, s, phi, phi2, b, mask, sd, r32, r16, bk, w, h,
                                partials);
         }
         return finish_check(check_id, (mixed && flush) ? 3 : 2,
@@ -1688,8 +1845,6 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                             ncheck);
     };
 
-    const dim3 sblk(SWEEP_BX, SWEEP_BY);
-    const dim3 sgrid(div_up(div_up(w, 2), SWEEP_BX), div_up(h, SWEEP_BY));
     // blocked geometry
     constexpr int BH = CD_BK_H;  // halo = half-sweeps per launch
     const int bix = BK_RX - 2 * BH, biy = BK_RY - 2 * BH;
@@ -1742,26 +1897,60 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     auto enqueue_blocked = [&](int first, int count_sweeps) -> int {
         return enqueue_blocked_om(first, count_sweeps, om2, om3, om4);
     };
-    auto enqueue_sweeps = [&](int first, int count_sweeps) -> int {
-        if (blocked) return enqueue_blocked(first, count_sweeps);
+    // natural layout: launches of several sweeps between the buffers b0 and b1;
+    // FP64 iterates continue in the buffer the last check found current, FP32
+    // corrections start in b0 (the check's flush cleared it)
+    int track_lid = 0;
+    auto enqueue_natural = [&](auto* b0, auto* b1, const auto* rhs, auto om, const auto* mean,
+                               int first, int count_sweeps) -> int {
+        using T = std::remove_pointer_t<decltype(b0)>;
+        const SweepTiles t = natural_tiles(w, h, sizeof(T) == 8, count_sweeps, track != 0,
+                                           cd_partials_bytes(nred));
+        const int most = t.ntiles == 1 ? (track ? kTrackSweeps : count_sweeps) : t.halo / 2;
+        const dim3 grid(sweep_grid(t.ntiles)), blk(64 * NAT_NW);
+        int cur = mixed ? 0 : ctx->host_status->cur;
+        float* tmax[2] = {reinterpret_cast<float*>(partials),
+                          reinterpret_cast<float*>(partials) + (size_t)t.ntiles * kTrackSweeps};
+        TrackArgs tr{};
+        tr.group = 1;
+        tr.tol = o->tol;
         CD_TRY(timer_begin());
-        for (int k = 0; k < count_sweeps; ++k) {
-            const int sw = first + k;
-            for (int color = 0; color < 2; ++color) {
-                if (mixed) {
-                    hipLaunchKernelGGL(k_rb_sweep<float>, sgrid, sblk, 0, s, e32, r32, mask, w,
-                                       h, color, (float)omega, &sd->rmean32, sd, track, sw);
-                } else {
-                    hipLaunchKernelGGL(k_rb_sweep<double>, sgrid, sblk, 0, s, phi, b, mask, w,
-                                       h, color, omega, &sd->bmean, sd, track, sw);
-                }
+        int launches = 0;
+        for (int done_sw = 0; done_sw < count_sweeps; ++launches) {
+            const int nsw = std::min(most, count_sweeps - done_sw);
+            T* in = cur ? b1 : b0;
+            T* out = cur ? b0 : b1;
+            if (track) {
+                tr.lid = ++track_lid;
+                hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, in, out, rhs, mask, t,
+                                   nsw, om, mean, sd, 1 - cur, tmax[launches & 1], tr);
+                tr.prev = tmax[launches & 1];
+                tr.nprev = nsw;
+                tr.first_prev = first + done_sw;
+            } else {
+                hipLaunchKernelGGL((k_rb_natural<T, false>), grid, blk, 0, s, in, out, rhs, mask, t,
+                                   nsw, om, mean, sd, 1 - cur, nullptr, tr);
             }
-            if (track) hipLaunchKernelGGL(k_maxcheck, dim3(1), dim3(64), 0, s, sd, sw, o->tol);
+            cur = 1 - cur;
+            done_sw += nsw;
+        }
+        if (track) {  // the last launch's own decision
+            tr.lid = ++track_lid;
+            tr.check_only = 1;
+            hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, cur ? b1 : b0,
+                               cur ? b0 : b1, rhs, mask, t, 0, om, mean, sd, 1 - cur,
+                               tmax[launches & 1], tr);
+            ++launches;
         }
         CD_CHECK_LAUNCH(ctx);
-        CD_TRY(timer_end(CD_KERNEL_SOR_SWEEP, 2LL * count_sweeps,
-                              (mixed ? 12.0 : 24.0) * (double)n * count_sweeps));
-        return CD_OK;
+        return timer_end(CD_KERNEL_SOR_SWEEP, launches,
+                         (mixed ? 12.0 : 24.0) * (double)n * count_sweeps);
+    };
+    auto enqueue_sweeps = [&](int first, int count_sweeps) -> int {
+        if (blocked) return enqueue_blocked(first, count_sweeps);
+        if (mixed)
+            return enqueue_natural(e32, e32b, r32, (float)omega, &sd->rmean32, first, count_sweeps);
+        return enqueue_natural(phi, phi2, b, omega, &sd->bmean, first, count_sweeps);
     };
 
     // ---- learned correction / capture geometry ------------------------------
@@ -2162,6 +2351,8 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         CD_CHECK_LAUNCH(ctx);
     }
     const SolveDev hs = *ctx->host_status;
+    if (!mixed && hs.cur)  // FP64 sweeps: the iterate ended in the second buffer
+        CD_HIP(ctx, hipMemcpyAsync(phi, phi2, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     if (mask && o->max_sweeps > 0) {
         hipLaunchKernelGGL(k_set_holes_nan, dim3(div_up((long long)n, CD_BLOCK)), dim3(CD_BLOCK), 0,
                            s, phi, mask, n);
@@ -2236,7 +2427,7 @@ constexpr NoallocLayout noalloc_layout(int w, int h) {
     const size_t nred = (size_t)((w + RED_BX - 1) / RED_BX) * ((h + RED_BY - 1) / RED_BY);
     NoallocLayout L{};
     size_t o = 0;
-    L.partials = o; o += al256(sizeof(double) * 4 * nred);
+    L.partials = o; o += al256(cd_partials_bytes(nred));
     L.sd = o;       o += al256(sizeof(SolveDev));
     L.e32 = o;      o += al256(sizeof(float) * npk);
     L.e32b = o;     o += al256(sizeof(float) * npk);
@@ -2311,6 +2502,8 @@ int cd_poisson_solve_device_noalloc(cd_context* ctx, const double* d_rhs, double
     ws.e32 = reinterpret_cast<float*>(base + L.e32);
     ws.e32b = reinterpret_cast<float*>(base + L.e32b);
     ws.r = base + L.r;
+    // FP64 sweeps use neither correction: their second buffer lies over both
+    ws.phi2 = reinterpret_cast<double*>(base + L.e32);
     uint8_t* mask = base + L.mask;
     double* fill = reinterpret_cast<double*>(base + L.fill);
     long long holes = 0;
@@ -2332,7 +2525,7 @@ int cd_poisson_solve_device(cd_context* ctx, const double* d_rhs, double* d_phi,
     cd_solve_work_sizes(width, height, &nred, &npk);
     // hole mask: only used by the solve when the right-hand side contains NaN
     CD_TRY(ctx->ensure(ctx->mask, n));
-    CD_TRY(ctx->ensure(ctx->partials, sizeof(double) * 4 * nred));  // as the solve
+    CD_TRY(ctx->ensure(ctx->partials, cd_partials_bytes(nred)));  // as the solve
     CD_TRY(ctx->ensure(ctx->fill, sizeof(double) * 4));
     long long holes = 0;
     CD_TRY(cd_hole_mask(ctx, d_rhs, width, height, ctx->mask.as<uint8_t>(),
