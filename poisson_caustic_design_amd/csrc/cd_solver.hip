@@ -391,10 +391,11 @@ __global__ void k_check(const double* __restrict__ partials, int nblocks, SolveD
 //   delta = omega / cnt * (sum - cnt * val - rhs)   (solver.cpp:47, 56)
 // with the operations, and hence the bits, of one half-sweep over the whole
 // grid per launch; colour 0 is x+y even.  A neighbour outside the grid or on a
-// hole holds zero in the region, so it drops out of the sum; such a cell is
-// never updated (a select, not a zero factor: an isolated cell's value may be
-// infinite).  oc = omega / cnt and cnt come per cell on tiles at the grid border
-// and with a mask, and are constants elsewhere.
+// hole holds zero in the region, so it drops out of the sum; its own update has
+// the factor oc = 0 (and with a mask a select: a cell with no neighbour left has
+// an infinite update, which 0 would turn into a NaN beside it).  oc = omega / cnt
+// and cnt come per cell on tiles at the grid border and with a mask, and are
+// constants elsewhere.
 //
 // A half-sweep per launch was bound by its launches: two of 3.8 us (plus gaps)
 // per sweep on a 512 x 512 grid, where 8 sweeps in one launch take about 11 us.
@@ -415,7 +416,8 @@ __device__ __forceinline__ double nat_fma(double a, double b, double c) { return
 
 // Rows K0 <= k < K1 of a half-sweep of colour C; mx[p] takes the largest
 // |update| of the lane's cells of column parity p.
-template <typename T, int C, bool GENERAL, bool TRACK, int K0, int K1>
+enum { NAT_INNER = 0, NAT_EDGE = 1, NAT_MASK = 2 };
+template <typename T, int C, int KIND, bool TRACK, int K0, int K1>
 __device__ __forceinline__ void nat_half(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
                                          const NatCells<T>& cl, T oc4, T up_row, T down_row,
                                          T (&mx)[2]) {
@@ -430,22 +432,18 @@ __device__ __forceinline__ void nat_half(T (&ev)[2][NAT_R], const T (&rv)[2][NAT
         const T s = left + up + right + down;
         const T v = ev[C][k];
         // (4 v is exact: the fused form has the unfused one's bits)
-        const T res = GENERAL ? s - cl.cnt[C][k] * v : nat_fma((T)-4, v, s);
-        const T d = (GENERAL ? cl.oc[C][k] : oc4) * (res - rv[C][k]);
-        if (GENERAL) {
-            const bool live = (cl.live >> (C * NAT_R + k)) & 1u;
-            ev[C][k] = live ? v + d : (T)0;
-            if (TRACK && live) mx[p] = fmax(mx[p], fabs(d));
-        } else {
-            ev[C][k] = v + d;
-            if (TRACK) mx[p] = fmax(mx[p], fabs(d));
-        }
+        const T res = KIND ? s - cl.cnt[C][k] * v : nat_fma((T)-4, v, s);
+        const T d = (KIND ? cl.oc[C][k] : oc4) * (res - rv[C][k]);
+        const T nv = v + d;
+        if (KIND == NAT_MASK) ev[C][k] = (cl.live >> (C * NAT_R + k)) & 1u ? nv : (T)0;
+        else ev[C][k] = nv;
+        if (TRACK) mx[p] = fmax(mx[p], fabs(d));  // (0, or a NaN that fmax drops, where oc = 0)
     }
 }
 
 // Everything between the loads and the stores of a region: nsweeps sweeps.
 // edge_up / edge_down: the wave's first / last row has no row beyond it.
-template <typename T, bool GENERAL, bool TRACK>
+template <typename T, int KIND, bool TRACK>
 __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
                                         const NatCells<T>& cl, T (*xch)[NAT_NW][2][64], T oc4,
                                         bool edge_up, bool edge_down, int wave, int lane,
@@ -460,23 +458,23 @@ __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_
         T mx[2] = {(T)0, (T)0};
         T up, down;
         publish(1);
-        nat_half<T, 0, GENERAL, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
+        nat_half<T, 0, KIND, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
         __syncthreads();
         up = xch[1][wu][1][lane];
         down = xch[1][wd][0][lane];
-        if (GENERAL && edge_up) up = (T)0;
-        if (GENERAL && edge_down) down = (T)0;
-        nat_half<T, 0, GENERAL, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
-        nat_half<T, 0, GENERAL, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
+        if (KIND && edge_up) up = (T)0;
+        if (KIND && edge_down) down = (T)0;
+        nat_half<T, 0, KIND, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
+        nat_half<T, 0, KIND, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
         publish(0);
-        nat_half<T, 1, GENERAL, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
+        nat_half<T, 1, KIND, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
         __syncthreads();
         up = xch[0][wu][1][lane];
         down = xch[0][wd][0][lane];
-        if (GENERAL && edge_up) up = (T)0;
-        if (GENERAL && edge_down) down = (T)0;
-        nat_half<T, 1, GENERAL, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
-        nat_half<T, 1, GENERAL, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
+        if (KIND && edge_up) up = (T)0;
+        if (KIND && edge_down) down = (T)0;
+        nat_half<T, 1, KIND, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
+        nat_half<T, 1, KIND, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
         if (TRACK) {
             // non-negative floats order like their bit patterns
             const float m = fmaxf(track0 ? (float)mx[0] : 0.f, track1 ? (float)mx[1] : 0.f);
@@ -544,8 +542,8 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
                 if (live) cl.live |= 1u << (c * NAT_R + k);
                 else ev[c][k] = (T)0;
                 cl.cnt[c][k] = (T)n;
-                cl.oc[c][k] = omega / (T)n;
-                rv[c][k] = rv[c][k] - rm;
+                cl.oc[c][k] = live ? omega / (T)n : (T)0;
+                rv[c][k] = live ? rv[c][k] - rm : (T)0;
             }
     } else {
 #pragma unroll
@@ -560,12 +558,16 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     const bool rows_ok = (g.top || dy0 >= hl) && (g.bottom || dy0 + NAT_R <= NAT_RY - hl);
     auto col_ok = [&](int dx) { return rows_ok && (g.left || dx >= hl) && (g.right || dx < SW_RX - hl); };
     const bool t0 = TRACK && col_ok(2 * lane), t1 = TRACK && col_ok(2 * lane + 1);
-    if (general)
-        nat_run<T, true, TRACK>(ev, rv, cl, xch, oc4, g.top && wave == 0,
-                                g.bottom && wave == NAT_NW - 1, wave, lane, nsweeps, smax, t0, t1);
+    const bool up0 = g.top && wave == 0, down0 = g.bottom && wave == NAT_NW - 1;
+    if (mask)
+        nat_run<T, NAT_MASK, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, smax,
+                                    t0, t1);
+    else if (general)
+        nat_run<T, NAT_EDGE, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, smax,
+                                    t0, t1);
     else
-        nat_run<T, false, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, smax, t0,
-                                 t1);
+        nat_run<T, NAT_INNER, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, smax,
+                                     t0, t1);
 #pragma unroll
     for (int k = 0; k < NAT_R; ++k) {
         const int y = Yw + k;
@@ -1092,19 +1094,21 @@ __global__ void k_set_holes_nan(double* __restrict__ phi, const uint8_t* __restr
 inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
 
 // Tiles of the natural-layout sweeps: the halo (twice the sweeps of a launch)
-// that the cost model finds cheapest per sweep.  A launch costs NAT_FIXED_US
-// (dispatch, loads, stores) plus, per half-sweep, the time of a workgroup,
-// times the workgroups per CU past one.  tmax_bytes: room for a tracking
-// launch's two arrays of per-tile maxima.
+// that is cheapest per sweep by what launches measured: about 5 us of dispatch,
+// loads and stores, and 0.43 us (FP64) or 0.28 us (FP32) per half-sweep and
+// round of one workgroup per CU.  At 400 x 400 in FP64 halos of 8 / 16 / 24 / 28
+// take 2.18 / 1.49 / 1.29 / 1.25 us per sweep; at 700 x 700 the 369 tiles of halo
+// 24 need a second round and take 2.12, halo 20 1.41.  tmax_bytes: room for a
+// tracking launch's two arrays of per-tile maxima.
 SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t tmax_bytes) {
-    const double half_us = fp64 ? 0.36 : 0.30, fixed_us = 5.5;
+    const double half_us = fp64 ? 0.43 : 0.28, fixed_us = 5.0;
     SweepTiles best = sweep_tiles(w, h, NAT_RY, 4);
     double best_cost = INFINITY;
     for (int halo = 4; halo <= 28; halo += 4) {
         const SweepTiles t = sweep_tiles(w, h, NAT_RY, halo);
         if (track && 2 * sizeof(float) * kTrackSweeps * (size_t)t.ntiles > tmax_bytes) continue;
         const int sweeps = std::min(halo / 2, std::max(batch, 1));
-        const double cost = (fixed_us + 2 * sweeps * half_us * std::max(1.0, t.ntiles / 256.0)) / sweeps;
+        const double cost = (fixed_us + 2 * sweeps * half_us * div_up(t.ntiles, 256)) / sweeps;
         if (cost < best_cost) {
             best_cost = cost;
             best = t;
