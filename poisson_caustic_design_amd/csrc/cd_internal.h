@@ -72,7 +72,6 @@ struct SolveDev {
     double last_max_update;
     float rmean32;       // mean of the last FP32 residual (projected out in sweeps)
     int cur;             // blocked path: ping-pong buffer holding the current correction
-    unsigned int maxupd_bits[16];  // per-sweep max |delta| (float bits) for the max-update rule
     unsigned int seq;    // host mirror: written last by a check (the host waits for it)
     int stop_lid;        // max-update rule: the launch that found the stop (INT_MAX: none)
 };

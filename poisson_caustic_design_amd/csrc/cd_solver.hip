@@ -106,7 +106,6 @@ __global__ void k_rhs_finish(const double* __restrict__ partials, int nblocks, S
             st->rmean32 = 0.f;
             st->cur = 0;
             st->stop_lid = INT_MAX;
-            for (int k = 0; k < 16; ++k) st->maxupd_bits[k] = 0u;
         } else {
             st->bnorm = sqrt(s);
         }
@@ -447,7 +446,7 @@ template <typename T, int KIND, bool TRACK>
 __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
                                         const NatCells<T>& cl, T (*xch)[NAT_NW][2][64], T oc4,
                                         bool edge_up, bool edge_down, int wave, int lane,
-                                        int nsweeps, unsigned (*smax)[64], bool track0,
+                                        int nsweeps, float (*smax)[NAT_NW][64], bool track0,
                                         bool track1) {
     const int wu = max(wave - 1, 0), wd = min(wave + 1, NAT_NW - 1);
     auto publish = [&](int c) {
@@ -476,9 +475,7 @@ __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_
         nat_half<T, 1, KIND, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
         nat_half<T, 1, KIND, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
         if (TRACK) {
-            // non-negative floats order like their bit patterns
-            const float m = fmaxf(track0 ? (float)mx[0] : 0.f, track1 ? (float)mx[1] : 0.f);
-            atomicMax(&smax[j][lane], __float_as_uint(m));
+            smax[j][wave][lane] = fmaxf(track0 ? (float)mx[0] : 0.f, track1 ? (float)mx[1] : 0.f);
         }
     }
 }
@@ -487,26 +484,12 @@ template <typename T, bool TRACK>
 __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     const T* ein, T* eout, const T* __restrict__ r, const uint8_t* __restrict__ mask,
     SweepTiles tiles, int nsweeps, T omega, const T* __restrict__ rmean, SolveDev* st,
-    int out_index, float* __restrict__ tmax, TrackArgs track) {
+    int out_index, TrackArgs track) {
     __shared__ T xch[2][NAT_NW][2][64];
-    __shared__ unsigned smax[TRACK ? kTrackSweeps : 1][64];
-    __shared__ float red[TRACK ? NAT_NW * kTrackSweeps : 1];
+    __shared__ float smax[TRACK ? kTrackSweeps : 1][NAT_NW][64];
+    __shared__ unsigned red[TRACK ? NAT_NW : 1];
     const int tile = tile_of_block();
     if (tile >= tiles.ntiles) return;
-    if (TRACK) {
-        if (st->stop_lid < track.lid) return;
-        const TrackPlan plan = track_decide<NAT_NW>(track, st, tiles.ntiles, nsweeps, red);
-        if (plan.nsweeps == 0) return;
-        nsweeps = plan.nsweeps;
-        if (plan.redo) {
-            const T* in = eout;
-            eout = const_cast<T*>(ein);
-            ein = in;
-            out_index ^= 1;
-        }
-        for (int i = threadIdx.x; i < kTrackSweeps * 64; i += 64 * NAT_NW) (&smax[0][0])[i] = 0u;
-        __syncthreads();
-    }
     const Region g = region_of(tiles, tile);
     const int w = tiles.w, h = tiles.h;
     const int lane = threadIdx.x & 63;
@@ -517,15 +500,34 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     NatCells<T> cl;
     uint8_t mk[2][NAT_R];
     // branch-free loads from clamped addresses: all in flight together
+    auto cell = [&](int c, int k) {
+        return (size_t)min(Yw + k, h - 1) * w + min(x0 + ((k + c) & 1), w - 1);
+    };
+    const unsigned words = TRACK ? track_load<NAT_NW>(track, tiles.ntiles) : 0u;
 #pragma unroll
     for (int k = 0; k < NAT_R; ++k)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const size_t i = (size_t)min(Yw + k, h - 1) * w + min(x0 + ((k + c) & 1), w - 1);
+            const size_t i = cell(c, k);
             ev[c][k] = ein[i];
             rv[c][k] = r[i];
             mk[c][k] = mask ? mask[i] : (uint8_t)0;
         }
+    if (TRACK) {
+        const TrackPlan plan =
+            track_decide<NAT_NW>(track, st, tiles.ntiles, nsweeps, words, red);
+        if (plan.nsweeps == 0) return;
+        nsweeps = plan.nsweeps;
+        if (plan.redo) {
+            const T* in = eout;
+            eout = const_cast<T*>(ein);
+            out_index ^= 1;
+#pragma unroll
+            for (int k = 0; k < NAT_R; ++k)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) ev[c][k] = in[cell(c, k)];
+        }
+    }
     const bool general = mask || g.left || g.right || g.top || g.bottom;
     const T oc4 = omega / (T)4;
     if (general) {
@@ -578,287 +580,162 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
             if (x >= g.xs0 && x < g.xs1) eout[(size_t)y * w + x] = ev[c][k];
         }
     }
-    if (TRACK) {
-        __syncthreads();
-        for (int j = wave; j < nsweeps; j += NAT_NW) {
-            const float m = cd_wave_max(__uint_as_float(smax[j][lane]));
-            if (lane == 0) tmax[(size_t)tile * kTrackSweeps + j] = m;
-        }
-    }
+    if (TRACK) track_store<NAT_NW>(track, smax, red, tile, nsweeps, wave, lane);
     if (threadIdx.x == 0) st->cur = out_index;  // same value from every workgroup
 }
 
 // ---------------------------------------------------------------------------
-// Temporally blocked red-black SOR (FP32, packed layout, no holes).
+// Temporally blocked red-black SOR (FP32, bricked layout, no holes).
 //
-// A workgroup of W waves owns a region of W*R rows x 128 columns; the halo is
-// H cells on every side.  Lane l of wave v keeps packed column l (cells
-// 2l and 2l+1 of every row, one per colour) of rows v*R .. v*R+R-1 in
-// registers, with the cells' scaled right-hand side.  Up/down neighbours of a
+// Regions as described in cd_sweeps.h, NW = 16 waves of R rows each, with the
+// cells' right-hand side in registers beside them.  Up/down neighbours of a
 // cell are the other colour in the rows above/below: registers of the same
 // lane, except at a wave's first/last row, which comes through a small LDS
-// exchange.  Left/right neighbours are the other colour in the same row at
-// packed column l-1+p or l+p (p = column parity of the cell): the same lane or
-// the adjacent lane, fetched with a DPP wave shift folded into the first add.
-// Half-sweep s (1-based) updates the cells at distance >= s from the region
-// border, whose neighbours are exact at that point; after nhalf <= H
-// half-sweeps the interior (distance >= H) equals nhalf global half-sweeps
-// and is written to the other ping-pong buffer.
+// exchange.  Left/right neighbours are the other colour in the same row: the
+// same lane or the adjacent lane, fetched with a DPP wave shift folded into the
+// first add.
+//
+// Residual rule: the right-hand side holds nq = -oc r per cell (oc = omega /
+// cnt, cnt = in-grid neighbours; 0 outside the grid), and
+//     v' = oc S + ((1 - omega) v + nq),   S = sum of the in-grid neighbours,
+// which is v + oc (S - cnt v - r), the reference operator's SOR update
+// (solver.cpp:29-47), in five VALU operations per cell (three adds, two FMAs).
+// Cells outside the grid have oc = nq = 0 and value 0, and stay 0: they drop
+// out of S by themselves.  Max-update rule (TRACK): the right-hand side holds r
+// and the update oc (S - cnt v - r) is formed explicitly, as the stop test
+// tracks it; a neighbour outside the grid contributes the cell's own value.
+//
+// What bounds it: dispatch, loads and stores take 4.3 us (R = 4) to 6.6 us
+// (R = 8) of a launch whatever its sweeps; a half-sweep of one region per CU
+// 0.19 to 0.28 us (0.13 / 0.27 us of it VALU issue, the rest the exchange's
+// latency), a further region per CU 2.9 us (R = 4, 5 sweeps) to 5.6 us (R = 8, 8
+// sweeps), where VALU issue and memory phases of two resident workgroups
+// overlap.  Taller regions lose less of their work to the halo, shorter ones
+// have the faster half-sweep, more sweeps per launch spread the fixed part over
+// a wider halo: blocked_plan weighs these.  Registers: 64 VGPRs (R = 8) keep two
+// workgroups per CU; row and column kinds per wave instead of a factor per cell
+// made room for that (102 VGPRs before, one workgroup per CU, 21.9 us for 8
+// sweeps at 2048 x 2048 against 16.1).  Measured and not taken: 8 waves of 16
+// rows 19.1 us, 12 of 8 18.1, 8 of 8 18.6, 4 of 16 23.6, 16 of 10 24.9.
 // ---------------------------------------------------------------------------
-// Geometry is fixed at compile time; CD_BK_W / CD_BK_R / CD_BK_H exist to
-// compare variants on the hardware.  The kernel is bound by vector
-// ALU issue and by the load phase that precedes the sweeps (a round of
-// resident workgroups loads, then sweeps): the interior update takes five
-// VALU operations per cell (three adds, the first carrying the DPP shift, and
-// two FMAs), border tiles six.  Measured at 2048^2, 5 sweeps per launch:
-// 14.3-14.8 us per launch with these updates against 17.6-18.0 us for the
-// earlier form (fma(-4, v, sum) - r, then fma(oc, t, v); selects on border
-// tiles; 64-bit per-lane addresses); right-hand side in LDS 15.0-15.4 us.
-// Halo (= half-sweeps per launch): H = 6 / 8 / 10 / 12 give 3.76 / 3.27 /
-// 2.94 / 2.99 us per sweep at 2048^2 and 1.96 / 1.56 / 1.36 / 1.45 at 1024^2;
-// 16 waves x 6 rows 3.14 and 1.69.  Earlier geometry comparisons (4 sweeps per
-// launch, same 128 x 64 region): 4 waves x 16 rows 22.1 us, 8 x 8 17.0 us,
-// 12 x 6 17.7 us, 16 x 4 16.8 us; 8 x 12 and 8 x 16 (taller regions, fewer
-// workgroups) 21.7 and 27.0 us.  A persistent variant (one round of
-// workgroups walking the tiles, the next tile's loads issued before the
-// current tile's sweeps) measured 21.1-21.5 us against 17.6-18.0 us: the
-// loop-carried registers cost copies in every half-sweep and the static tile
-// split loses the dispatcher's load balance; two tiles per workgroup (the
-// second's loads issued before the first's sweeps) 17.2 us against 14.8 us;
-// delaying the start of a quarter of the first round's workgroups by 0.9-2.6
-// us (to stagger the load and sweep phases) 15.2-16.6 us.
-// H = 10 also keeps the learned iteration's 8 smoothing sweeps at two
-// launches.
-#ifndef CD_BK_R
-#define CD_BK_R 4
-#endif
-#ifndef CD_BK_H
-#define CD_BK_H 10
-#endif
-#ifndef CD_BK_W
-#define CD_BK_W 16
-#endif
 // cache policy bits of the blocked kernel's stores
 #ifndef CD_BK_STORE_POLICY
 #define CD_BK_STORE_POLICY 16  // sc1: written through, not left dirty in L2
 #endif
-constexpr int BK_RX = 128;      // region columns (64 packed columns, one per lane)
-constexpr int BK_R = CD_BK_R;   // rows per wave
-constexpr int BK_NW = CD_BK_W;  // waves per workgroup
+constexpr int BK_NW = 16;  // waves per workgroup
 constexpr int BK_THREADS = 64 * BK_NW;
-constexpr int BK_RY = BK_NW * BK_R;
 
-// Right-hand side of the region in the registers of the owning thread:
-// element (colour c, row k of the wave).  (In LDS it measured 4% slower.)
-template <int R>
-struct RhsRegsT {
-    float v[2][R];
-    __device__ __forceinline__ float get(int c, int k, int, int) const { return v[c][k]; }
-    __device__ __forceinline__ void set(int c, int k, int, int, float x) { v[c][k] = x; }
+// What a wave's rows meet: nothing but cells with four neighbours; also the
+// left or right grid border; also rows at or beyond the top or bottom border
+// (or, under the max-update rule, an odd width's right border).
+enum { BK_INNER = 0, BK_SIDE = 1, BK_ENDS = 2 };
+
+// Per-lane facts of a region.  Index p: the lane's cell of column parity p.
+struct BlockCells {
+    float om4, c1;             // omega / 4, 1 - omega
+    float oc[2], oc_end[2];    // omega / cnt in a row with both neighbour rows, with one
+    bool miss_l;               // cell 0 has no left neighbour
+    bool miss_r[2];            // the cell has no right neighbour
+    unsigned end_rows;         // bit k: row k of the wave has one neighbour row
+    unsigned out_rows;         // bit k: row k lies outside the grid
+    bool first, last;          // the wave's row 0 / R-1 has no row above / below it
 };
-using RhsRegs = RhsRegsT<BK_R>;
-
-// Per-lane facts of a region for the sweep helpers: packed column `lane`
-// holds cells x0 = X0 + 2 lane and x0 + 1 of rows Yw .. Yw + R - 1.
-struct SweepGeom {
-    int lane, dx0, dx1;     // region-border distances of the lane's two columns
-    int dyw, Yw, h;         // first region row and grid row of the wave, grid height
-    bool l0, l1, r0, r1;    // the two cells have a left / right neighbour in the grid
-    bool in0, in1;          // the two cells lie in the grid
-    float wl0, wl1, wr0, wr1;  // the same as weights 1 / 0
-    float om2, om3, om4;    // omega / cnt
-    float c1;               // 1 - omega
-};
-
-__device__ __forceinline__ SweepGeom sweep_geom(int X0, int RX, int RY, int R, int Yw, int dyw,
-                                                int w, int h, float om2, float om3, float om4,
-                                                float c1) {
-    SweepGeom g;
-    g.lane = threadIdx.x & 63;
-    const int x0 = X0 + 2 * g.lane;
-    g.dx0 = min(2 * g.lane, RX - 1 - 2 * g.lane);
-    g.dx1 = min(2 * g.lane + 1, RX - 2 - 2 * g.lane);
-    g.dyw = dyw;
-    g.Yw = Yw;
-    g.h = h;
-    g.in0 = (unsigned)x0 < (unsigned)w;
-    g.in1 = (unsigned)(x0 + 1) < (unsigned)w;
-    g.l0 = x0 > 0;
-    g.l1 = x0 + 1 > 0;
-    g.r0 = x0 < w - 1;
-    g.r1 = x0 + 1 < w - 1;
-    g.wl0 = g.l0 ? 1.f : 0.f;
-    g.wl1 = g.l1 ? 1.f : 0.f;
-    g.wr0 = g.r0 ? 1.f : 0.f;
-    g.wr1 = g.r1 ? 1.f : 0.f;
-    g.om2 = om2;
-    g.om3 = om3;
-    g.om4 = om4;
-    g.c1 = c1;
-    return g;
-}
 
 // Rows K0 <= k < K1 of one half-sweep of colour C.  Only rows 0 and R-1 read
-// up_row / down_row (the neighbouring waves' rows).
+// up_row / down_row (the neighbouring waves' rows).  mx[p]: largest |update|.
 //
-// Residual rule (!TRACK): the right-hand side holds nq = -oc r per cell
-// (oc = omega / cnt, cnt = in-grid neighbours; 0 outside the grid), and
-//     v' = oc S + ((1 - omega) v + nq),   S = sum of the in-grid neighbours,
-// which is v + oc (S - cnt v - r), the reference operator's SOR update
-// (solver.cpp:29-47), in two FMAs after the neighbour sum.  On border tiles
-// (EDGE) S is a weighted sum with weight 0 for a neighbour outside the grid
-// and oc comes per cell from `occ`; weights 1 and oc = omega / 4 give the
-// interior path's operations, hence its bits.  Cells outside the grid have
-// oc = nq = 0 and value 0, and stay 0.
-// Max-update rule (TRACK): the right-hand side holds r; the update
-// oc (S - cnt v - r) is formed explicitly, as the stop test tracks it.
-template <int C, int H, bool EDGE, bool TRACK, int R, int RY, int K0, int K1, typename RV>
-__device__ __forceinline__ void blocked_half(float (&ev)[2][R], const RV& rv, const SweepGeom g,
-                                             const float (&occ)[2][R], float up_row,
-                                             float down_row, float& mx) {
+// Every cell of the region is updated.  A cell at distance d from an inner
+// region border takes stale neighbours, but after half-sweep s only cells at
+// distance >= s are exact, and those read cells at distance >= s-1 only: the
+// stale values never reach the stored cells (distance >= halo) and stay finite
+// (each update is a bounded combination of finite values).
+template <int C, int KIND, bool TRACK, int R, int K0, int K1>
+__device__ __forceinline__ void blocked_half(float (&ev)[2][R], const float (&rv)[2][R],
+                                             const BlockCells& g, unsigned end_rows,
+                                             unsigned out_rows, float up_row, float down_row,
+                                             float (&mx)[2]) {
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
         const int p = (k + C) & 1;  // column parity of colour-C cells in row k (R even)
         const float o = ev[1 - C][k];
-        const float up = k > 0 ? ev[1 - C][k - 1] : up_row;
-        const float down = k < R - 1 ? ev[1 - C][k + 1] : down_row;
-        const int dy = min(g.dyw + k, RY - 1 - (g.dyw + k));
-        const int dx = p ? g.dx1 : g.dx0;
+        float up = k > 0 ? ev[1 - C][k - 1] : up_row;
+        float down = k < R - 1 ? ev[1 - C][k + 1] : down_row;
+        float left = p ? o : lane_prev(o);
+        float right = p ? lane_next(o) : o;
         const float v = ev[C][k];
-        if (!TRACK) {
-            const float nq = rv.get(C, k, g.dyw, g.lane);
-            if (EDGE) {
-                const int Y = g.Yw + k;
-                const float wu = Y > 0 ? 1.f : 0.f, wd = Y < g.h - 1 ? 1.f : 0.f;  // uniform
-                const float wl = p ? g.wl1 : g.wl0, wr = p ? g.wr1 : g.wr0;
-                float sum = (p ? o : lane_prev(o)) * wl;
-                sum = __builtin_fmaf(wu, up, sum);
-                sum = __builtin_fmaf(wr, p ? lane_next(o) : o, sum);
-                sum = __builtin_fmaf(wd, down, sum);
-                ev[C][k] = __builtin_fmaf(occ[C][k], sum, __builtin_fmaf(g.c1, v, nq));
-            } else {
-                // Interior region: every cell is updated.  A cell at distance
-                // d < s from the region border takes stale neighbours, but
-                // after half-sweep s only cells at distance >= s are exact, and
-                // those read cells at distance >= s-1 only: the stale values
-                // never reach the stored interior (distance >= H >= nhalf) and
-                // stay finite (each update is a bounded combination of finite
-                // values).
-                const float left = p ? o : lane_prev(o);
-                const float right = p ? lane_next(o) : o;
-                const float sum = left + up + right + down;
-                ev[C][k] = __builtin_fmaf(g.om4, sum, __builtin_fmaf(g.c1, v, nq));
+        float oc = KIND == BK_INNER ? g.om4 : g.oc[p];
+        if (KIND == BK_ENDS) {
+            oc = (end_rows >> k) & 1u ? g.oc_end[p] : oc;
+            oc = (out_rows >> k) & 1u ? 0.f : oc;
+        }
+        if (TRACK) {
+            if (KIND != BK_INNER) {
+                if (p == 0) left = g.miss_l ? v : left;
+                // (cell 0 has no right neighbour only where the width is odd)
+                if (p == 1 || KIND == BK_ENDS) right = g.miss_r[p] ? v : right;
             }
+            if (KIND == BK_ENDS) {
+                if (k == 0) up = g.first ? v : up;
+                // (row k is the last in the grid where row k + 1 is not in it)
+                const bool below = k < R - 1 ? ((out_rows >> (k + 1)) & 1u) != 0 : g.last;
+                down = below ? v : down;
+            }
+            const float t = __builtin_fmaf(-4.f, v, left + up + right + down) - rv[C][k];
+            const float dl = oc * t;
+            ev[C][k] = v + dl;
+            mx[p] = fmaxf(mx[p], fabsf(dl));  // (0, or a NaN that fmaxf drops, where oc = 0)
         } else {
-            const float left = p ? o : lane_prev(o);
-            const float right = p ? lane_next(o) : o;
-            if (EDGE) {
-                // A neighbour outside the grid contributes the cell's own
-                // value: the sum is then the sum over the in-grid neighbours
-                // plus (4 - cnt) v, so fma(-4, v, sum) = sum_in - cnt v, and
-                // omega/cnt (om4 / om3 / om2) scales the update.  Cells outside
-                // the grid keep their value (0); they are never read by cells
-                // inside it.  The grid border lies at least H cells inside the
-                // region, so every in-grid cell is updated: stale values near
-                // the region border never reach the stored interior.
-                // (Branch-free: uniform per-row branches here keep the
-                // compiler from interleaving the rows' dependent chains.)
-                const int Y = g.Yw + k;
-                const bool lu = Y > 0, ld = Y < g.h - 1;  // uniform over the wave
-                const bool ll = p ? g.l1 : g.l0, lr = p ? g.r1 : g.r0;
-                const bool in = (p ? g.in1 : g.in0) && Y >= 0 && Y < g.h;
-                const float sum = (ll ? left : v) + (lu ? up : v) + (lr ? right : v) + (ld ? down : v);
-                const int miss = (int)!ll + (int)!lr + (int)!lu + (int)!ld;
-                const float oc = miss == 0 ? g.om4 : (miss == 1 ? g.om3 : g.om2);
-                const float t = __builtin_fmaf(-4.f, v, sum) - rv.get(C, k, g.dyw, g.lane);
-                const float dl = oc * t;
-                ev[C][k] = in ? v + dl : v;
-                if (in && dx >= H && dy >= H) mx = fmaxf(mx, fabsf(dl));
-            } else {
-                const float t = __builtin_fmaf(-4.f, v, left + up + right + down) -
-                                rv.get(C, k, g.dyw, g.lane);
-                const float dl = g.om4 * t;
-                ev[C][k] = v + dl;
-                if (dx >= H && dy >= H) mx = fmaxf(mx, fabsf(dl));
-            }
+            const float sum = left + up + right + down;
+            ev[C][k] = __builtin_fmaf(oc, sum, __builtin_fmaf(g.c1, v, rv[C][k]));
         }
     }
 }
 
-template <int C, int H, bool EDGE, bool TRACK, int R, int NW, typename RV>
-__device__ __forceinline__ void blocked_step(float (&ev)[2][R], const RV& rv,
-                                             float (*xch)[NW][2][64], const SweepGeom g,
-                                             const float (&occ)[2][R], int wave, float& mx) {
-    const int lane = g.lane;
+template <int C, int KIND, bool TRACK, int R>
+__device__ __forceinline__ void blocked_step(float (&ev)[2][R], const float (&rv)[2][R],
+                                             float (*xch)[BK_NW][2][64], const BlockCells& g,
+                                             int wave, int lane, float (&mx)[2]) {
     // publish this wave's first/last row of the colour the update reads
     xch[1 - C][wave][0][lane] = ev[1 - C][0];
     xch[1 - C][wave][1][lane] = ev[1 - C][R - 1];
+    // the row kinds are re-read each half-sweep, so that the factors derived
+    // from them are not kept in registers per row
+    unsigned er = __builtin_amdgcn_readfirstlane(g.end_rows);
+    unsigned ou = __builtin_amdgcn_readfirstlane(g.out_rows);
+    if (KIND == BK_ENDS) asm volatile("" : "+s"(er), "+s"(ou));
     // the inner rows need only this wave's registers: update them while the
     // other waves reach the barrier (the order of the updates of one colour
     // does not matter: they read only the other colour)
-    blocked_half<C, H, EDGE, TRACK, R, R * NW, 1, R - 1>(ev, rv, g, occ, 0.f, 0.f, mx);
+    blocked_half<C, KIND, TRACK, R, 1, R - 1>(ev, rv, g, er, ou, 0.f, 0.f, mx);
     __syncthreads();
-    const float up_row = xch[1 - C][wave > 0 ? wave - 1 : 0][1][lane];
-    const float down_row = xch[1 - C][wave < NW - 1 ? wave + 1 : NW - 1][0][lane];
-    blocked_half<C, H, EDGE, TRACK, R, R * NW, 0, 1>(ev, rv, g, occ, up_row, down_row, mx);
-    blocked_half<C, H, EDGE, TRACK, R, R * NW, R - 1, R>(ev, rv, g, occ, up_row, down_row, mx);
-}
-
-// nhalf <= H half-sweeps, colours alternating from 0; mxs[j] receives the
-// largest |update| of sweep j over the cells the launch stores (TRACK)
-template <int H, bool EDGE, bool TRACK, int R, int NW, typename RV>
-__device__ __forceinline__ void blocked_run(float (&ev)[2][R], const RV& rv,
-                                            float (*xch)[NW][2][64], const SweepGeom g,
-                                            const float (&occ)[2][R], int wave, int nhalf,
-                                            float (&mxs)[H / 2]) {
-#pragma unroll
-    for (int j = 0; j < H / 2; ++j) {
-        const int s = 2 * j + 1;
-        if (s > nhalf) break;
-        float mx = 0.f;
-        blocked_step<0, H, EDGE, TRACK, R, NW>(ev, rv, xch, g, occ, wave, mx);
-        if (s + 1 <= nhalf) blocked_step<1, H, EDGE, TRACK, R, NW>(ev, rv, xch, g, occ, wave, mx);
-        mxs[j] = fmaxf(mxs[j], mx);
+    float up_row = xch[1 - C][wave > 0 ? wave - 1 : 0][1][lane];
+    float down_row = xch[1 - C][wave < BK_NW - 1 ? wave + 1 : BK_NW - 1][0][lane];
+    if (KIND == BK_ENDS && !TRACK) {
+        up_row = g.first ? 0.f : up_row;
+        down_row = g.last ? 0.f : down_row;
     }
+    blocked_half<C, KIND, TRACK, R, 0, 1>(ev, rv, g, er, ou, up_row, down_row, mx);
+    blocked_half<C, KIND, TRACK, R, R - 1, R>(ev, rv, g, er, ou, up_row, down_row, mx);
 }
 
-// Right-hand side of the sweeps, per cell: r - mean (TRACK) or
-// nq = (mean - r) oc (residual rule, see blocked_half).  On interior tiles
-// every cell lies in the grid with four neighbours (oc = omega / 4); on border
-// tiles cells outside the grid get value 0 and nq = oc = 0.
-template <bool EDGE, bool TRACK, typename RT, typename RV>
-__device__ __forceinline__ void region_setup(float (&ev)[2][BK_R], const RT (&rr)[2][BK_R], RV& rv,
-                                             float (&occ)[2][BK_R], const SweepGeom g, float rm) {
-#pragma unroll
-    for (int k = 0; k < BK_R; ++k) {
-        const int Y = g.Yw + k;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int p = (k + c) & 1;
-            const float rc = rhs_to_f32(rr[c][k]);
-            if (!EDGE) {
-                rv.set(c, k, g.dyw, g.lane, TRACK ? rc - rm : (rm - rc) * g.om4);
-                continue;
-            }
-            const bool in = (p ? g.in1 : g.in0) && Y >= 0 && Y < g.h;
-            ev[c][k] = in ? ev[c][k] : 0.f;
-            if (TRACK) {
-                rv.set(c, k, g.dyw, g.lane, in ? rc - rm : 0.f);
-            } else {
-                const int miss = (int)!(p ? g.l1 : g.l0) + (int)!(p ? g.r1 : g.r0) +
-                                 (int)!(Y > 0) + (int)!(Y < g.h - 1);
-                const float oc = in ? (miss == 0 ? g.om4 : (miss == 1 ? g.om3 : g.om2)) : 0.f;
-                occ[c][k] = oc;
-                rv.set(c, k, g.dyw, g.lane, (rm - rc) * oc);
-            }
+// nsweeps sweeps of a region.  The waves of a workgroup may take this with
+// different KINDs (a choice uniform over the wave): each executes the same
+// number of barriers.
+template <int KIND, bool TRACK, int R>
+__device__ __forceinline__ void blocked_run(float (&ev)[2][R], const float (&rv)[2][R],
+                                            float (*xch)[BK_NW][2][64], const BlockCells& g,
+                                            int wave, int lane, int nsweeps,
+                                            float (*smax)[BK_NW][64], bool track0, bool track1) {
+    for (int j = 0; j < nsweeps; ++j) {
+        float mx[2] = {0.f, 0.f};
+        blocked_step<0, KIND, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
+        blocked_step<1, KIND, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
+        if (TRACK) {
+            smax[j][wave][lane] = fmaxf(track0 ? mx[0] : 0.f, track1 ? mx[1] : 0.f);
         }
     }
 }
 
-// The right-hand side is BF16 under the residual rule (every FP64 check
-// re-rounds the current residual, so the rounding never reaches the result)
-// and FP32 under the max-update rule (TRACK), which cannot see the smooth
-// error a rounded right-hand side leaves behind.
 // The intermediate-grid correction em (bricked, wm x hm, fm x fm fine cells
 // per cell), which the learned iteration's first fine smoothing launch
 // interpolates bilinearly at the fine cell centres as it loads its region.
@@ -868,33 +745,32 @@ struct MidGrid {
     int wm, hm, fm;
 };
 
-// Loads of one region: packed column `lane` of the wave's BK_R rows, both
-// colours, from the correction and the right-hand side.  Rows and columns are
-// clamped into the grid (cells outside it are masked by region_setup).
+// Loads of one region: packed column `lane` of the wave's R rows, both colours,
+// from the correction and the right-hand side.  Rows and columns are clamped
+// into the grid.
 // PROLONG: the correction is the intermediate-grid correction interpolated
 // bilinearly at the cell centres (u, v) = ((x, y) + 0.5) / fm - 0.5, not ein;
 // the workgroup first stages the intermediate cells its region needs in
 // `patch` (each is read by up to 4 fm^2 fine cells), with the intermediate
 // grid's border clamping.  All waves of the workgroup must call it.
-constexpr int kPatchMax = (BK_RX / 2 + 2) * (BK_RY / 2 + 2);  // fm >= 2
-template <int H, bool PROLONG, typename RT>
-__device__ __forceinline__ void region_load(float (&ev)[2][BK_R], RT (&rr)[2][BK_R],
+template <int R>
+constexpr int kPatchMax = (SW_RX / 2 + 2) * (BK_NW * R / 2 + 2);  // fm >= 2
+template <int R, bool PROLONG, typename RT>
+__device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R],
                                             __amdgpu_buffer_rsrc_t ein_rs,
                                             __amdgpu_buffer_rsrc_t r_rs, const Brick& bk,
-                                            const MidGrid& mid, float* patch, int tile,
-                                            int tiles_x, int w, int h, int wave, int lane) {
-    constexpr int IX = BK_RX - 2 * H, IY = BK_RY - 2 * H;
-    const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
-    const int X0 = tx * IX - H, Y0 = ty * IY - H, Yw = Y0 + BK_R * wave;
-    const int j = min(max(X0 / 2 + lane, 0), (w + 1) / 2 - 1);
+                                            const MidGrid& mid, float* patch, int X0, int Y0,
+                                            int w, int h, int wave, int lane) {
+    const int Yw = Y0 + R * wave;
+    const int j = min(X0 / 2 + lane, (w + 1) / 2 - 1);
     const unsigned col = brick_col(j);
     int pi0[2] = {0, 0}, pj0 = 0, pw = 0;
     float ptu[2] = {0.f, 0.f};
     const float inv = PROLONG ? 1.f / mid.fm : 0.f;
     if (PROLONG) {
         // intermediate cells I0..I1 x J0..J1 cover the region's (clamped) cells
-        const int xa = min(max(X0, 0), w - 1), xb = min(max(X0 + BK_RX - 1, 0), w - 1);
-        const int ya = min(max(Y0, 0), h - 1), yb = min(max(Y0 + BK_RY - 1, 0), h - 1);
+        const int xa = min(X0, w - 1), xb = min(X0 + SW_RX - 1, w - 1);
+        const int ya = min(Y0, h - 1), yb = min(Y0 + BK_NW * R - 1, h - 1);
         const int I0 = (int)floorf((xa + 0.5f) * inv - 0.5f);
         const int I1 = (int)floorf((xb + 0.5f) * inv - 0.5f) + 1;
         pj0 = (int)floorf((ya + 0.5f) * inv - 0.5f);
@@ -918,8 +794,8 @@ __device__ __forceinline__ void region_load(float (&ev)[2][BK_R], RT (&rr)[2][BK
         __syncthreads();
     }
 #pragma unroll
-    for (int k = 0; k < BK_R; ++k) {
-        const int Yc = min(max(Yw + k, 0), h - 1);
+    for (int k = 0; k < R; ++k) {
+        const int Yc = min(Yw + k, h - 1);
         int r0 = 0;
         float tv = 0.f;
         if (PROLONG) {
@@ -945,134 +821,131 @@ __device__ __forceinline__ void region_load(float (&ev)[2][BK_R], RT (&rr)[2][BK
     }
 }
 
-// Setup, nhalf half-sweeps and the store of one loaded region; mxs[j] takes
-// the max with the largest |update| of sweep j (TRACK).
-template <int H, bool TRACK, typename RT>
-__device__ __forceinline__ void blocked_tile(float (&ev)[2][BK_R], const RT (&rr)[2][BK_R],
-                                             float (*xch)[BK_NW][2][64], float (&mxs)[H / 2],
-                                             __amdgpu_buffer_rsrc_t eout_rs, const Brick& bk,
-                                             int tile, int tiles_x, int w, int h, int nhalf,
-                                             float om2, float om3, float om4, float rm, int wave,
-                                             int lane) {
-    constexpr int IX = BK_RX - 2 * H, IY = BK_RY - 2 * H;
-    const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
-    const int X0 = tx * IX - H, Y0 = ty * IY - H;
-    const int wp = (w + 1) / 2;
-    const int Yw = Y0 + BK_R * wave;  // first global row of this wave
-    const int dyw = BK_R * wave;      // first region row of this wave
-    const unsigned col = brick_col(min(max(X0 / 2 + lane, 0), wp - 1));
-    RhsRegs rv;
-    const SweepGeom g = sweep_geom(X0, BK_RX, BK_RY, BK_R, Yw, dyw, w, h, om2, om3, om4,
-                                   1.f - 4.f * om4);
-    const bool edge = X0 < 1 || X0 + BK_RX > w - 1 || Y0 < 1 || Y0 + BK_RY > h - 1;
-    float occ[2][BK_R];  // border tiles: omega / cnt per cell, 0 outside the grid
-    if (edge) {
-        region_setup<true, TRACK>(ev, rr, rv, occ, g, rm);
-        blocked_run<H, true, TRACK, BK_R, BK_NW>(ev, rv, xch, g, occ, wave, nhalf, mxs);
-    } else {
-        region_setup<false, TRACK>(ev, rr, rv, occ, g, rm);
-        blocked_run<H, false, TRACK, BK_R, BK_NW>(ev, rv, xch, g, occ, wave, nhalf, mxs);
-    }
-    // write the interior
-#pragma unroll
-    for (int k = 0; k < BK_R; ++k) {
-        const int Y = Yw + k;
-        const int dy = min(dyw + k, BK_RY - 1 - (dyw + k));
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int p = (k + c) & 1;
-            const int dx = p ? g.dx1 : g.dx0;
-            if (dx >= H && dy >= H && (unsigned)Y < (unsigned)h && (p ? g.in1 : g.in0))
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ev[c][k]), eout_rs, col * 4u,
-                                                      (unsigned)brick_row(bk, c, Y) * 4u,
-                                                      CD_BK_STORE_POLICY);
-        }
-    }
-}
-
-// workgroups of a k_rb_blocked launch over ntiles tiles (a multiple of 8)
-inline int blocked_grid(int ntiles) { return (ntiles + 7) / 8 * 8; }
-
-// FULL: nhalf == H, known at compile time (every launch but a batch's last),
-// which leaves the half-sweeps free of branches.  PROLONG: the sweeps start
+// The right-hand side is BF16 under the residual rule (every FP64 check
+// re-rounds the current residual, so the rounding never reaches the result)
+// and FP32 under the max-update rule (TRACK), which cannot see the smooth
+// error a rounded right-hand side leaves behind.  PROLONG: the sweeps start
 // from `mid` interpolated at the cells instead of from ein.
-template <int H, bool TRACK, bool FULL, bool PROLONG = false>
-__global__ __launch_bounds__(BK_THREADS) void k_rb_blocked(const float* __restrict__ ein,
-                                                    float* __restrict__ eout,
-                                                    const void* __restrict__ rhs,
-                                                    Brick bk, int w, int h,
-                                                    int tiles_x, int ntiles, int nhalf,
-                                                    float om2, float om3, float om4,
-                                                    const float* __restrict__ rmean,
-                                                    SolveDev* st, int out_index, MidGrid mid) {
-    static_assert(H % 2 == 0 && H >= 2 && 2 * H < BK_RY && BK_R % 2 == 0, "geometry");
+template <int R, bool TRACK, bool PROLONG>
+__global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) ? 4 : 8) void k_rb_blocked(
+    const float* ein, float* eout, const void* __restrict__ rhs, Brick bk, SweepTiles tiles,
+    int nsweeps, float om2, float om3, float om4, const float* __restrict__ rmean, SolveDev* st,
+    int out_index, MidGrid mid, TrackArgs track) {
+    static_assert(R % 2 == 0, "colours alternate by row");
     __shared__ float xch[2][BK_NW][2][64];
-    __shared__ float smax[BK_NW][H / 2];
-    // XCD-aware tile order: gridDim.x is a multiple of 8 and consecutive
-    // workgroups go round-robin to the 8 XCDs; give each XCD a contiguous band
-    // of tiles so halo re-reads hit its own L2.
-    const int per = gridDim.x >> 3;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (tile >= ntiles) return;
+    __shared__ float smax[TRACK ? kTrackSweeps : 1][BK_NW][64];
+    __shared__ unsigned red[TRACK ? BK_NW : 1];
+    __shared__ float patch[PROLONG ? kPatchMax<R> : 1];
+    const int tile = tile_of_block();
+    if (tile >= tiles.ntiles) return;
+    const Region rg = region_of(tiles, tile);
+    const int w = tiles.w, h = tiles.h;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     using RT = typename std::conditional<TRACK, float, unsigned short>::type;
     const size_t npk = 2 * bk.plane;
     const __amdgpu_buffer_rsrc_t ein_rs = plane_rsrc(ein, npk * sizeof(float));
     const __amdgpu_buffer_rsrc_t r_rs = plane_rsrc(rhs, npk * sizeof(RT));
-    const __amdgpu_buffer_rsrc_t eout_rs = plane_rsrc(eout, npk * sizeof(float));
-    float ev[2][BK_R];
-    RT rr[2][BK_R];
-    __shared__ float patch[PROLONG ? kPatchMax : 1];
-    region_load<H, PROLONG>(ev, rr, ein_rs, r_rs, bk, mid, patch, tile, tiles_x, w, h, wave,
-                            lane);
-    // Max-update rule: the stop flag can be set between the launches of one
-    // batch (k_maxcheck_blocked), and a finished solve leaves the buffers
-    // untouched.  Residual rule: only a check sets it, and no sweeps are
-    // enqueued after a check that stopped the solve, so the flag is not read
-    // (reading it first would hold every load behind two dependent scalar
-    // loads).
-    if (TRACK && st->done) return;
-    const float rm = *rmean;
-    float mxs[H / 2];
-#pragma unroll
-    for (int j = 0; j < H / 2; ++j) mxs[j] = 0.f;
-    blocked_tile<H, TRACK>(ev, rr, xch, mxs, eout_rs, bk, tile, tiles_x, w, h, FULL ? H : nhalf,
-                           om2, om3, om4, rm, wave, lane);
+    __amdgpu_buffer_rsrc_t eout_rs = plane_rsrc(eout, npk * sizeof(float));
+    float ev[2][R], rv[2][R];
+    RT rr[2][R];
+    const unsigned words = TRACK ? track_load<BK_NW>(track, tiles.ntiles) : 0u;
+    region_load<R, PROLONG>(ev, rr, ein_rs, r_rs, bk, mid, patch, rg.X0, rg.Y0, w, h, wave, lane);
+    // Max-update rule: the solve can have stopped in an earlier launch of the
+    // batch, and then leaves the buffers untouched.  Residual rule: only a check
+    // stops it, and no sweeps are enqueued after that.
     if (TRACK) {
-#pragma unroll
-        for (int j = 0; j < H / 2; ++j) {
-            const float m = cd_wave_max(mxs[j]);
-            if (lane == 0) smax[wave][j] = m;
-        }
-        __syncthreads();
-        if (threadIdx.x < H / 2 && 2 * (int)threadIdx.x < nhalf) {
-            const int j = threadIdx.x;
-            float m = smax[0][j];
-            for (int wv = 1; wv < BK_NW; ++wv) m = fmaxf(m, smax[wv][j]);
-            atomicMax(&st->maxupd_bits[j], __float_as_uint(m));
+        const TrackPlan plan =
+            track_decide<BK_NW>(track, st, tiles.ntiles, nsweeps, words, red);
+        if (plan.nsweeps == 0) return;
+        nsweeps = plan.nsweeps;
+        if (plan.redo) {
+            out_index ^= 1;
+            region_load<R, PROLONG>(ev, rr, eout_rs, r_rs, bk, mid, patch, rg.X0, rg.Y0, w, h,
+                                    wave, lane);
+            eout_rs = ein_rs;
         }
     }
-    if (threadIdx.x == 0) st->cur = out_index;  // same value from every workgroup
-}
+    const float rm = *rmean;
 
-// max-update stop rule over the sweeps of one blocked launch (solver.cpp:142).
-// The launch has applied all of its nsweeps sweeps, so a stop at any of them
-// counts the whole launch.
-__global__ void k_maxcheck_blocked(SolveDev* st, int first_sweep, int nsweeps, double tol) {
-    if (threadIdx.x != 0) return;
-    if (!st->done) {
-        for (int j = 0; j < nsweeps; ++j) {
-            const float mu = __uint_as_float(st->maxupd_bits[j]);
-            st->last_max_update = (double)mu;
-            if ((double)mu < tol) {
-                st->done = 1;
-                st->sweeps_at_done = first_sweep + nsweeps;
-                break;
+    const int Yw = rg.Y0 + R * wave, x0 = rg.X0 + 2 * lane;
+    BlockCells g;
+    g.om4 = om4;
+    g.c1 = 1.f - 4.f * om4;
+    g.first = Yw == 0;
+    g.last = Yw + R >= h;
+    g.end_rows = 0u;
+    g.out_rows = 0u;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        if (Yw + k == 0 || Yw + k == h - 1) g.end_rows |= 1u << k;
+        if (Yw + k >= h) g.out_rows |= 1u << k;
+    }
+    g.miss_l = x0 == 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const bool in = x0 + p < w;
+        const bool side = x0 + p == 0 || x0 + p == w - 1;
+        g.miss_r[p] = x0 + p >= w - 1;
+        g.oc[p] = in ? (side ? om3 : om4) : 0.f;
+        g.oc_end[p] = in ? (side ? om2 : om3) : 0.f;
+    }
+    // (uniform over the wave)
+    const int kind = (g.first || g.last || (TRACK && rg.right && (w & 1))) ? BK_ENDS
+                     : (rg.left || rg.right) ? BK_SIDE : BK_INNER;
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int p = (k + c) & 1;
+            const float rc = rhs_to_f32(rr[c][k]);
+            float oc = g.om4;
+            if (kind != BK_INNER) {
+                const bool out = (g.out_rows >> k) & 1u;
+                oc = out ? 0.f : (g.end_rows >> k) & 1u ? g.oc_end[p] : g.oc[p];
+                const bool in = !out && x0 + p < w;
+                ev[c][k] = in ? ev[c][k] : 0.f;
+                if (TRACK) rv[c][k] = in ? rc - rm : 0.f;
+                else rv[c][k] = (rm - rc) * oc;
+            } else {
+                rv[c][k] = TRACK ? rc - rm : (rm - rc) * oc;
             }
         }
+    // the cells whose updates count for the stop rule: those at distance >= halo
+    // from the region's inner borders (all exact; two tiles may count one)
+    bool t0 = false, t1 = false;
+    if (TRACK) {
+        const int hl = tiles.halo, dy0 = R * wave;  // halo is a multiple of R
+        const bool rows_ok = (rg.top || dy0 >= hl) && (rg.bottom || dy0 + R <= BK_NW * R - hl);
+        auto col_ok = [&](int dx) {
+            return rows_ok && (rg.left || dx >= hl) && (rg.right || dx < SW_RX - hl);
+        };
+        t0 = col_ok(2 * lane);
+        t1 = col_ok(2 * lane + 1);
     }
-    for (int j = 0; j < 16; ++j) st->maxupd_bits[j] = 0u;
+    if (kind == BK_INNER)
+        blocked_run<BK_INNER, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
+    else if (kind == BK_SIDE)
+        blocked_run<BK_SIDE, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
+    else
+        blocked_run<BK_ENDS, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
+    // store
+    const unsigned col = brick_col(min(rg.X0 / 2 + lane, (w + 1) / 2 - 1));
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int Y = Yw + k;
+        if (Y < rg.ys0 || Y >= rg.ys1) continue;  // uniform
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int x = x0 + ((k + c) & 1);
+            if (x >= rg.xs0 && x < rg.xs1)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ev[c][k]), eout_rs, col * 4u,
+                                                      (unsigned)brick_row(bk, c, Y) * 4u,
+                                                      CD_BK_STORE_POLICY);
+        }
+    }
+    if (TRACK) track_store<BK_NW>(track, smax, red, tile, nsweeps, wave, lane);
+    if (threadIdx.x == 0) st->cur = out_index;  // same value from every workgroup
 }
 
 // Reopen a solve whose max-update stop is to be confirmed on a fresh
@@ -1082,7 +955,6 @@ __global__ void k_reopen(SolveDev* st) {
     st->done = 0;
     st->stop_lid = INT_MAX;
     st->sweeps_at_done = -1;
-    for (int j = 0; j < 16; ++j) st->maxupd_bits[j] = 0u;
 }
 
 __global__ void k_set_holes_nan(double* __restrict__ phi, const uint8_t* __restrict__ mask,
@@ -1098,15 +970,15 @@ inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
 // loads and stores, and 0.43 us (FP64) or 0.28 us (FP32) per half-sweep and
 // round of one workgroup per CU.  At 400 x 400 in FP64 halos of 8 / 16 / 24 / 28
 // take 2.18 / 1.49 / 1.29 / 1.25 us per sweep; at 700 x 700 the 369 tiles of halo
-// 24 need a second round and take 2.12, halo 20 1.41.  tmax_bytes: room for a
-// tracking launch's two arrays of per-tile maxima.
-SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t tmax_bytes) {
+// 24 need a second round and take 2.12, halo 20 1.41.  track_room: bytes for a
+// tracking launch's two TrackOut.
+SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t track_room) {
     const double half_us = fp64 ? 0.43 : 0.28, fixed_us = 5.0;
     SweepTiles best = sweep_tiles(w, h, NAT_RY, 4);
     double best_cost = INFINITY;
     for (int halo = 4; halo <= 28; halo += 4) {
         const SweepTiles t = sweep_tiles(w, h, NAT_RY, halo);
-        if (track && 2 * sizeof(float) * kTrackSweeps * (size_t)t.ntiles > tmax_bytes) continue;
+        if (track && track_bytes(t.ntiles) > track_room) continue;
         const int sweeps = std::min(halo / 2, std::max(batch, 1));
         const double cost = (fixed_us + 2 * sweeps * half_us * div_up(t.ntiles, 256)) / sweeps;
         if (cost < best_cost) {
@@ -1115,6 +987,95 @@ SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t 
         }
     }
     return best;
+}
+
+// A max-update stop of the blocked sweeps falls at the end of a group of this
+// many sweeps, counted from the last check.
+constexpr int kStopGroup = 5;
+
+// How a batch of sweeps is cut into launches: sweeps per launch, rows per wave.
+struct BlockedPlan {
+    int rows, sweeps;
+    SweepTiles t;
+};
+
+// Time of a launch of `sweeps` sweeps over ntiles regions of 16 waves x `rows`
+// rows, in us: a first region per CU, then every further one.  Fitted to
+// launches of 5 to 16 sweeps on grids of 128 to 4096 squared (rows 4: 6.2 us for
+// 5 sweeps of up to 256 regions, 9.7 for 14; rows 8: 11.2 for 8, 16.1 with two
+// regions per CU, 50.3 with eight).  Tracking launches have about twice the VALU
+// work per sweep and, at 8 rows, one workgroup per CU.
+double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
+    struct Cost { double first, first_half, next, next_half; };
+    static constexpr Cost cost[2][3] = {
+        {{4.3, 0.194, 2.45, 0.042}, {5.2, 0.234, 3.2, 0.093}, {6.6, 0.283, 3.9, 0.125}},
+        {{5.7, 0.345, 3.0, 0.135}, {7.4, 0.45, 4.2, 0.17}, {8.8, 0.525, 8.0, 0.36}}};
+    const Cost& c = cost[track][(rows - 4) / 2];
+    const int halves = 2 * sweeps;
+    return c.first + c.first_half * halves +
+           (c.next + c.next_half * halves) * (div_up(ntiles, 256) - 1);
+}
+
+// The cut of a batch of `batch` sweeps on a w x h grid that blocked_launch_us
+// finds cheapest.  Per sweep, measured: 2048 x 2048 1.87 us (8 rows, 9 sweeps;
+// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 1.01 (8, 16; 1.31), 400 x 400 0.74
+// (4, 14; 1.29).  Tracking launches take whole groups, a halo of whole waves,
+// and need room for two TrackOut in track_room bytes.
+BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room) {
+    BlockedPlan best{4, kStopGroup, sweep_tiles(w, h, BK_NW * 4, 2 * kStopGroup)};
+    double best_us = INFINITY;
+    batch = std::max(batch, 1);
+    for (int rows = 4; rows <= 8; rows += 2) {
+        const int ry = BK_NW * rows, unit = track ? kStopGroup : 1;
+        const int most = track ? kTrackSweeps / unit * unit : 16;
+        for (int sweeps = unit; sweeps <= most; sweeps += unit) {
+            const int halo = track ? div_up(2 * sweeps, rows) * rows : 2 * sweeps;
+            if (ry - 2 * halo < 8) break;
+            SweepTiles t = sweep_tiles(w, h, ry, halo);
+            if (track && track_bytes(t.ntiles) > track_room) continue;
+            // a grid of one region takes any number of sweeps
+            const int per = t.ntiles > 1 ? sweeps : track ? most : batch;
+            const int full = batch / per, rest = batch % per;
+            const double us = full * blocked_launch_us(rows, per, t.ntiles, track) +
+                              (rest ? blocked_launch_us(rows, rest, t.ntiles, track) : 0.0);
+            if (us < best_us) {
+                best_us = us;
+                best = BlockedPlan{rows, per, t};
+            }
+        }
+    }
+    return best;
+}
+
+template <int R>
+void launch_blocked_rows(bool track, const MidGrid* pro, dim3 grid, hipStream_t s,
+                         const float* ein, float* eout, const void* rhs, const Brick& bk,
+                         const SweepTiles& t, int nsweeps, float om2, float om3, float om4,
+                         const float* rmean, SolveDev* st, int out_index, const TrackArgs& tr) {
+    const dim3 blk(BK_THREADS);
+    const MidGrid mid = pro ? *pro : MidGrid{};
+    if (track)
+        hipLaunchKernelGGL((k_rb_blocked<R, true, false>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+    else if (pro)
+        hipLaunchKernelGGL((k_rb_blocked<R, false, true>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+    else
+        hipLaunchKernelGGL((k_rb_blocked<R, false, false>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+}
+
+// one launch of nsweeps sweeps from ein to eout
+void launch_blocked(const BlockedPlan& pl, bool track, const MidGrid* pro, hipStream_t s,
+                    const float* ein, float* eout, const void* rhs, const Brick& bk, int nsweeps,
+                    float om2, float om3, float om4, const float* rmean, SolveDev* st,
+                    int out_index, const TrackArgs& tr) {
+    const dim3 grid(sweep_grid(pl.t.ntiles));
+    switch (pl.rows) {
+    case 4: launch_blocked_rows<4>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
+    case 6: launch_blocked_rows<6>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
+    default: launch_blocked_rows<8>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
+    }
 }
 
 // Over-relaxation factor.  > 0: as given.  < 0: the reference's
@@ -1849,48 +1810,41 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                             ncheck);
     };
 
-    // blocked geometry
-    constexpr int BH = CD_BK_H;  // halo = half-sweeps per launch
-    const int bix = BK_RX - 2 * BH, biy = BK_RY - 2 * BH;
-    const int tiles_x = div_up(w, bix), tiles_y = div_up(h, biy);
-    const int ntiles = tiles_x * tiles_y;
-    const int bgrid = blocked_grid(ntiles);
     const float om = (float)omega;
     const float om2 = om / 2.f, om3 = om / 3.f, om4 = om / 4.f;
-    // pro: the first launch starts from this intermediate-grid correction,
-    // interpolated at the cells, instead of from e32
+    int track_lid = 0;  // tracking launches of this solve
+    // count_sweeps sweeps in launches between e32 and e32b, the first reading
+    // e32; pro: it starts from this intermediate-grid correction, interpolated
+    // at the cells, instead
     auto enqueue_blocked_om = [&](int first, int count_sweeps, float om2, float om3, float om4,
                                   const MidGrid* pro = nullptr) -> int {
         CD_TRY(timer_begin());
+        const BlockedPlan pl = blocked_plan(w, h, count_sweeps, track != 0, cd_partials_bytes(nred));
+        TrackArgs tr{};
+        tr.group = kStopGroup;
+        tr.tol = o->tol;
         int launches = 0;
-        const MidGrid none{};
-        for (int done_sw = 0; done_sw < count_sweeps;) {
-            const int nsw = std::min(BH / 2, count_sweeps - done_sw);
-            const bool full = 2 * nsw == BH;
-            const int in = launches & 1;
-            float* ein = in ? e32b : e32;
-            float* eout = in ? e32 : e32b;
-            if (track) {
-                hipLaunchKernelGGL(full ? (k_rb_blocked<BH, true, true>) : (k_rb_blocked<BH, true, false>),
-                                   dim3(bgrid), dim3(BK_THREADS), 0, s, ein, eout, r32, bk, w, h,
-                                   tiles_x, ntiles, 2 * nsw, om2, om3, om4, &sd->rmean32, sd,
-                                   1 - in, none);
-                hipLaunchKernelGGL(k_maxcheck_blocked, dim3(1), dim3(64), 0, s, sd,
-                                   first + done_sw, nsw, o->tol);
-            } else if (pro && launches == 0) {
-                hipLaunchKernelGGL(full ? (k_rb_blocked<BH, false, true, true>)
-                                        : (k_rb_blocked<BH, false, false, true>),
-                                   dim3(bgrid), dim3(BK_THREADS), 0, s, ein, eout, r16, bk, w, h,
-                                   tiles_x, ntiles, 2 * nsw, om2, om3, om4, &sd->rmean32, sd,
-                                   1 - in, *pro);
-            } else {
-                hipLaunchKernelGGL(full ? (k_rb_blocked<BH, false, true>) : (k_rb_blocked<BH, false, false>),
-                                   dim3(bgrid), dim3(BK_THREADS), 0, s, ein, eout, r16, bk, w, h,
-                                   tiles_x, ntiles, 2 * nsw, om2, om3, om4, &sd->rmean32, sd,
-                                   1 - in, none);
-            }
-            ++launches;
+        float* bufs[2] = {e32, e32b};
+        const void* rhs = track ? (const void*)r32 : (const void*)r16;
+        for (int done_sw = 0; done_sw < count_sweeps; ++launches) {
+            const int nsw = std::min(pl.sweeps, count_sweeps - done_sw);
+            float* ein = bufs[launches & 1];
+            float* eout = bufs[1 - (launches & 1)];
+            tr.lid = ++track_lid;
+            tr.out = track_out(partials, pl.t.ntiles, launches & 1);
+            launch_blocked(pl, track != 0, launches == 0 ? pro : nullptr, s, ein, eout, rhs, bk,
+                           nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr);
+            tr.prev = tr.out;
+            tr.nprev = nsw;
+            tr.first_prev = first + done_sw;
             done_sw += nsw;
+        }
+        if (track) {  // the last launch's own decision
+            tr.lid = ++track_lid;
+            tr.check_only = 1;
+            launch_blocked(pl, true, nullptr, s, bufs[launches & 1], bufs[1 - (launches & 1)], rhs,
+                           bk, 0, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr);
+            ++launches;
         }
         CD_CHECK_LAUNCH(ctx);
         // algorithmic bytes: 12 B per cell per red+black sweep (e read, e write,
@@ -1904,7 +1858,6 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     // natural layout: launches of several sweeps between the buffers b0 and b1;
     // FP64 iterates continue in the buffer the last check found current, FP32
     // corrections start in b0 (the check's flush cleared it)
-    int track_lid = 0;
     auto enqueue_natural = [&](auto* b0, auto* b1, const auto* rhs, auto om, const auto* mean,
                                int first, int count_sweeps) -> int {
         using T = std::remove_pointer_t<decltype(b0)>;
@@ -1913,8 +1866,6 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         const int most = t.ntiles == 1 ? (track ? kTrackSweeps : count_sweeps) : t.halo / 2;
         const dim3 grid(sweep_grid(t.ntiles)), blk(64 * NAT_NW);
         int cur = mixed ? 0 : ctx->host_status->cur;
-        float* tmax[2] = {reinterpret_cast<float*>(partials),
-                          reinterpret_cast<float*>(partials) + (size_t)t.ntiles * kTrackSweeps};
         TrackArgs tr{};
         tr.group = 1;
         tr.tol = o->tol;
@@ -1926,14 +1877,15 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             T* out = cur ? b0 : b1;
             if (track) {
                 tr.lid = ++track_lid;
+                tr.out = track_out(partials, t.ntiles, launches & 1);
                 hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, in, out, rhs, mask, t,
-                                   nsw, om, mean, sd, 1 - cur, tmax[launches & 1], tr);
-                tr.prev = tmax[launches & 1];
+                                   nsw, om, mean, sd, 1 - cur, tr);
+                tr.prev = tr.out;
                 tr.nprev = nsw;
                 tr.first_prev = first + done_sw;
             } else {
                 hipLaunchKernelGGL((k_rb_natural<T, false>), grid, blk, 0, s, in, out, rhs, mask, t,
-                                   nsw, om, mean, sd, 1 - cur, nullptr, tr);
+                                   nsw, om, mean, sd, 1 - cur, tr);
             }
             cur = 1 - cur;
             done_sw += nsw;
@@ -1942,8 +1894,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             tr.lid = ++track_lid;
             tr.check_only = 1;
             hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, cur ? b1 : b0,
-                               cur ? b0 : b1, rhs, mask, t, 0, om, mean, sd, 1 - cur,
-                               tmax[launches & 1], tr);
+                               cur ? b0 : b1, rhs, mask, t, 0, om, mean, sd, 1 - cur, tr);
             ++launches;
         }
         CD_CHECK_LAUNCH(ctx);
@@ -2073,7 +2024,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const int nsmooth = arch ? std::max(1, arch->smooth_sweeps) : 4;
     // the smoothing launches start from e32; after `nl` launches the result
     // sits in e32 (nl even) or e32b (nl odd)
-    const int smooth_launches = div_up(nsmooth, BH / 2);
+    const int smooth_launches = div_up(nsmooth, blocked_plan(w, h, nsmooth, false, 0).sweeps);
     // packed-element kernels: grid (packed width / 256, rows, 2 planes); the
     // dot products stride over rows so that their partials fit nred blocks
     const int pbx = div_up(bk.wpb, 256);
@@ -2166,16 +2117,13 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             hipLaunchKernelGGL(k_restrict_to_mid, dim3(pbm, hm, 2), dim3(256), 0, s, r16, bk, sd,
                                fm, wm, hm, bkm, rm, ctx->lc_y.as<float>(), stats + 2, lf / fm,
                                lwc, lhc, nscale, em[0]);
-            const int tx = div_up(wm, bix), ntm = tx * div_up(hm, biy);
-            const int gm = blocked_grid(ntm);
+            const BlockedPlan pm = blocked_plan(wm, hm, mid_sweeps, false, 0);
             int cur_m = 0;
             for (int done_sw = 0; done_sw < mid_sweeps;) {
-                const int nsw = std::min(BH / 2, mid_sweeps - done_sw);
-                hipLaunchKernelGGL(2 * nsw == BH ? (k_rb_blocked<BH, false, true>) : (k_rb_blocked<BH, false, false>),
-                                   dim3(gm), dim3(BK_THREADS), 0, s, em[cur_m],
-                                   em[1 - cur_m], rm, bkm, wm, hm, tx, ntm, 2 * nsw, oms / 2.f,
-                                   oms / 3.f, oms / 4.f, ctx->fcg_zero.as<float>(), sd, 0,
-                                   MidGrid{});
+                const int nsw = std::min(pm.sweeps, mid_sweeps - done_sw);
+                launch_blocked(pm, false, nullptr, s, em[cur_m], em[1 - cur_m], rm, bkm, nsw,
+                               oms / 2.f, oms / 3.f, oms / 4.f, ctx->fcg_zero.as<float>(), sd, 0,
+                               TrackArgs{});
                 cur_m = 1 - cur_m;
                 done_sw += nsw;
             }
@@ -2307,7 +2255,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     // sweeps does, the solve goes on (and a later stop is confirmed the same
     // way).  FP64 sweeps read b itself and stop at once.
     const bool confirm_stop = track && mixed;
-    const int confirm_sweeps = blocked ? BH / 2 : 4;
+    const int confirm_sweeps = blocked ? kStopGroup : 4;
     bool confirming = false;
     while (!done && cum < o->max_sweeps) {
         const int nsw = std::min(confirming ? confirm_sweeps : k, o->max_sweeps - cum);

@@ -103,70 +103,150 @@ __device__ __forceinline__ double lane_next(double v) {
 // ---------------------------------------------------------------------------
 // Max-update stop rule (solver.cpp:142) over launches of several sweeps.
 //
-// A launch leaves the largest |update| of each of its sweeps over the cells it
-// stores, per tile, in tmax (kTrackSweeps slots a tile; two such arrays,
-// alternating).  The next launch of the batch first reduces the previous
-// launch's array: the solve stops with the group of `group` sweeps that holds
-// the first sweep below tol.  If that group ends the previous launch there is
-// nothing left to do; otherwise the launch repeats the previous one from its
-// input, which the ping-pong still holds, up to the end of that group.  Every
-// workgroup reaches the same decision from the same array; the first one
-// records it (stop_lid: the launch that found the stop; launches after it
-// return at once, the workgroups of that launch itself do not look at it).
+// A tile of a launch leaves a word with bit j set when some cell it stores moved
+// by tol or more in the launch's sweep j, and the largest |update| of each sweep
+// (TrackOut; two of them, alternating).  The next launch of the batch ORs the
+// previous one's words: the solve stops with the group of `group` sweeps that
+// holds the first sweep whose bit is clear.  If that group ends the previous
+// launch there is nothing left to do; otherwise the launch repeats the previous
+// one from its input, which the ping-pong still holds, up to the end of that
+// group.  Every workgroup reaches the same decision from the same words; the
+// first one records it (stop_lid: the launch that found the stop; launches
+// after it return at once, the workgroups of that launch itself do not look at
+// it) with the largest update of the sweep.  The words are read beside the
+// region's loads, which the decision would otherwise hold back; a word shared
+// by all tiles (atomicOr) cost 0.6 us of a launch at 50 tiles and 9 us at 1000.
 // ---------------------------------------------------------------------------
-constexpr int kTrackSweeps = 16;  // most sweeps of a tracking launch
+constexpr int kTrackSlots = 16;   // floats of maxima per tile
+constexpr int kTrackSweeps = 15;  // most sweeps of a tracking launch
+
+struct TrackOut {
+    unsigned* bits;  // [ntiles]
+    float* maxima;   // [ntiles][kTrackSlots]
+};
+// bytes of two TrackOut for ntiles tiles, and their placement in `base`
+inline size_t track_bytes(int ntiles) { return 2 * (size_t)ntiles * 4 * (1 + kTrackSlots); }
+inline TrackOut track_out(void* base, int ntiles, int which) {
+    unsigned* u = static_cast<unsigned*>(base) + (size_t)which * ntiles * (1 + kTrackSlots);
+    return {u, reinterpret_cast<float*>(u + ntiles)};
+}
 
 struct TrackArgs {
-    float* tmax;        // this launch's array
-    const float* prev;  // the previous launch's array, null for a batch's first
-    int nprev;          // sweeps of the previous launch
-    int first_prev;     // sweeps of the solve before it
-    int group;          // sweeps the stop is rounded up to
-    int lid;            // launch number within the solve
-    int check_only;     // after a batch's last launch: decide, at most repeat it
+    TrackOut out;    // this launch's
+    TrackOut prev;   // the previous launch's, null for a batch's first
+    int nprev;       // sweeps of the previous launch
+    int first_prev;  // sweeps of the solve before it
+    int group;       // sweeps the stop is rounded up to
+    int lid;         // launch number within the solve
+    int check_only;  // after a batch's last launch: decide, at most repeat it
     double tol;
 };
 
-// The sweep decision of a tracking launch, the same in every workgroup.
+// The decision of a tracking launch, the same in every workgroup.
 struct TrackPlan {
     int nsweeps;  // sweeps to take (0: nothing to do)
     bool redo;    // from the previous launch's input to its output
 };
 
-// red: LDS of NW * kTrackSweeps floats.  All threads of the workgroup (64*NW)
-// must call it.
+// Reductions of a wave by DPP (row shifts, then row broadcasts): the result of
+// lane 63, in every lane.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned dpp_or0(unsigned v) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <typename Op>
+__device__ __forceinline__ unsigned wave_reduce(unsigned v, Op op) {
+    v = op(v, dpp_or0<0x111, 0xf>(v));
+    v = op(v, dpp_or0<0x112, 0xf>(v));
+    v = op(v, dpp_or0<0x114, 0xf>(v));
+    v = op(v, dpp_or0<0x118, 0xf>(v));
+    v = op(v, dpp_or0<0x142, 0xa>(v));
+    v = op(v, dpp_or0<0x143, 0xc>(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+    return wave_reduce(v, [](unsigned a, unsigned b) { return a | b; });
+}
+// largest of non-negative floats, which order like their bit patterns
+__device__ __forceinline__ float wave_max_pos(float v) {
+    return __uint_as_float(
+        wave_reduce(__float_as_uint(v), [](unsigned a, unsigned b) { return max(a, b); }));
+}
+
+// this thread's part of the previous launch's words
+template <int NW>
+__device__ __forceinline__ unsigned track_load(const TrackArgs& a, int ntiles) {
+    if (!a.prev.bits) return 0u;
+    // (the first load is unconditional, so that nothing waits for it here)
+    unsigned w = a.prev.bits[min((int)threadIdx.x, ntiles - 1)];
+    for (int i = threadIdx.x + 64 * NW; i < ntiles; i += 64 * NW) w |= a.prev.bits[i];
+    return w;
+}
+
+// words: track_load's; red: LDS of NW (<= 16) words.  All threads of the
+// workgroup (64*NW) must call it.
 template <int NW>
 __device__ __forceinline__ TrackPlan track_decide(const TrackArgs& a, SolveDev* st, int ntiles,
-                                                  int nsweeps, float* red) {
+                                                  int nsweeps, unsigned words, unsigned* red) {
+    static_assert(NW <= 16, "one row of lanes reads the waves' words");
     TrackPlan p{a.check_only ? 0 : nsweeps, false};
-    if (!a.prev) return p;
-    static_assert(kTrackSweeps == 16, "lane j of 16 takes sweep j");
-    float m = 0.f;
-    for (int i = threadIdx.x; i < ntiles * kTrackSweeps; i += 64 * NW) m = fmaxf(m, a.prev[i]);
-    m = fmaxf(m, __shfl_xor(m, 16, 64));
-    m = fmaxf(m, __shfl_xor(m, 32, 64));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane < kTrackSweeps) red[wave * kTrackSweeps + lane] = m;
+    if (st->stop_lid < a.lid) return TrackPlan{0, false};
+    if (!a.prev.bits) return p;
+    words = wave_or(words);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = words;
     __syncthreads();
-    float mj = lane < kTrackSweeps ? red[lane] : 0.f;
-    if (lane < kTrackSweeps)
-        for (int v = 1; v < NW; ++v) mj = fmaxf(mj, red[v * kTrackSweeps + lane]);
-    const unsigned long long below = __ballot(lane < a.nprev && (double)mj < a.tol);
-    const int stop = below ? __ffsll((long long)below) - 1 : -1;
-    const float last = __shfl(mj, stop >= 0 ? stop : a.nprev - 1, 64);
-    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-    if (first) st->last_max_update = (double)last;
+    const unsigned over = wave_or(red[min((int)threadIdx.x & 15, NW - 1)]);
+    const unsigned clear = ~over & ((1u << a.nprev) - 1u);
+    const int stop = clear ? __ffs((int)clear) - 1 : -1;
+    const int end = stop >= 0 ? min((stop / a.group + 1) * a.group, a.nprev) : 0;
     if (stop >= 0) {
-        const int end = min((stop / a.group + 1) * a.group, a.nprev);
         p.nsweeps = end < a.nprev ? end : 0;
         p.redo = true;
-        if (first) {
-            st->sweeps_at_done = a.first_prev + end;
-            st->done = 1;
-            __hip_atomic_store(&st->stop_lid, a.lid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (blockIdx.x == 0 && (stop >= 0 || a.check_only)) {
+        const int j = stop >= 0 ? stop : a.nprev - 1;
+        float m = 0.f;
+        for (int i = threadIdx.x; i < ntiles; i += 64 * NW)
+            m = fmaxf(m, a.prev.maxima[(size_t)i * kTrackSlots + j]);
+        m = wave_max_pos(m);
+        __syncthreads();  // red has been read
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = __float_as_uint(m);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int v = 1; v < NW; ++v) m = fmaxf(m, __uint_as_float(red[v]));
+            st->last_max_update = (double)m;
+            if (stop >= 0) {
+                st->sweeps_at_done = a.first_prev + end;
+                st->done = 1;
+                __hip_atomic_store(&st->stop_lid, a.lid, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
     }
     return p;
+}
+
+// The end of a tracking launch's workgroup: its tile's largest updates from
+// those of the lanes, one wave per sweep, and the tile's word.
+template <int NW>
+__device__ __forceinline__ void track_store(const TrackArgs& a, const float (*smax)[NW][64],
+                                            unsigned* red, int tile, int nsweeps, int wave,
+                                            int lane) {
+    __syncthreads();
+    unsigned over = 0u;
+    for (int j = wave; j < nsweeps; j += NW) {
+        float m = smax[j][0][lane];
+        for (int v = 1; v < NW; ++v) m = fmaxf(m, smax[j][v][lane]);
+        m = wave_max_pos(m);
+        if (lane == 0) a.out.maxima[(size_t)tile * kTrackSlots + j] = m;
+        if (!((double)m < a.tol)) over |= 1u << j;
+    }
+    if (lane == 0) red[wave] = over;
+    __syncthreads();
+    if (wave == 0) {
+        over = wave_or(red[min(lane & 15, NW - 1)]);
+        if (lane == 0) a.out.bits[tile] = over;
+    }
 }
 
 }  // namespace

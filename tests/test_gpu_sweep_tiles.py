@@ -2,8 +2,9 @@
 grids of one region, one cell more or less, odd sides, many tiles, several
 launches.  FP64 sweeps equal the oracle's red-black iterates to FP64 rounding;
 with holes (FP32 sweeps on an FP32 right-hand side) to FP32 rounding of the
-update; and a max-update stop inside a launch ends at the sweep at which the
-oracle stops."""
+update, on the bricked layout to the rounding of its right-hand side; and a
+max-update stop inside a launch ends at the sweep at which the oracle stops, or
+at the iterate of the same number of sweeps taken without a stop."""
 import numpy as np
 import pytest
 
@@ -73,3 +74,102 @@ def test_fp64_max_update_stops_at_the_oracle_sweep(ctx, oracle, rng, w, h):
         assert st.status == capi.OK and st.sweeps == rst.sweeps
         assert st.last_max_update < tol
         assert np.abs(g - ref).max() <= 1e-11 * np.abs(ref).max()
+
+
+def bf16(a):
+    u = np.asarray(a, dtype=np.float32).view(np.uint32).astype(np.uint64)
+    return ((((u + 0x7FFF + ((u >> 16) & 1)) >> 16) << 16).astype(np.uint32)).view(np.float32)
+
+
+def residual_rule_sweeps(b, p0, k, omega):
+    """One batch of k sweeps under the residual rule, restated in numpy: FP32 on a
+    correction e of p0, right-hand side the FP64 residual rounded to BF16, the
+    update v' = oc S + ((1 - omega) v + nq), nq = (mean - r) oc, with fused
+    multiply-adds (long double, rounded once to FP32)."""
+    h, w = b.shape
+    f32, ld = np.float32, np.longdouble
+    pad = lambda a: np.pad(a, 1)
+    one = pad(np.ones((h, w)))
+    nb = [(slice(1, -1), slice(0, -2)), (slice(0, -2), slice(1, -1)),   # left, up
+          (slice(1, -1), slice(2, None)), (slice(2, None), slice(1, -1))]  # right, down
+    cnt = sum(one[n] for n in nb)
+    q = pad(p0)
+    r = (b - b.mean()) - (((q[nb[0]] + q[nb[1]]) + q[nb[2]]) + q[nb[3]] - cnt * p0)
+    om = f32(omega)
+    oc = np.choose(4 - cnt.astype(int), [om / f32(4), om / f32(3), om / f32(2)])
+    nq = (f32(r.mean()) - bf16(r)) * oc
+    c1 = f32(1) - f32(4) * (om / f32(4))
+    fma = lambda a, x, c: (a.astype(ld) * x.astype(ld) + c.astype(ld)).astype(f32)
+    e = np.zeros((h, w), dtype=f32)
+    colour = np.add.outer(np.arange(h), np.arange(w)) & 1
+    for _ in range(k):
+        for c in (0, 1):
+            q = pad(e)
+            s = ((q[nb[0]] + q[nb[1]]) + q[nb[2]]) + q[nb[3]]
+            v = fma(oc, s, fma(np.full_like(e, c1), e, nq))
+            e = np.where(colour == c, v, e)
+    return p0 + e.astype(np.float64)
+
+
+# regions of 64, 96 and 128 rows; launches of 5 to 16 sweeps
+BLOCKED = SIZES + [(128, 96), (129, 97), (128, 128), (127, 129), (640, 1030), (1024, 700)]
+
+
+@pytest.mark.parametrize("w,h", BLOCKED)
+@pytest.mark.parametrize("k", [3, 16, 41])
+def test_blocked_sweeps_residual_rule(ctx, rng, w, h, k):
+    """The sweeps equal their restatement to a few FP32 roundings of the update
+    (the mean of r, about 1e-17, and ties of its BF16 rounding are all that can
+    differ; an indexing or ordering error is O(1))."""
+    b, _, p0 = make(rng, w, h, False)
+    o = capi.default_opts(max_sweeps=k, stop=capi.STOP_RESIDUAL, tol=0.0, omega=1.6,
+                          check_every=k)
+    g, st = ctx.poisson_solve(b, p0, o)
+    ref = residual_rule_sweeps(b, p0, k, 1.6)
+    assert st.sweeps == k
+    assert np.abs(g - ref).max() <= 2.0 ** -20 * np.abs(ref - p0).max(), (w, h)
+
+
+@pytest.mark.parametrize("w,h", BLOCKED)
+@pytest.mark.parametrize("k", [3, 16, 41])
+def test_blocked_sweeps_max_update_rule(ctx, oracle, rng, w, h, k):
+    """FP32 sweeps on an FP32 right-hand side: 2^-24 per operation, about 8
+    operations a sweep."""
+    b, _, p0 = make(rng, w, h, False)
+    o = capi.default_opts(max_sweeps=k, stop=capi.STOP_MAX_UPDATE, tol=0.0, omega=1.6,
+                          check_every=k)
+    g, st = ctx.poisson_solve(b, p0, o)
+    ref, _ = oracle.poisson_sor(b, p0, k, max_update_tol=1e-300, ordering=RED_BLACK, omega=1.6)
+    assert st.sweeps == k
+    scale = np.abs(ref - p0).max()
+    assert np.abs(g - ref).max() <= 8 * k * 2.0 ** -24 * scale, (w, h)
+
+
+@pytest.mark.parametrize("w,h", [(61, 40), (128, 64), (200, 136), (333, 129), (640, 520)])
+def test_max_update_stop_inside_a_launch_keeps_that_iterate(ctx, rng, w, h):
+    """The first sweep below the threshold, found from runs of 1, 2, ... sweeps,
+    ends the batch with its group of 5, wherever in a launch that falls: the
+    result is bit-equal to that many sweeps taken with no stop (tolerance 0) and
+    the 5 that confirm it (whatever the stop, the reported count is the
+    enqueued batch's)."""
+    b, _, p0 = make(rng, w, h, False)
+    kw = dict(stop=capi.STOP_MAX_UPDATE, omega=1.5)
+    mu = [np.inf]
+    while mu[-1] >= 1e-2 and len(mu) < 200:
+        n = len(mu)
+        _, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=0.0, check_every=n, max_sweeps=n,
+                                                           **kw))
+        mu.append(st.last_max_update)
+    stops = set()
+    for tol in np.geomspace(mu[3], min(mu) * 1.01, 12):
+        j = next(i for i, m in enumerate(mu) if m < tol)
+        s = (j + 4) // 5 * 5
+        g, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=tol, check_every=1000, **kw))
+        if st.checks != 3:
+            continue  # the confirming sweeps did not meet the rule: more batches follow
+        f, _ = ctx.poisson_solve(b, p0, capi.default_opts(tol=0.0, check_every=s, max_sweeps=s + 5,
+                                                          **kw))
+        assert st.status == capi.OK and st.last_max_update < tol
+        assert np.array_equal(f, g), (tol, j)
+        stops.add(s)
+    assert len(stops) >= 3
