@@ -470,67 +470,170 @@ __global__ __launch_bounds__(256) void k_conv_pair_tile(
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient dW[co][k] += sum_p gm[p][co] * xs[p][k], gm = g*(mask>0),
-// xs the 3x3-shifted (concatenated) input: MFMA with M = output channels,
-// N = k, reduction over pixels in steps of 32.  grid: (co blocks, k blocks,
-// pixel chunks); each wave reduces `ppw` pixels and adds its 16x16 tile with
-// FP32 atomics.
+// Weight gradient dW[co][tap*cin + ci] += sum_p gm[p][co] * x[p + tap][ci],
+// gm = g*(mask>0), x the (concatenated) input, zero outside the image: MFMA with
+// M = output channels, N = input channels of one tap, K = pixels.
+//
+// A workgroup (4 waves) stages an 8 x 32 pixel tile in LDS, channel-major so
+// that a fragment's 8 consecutive pixels of a row are 16 contiguous bytes: the
+// gradient of NCO*16 output channels rounded to BF16, and the input of NCI*16
+// channels with a one-pixel rim, its columns shifted by one so that tap dx = 0
+// starts aligned.  One 16-byte and one 4-byte read per input row then give the
+// fragments of all three dx (dx = 2 is the same words one dword on, dx = 1 a
+// 16-bit funnel shift).  Wave w takes 16 input channels (w % NCI), all 9 taps and
+// all NCO blocks, and every (4 / NCI)-th group of 4 x 8 pixels.  The waves'
+// sums meet in LDS and go out with FP32 atomics, one set per workgroup, after
+// as many tiles as the grid leaves it.
+//
+// Bound by the staging's LDS stores and loads (each input pixel is read once
+// per 32 output channels).  Gathering each fragment from global memory, element
+// by element with a division per pixel, took 97 us per convolution at 8 x 128 x
+// 128 (18 of them, 1.75 of the 2.16 ms of a training gradient).
+// grid: (workgroups over the tiles, ceil(cin / (16 NCI)), ceil(cg / (16 NCO))).
 // ---------------------------------------------------------------------------
+constexpr int WG_TR = 8, WG_TC = 32;             // tile rows, columns
+constexpr int WG_XROW = (WG_TC + 8) / 2;         // dwords per staged input row
+// dwords per channel, multiples of 4 with 8 channels' starts on distinct banks
+constexpr int WG_XCH = (WG_TR + 2) * WG_XROW + 4;
+constexpr int WG_GCH = WG_TR * WG_TC / 2 + 4;
+
+template <int NCI, int NCO>
 __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
                                                const u16* __restrict__ x2, int c1, int c2,
                                                const float* __restrict__ g,
                                                const u16* __restrict__ mask, int cg, int B,
                                                int H, int W, float* __restrict__ dw, int kpad,
-                                               int ppw) {
+                                               int tiles_x, int tiles_y) {
+    constexpr int KP = 4 / NCI;    // waves sharing 16 input channels
+    constexpr int XG = 2 * NCI;    // groups of 8 input channels
+    constexpr int XDW = NCI * 16 * WG_XCH + XG * 4, GDW = NCO * 16 * WG_GCH;
+    static_assert(NCI * 64 * 36 * NCO <= XDW + GDW, "the waves' sums fit the staging buffer");
+    __shared__ __align__(16) unsigned lds[XDW + GDW];
+    unsigned* xs = lds;
+    unsigned* gs = lds + XDW;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int co = blockIdx.x * 16 + (lane & 15);
-    const int kcol = blockIdx.y * 16 + (lane & 15);
+    const int cb = wave % NCI, kpart = wave / NCI;
     const int cin = c1 + c2;
-    const int K = 9 * cin;
-    const long long npix = (long long)B * H * W;
-    const long long pbeg = ((long long)blockIdx.z * 4 + wave) * ppw;
-    int tap = 0, ci = 0, dy = 0, dx = 0;
-    const bool kvalid = kcol < K;
-    if (kvalid) {
-        tap = kcol / cin;
-        ci = kcol - tap * cin;
-        dy = tap / 3 - 1;
-        dx = tap % 3 - 1;
-    }
-    const bool cvalid = co < cg;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (long long ps = pbeg; ps < pbeg + ppw && ps < npix; ps += 32) {
-        V8 a, b;
+    const int ci0 = blockIdx.y * NCI * 16, co0 = blockIdx.z * NCO * 16;
+    floatx4 acc[9][NCO];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const long long p = ps + 8 * (lane >> 4) + j;
-            float gv = 0.f;
-            u16 xv = 0;
-            if (p < npix) {
-                if (cvalid) {
-                    gv = g[p * cg + co];
-                    if (mask && !(from_bf16(mask[p * cg + co]) > 0.f)) gv = 0.f;
-                }
-                if (kvalid) {
-                    const int xx = (int)(p % W) + dx;
-                    const long long t = p / W;
-                    const int yy = (int)(t % H) + dy;
-                    if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
-                        const long long q = (t / H * H + yy) * W + xx;
-                        xv = ci < c1 ? x1[q * c1 + ci] : x2[q * c2 + (ci - c1)];
-                    }
-                }
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int m = 0; m < NCO; ++m) acc[t][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int ntiles = tiles_x * tiles_y * B;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, b = tile / (tiles_x * tiles_y);
+        const int xo = tx * WG_TC, yo = ty * WG_TR;
+        const long long img = (long long)b * H * W;
+        __syncthreads();  // the previous tile has been read
+        for (int it = threadIdx.x; it < (WG_TR + 2) * (WG_TC / 2 + 1) * XG; it += 256) {
+            const int gi = it % XG, t = it / XG;
+            const int pair = t % (WG_TC / 2 + 1), row = t / (WG_TC / 2 + 1);
+            const int ci = ci0 + gi * 8, yy = yo + row - 1, xx = xo + 2 * pair - 1;
+            const u16* src = ci < c1 ? x1 + ci : x2 + (ci - c1);
+            const int cs = ci < c1 ? c1 : c2;
+            const bool rok = ci < cin && yy >= 0 && yy < H;
+            V8 v[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                v[e].u = make_uint4(0, 0, 0, 0);
+                if (rok && xx + e >= 0 && xx + e < W)
+                    v[e].u = *reinterpret_cast<const uint4*>(src + (img + (long long)yy * W + xx + e) * cs);
             }
-            a.h[j] = to_bf16(gv);
-            b.h[j] = xv;
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc, 0, 0, 0);
-    }
+            unsigned* dst = xs + gi * (8 * WG_XCH + 4) + row * WG_XROW + pair;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int m = blockIdx.x * 16 + 4 * (lane >> 4) + r;  // output channel row of D
-        if (m < cg && kvalid) atomicAdd(dw + (size_t)m * kpad + kcol, acc[r]);
+            for (int e = 0; e < 8; ++e)
+                dst[e * WG_XCH] = (unsigned)v[0].h[e] | ((unsigned)v[1].h[e] << 16);
+        }
+        for (int it = threadIdx.x; it < WG_TR * (WG_TC / 2) * 4 * NCO; it += 256) {
+            const int q = it % (4 * NCO), t = it / (4 * NCO);
+            const int pair = t % (WG_TC / 2), row = t / (WG_TC / 2);
+            const int co = co0 + 4 * q, yy = yo + row, xx = xo + 2 * pair;
+            unsigned o[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (co >= cg || yy >= H || xx + e >= W) continue;
+                const long long p = (img + (long long)yy * W + xx + e) * cg + co;
+                const float4 gv = *reinterpret_cast<const float4*>(g + p);
+                float f[4] = {gv.x, gv.y, gv.z, gv.w};
+                if (mask) {
+                    const ushort4 mv = *reinterpret_cast<const ushort4*>(mask + p);
+                    const u16 m[4] = {mv.x, mv.y, mv.z, mv.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (!(from_bf16(m[k]) > 0.f)) f[k] = 0.f;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) o[k] |= (unsigned)to_bf16(f[k]) << (16 * e);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) gs[(4 * q + k) * WG_GCH + row * (WG_TC / 2) + pair] = o[k];
+        }
+        __syncthreads();
+        // this lane's channel of the input block
+        const int ch = cb * 16 + (lane & 15);
+        const unsigned* xc = xs + ch * WG_XCH + (ch >> 3) * 4;
+        const unsigned* gc = gs + (lane & 15) * WG_GCH;
+        for (int ks = kpart; ks < (WG_TR / 4) * (WG_TC / 8); ks += KP) {
+            const int row = (ks / (WG_TC / 8)) * 4 + (lane >> 4), col = (ks % (WG_TC / 8)) * 4;
+            V8 a[NCO];
+#pragma unroll
+            for (int m = 0; m < NCO; ++m)
+                a[m].u = *reinterpret_cast<const uint4*>(gc + m * 16 * WG_GCH + row * (WG_TC / 2) + col);
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+                const unsigned* xr = xc + (row + dy) * WG_XROW + col;
+                const uint4 d = *reinterpret_cast<const uint4*>(xr);
+                const unsigned d4 = xr[4];
+                V8 bx[3];
+                bx[0].u = d;
+                bx[1].u = make_uint4(__builtin_amdgcn_alignbit(d.y, d.x, 16),
+                                     __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                                     __builtin_amdgcn_alignbit(d.w, d.z, 16),
+                                     __builtin_amdgcn_alignbit(d4, d.w, 16));
+                bx[2].u = make_uint4(d.y, d.z, d.w, d4);
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                    for (int m = 0; m < NCO; ++m)
+                        acc[3 * dy + dx][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a[m].v, bx[dx].v, acc[3 * dy + dx][m], 0, 0, 0);
+            }
+        }
     }
+    // sum over the waves of an input block, one after the other
+    float* red = reinterpret_cast<float*>(lds) + (cb * 64 + lane);
+    for (int k = 1; k < KP; ++k) {
+        __syncthreads();
+        if (kpart == k)
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int m = 0; m < NCO; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        red[((t * NCO + m) * 4 + r) * NCI * 64] = acc[t][m][r];
+        __syncthreads();
+        if (kpart == 0)
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int m = 0; m < NCO; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[t][m][r] += red[((t * NCO + m) * 4 + r) * NCI * 64];
+    }
+    const int ci = ci0 + cb * 16 + (lane & 15);
+    if (kpart != 0 || ci >= cin) return;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int m = 0; m < NCO; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int co = co0 + m * 16 + 4 * (lane >> 4) + r;  // output channel row of D
+                if (co < cg) atomicAdd(dw + (size_t)co * kpad + t * cin + ci, acc[t][m][r]);
+            }
 }
 
 // ---- elementwise / pooling ---------------------------------------------------
@@ -1117,11 +1220,19 @@ int launch_wgrad(cd_net* n, const NetConv& cv, int B, int H, int W) {
     const u16* x2 = cv.in2 < 0 ? nullptr : n->t[cv.in2].act.as<u16>();
     const float* g = cv.out < 0 ? n->ghead.as<float>() : n->t[cv.out].grad.as<float>();
     const u16* mask = (cv.out >= 0 && cv.relu) ? n->t[cv.out].act.as<u16>() : nullptr;
-    const long long npix = (long long)B * H * W;
-    const int ppw = 1024;
-    dim3 grid(div_up(cv.coutA, 16), div_up(cv.K, 16), div_up(npix, 4LL * ppw));
-    hipLaunchKernelGGL(k_wgrad, grid, dim3(256), 0, c->stream, x1, x2, cv.c1, cv.c2, g, mask,
-                       cv.coutA, B, H, W, n->gw.as<float>() + cv.woff, cv.kpad, ppw);
+    const int cin = cv.c1 + cv.c2;
+    const int nci = div_up(cin, 16) % 2 == 0 ? 2 : 1, nco = cv.coutA > 16 ? 2 : 1;
+    const int tx = div_up(W, WG_TC), ty = div_up(H, WG_TR);
+    const int gy = div_up(cin, 16 * nci), gz = div_up(cv.coutA, 16 * nco);
+    // about three workgroups per CU (their LDS), each over several tiles where
+    // the image has more: fewer atomics
+    const int gx = std::min(tx * ty * B, std::max(1, 768 / (gy * gz)));
+#define WGRAD(CI, CO) hipLaunchKernelGGL((k_wgrad<CI, CO>), dim3(gx, gy, gz), dim3(256), 0, c->stream, x1, x2, cv.c1, cv.c2, g, mask, cv.coutA, B, H, W, n->gw.as<float>() + cv.woff, cv.kpad, tx, ty)
+    if (nci == 1 && nco == 1) WGRAD(1, 1);
+    else if (nci == 1) WGRAD(1, 2);
+    else if (nco == 1) WGRAD(2, 1);
+    else WGRAD(2, 2);
+#undef WGRAD
     CD_CHECK_LAUNCH(c);
     return CD_OK;
 }
