@@ -46,8 +46,7 @@ union V8 {
 //   IN 0: BF16 input = channel concatenation of x1 (c1 ch) and x2 (c2 ch)
 //   IN 1: FP32 input g (c1 ch), multiplied by (mask > 0) when mask != NULL
 //   OUT 0: BF16 output (cy ch), optional ReLU
-//   OUT 1: FP32 output split by channel into y1 (cy ch) and y2 (cy2 ch),
-//          optionally accumulated
+//   OUT 1: FP32 output split by channel into y1 (cy ch) and y2 (cy2 ch)
 // wt: BF16 weights [nb*16][kpad], kpad a multiple of 32, zero padded.
 // One workgroup = 4 waves = 64 consecutive pixels; a wave computes 16 pixels
 // by NB*16 output channels.
@@ -60,8 +59,7 @@ __global__ __launch_bounds__(256) void k_conv3x3(const u16* __restrict__ x1,
                                                  const u16* __restrict__ wt, int kpad, int B,
                                                  int H, int W, u16* __restrict__ ybf,
                                                  float* __restrict__ y1, float* __restrict__ y2,
-                                                 int cy, int cy2, int relu, int accumulate,
-                                                 int mode1) {
+                                                 int cy, int cy2, int relu, int mode1) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const long long npix = (long long)B * H * W;
     const long long p0 = (long long)blockIdx.x * 64 + wave * 16;
@@ -162,7 +160,7 @@ __global__ __launch_bounds__(256) void k_conv3x3(const u16* __restrict__ x1,
                 float* dst = nullptr;
                 if (ch < cy) dst = y1 + p * cy + ch;
                 else if (ch - cy < cy2) dst = y2 + p * cy2 + (ch - cy);
-                if (dst) *dst = accumulate ? *dst + v : v;
+                if (dst) *dst = v;
             }
         }
     }
@@ -178,7 +176,9 @@ __global__ __launch_bounds__(256) void k_conv3x3(const u16* __restrict__ x1,
 // so every output is bit-identical to it; the tiles cut the latency chain of
 // the per-chunk global gathers, which sets the time of these small layers.
 //   OUT 0: BF16 output ybf [B][H][W][cy] (ReLU optional);
-//   OUT 1: FP32 output yf [B][H][W][cy].
+//   OUT 1: FP32 output yf [B][H][W][cy]; OUT 2: yf (cy ch) and y2 (cy2 ch).
+//   IN 1: FP32 gradient g (c1 ch, masked) in place of x1, x2, for the input
+//   gradient (transposed weights), as k_conv3x3<NB, 1, 1>.
 // grid: (ceil(W/8), ceil(H/8), B * cblocks), output channels
 // [16*NB*cblk, 16*NB*(cblk+1)) with cblk = blockIdx.z % cblocks.
 // LDS: 100 * (cin + 8) + NB*16 * (kpad + 8) u16 (row paddings spread banks).
@@ -252,6 +252,51 @@ __device__ __forceinline__ void stage_patch(u16* __restrict__ xs, int xstride,
             if (px < NP)
                 *reinterpret_cast<uint4*>(xs + px * xstride + ci) =
                     ok[u] ? v[u] : make_uint4(0, 0, 0, 0);
+        }
+    }
+}
+
+// The same for an FP32 gradient g of c channels, rounded to BF16 and zeroed where
+// mask (NULL: none) is not positive, as k_conv3x3 with IN 1 reads it.
+template <int P>
+__device__ __forceinline__ void stage_grad(u16* __restrict__ xs, int xstride,
+                                           const float* __restrict__ g,
+                                           const u16* __restrict__ mask, int c, int H, int W,
+                                           int b, int oy, int ox) {
+    constexpr int SB = 4;
+    constexpr int NP = P * P;
+    const int ng = c >> 3;
+    const int pstride = 256 / ng;
+    const int ci = (threadIdx.x % ng) * 8;
+    if (threadIdx.x >= pstride * ng) return;
+    for (int pb = threadIdx.x / ng; pb < NP; pb += SB * pstride) {
+        float4 v0[SB], v1[SB];
+        V8 m[SB];
+        bool ok[SB];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+            const int px = pb + u * pstride;
+            const int yy = oy + px / P, xx = ox + px % P;
+            ok[u] = px < NP && yy >= 0 && yy < H && xx >= 0 && xx < W;
+            const long long q = (((long long)b * H + min(max(yy, 0), H - 1)) * W +
+                                 min(max(xx, 0), W - 1)) * c + ci;
+            v0[u] = *reinterpret_cast<const float4*>(g + q);
+            v1[u] = *reinterpret_cast<const float4*>(g + q + 4);
+            if (mask) m[u].u = *reinterpret_cast<const uint4*>(mask + q);
+        }
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+            const int px = pb + u * pstride;
+            if (px >= NP) continue;
+            const float gv[8] = {v0[u].x, v0[u].y, v0[u].z, v0[u].w,
+                                 v1[u].x, v1[u].y, v1[u].z, v1[u].w};
+            V8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool on = ok[u] && !(mask && !(from_bf16(m[u].h[e]) > 0.f));
+                o.h[e] = on ? to_bf16(gv[e]) : (u16)0;
+            }
+            *reinterpret_cast<uint4*>(xs + px * xstride + ci) = o.u;
         }
     }
 }
@@ -335,13 +380,17 @@ __device__ __forceinline__ void conv_lds(floatx4 (&acc)[MT][NB], const u16* __re
     }
 }
 
-template <int NB, int OUT>
+template <int NB, int OUT, int IN = 0>
 __global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1,
                                                       const u16* __restrict__ x2, int c1, int c2,
                                                       const u16* __restrict__ wt, int kpad, int H,
                                                       int W, int cblocks, u16* __restrict__ ybf,
                                                       float* __restrict__ yf, int cy, int relu,
-                                                      int mode1) {
+                                                      int mode1,
+                                                      const float* __restrict__ g = nullptr,
+                                                      const u16* __restrict__ mask = nullptr,
+                                                      float* __restrict__ y2 = nullptr,
+                                                      int cy2 = 0) {
     extern __shared__ uint4 tile_lds[];
     u16* xs = reinterpret_cast<u16*>(tile_lds);
     const int cin = c1 + c2;
@@ -349,7 +398,10 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1
     u16* ws = xs + 100 * xstride;                     // 16-byte aligned: xstride % 8 == 0
     const int cblk = blockIdx.z % cblocks, b = blockIdx.z / cblocks;
     const int tx0 = blockIdx.x * CT, ty0 = blockIdx.y * CT;
-    stage_patch<10>(xs, xstride, x1, x2, c1, c2, H, W, b, ty0 - 1, tx0 - 1, mode1);
+    if (IN == 0)
+        stage_patch<10>(xs, xstride, x1, x2, c1, c2, H, W, b, ty0 - 1, tx0 - 1, mode1);
+    else
+        stage_grad<10>(xs, xstride, g, mask, c1, H, W, b, ty0 - 1, tx0 - 1);
     stage_weights(ws, wt + (size_t)cblk * NB * 16 * kpad, NB * 16, kpad);
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -367,14 +419,16 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1
             const int row = 4 * (lane >> 4) + r;
             const int yy = ty0 + 2 * wave + (row >> 3), xx = tx0 + (row & 7);
             const int ch = (cblk * NB + nb) * 16 + (lane & 15);
-            if (yy >= H || xx >= W || ch >= cy) continue;
+            if (yy >= H || xx >= W || ch >= cy + (OUT == 2 ? cy2 : 0)) continue;
             const long long p = ((long long)b * H + yy) * W + xx;
             float v = acc[nb][r];
             if (OUT == 0) {
                 if (relu) v = fmaxf(v, 0.f);
                 ybf[p * cy + ch] = to_bf16(v);
-            } else {
+            } else if (OUT == 1 || ch < cy) {
                 yf[p * cy + ch] = v;
+            } else {
+                y2[p * cy2 + ch - cy] = v;
             }
         }
     }
@@ -488,7 +542,7 @@ __global__ __launch_bounds__(256) void k_conv_pair_tile(
 // Bound by the staging's LDS stores and loads (each input pixel is read once
 // per 32 output channels).  Gathering each fragment from global memory, element
 // by element with a division per pixel, took 97 us per convolution at 8 x 128 x
-// 128 (18 of them, 1.75 of the 2.16 ms of a training gradient).
+// 128 (18 of them, 1.75 of the 2.16 ms of a training gradient); 16 us now.
 // grid: (workgroups over the tiles, ceil(cin / (16 NCI)), ceil(cg / (16 NCO))).
 // ---------------------------------------------------------------------------
 constexpr int WG_TR = 8, WG_TC = 32;             // tile rows, columns
@@ -526,45 +580,71 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
         const int xo = tx * WG_TC, yo = ty * WG_TR;
         const long long img = (long long)b * H * W;
         __syncthreads();  // the previous tile has been read
-        for (int it = threadIdx.x; it < (WG_TR + 2) * (WG_TC / 2 + 1) * XG; it += 256) {
+        // all of a thread's loads are issued before its first LDS store
+        constexpr int XN = (WG_TR + 2) * (WG_TC / 2 + 1) * XG, XIT = (XN + 255) / 256;
+        constexpr int GN = WG_TR * (WG_TC / 2) * 4 * NCO, GIT = GN / 256;
+        static_assert(GN % 256 == 0, "whole rounds");
+        V8 xv[XIT][2];
+        float4 gv[GIT][2];
+        ushort4 mv[GIT][2];
+#pragma unroll
+        for (int u = 0; u < XIT; ++u) {
+            const int it = threadIdx.x + 256 * u;
             const int gi = it % XG, t = it / XG;
             const int pair = t % (WG_TC / 2 + 1), row = t / (WG_TC / 2 + 1);
             const int ci = ci0 + gi * 8, yy = yo + row - 1, xx = xo + 2 * pair - 1;
             const u16* src = ci < c1 ? x1 + ci : x2 + (ci - c1);
             const int cs = ci < c1 ? c1 : c2;
-            const bool rok = ci < cin && yy >= 0 && yy < H;
-            V8 v[2];
+            const bool rok = it < XN && ci < cin && yy >= 0 && yy < H;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                v[e].u = make_uint4(0, 0, 0, 0);
+                xv[u][e].u = make_uint4(0, 0, 0, 0);
                 if (rok && xx + e >= 0 && xx + e < W)
-                    v[e].u = *reinterpret_cast<const uint4*>(src + (img + (long long)yy * W + xx + e) * cs);
+                    xv[u][e].u = *reinterpret_cast<const uint4*>(
+                        src + (img + (long long)yy * W + xx + e) * cs);
             }
-            unsigned* dst = xs + gi * (8 * WG_XCH + 4) + row * WG_XROW + pair;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                dst[e * WG_XCH] = (unsigned)v[0].h[e] | ((unsigned)v[1].h[e] << 16);
         }
-        for (int it = threadIdx.x; it < WG_TR * (WG_TC / 2) * 4 * NCO; it += 256) {
+#pragma unroll
+        for (int u = 0; u < GIT; ++u) {
+            const int it = threadIdx.x + 256 * u;
             const int q = it % (4 * NCO), t = it / (4 * NCO);
             const int pair = t % (WG_TC / 2), row = t / (WG_TC / 2);
             const int co = co0 + 4 * q, yy = yo + row, xx = xo + 2 * pair;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                gv[u][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+                mv[u][e] = make_ushort4(0x3f80, 0x3f80, 0x3f80, 0x3f80);  // 1.0: not masked
+                if (co < cg && yy < H && xx + e < W) {
+                    const long long p = (img + (long long)yy * W + xx + e) * cg + co;
+                    gv[u][e] = *reinterpret_cast<const float4*>(g + p);
+                    if (mask) mv[u][e] = *reinterpret_cast<const ushort4*>(mask + p);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < XIT; ++u) {
+            const int it = threadIdx.x + 256 * u;
+            const int gi = it % XG, t = it / XG;
+            const int pair = t % (WG_TC / 2 + 1), row = t / (WG_TC / 2 + 1);
+            if (it >= XN) continue;
+            unsigned* dst = xs + gi * (8 * WG_XCH + 4) + row * WG_XROW + pair;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                dst[e * WG_XCH] = (unsigned)xv[u][0].h[e] | ((unsigned)xv[u][1].h[e] << 16);
+        }
+#pragma unroll
+        for (int u = 0; u < GIT; ++u) {
+            const int it = threadIdx.x + 256 * u;
+            const int q = it % (4 * NCO), t = it / (4 * NCO);
+            const int pair = t % (WG_TC / 2), row = t / (WG_TC / 2);
             unsigned o[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                if (co >= cg || yy >= H || xx + e >= W) continue;
-                const long long p = (img + (long long)yy * W + xx + e) * cg + co;
-                const float4 gv = *reinterpret_cast<const float4*>(g + p);
-                float f[4] = {gv.x, gv.y, gv.z, gv.w};
-                if (mask) {
-                    const ushort4 mv = *reinterpret_cast<const ushort4*>(mask + p);
-                    const u16 m[4] = {mv.x, mv.y, mv.z, mv.w};
+                const float f[4] = {gv[u][e].x, gv[u][e].y, gv[u][e].z, gv[u][e].w};
+                const u16 m[4] = {mv[u][e].x, mv[u][e].y, mv[u][e].z, mv[u][e].w};
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (!(from_bf16(m[k]) > 0.f)) f[k] = 0.f;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) o[k] |= (unsigned)to_bf16(f[k]) << (16 * e);
+                for (int k = 0; k < 4; ++k)
+                    if (from_bf16(m[k]) > 0.f) o[k] |= (unsigned)to_bf16(f[k]) << (16 * e);
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) gs[(4 * q + k) * WG_GCH + row * (WG_TC / 2) + pair] = o[k];
@@ -709,7 +789,7 @@ __global__ void k_upsample2(const u16* __restrict__ x, u16* __restrict__ y, int 
     y[i] = x[(((long long)b * (H / 2) + yy / 2) * (W / 2) + xx / 2) * C + c];
 }
 
-// dx[coarse] += sum of the 4 fine gradients
+// dx[coarse] = sum of the 4 fine gradients
 __global__ void k_upsample2_bwd(const float* __restrict__ dy, float* __restrict__ dx, int B, int H,
                                 int W, int C) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -723,7 +803,7 @@ __global__ void k_upsample2_bwd(const float* __restrict__ dy, float* __restrict_
     const int yo = (int)(t % Ho);
     const int b = (int)(t / Ho);
     const long long base = (((long long)b * H + 2 * yo) * W + 2 * xo) * C + c;
-    dx[i] += dy[base] + dy[base + C] + dy[base + (long long)W * C] + dy[base + (long long)W * C + C];
+    dx[i] = dy[base] + dy[base + C] + dy[base + (long long)W * C] + dy[base + (long long)W * C + C];
 }
 
 // supervised loss on the output y (FP32 [npix]): partial sums of (y - t)^2
@@ -1091,6 +1171,8 @@ size_t tiled_lds_limit(cd_context* c) {
     const void* fns[] = {reinterpret_cast<const void*>(&k_conv3x3_tile<1, 0>),
                          reinterpret_cast<const void*>(&k_conv3x3_tile<2, 0>),
                          reinterpret_cast<const void*>(&k_conv3x3_tile<1, 1>),
+                         reinterpret_cast<const void*>(&k_conv3x3_tile<1, 2, 1>),
+                         reinterpret_cast<const void*>(&k_conv3x3_tile<2, 2, 1>),
                          reinterpret_cast<const void*>(&k_conv_pair_tile<1, 1>),
                          reinterpret_cast<const void*>(&k_conv_pair_tile<2, 2>),
                          reinterpret_cast<const void*>(&k_head_smooth<6>)};
@@ -1172,13 +1254,13 @@ int launch_conv(cd_net* n, const NetConv& cv, int B, int H, int W, bool grad_inp
         const u16* wt = n->wbf.as<u16>() + cv.woff;
         const int nb = cv.coutpad / 16;
         if (cv.out < 0) {  // head: FP32 output [npix][8]
-#define CONV_F(NB) hipLaunchKernelGGL((k_conv3x3<NB, 0, 1>), dim3(blocks), dim3(256), 0, s, x1, x2, cv.c1, cv.c2, (const float*)nullptr, (const u16*)nullptr, wt, cv.kpad, B, H, W, (u16*)nullptr, n->head.as<float>(), (float*)nullptr, 8, 0, 0, 0, mode1)
+#define CONV_F(NB) hipLaunchKernelGGL((k_conv3x3<NB, 0, 1>), dim3(blocks), dim3(256), 0, s, x1, x2, cv.c1, cv.c2, (const float*)nullptr, (const u16*)nullptr, wt, cv.kpad, B, H, W, (u16*)nullptr, n->head.as<float>(), (float*)nullptr, 8, 0, 0, mode1)
             if (nb == 1) CONV_F(1);
             else return CD_ERR_BAD_ARG;
 #undef CONV_F
         } else {
             u16* y = n->t[cv.out].act.as<u16>();
-#define CONV_B(NB) hipLaunchKernelGGL((k_conv3x3<NB, 0, 0>), dim3(blocks), dim3(256), 0, s, x1, x2, cv.c1, cv.c2, (const float*)nullptr, (const u16*)nullptr, wt, cv.kpad, B, H, W, y, (float*)nullptr, (float*)nullptr, cv.coutA, 0, cv.relu, 0, mode1)
+#define CONV_B(NB) hipLaunchKernelGGL((k_conv3x3<NB, 0, 0>), dim3(blocks), dim3(256), 0, s, x1, x2, cv.c1, cv.c2, (const float*)nullptr, (const u16*)nullptr, wt, cv.kpad, B, H, W, y, (float*)nullptr, (float*)nullptr, cv.coutA, 0, cv.relu, mode1)
             switch (nb) {
                 case 1: CONV_B(1); break;
                 case 2: CONV_B(2); break;
@@ -1198,7 +1280,22 @@ int launch_conv(cd_net* n, const NetConv& cv, int B, int H, int W, bool grad_inp
         float* d1 = n->t[cv.in1].grad.as<float>();
         float* d2 = cv.in2 < 0 ? nullptr : n->t[cv.in2].grad.as<float>();
         const int nb = cv.cinpad / 16;
-#define CONV_G(NB) hipLaunchKernelGGL((k_conv3x3<NB, 1, 1>), dim3(blocks), dim3(256), 0, s, (const u16*)nullptr, (const u16*)nullptr, cv.coutA, 0, g, mask, wt, cv.kpadT, B, H, W, (u16*)nullptr, d1, d2, cv.c1, cv.c2, 0, 1, 0)
+        // on tiles where their LDS allows, as the forward convolutions: 9 to 25 us
+        // by per-chunk global gathers, 5 to 7 on tiles at 8 x 128 x 128
+        const int nbg = nb % 2 == 0 && tiles_t * (nb / 2) >= kConvWideMinBlocks ? 2 : 1;
+        const size_t lds_g = sizeof(u16) * (100 * (size_t)(cv.coutA + 8) +
+                                            (size_t)nbg * 16 * (cv.kpadT + 8));
+        if (cv.coutA <= 256 && lds_g <= tiled_lds_limit(c)) {
+            const int cblocks = nb / nbg;
+            const dim3 grid(div_up(W, CT), div_up(H, CT), B * cblocks);
+            auto kernel = nbg == 2 ? k_conv3x3_tile<2, 2, 1> : k_conv3x3_tile<1, 2, 1>;
+            hipLaunchKernelGGL(kernel, grid, dim3(256), lds_g, s, (const u16*)nullptr,
+                               (const u16*)nullptr, cv.coutA, 0, wt, cv.kpadT, H, W, cblocks,
+                               (u16*)nullptr, d1, cv.c1, 0, 0, g, mask, d2, cv.c2);
+            CD_CHECK_LAUNCH(c);
+            return CD_OK;
+        }
+#define CONV_G(NB) hipLaunchKernelGGL((k_conv3x3<NB, 1, 1>), dim3(blocks), dim3(256), 0, s, (const u16*)nullptr, (const u16*)nullptr, cv.coutA, 0, g, mask, wt, cv.kpadT, B, H, W, (u16*)nullptr, d1, d2, cv.c1, cv.c2, 0, 0)
         switch (nb) {
             case 1: CONV_G(1); break;
             case 2: CONV_G(2); break;
@@ -1224,9 +1321,10 @@ int launch_wgrad(cd_net* n, const NetConv& cv, int B, int H, int W) {
     const int nci = div_up(cin, 16) % 2 == 0 ? 2 : 1, nco = cv.coutA > 16 ? 2 : 1;
     const int tx = div_up(W, WG_TC), ty = div_up(H, WG_TR);
     const int gy = div_up(cin, 16 * nci), gz = div_up(cv.coutA, 16 * nco);
-    // about three workgroups per CU (their LDS), each over several tiles where
-    // the image has more: fewer atomics
-    const int gx = std::min(tx * ty * B, std::max(1, 768 / (gy * gz)));
+    // up to 1.5 workgroups per CU, each over several tiles where the image has
+    // more: fewer atomics (768 to 3072 workgroups 20 us against 16 at 8 x 128 x
+    // 128, 48 to 16 channels)
+    const int gx = std::min(tx * ty * B, std::max(1, 384 / (gy * gz)));
 #define WGRAD(CI, CO) hipLaunchKernelGGL((k_wgrad<CI, CO>), dim3(gx, gy, gz), dim3(256), 0, c->stream, x1, x2, cv.c1, cv.c2, g, mask, cv.coutA, B, H, W, n->gw.as<float>() + cv.woff, cv.kpad, tx, ty)
     if (nci == 1 && nco == 1) WGRAD(1, 1);
     else if (nci == 1) WGRAD(1, 2);
@@ -1471,13 +1569,12 @@ int forward(cd_net* n, int B, int H, int W, bool fused = false) {
     return CD_OK;
 }
 
-// backward pass: n->ghead holds dL/dhead; accumulates n->gw
+// backward pass: n->ghead holds dL/dhead; accumulates n->gw.  A tensor's first
+// gradient is stored, so that none needs zeroing (21 launches): every tensor has
+// one consumer but the skips, whose decoder convolution comes before their
+// pooling here, and only the pooling adds.
 int backward(cd_net* n, int B, int H, int W) {
     cd_context* c = n->ctx;
-    for (auto& t : n->t) {
-        const long long px = (long long)B * (H >> t.level) * (W >> t.level);
-        CD_TRY(zero(c, t.grad.as<float>(), px * t.C));
-    }
     const int L = n->arch.levels;
     for (int idx = (int)n->convs.size() - 1; idx >= 0; --idx) {
         const NetConv& cv = n->convs[idx];
