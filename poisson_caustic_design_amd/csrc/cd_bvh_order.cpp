@@ -18,6 +18,9 @@
 #include <cfloat>
 #include <cmath>
 #include <limits>
+#include <new>
+#include <system_error>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -27,12 +30,28 @@ namespace {
 
 constexpr int kLeafSize = 5;   // build_target_bvh(5, 30), mesh.cpp:235
 constexpr int kMaxDepth = 30;
+// Ranges of at least kParallel triangles at the first kParallelDepth levels take
+// a thread for one half (at most 7 more): a thread costs about 20 us, the build
+// of 8192 triangles about 500.
+constexpr int kParallel = 8192;
+constexpr int kParallelDepth = 3;
+
+// A triangle as the build sees it; the array is permuted with the ids, so that
+// every pass over a range reads memory in order.
+struct Tri {
+    double c[2];           // centroid
+    double mn[2], mx[2];   // bounding box of the vertices
+    int id;
+};
+
+// std::fmin / std::fmax against a bound that is never NaN: a NaN v keeps it.
+inline double lower(double bound, double v) { return v < bound ? v : bound; }
+inline double upper(double bound, double v) { return v > bound ? v : bound; }
 
 struct OrderBuilder {
     const double* xy;
     int mx, T;
-    std::vector<double> cx, cy;  // centroids, permuted with the ids
-    int* ids;
+    std::vector<Tri> tri;
 
     void vertices(int t, int v[3]) const {  // mesh.cpp:57-63
         const int cell = t >> 1, cw = mx - 1;
@@ -42,10 +61,12 @@ struct OrderBuilder {
     }
 
     // area-weighted polygon centroid, polygon_utils.cpp:238-263 (a triangle
-    // of zero area yields non-finite coordinates there as here)
-    void centroid(int t, double& ox, double& oy) const {
+    // of zero area yields non-finite coordinates there as here), and the box
+    Tri triangle(int t) const {
         int v[3];
         vertices(t, v);
+        const double inf = std::numeric_limits<double>::infinity();
+        Tri r{{0.0, 0.0}, {inf, inf}, {-inf, -inf}, t};
         double sa = 0.0, sx = 0.0, sy = 0.0;
         for (int k = 0; k < 3; ++k) {
             const double x0 = xy[2 * v[k]], y0 = xy[2 * v[k] + 1];
@@ -54,60 +75,72 @@ struct OrderBuilder {
             sa += a;
             sx += (x0 + x1) * a;
             sy += (y0 + y1) * a;
+            r.mn[0] = lower(r.mn[0], x0);
+            r.mn[1] = lower(r.mn[1], y0);
+            r.mx[0] = upper(r.mx[0], x0);
+            r.mx[1] = upper(r.mx[1], y0);
         }
         sa *= 0.5;
-        ox = sx / (6 * sa);
-        oy = sy / (6 * sa);
+        r.c[0] = sx / (6 * sa);
+        r.c[1] = sy / (6 * sa);
+        return r;
     }
 
-    // two-sided partition of bvh.cpp:50-76; the split value arrives as float
-    int split(int start, int end, int dim, float split_value) {
+    // two-sided partition of bvh.cpp:50-76; the split value arrives as float.
+    // next: the centroid coordinate after the range's last entry.
+    int split(int start, int end, int dim, float split_value, double next) {
         const double s = split_value;
-        std::vector<double>& c = dim ? cy : cx;
+        Tri* t = tri.data();
         int left = start, right = end - 1;
         while (left < right) {
-            while (left < end && c[left] < s) ++left;
-            while (right >= start && c[right] >= s) --right;
+            while (left < end && t[left].c[dim] < s) ++left;
+            while (right >= start && t[right].c[dim] >= s) --right;
             if (left >= right) break;
-            std::swap(cx[left], cx[right]);
-            std::swap(cy[left], cy[right]);
-            std::swap(ids[left], ids[right]);
+            std::swap(t[left], t[right]);
             ++left;
             --right;
         }
-        // the reference reads the centroid at `left` even when left == end:
-        // inside the array that is the next range's first entry; past its
-        // end (undefined there) it is taken as not below the split value
-        const double cl = left < T ? c[left] : std::numeric_limits<double>::quiet_NaN();
+        // the reference reads the centroid at `left` even when left == end
+        const double cl = left < end ? t[left].c[dim] : next;
         return cl <= s ? std::min(end, left + 1) : left;
     }
 
-    void node(int start, int end, int level) {
-        double mnx = std::numeric_limits<double>::infinity(), mny = mnx;
-        double mxx = -mnx, mxy = -mnx;
-        for (int i = start; i < end; ++i) {
-            int v[3];
-            vertices(ids[i], v);
-            for (int k = 0; k < 3; ++k) {
-                const double x = xy[2 * v[k]], y = xy[2 * v[k] + 1];
-                mnx = std::fmin(mnx, x);
-                mny = std::fmin(mny, y);
-                mxx = std::fmax(mxx, x);
-                mxy = std::fmax(mxy, y);
+    // next: the centroid of the entry after the range.  The walk takes the
+    // first half before the second, so while a range is being partitioned that
+    // entry is the one its ancestors' splits put there: a value of the call,
+    // which lets the halves go in parallel.  Past the array's end (undefined in
+    // the reference) it is NaN, not below any split value.
+    void node(int start, int end, int level, const double next[2]) {
+        const double inf = std::numeric_limits<double>::infinity();
+        double mn[2] = {inf, inf}, mx_[2] = {-inf, -inf};
+        if (end - start <= kLeafSize || level >= kMaxDepth) return;
+        for (int i = start; i < end; ++i)
+            for (int d = 0; d < 2; ++d) {
+                mn[d] = lower(mn[d], tri[i].mn[d]);
+                mx_[d] = upper(mx_[d], tri[i].mx[d]);
+            }
+        for (int d = 0; d < 2; ++d) {
+            mn[d] -= 0.5 * DBL_EPSILON;
+            mx_[d] += 0.5 * DBL_EPSILON;
+        }
+        const int dim = (mx_[0] - mn[0]) < (mx_[1] - mn[1]) ? 1 : 0;
+        const int m = split(start, end, dim, (float)(0.5 * (mx_[dim] + mn[dim])), next[dim]);
+        if (m == start || m == end) return;
+        const double mid[2] = {tri[m].c[0], tri[m].c[1]};
+        if (end - start >= kParallel && level < kParallelDepth) {
+            std::thread first;
+            try {
+                first = std::thread([&] { node(start, m, level + 1, mid); });
+            } catch (const std::system_error&) {  // no thread to be had: one after the other
+            }
+            if (first.joinable()) {
+                node(m, end, level + 1, next);
+                first.join();
+                return;
             }
         }
-        const double eps = DBL_EPSILON;
-        mnx -= 0.5 * eps;
-        mny -= 0.5 * eps;
-        mxx += 0.5 * eps;
-        mxy += 0.5 * eps;
-        if (end - start <= kLeafSize || level >= kMaxDepth) return;
-        const int dim = (mxx - mnx) < (mxy - mny) ? 1 : 0;
-        const double mid = dim == 0 ? 0.5 * (mxx + mnx) : 0.5 * (mxy + mny);
-        const int m = split(start, end, dim, (float)mid);
-        if (m == start || m == end) return;
-        node(start, m, level + 1);
-        node(m, end, level + 1);
+        node(start, m, level + 1, mid);
+        node(m, end, level + 1, next);
     }
 };
 
@@ -117,13 +150,15 @@ extern "C" int cd_bvh_first_hit_order(const double* xy, int mx, int my, int* ord
     if (!xy || !order || mx < 2 || my < 2) return CD_ERR_BAD_ARG;
     const long long T = 2LL * (mx - 1) * (my - 1);
     if (T > (long long)std::numeric_limits<int>::max() / 2) return CD_ERR_BAD_ARG;
-    OrderBuilder b{xy, mx, (int)T, {}, {}, order};
-    b.cx.resize(T);
-    b.cy.resize(T);
-    for (int t = 0; t < (int)T; ++t) {
-        order[t] = t;
-        b.centroid(t, b.cx[t], b.cy[t]);
+    try {
+        OrderBuilder b{xy, mx, (int)T, {}};
+        b.tri.reserve((size_t)T);
+        for (int t = 0; t < (int)T; ++t) b.tri.push_back(b.triangle(t));
+        const double nan = std::numeric_limits<double>::quiet_NaN(), past[2] = {nan, nan};
+        b.node(0, (int)T, 0, past);
+        for (int t = 0; t < (int)T; ++t) order[t] = b.tri[t].id;
+    } catch (const std::bad_alloc&) {
+        return CD_ERR_OOM;
     }
-    b.node(0, (int)T, 0);
     return CD_OK;
 }
