@@ -7,6 +7,7 @@
 #include <chrono>
 #include <climits>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <system_error>
 #include <thread>
@@ -801,6 +802,9 @@ int finish(cd_design* d, int nblocks, int ncomp, int op0, int op1, int op2, int 
 
 int read_scalars(cd_design* d, double* out, int n) {
     cd_context* c = d->ctx;
+    // (the pinned solve status is borrowed up to its sequence word, which only
+    // checks may write)
+    if (sizeof(double) * n > offsetof(SolveDev, seq)) return CD_ERR_BAD_ARG;
     CD_HIP(c, hipMemcpyAsync(c->host_status, d->scalars.ptr, sizeof(double) * n,
                              hipMemcpyDeviceToHost, c->stream));
     CD_HIP(c, hipStreamSynchronize(c->stream));

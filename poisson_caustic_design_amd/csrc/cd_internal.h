@@ -72,6 +72,10 @@ struct SolveDev {
     double last_max_update;
     float rmean32;       // mean of the last FP32 residual (projected out in sweeps)
     int cur;             // blocked path: ping-pong buffer holding the current correction
+    // a solve in one workgroup: what its next launch goes on from, if there is more
+    int cum, batch, confirming, more;
+    int holes;           // NaN cells of the right-hand side (nothing was solved)
+    int pad_;
     unsigned int seq;    // host mirror: written last by a check (the host waits for it)
     int stop_lid;        // max-update rule: the launch that found the stop (INT_MAX: none)
 };

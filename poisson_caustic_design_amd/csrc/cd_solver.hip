@@ -948,6 +948,313 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
     if (threadIdx.x == 0) st->cur = out_index;  // same value from every workgroup
 }
 
+// ---------------------------------------------------------------------------
+// A whole mixed-precision solve of a grid of one region (up to 128 x 128 cells)
+// in one launch of one workgroup: the iterate phi, the correction and the
+// right-hand side stay in registers; sweeps, checks and the choice of the next
+// batch are those of cd_solve_device_internal's loop, with the same operations
+// per cell (the reductions sum in another order).  Such a solve was bound by its
+// checks, each three launches and a round trip to the host for 10 us of sweeps:
+// 64 x 64 to 1e-6 took 665 us (490 with launches of a whole batch), 13 checks of
+// about 35 us.  Now 0.32 us a sweep, 5 us a check and 35 us for the launch.
+//
+// The kernel leaves phi alone and reports `holes` when b holds a NaN, and
+// returns at a check after kRegionSweeps sweeps (the host launches it again).
+// ---------------------------------------------------------------------------
+constexpr int kRegionSweeps = 16384;
+
+struct RegionArgs {
+    int w, h, max_sweeps, kmax, adaptive, check_holes, resume;
+    unsigned seq;
+    float om2, om3, om4;
+    double tol, margin;
+};
+
+// Sums of N doubles over the workgroup of 16 waves, in every thread.
+template <int N>
+__device__ __forceinline__ void region_sum(double (&v)[N], double (*red)[BK_NW], int wave, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = cd_wave_sum(v[i]);
+    __syncthreads();  // red has been read
+    if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < N; ++i) red[i][wave] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        double t = red[i][lane & (BK_NW - 1)];
+#pragma unroll
+        for (int o = BK_NW / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        v[i] = t;
+    }
+}
+
+template <int R, bool TRACK>
+__global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __restrict__ b,
+                                                             double* __restrict__ phi,
+                                                             RegionArgs a, SolveDev* st,
+                                                             SolveDev* host_st) {
+    __shared__ float xch[2][BK_NW][2][64];
+    __shared__ double xphi[BK_NW][2][2][64];
+    __shared__ double red[2][BK_NW];
+    __shared__ float smax[TRACK ? kStopGroup : 1][BK_NW][64];
+    __shared__ float redm[kStopGroup];
+    const int w = a.w, h = a.h;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int Yw = R * wave, x0 = 2 * lane;
+    auto in_grid = [&](int c, int k) { return x0 + ((k + c) & 1) < w && Yw + k < h; };
+    // clamped cell addresses: a uniform row and one of two lane offsets
+    const unsigned col[2] = {(unsigned)min(x0, w - 1), (unsigned)min(x0 + 1, w - 1)};
+    auto row = [&](int k) { return (unsigned)(min(Yw + k, h - 1) * w); };
+    const double count = (double)w * h;
+
+    // right-hand side statistics (k_rhs_moments)
+    double bmean, bnorm, holes;
+    {
+        double bv[2][R], s[2] = {0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) bv[c][k] = (b + row(k))[col[(k + c) & 1]];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (!in_grid(c, k)) continue;
+                if (isnan(bv[c][k])) s[1] += 1.0;
+                else s[0] += bv[c][k];
+            }
+        region_sum(s, red, wave, lane);
+        bmean = s[0] / count;
+        holes = s[1];
+        double q[1] = {0.0};
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                if (in_grid(c, k) && !isnan(bv[c][k])) {
+                    const double d = bv[c][k] - bmean;
+                    q[0] += d * d;
+                }
+        region_sum(q, red, wave, lane);
+        bnorm = sqrt(q[0]);
+    }
+
+    BlockCells g;
+    g.om4 = a.om4;
+    g.c1 = 1.f - 4.f * a.om4;
+    g.first = Yw == 0;
+    g.last = Yw + R >= h;
+    g.end_rows = 0u;
+    g.out_rows = 0u;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        if (Yw + k == 0 || Yw + k == h - 1) g.end_rows |= 1u << k;
+        if (Yw + k >= h) g.out_rows |= 1u << k;
+    }
+    g.miss_l = x0 == 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const bool in = x0 + p < w;
+        const bool side = x0 + p == 0 || x0 + p == w - 1;
+        g.miss_r[p] = x0 + p >= w - 1;
+        g.oc[p] = in ? (side ? a.om3 : a.om4) : 0.f;
+        g.oc_end[p] = in ? (side ? a.om2 : a.om3) : 0.f;
+    }
+    const bool ends = g.first || g.last || (TRACK && (w & 1));  // (uniform over the wave)
+
+    double ph[2][R];
+    float ev[2][R], rv[2][R];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double v = (phi + row(k))[col[(k + c) & 1]];
+            ph[c][k] = in_grid(c, k) ? v : 0.0;
+            ev[c][k] = 0.f;
+        }
+
+    // FP64 check of phi + e (k_flush_packed, k_residual, k_check): folds e, leaves
+    // the sweeps' right-hand side in rv; returns the relative residual
+    double rnorm = 0.0, rsum = 0.0;
+    float rm = 0.f;
+    auto check = [&]() -> double {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                ph[c][k] += (double)ev[c][k];
+                ev[c][k] = 0.f;
+            }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            xphi[wave][c][0][lane] = ph[c][0];
+            xphi[wave][c][1][lane] = ph[c][R - 1];
+        }
+        __syncthreads();
+        double s[2] = {0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int p = (k + c) & 1, x = x0 + p, y = Yw + k;
+                const double o = ph[1 - c][k];
+                double up = k > 0 ? ph[1 - c][k > 0 ? k - 1 : 0]
+                                  : xphi[wave > 0 ? wave - 1 : 0][1 - c][1][lane];
+                double down = k < R - 1 ? ph[1 - c][k < R - 1 ? k + 1 : 0]
+                                        : xphi[wave < BK_NW - 1 ? wave + 1 : 0][1 - c][0][lane];
+                if (k == 0 && g.first) up = 0.0;
+                if (k == R - 1 && g.last) down = 0.0;
+                const double left = p ? o : lane_prev(o), right = p ? lane_next(o) : o;
+                const double cnt = (double)((x > 0) + (y > 0) + (x < w - 1) + (y < h - 1));
+                double v = ((b + row(k))[col[p]] - bmean) -
+                           ((left + up + right + down) - cnt * ph[c][k]);
+                if (!in_grid(c, k)) v = 0.0;
+                s[0] += v;
+                s[1] += v * v;
+                rv[c][k] = TRACK ? (float)v : bf16_to_f32(f32_to_bf16((float)v));
+            }
+        region_sum(s, red, wave, lane);
+        const double mean = s[0] / count, rn2 = s[1] - count * mean * mean;
+        rsum = s[0];
+        rnorm = rn2 > 0.0 ? sqrt(rn2) : (rn2 == rn2 ? 0.0 : rn2);
+        rm = (float)mean;
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int p = (k + c) & 1;
+                const bool out = (g.out_rows >> k) & 1u;
+                const float oc = out ? 0.f : (g.end_rows >> k) & 1u ? g.oc_end[p] : g.oc[p];
+                if (TRACK) rv[c][k] = in_grid(c, k) ? rv[c][k] - rm : 0.f;
+                else rv[c][k] = (rm - rv[c][k]) * oc;
+            }
+        return bnorm > 0 ? rnorm / bnorm : (rnorm > 0 ? INFINITY : 0.0);
+    };
+    auto sweep = [&](int n) {
+        n = __builtin_amdgcn_readfirstlane(n);  // (the same in every thread)
+        if (ends) blocked_run<BK_ENDS, TRACK, R>(ev, rv, xch, g, wave, lane, n, smax, true, true);
+        else blocked_run<BK_SIDE, TRACK, R>(ev, rv, xch, g, wave, lane, n, smax, true, true);
+    };
+    // the first of n <= kStopGroup sweeps whose largest update is below tol
+    double last_max = a.resume ? st->last_max_update : INFINITY;
+    auto stopped = [&](int n) -> bool {
+        __syncthreads();
+        if (wave < n) {  // one wave per sweep
+            float m = 0.f;
+            for (int v = 0; v < BK_NW; ++v) m = fmaxf(m, smax[wave][v][lane]);
+            m = wave_max_pos(m);
+            if (lane == 0) redm[wave] = m;
+        }
+        __syncthreads();  // (also: smax has been read)
+        for (int j = 0; j < n; ++j) {
+            last_max = (double)redm[j];
+            if (last_max < a.tol) return true;
+        }
+        return false;
+    };
+
+    // the solve (cd_solve_device_internal's loop), resumed where it was left
+    const bool resume = a.resume != 0;
+    int cum = resume ? st->cum : 0, checks = resume ? st->checks : 0;
+    int k = resume ? st->batch : a.adaptive ? min(a.kmax, max(8, a.kmax / 4)) : a.kmax;
+    int at_done = resume ? st->sweeps_at_done : -1;
+    bool confirming = resume && st->confirming, done = false, more = false;
+    double rel = INFINITY, rel0 = resume ? st->rel0 : INFINITY, prev = 0.0;
+    const bool valid = !(a.check_holes && holes > 0.0);
+    if (valid) {
+        rel = check();
+        if (!resume) {
+            rel0 = rel;
+            ++checks;
+            done = !TRACK && rel <= a.tol;
+        }
+        prev = rel;
+        const int until = cum > INT_MAX - kRegionSweeps ? INT_MAX : cum + kRegionSweeps;
+        // (a non-finite first residual still takes one batch, as the launches do)
+        while (!done && cum < a.max_sweeps) {
+            if (cum >= until) { more = true; break; }
+            const int nsw = min(confirming ? kStopGroup : k, a.max_sweeps - cum);
+            if (!TRACK) {
+                sweep(nsw);
+            } else {
+                for (int j = 0; j < nsw && !done; j += kStopGroup) {
+                    const int n = min(kStopGroup, nsw - j);
+                    sweep(n);
+                    if (stopped(n)) {
+                        done = true;
+                        at_done = cum + j + n;
+                    }
+                }
+            }
+            cum += nsw;
+            rel = check();
+            ++checks;
+            if (!TRACK) done = rel <= a.tol;
+            if (!isfinite(rel)) break;
+            if (TRACK) {
+                if (done && !confirming && cum < a.max_sweeps) {
+                    confirming = true;
+                    done = false;
+                    at_done = -1;
+                    continue;
+                }
+                confirming = false;
+            }
+            if (a.adaptive && !done) {
+                // geometric rate over the last batch, rho = (rel / prev)^(1 / nsw)
+                const double lr = prev > 0 && rel > 0 && rel < prev ? log(rel / prev) / nsw : 0.0;
+                int want = a.kmax;
+                if (lr < -1.0000005000003333e-6) {  // rho < 0.999999
+                    // (out of int's range, as for a tolerance of 0: the fewest)
+                    const double need = ceil(log(a.tol / rel) / lr * a.margin) + 2.0;
+                    want = fabs(need) < 2147483647.0 ? (int)need : 0;
+                }
+                k = max(8, min(a.kmax, want));
+                prev = rel;
+            }
+        }
+#pragma unroll
+        for (int kk = 0; kk < R; ++kk)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                if (in_grid(c, kk)) (phi + row(kk))[col[(kk + c) & 1]] = ph[c][kk];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        SolveDev o{};
+        o.holes = valid ? 0 : (int)holes;
+        o.done = done;
+        o.done_check = done ? checks - 1 : -1;
+        o.stop_lid = INT_MAX;
+        o.bsum = bmean * count;
+        o.sweeps_at_done = at_done;
+        o.checks = checks;
+        o.bmean = bmean;
+        o.bnorm = bnorm;
+        o.rsum = rsum;
+        o.rnorm = rnorm;
+        o.rel = rel;
+        o.rel0 = rel0;
+        o.last_max_update = last_max;
+        o.rmean32 = rm;
+        o.cum = cum;
+        o.batch = k;
+        o.confirming = confirming;
+        o.more = more;
+        o.seq = a.seq;
+        *st = o;
+        // the host waits for the sequence word, which goes last
+        const unsigned* src = reinterpret_cast<const unsigned*>(&o);
+        unsigned* dst = reinterpret_cast<unsigned*>(host_st);
+        constexpr int kSeq = (int)(offsetof(SolveDev, seq) / 4);
+        for (int i = 0; i < (int)(sizeof(SolveDev) / 4); ++i)
+            if (i != kSeq) dst[i] = src[i];
+        __hip_atomic_store(dst + kSeq, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // Reopen a solve whose max-update stop is to be confirmed on a fresh
 // right-hand side (the sweeps that stopped it read r rounded at the last check).
 __global__ void k_reopen(SolveDev* st) {
@@ -988,10 +1295,6 @@ SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t 
     }
     return best;
 }
-
-// A max-update stop of the blocked sweeps falls at the end of a group of this
-// many sweeps, counted from the last check.
-constexpr int kStopGroup = 5;
 
 // How a batch of sweeps is cut into launches: sweeps per launch, rows per wave.
 struct BlockedPlan {
@@ -1686,6 +1989,83 @@ int cd_wait_status(cd_context* ctx, unsigned seq) {
     return CD_OK;
 }
 
+namespace {
+
+// Whether cd_solve_region takes this solve: mixed precision, at most 128 x 128
+// cells, batches a launch can hold, no network and no training-pair capture.
+bool region_solve_applies(const cd_context* ctx, int w, int h, const cd_solve_opts* o) {
+    if (w < 2 || h < 2 || w > SW_RX || h > 8 * BK_NW) return false;
+    if (o->precision != CD_PREC_MIXED) return false;
+    if (o->stop != CD_STOP_RESIDUAL && o->stop != CD_STOP_MAX_UPDATE) return false;
+    if ((o->learned_init && ctx->net) || ctx->cap_x) return false;
+    const int kmax = o->check_every > 0 ? o->check_every : auto_check_every(w, h);
+    return std::min(kmax, o->max_sweeps) <= kRegionSweeps;
+}
+
+void solve_stats(const SolveDev& hs, const cd_solve_opts* o, int cum, int status,
+                 std::chrono::steady_clock::time_point start, cd_solve_stats* out) {
+    std::memset(out, 0, sizeof(*out));
+    out->status = status;
+    // the residual rule stops at the last check, after all enqueued sweeps
+    out->sweeps = (hs.done && o->stop == CD_STOP_MAX_UPDATE) ? hs.sweeps_at_done : cum;
+    out->checks = hs.checks;
+    out->rel_residual = hs.rel;
+    out->initial_rel_residual = hs.rel0;
+    out->last_max_update = hs.last_max_update;
+    out->elapsed_ms = std::chrono::duration<double, std::milli>(
+                          std::chrono::steady_clock::now() - start).count();
+}
+
+// The whole solve in k_solve_region launches.  holes: NaN cells found in b when
+// check_holes (phi is then untouched and nothing is solved).
+int cd_solve_region(cd_context* ctx, const double* b, double* phi, int w, int h,
+                    const cd_solve_opts* o, SolveDev* sd, bool timers, bool check_holes,
+                    int* holes, cd_solve_stats* st_out) {
+    const auto t_start = std::chrono::steady_clock::now();
+    const bool track = o->stop == CD_STOP_MAX_UPDATE;
+    const float om = (float)cd_sor_omega(o->omega, w, h);
+    RegionArgs a{};
+    a.w = w;
+    a.h = h;
+    a.max_sweeps = o->max_sweeps;
+    a.kmax = o->check_every > 0 ? o->check_every : auto_check_every(w, h);
+    a.adaptive = o->check_every <= 0 && !track;
+    a.check_holes = check_holes;
+    a.om2 = om / 2.f;
+    a.om3 = om / 3.f;
+    a.om4 = om / 4.f;
+    a.tol = o->tol;
+    a.margin = CD_CHECK_MARGIN;
+    const int rows = h <= 2 * BK_NW ? 2 : h <= 4 * BK_NW ? 4 : 8;
+    auto kernel = rows == 2 ? (track ? k_solve_region<2, true> : k_solve_region<2, false>)
+                : rows == 4 ? (track ? k_solve_region<4, true> : k_solve_region<4, false>)
+                            : (track ? k_solve_region<8, true> : k_solve_region<8, false>);
+    for (;;) {
+        a.seq = ++ctx->status_seq;
+        const int before = a.resume ? ctx->host_status->cum : 0;
+        if (timers) CD_TRY(ctx->timer_begin());
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(BK_THREADS), 0, ctx->stream, b, phi, a, sd,
+                           ctx->host_status);
+        CD_CHECK_LAUNCH(ctx);
+        CD_TRY(cd_wait_status(ctx, a.seq));
+        const SolveDev& hs = *ctx->host_status;
+        if (timers)
+            CD_TRY(ctx->timer_end(CD_KERNEL_SOR_SWEEP, 1, 12.0 * w * h * (hs.cum - before)));
+        if (holes) *holes = hs.holes;
+        if (hs.holes) return CD_OK;
+        if (!hs.more) break;
+        a.resume = 1;
+    }
+    const SolveDev hs = *ctx->host_status;
+    CD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (timers) CD_TRY(ctx->resolve_timers());
+    const int status = !std::isfinite(hs.rel) ? CD_ERR_NAN : hs.done ? CD_OK : CD_ERR_NOT_CONVERGED;
+    if (st_out) solve_stats(hs, o, hs.cum, status, t_start, st_out);
+    return status;
+}
+
+}  // namespace
+
 int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, const uint8_t* mask,
                              long long valid_cells, int w, int h, const cd_solve_opts* o,
                              cd_solve_stats* st_out, const SolveWork* work) {
@@ -1696,6 +2076,12 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const bool mixed = o->precision == CD_PREC_MIXED;
     const size_t n = (size_t)w * h;
     const double count = (double)valid_cells;
+    if (!mask && region_solve_applies(ctx, w, h, o)) {
+        if (!work) CD_TRY(ctx->ensure(ctx->solve_dev, sizeof(SolveDev)));
+        return cd_solve_region(ctx, b, phi, w, h, o,
+                               work ? work->sd : ctx->solve_dev.as<SolveDev>(), !work, false,
+                               nullptr, st_out);
+    }
 
     // workspace
     const dim3 rblk(RED_BX, RED_BY);
@@ -2316,18 +2702,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     if (!std::isfinite(hs.rel)) status = CD_ERR_NAN;
     else if (!hs.done) status = CD_ERR_NOT_CONVERGED;
     if (st_out) {
-        std::memset(st_out, 0, sizeof(*st_out));
-        st_out->status = status;
-        // the residual rule stops at the last check, after all enqueued sweeps
-        st_out->sweeps = (hs.done && o->stop == CD_STOP_MAX_UPDATE) ? hs.sweeps_at_done : cum;
-        st_out->checks = hs.checks;
-        st_out->rel_residual = hs.rel;
-        st_out->initial_rel_residual = hs.rel0;
-        st_out->last_max_update = hs.last_max_update;
+        solve_stats(hs, o, cum, status, t_start, st_out);
         st_out->learned_applied = learned_applied;
         st_out->learned_rejected = learned_rejected;
-        st_out->elapsed_ms = std::chrono::duration<double, std::milli>(
-                                 std::chrono::steady_clock::now() - t_start).count();
     }
     return status;
 }
@@ -2458,6 +2835,12 @@ int cd_poisson_solve_device_noalloc(cd_context* ctx, const double* d_rhs, double
     ws.phi2 = reinterpret_cast<double*>(base + L.e32);
     uint8_t* mask = base + L.mask;
     double* fill = reinterpret_cast<double*>(base + L.fill);
+    if (region_solve_applies(ctx, width, height, opts)) {
+        int found = 0;
+        const int rc = cd_solve_region(ctx, d_rhs, d_phi, width, height, opts, ws.sd, false, true,
+                                       &found, stats);
+        if (!found) return rc;
+    }
     long long holes = 0;
     CD_TRY(cd_hole_mask(ctx, d_rhs, width, height, mask, ws.partials, fill,
                         reinterpret_cast<double*>(ctx->host_status), &holes));
@@ -2475,6 +2858,13 @@ int cd_poisson_solve_device(cd_context* ctx, const double* d_rhs, double* d_phi,
     const size_t n = (size_t)width * height;
     size_t nred, npk;
     cd_solve_work_sizes(width, height, &nred, &npk);
+    if (region_solve_applies(ctx, width, height, opts)) {
+        CD_TRY(ctx->ensure(ctx->solve_dev, sizeof(SolveDev)));
+        int found = 0;
+        const int rc = cd_solve_region(ctx, d_rhs, d_phi, width, height, opts,
+                                       ctx->solve_dev.as<SolveDev>(), true, true, &found, stats);
+        if (!found) return rc;
+    }
     // hole mask: only used by the solve when the right-hand side contains NaN
     CD_TRY(ctx->ensure(ctx->mask, n));
     CD_TRY(ctx->ensure(ctx->partials, cd_partials_bytes(nred)));  // as the solve

@@ -117,6 +117,10 @@ __device__ __forceinline__ double lane_next(double v) {
 // region's loads, which the decision would otherwise hold back; a word shared
 // by all tiles (atomicOr) cost 0.6 us of a launch at 50 tiles and 9 us at 1000.
 // ---------------------------------------------------------------------------
+// A max-update stop of the blocked sweeps falls at the end of a group of this
+// many sweeps, counted from the last check.
+constexpr int kStopGroup = 5;
+
 constexpr int kTrackSlots = 16;   // floats of maxima per tile
 constexpr int kTrackSweeps = 15;  // most sweeps of a tracking launch
 

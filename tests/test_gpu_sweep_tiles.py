@@ -173,3 +173,49 @@ def test_max_update_stop_inside_a_launch_keeps_that_iterate(ctx, rng, w, h):
         assert np.array_equal(f, g), (tol, j)
         stops.add(s)
     assert len(stops) >= 3
+
+
+# grids of one region run whole solves in one launch; one cell more does not
+REGION = [(2, 2), (5, 3), (31, 32), (64, 33), (100, 64), (127, 65), (128, 128)]
+
+
+@pytest.mark.parametrize("w,h", REGION)
+def test_one_region_solves_match_larger_route(ctx, rng, w, h):
+    """The one-launch solve against the solve of the same problem through the
+    hole-mask route's FP64 sweeps: both end at the tolerance, so the mean-free
+    solutions agree to it (the residual's factor on the error is below
+    (n / pi)^2 / 4 < 420 at 128)."""
+    b, _, p0 = make(rng, w, h, False)
+    tol = 1e-10
+    g, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=tol))
+    ref, sr = ctx.poisson_solve(b, p0, capi.default_opts(tol=tol, precision=capi.PREC_FP64))
+    assert st.status == sr.status == capi.OK and st.rel_residual <= tol
+    assert st.checks >= 2 and st.initial_rel_residual > tol
+    d = (g - g.mean()) - (ref - ref.mean())
+    assert np.abs(d).max() <= 2 * 420 * tol * np.linalg.norm(b)
+
+
+def test_one_region_solve_statuses(ctx, rng):
+    b, _, p0 = make(rng, 40, 30, False)
+    # cap, in the middle of a batch and of a group
+    for stop in (capi.STOP_RESIDUAL, capi.STOP_MAX_UPDATE):
+        _, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=1e-14, stop=stop, max_sweeps=33))
+        assert st.status == capi.NOT_CONVERGED and st.sweeps == 33
+    # no sweeps at all leave the start as it is
+    g, st = ctx.poisson_solve(b, p0, capi.default_opts(max_sweeps=0))
+    assert st.status == capi.NOT_CONVERGED and st.sweeps == 0 and np.array_equal(g, p0)
+    # non-finite values end the solve as such
+    bad = p0.copy()
+    bad[3, 4] = np.inf
+    _, st = ctx.poisson_solve(b, bad, capi.default_opts(), allow=(capi.NAN_,))
+    assert st.status == capi.NAN_
+    # more sweeps than one launch takes: it goes on from its last check
+    g, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=0.0, max_sweeps=40000, check_every=1000))
+    assert st.status == capi.NOT_CONVERGED and st.sweeps == 40000 and st.checks == 41
+    ref, _ = ctx.poisson_solve(b, p0, capi.default_opts(tol=1e-12, precision=capi.PREC_FP64))
+    d = (g - g.mean()) - (ref - ref.mean())
+    assert np.abs(d).max() <= 1e-9 * np.abs(ref).max()
+    # holes leave it for the route that handles them, the start still in place
+    b[4, 5] = np.nan
+    g, st = ctx.poisson_solve(b, p0, capi.default_opts(tol=1e-9))
+    assert st.status == capi.OK and np.isnan(g).sum() == 1
