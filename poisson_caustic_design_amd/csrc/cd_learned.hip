@@ -434,93 +434,282 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1
     }
 }
 
+// A compile-time value, or (0) the runtime one: sizes that are constants in the
+// instantiations for the shipped channel counts.
+template <int N>
+__device__ __forceinline__ int fixed_or(int runtime) { return N > 0 ? N : runtime; }
+
+// The input patch of a workgroup on its way to LDS: vector it = first +
+// threadIdx.x + NT*u of the P x P x cin/8 vectors (8 channels of a pixel each),
+// u < U, loaded by load() and stored by store(), so that other loads can be
+// issued in between.  A vector past the last is that one again, loaded and stored
+// where it lies: no branches, so every load is issued before the first store
+// waits.  Sources as for stage_patch; POOL: mode1 2.  CIN: channels (0: any).
+template <int P, int NT, int U, bool POOL, int CIN>
+struct PatchLoad {
+    uint4 v[U][POOL ? 4 : 1];
+    int px[U], gi[U];  // pixel and 8-channel group
+    __device__ __forceinline__ void load(const u16* __restrict__ x1, const u16* __restrict__ x2,
+                                         int c1, int c2, int H, int W, int b, int oy, int ox,
+                                         int mode1, int first) {
+        const int ng = fixed_or<CIN / 8>((c1 + c2) >> 3), last = P * P * ng - 1;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int it = min(first + (int)threadIdx.x + NT * u, last);
+            px[u] = it / ng;
+            gi[u] = it - px[u] * ng;
+            const int ci = gi[u] * 8;
+            const bool use2 = !POOL && ci >= c1;  // (a pooled input has no x2)
+            const u16* __restrict__ src = use2 ? x2 + (ci - c1) : x1 + ci;
+            const int cs = use2 ? c2 : c1;
+            const int yc = min(max(oy + px[u] / P, 0), H - 1);
+            const int xc = min(max(ox + px[u] % P, 0), W - 1);
+            if (POOL) {
+                const long long r0 = ((long long)b * (2 * H) + 2 * yc) * (2 * W) + 2 * xc;
+                const long long r1 = r0 + 2 * W;
+                v[u][0] = *reinterpret_cast<const uint4*>(src + r0 * cs);
+                v[u][POOL ? 1 : 0] = *reinterpret_cast<const uint4*>(src + (r0 + 1) * cs);
+                v[u][POOL ? 2 : 0] = *reinterpret_cast<const uint4*>(src + r1 * cs);
+                v[u][POOL ? 3 : 0] = *reinterpret_cast<const uint4*>(src + (r1 + 1) * cs);
+            } else {
+                const int up = (!use2 && mode1 == 1) ? 1 : 0;
+                const long long q = ((long long)b * (H >> up) + (yc >> up)) * (W >> up) + (xc >> up);
+                v[u][0] = *reinterpret_cast<const uint4*>(src + q * cs);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(u16* __restrict__ xs, int xstride, int H, int W, int oy,
+                                          int ox) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int yy = oy + px[u] / P, xx = ox + px[u] % P;
+            const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+            V8 o;
+            o.u = v[u][0];
+            if (POOL) {  // 2x2 average as k_avgpool2 takes it
+                V8 p[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[e].u = v[u][POOL ? e : 0];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    o.h[e] = to_bf16(0.25f * (from_bf16(p[0].h[e]) + from_bf16(p[1].h[e]) +
+                                              from_bf16(p[2].h[e]) + from_bf16(p[3].h[e])));
+            }
+            o.u = make_uint4(in ? o.u.x : 0, in ? o.u.y : 0, in ? o.u.z : 0, in ? o.u.w : 0);
+            *reinterpret_cast<uint4*>(xs + px[u] * xstride + gi[u] * 8) = o.u;
+        }
+    }
+};
+
+// The same for `rows` weight rows of kpad (LDS row stride kpad + 8; KPAD: 0 any).
+template <int NT, int U, int KPAD>
+struct WeightLoad {
+    uint4 v[U];
+    __device__ __forceinline__ static int at(int rows, int kv, int first, int u) {
+        return min(first + (int)threadIdx.x + NT * u, rows * kv - 1);
+    }
+    __device__ __forceinline__ void load(const u16* __restrict__ w, int rows, int kpad, int first) {
+        const int kv = fixed_or<KPAD / 8>(kpad >> 3);
+#pragma unroll
+        for (int u = 0; u < U; ++u)  // (rows are contiguous)
+            v[u] = reinterpret_cast<const uint4*>(w)[at(rows, kv, first, u)];
+    }
+    __device__ __forceinline__ void store(u16* __restrict__ ws, int rows, int kpad, int first) {
+        const int kv = fixed_or<KPAD / 8>(kpad >> 3);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int it = at(rows, kv, first, u), r = it / kv;
+            *reinterpret_cast<uint4*>(ws + r * (kv + 1) * 8 + (it - r * kv) * 8) = v[u];
+        }
+    }
+};
+
+// K of a 3x3 convolution over cin channels, padded to whole chunks
+constexpr int conv_kpad(int cin) { return (9 * cin + 31) / 32 * 32; }
+
+// The K loop of conv_lds for one block of 16 output channels (weight rows from
+// ws) and MT M-tiles, on a patch of side P.  CIN > 0: unrolled, all offsets
+// constants but for the lane's quarter of a chunk, so that the chunks' LDS reads
+// and MFMAs have no address chain between them.  CIN 0: conv_lds.  Same chunk
+// order, same bits.
+template <int CIN, int MT, int P>
+__device__ __forceinline__ void conv_chunks(floatx4 (&acc)[MT], const u16* __restrict__ xs,
+                                            int cin, const u16* __restrict__ ws, int kpad,
+                                            const int (&pbase)[MT], int lane) {
+    if (CIN == 0) {
+        floatx4 a2[MT][1];
+        conv_lds<1, MT, P>(a2, xs, cin + 8, cin, ws, kpad, pbase, lane);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = a2[m][0];
+        return;
+    }
+    constexpr int C = CIN > 0 ? CIN : 8, XS = C + 8, KP = conv_kpad(C);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int qd = lane >> 4;
+    const u16* wrow = ws + (lane & 15) * (KP + 8) + 8 * qd;
+    const u16* xm[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xm[m] = xs + pbase[m] * XS;
+#pragma unroll
+    for (int kc = 0; kc < KP; kc += 32) {
+        // patch offset of the lane's 8 consecutive k, one of four constants (past
+        // the last tap: anything, the fragment is zeroed)
+        auto offset = [&](int k) {
+            const int tap = k / C < 9 ? k / C : 0;
+            return ((tap / 3) * P + tap % 3) * XS + k % C;
+        };
+        int off;
+        if (C % 32 == 0) {
+            off = offset(kc) + 8 * qd;
+        } else {
+            off = qd == 0 ? offset(kc) : qd == 1 ? offset(kc + 8)
+                : qd == 2 ? offset(kc + 16) : offset(kc + 24);
+        }
+        V8 bw;
+        bw.u = *reinterpret_cast<const uint4*>(wrow + kc);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            V8 a;
+            a.u = *reinterpret_cast<const uint4*>(xm[m] + off);
+            if (kc + 32 > 9 * C) {
+                const bool in = kc + 8 * qd < 9 * C;
+                a.u = make_uint4(in ? a.u.x : 0, in ? a.u.y : 0, in ? a.u.z : 0, in ? a.u.w : 0);
+            }
+            acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, bw.v, acc[m], 0, 0, 0);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Two consecutive 3x3 convolutions of one resolution level in one launch
-// (inference): conv a reads its inputs as k_conv3x3_tile does (mode1) on the
-// 12x12 patch around an 8x8 output tile and computes the 10x10 region that
-// conv b needs (7 M-tiles of 16 pixels, two per wave), which stays in LDS as
-// BF16 (zero outside the image: conv b's padding); conv b then computes the
-// tile from it.  Every workgroup computes all output channels of both convs
-// (NBA*16 and NBB*16).  The A/B fragments and the K order of both are those of
-// k_conv3x3_tile, and the intermediate is rounded to BF16 as the stored tensor
-// is, so the output is bit-identical to the two launches; conv a's output is
-// not written (inference only).  wb_early: conv b's weights are staged with
-// conv a's at the start (separate LDS); else after conv a, over conv a's.
+// (inference), one 8x8 output tile per workgroup of 8 waves: conv a reads its
+// inputs as k_conv3x3_tile does (mode1; POOL: mode 2) on the 12x12 patch around
+// the tile and computes the 10x10 region that conv b needs (7 M-tiles of 16
+// pixels), which stays in LDS as BF16 (zero outside the image: conv b's padding);
+// conv b then computes the tile from it.  Every workgroup computes all output
+// channels of both convs (NB*16).  The A/B fragments and the K order of both are
+// those of k_conv3x3_tile, and the intermediate is rounded to BF16 as the stored
+// tensor is, so the output is bit-identical to the two launches; conv a's output
+// is not written.  wb_early: conv b's weights are staged with conv a's at the
+// start (separate LDS); else after conv a, over conv a's.
+//
+// Bound by latency: launch, one memory round trip, two short K loops.  The
+// patch's and both convolutions' weight loads are all issued before the first
+// LDS store (three round trips one after the other before), 8 waves share the
+// M-tiles by output block, and the K loops are unrolled for the chunk counts of
+// the shipped networks (CINA, CINB channels; 0: any): with the sizes at run time
+// the compiler put every weight load behind its predicate, next to its store, and
+// a division per chunk in front of the K loop.  On a 128 x 128 level 0, median of
+// a launch (8 -> 16, 16 -> 32 pooled, 32 -> 32 pooled, 64 -> 32, 48 -> 16
+// channels): 9.6, 11.7, 11.7, 11.7, 9.6 us before, 4.4, 6.0, 6.4, 7.3, 4.7 now.
 // grid: (ceil(W/8), ceil(H/8), B).  LDS (u16): 144 (cin + 8) + 100 (cya + 8) +
-// NBA*16 (kpada + 8) [+ NBB*16 (kpadb + 8)], or max of the two weight blocks.
+// NB*16 (kpada + 8) [+ NB*16 (kpadb + 8)], or max of the two weight blocks.
 // ---------------------------------------------------------------------------
-template <int NBA, int NBB>
-__global__ __launch_bounds__(256) void k_conv_pair_tile(
+constexpr int kPairThreads = 512;
+template <int NB, int CINA, int CINB, bool POOL>
+__global__ __launch_bounds__(kPairThreads) void k_conv_pair_tile(
     const u16* __restrict__ x1, const u16* __restrict__ x2, int c1, int c2,
     const u16* __restrict__ wa, int kpada, int cya, int relua, const u16* __restrict__ wb,
     int kpadb, int cyb, int relub, u16* __restrict__ ybf, int H, int W, int mode1,
     int wb_early) {
+    constexpr int NT = kPairThreads;
+    constexpr int KPA = CINA > 0 ? conv_kpad(CINA) : 0, KPB = CINB > 0 ? conv_kpad(CINB) : 0;
+    // vectors per thread of a round: all of them where the sizes are constants
+    constexpr int UP = CINA > 0 ? (144 * (CINA / 8) + NT - 1) / NT : 2;
+    constexpr int UA = CINA > 0 ? (NB * 2 * KPA + NT - 1) / NT : 4;
+    constexpr int UB = CINB > 0 ? (NB * 2 * KPB + NT - 1) / NT : 2;
     extern __shared__ uint4 tile_lds[];
-    const int cin = c1 + c2;
-    const int xstride = cin + 8, istride = cya + 8;
+    const int cin = fixed_or<CINA>(c1 + c2), cb = fixed_or<CINB>(cya);
+    const int ka = fixed_or<KPA>(kpada), kb = fixed_or<KPB>(kpadb);
+    const int xstride = cin + 8, istride = cb + 8;
     u16* xs = reinterpret_cast<u16*>(tile_lds);
     u16* ism = xs + 144 * xstride;
     u16* wsa = ism + 100 * istride;
-    u16* wsb = wb_early ? wsa + NBA * 16 * (kpada + 8) : wsa;
+    u16* wsb = wb_early ? wsa + NB * 16 * (ka + 8) : wsa;
     const int b = blockIdx.z;
     const int tx0 = blockIdx.x * CT, ty0 = blockIdx.y * CT;
-    stage_patch<12>(xs, xstride, x1, x2, c1, c2, H, W, b, ty0 - 2, tx0 - 2, mode1);
-    stage_weights(wsa, wa, NBA * 16, kpada);
-    if (wb_early) stage_weights(wsb, wb, NBB * 16, kpadb);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     {
-        // conv a: M-tiles wave and wave + 4 of the 10x10 region (pixels past
-        // 100 compute on pixel 0 and are dropped)
-        int pbase[2];
+        PatchLoad<12, NT, UP, POOL, CINA> pl;
+        WeightLoad<NT, UA, KPA> la;
+        WeightLoad<NT, UB, KPB> lb;
+        pl.load(x1, x2, c1, c2, H, W, b, ty0 - 2, tx0 - 2, mode1, 0);
+        la.load(wa, NB * 16, ka, 0);
+        lb.load(wb, NB * 16, kb, 0);
+        pl.store(xs, xstride, H, W, ty0 - 2, tx0 - 2);
+        la.store(wsa, NB * 16, ka, 0);
+        if (wb_early) lb.store(wsb, NB * 16, kb, 0);
+        // what did not fit the first round
+        for (int f = UP * NT; CINA == 0 && f < 18 * cin; f += UP * NT) {
+            pl.load(x1, x2, c1, c2, H, W, b, ty0 - 2, tx0 - 2, mode1, f);
+            pl.store(xs, xstride, H, W, ty0 - 2, tx0 - 2);
+        }
+        for (int f = UA * NT; CINA == 0 && f < NB * 2 * ka; f += UA * NT) {
+            la.load(wa, NB * 16, ka, f);
+            la.store(wsa, NB * 16, ka, f);
+        }
+        for (int f = UB * NT; CINB == 0 && wb_early && f < NB * 2 * kb; f += UB * NT) {
+            lb.load(wb, NB * 16, kb, f);
+            lb.store(wsb, NB * 16, kb, f);
+        }
+    }
+    __syncthreads();
+    // wave -> output block nb and M-tiles: with two blocks each wave takes two
+    // M-tiles of conv a and one of conv b, with one block one of each
+    const int nb = NB == 2 ? wave & 1 : 0, mg = NB == 2 ? wave >> 1 : wave;
+    const int ch = nb * 16 + (lane & 15);
+    {
+        // (pixels past 100 compute on pixel 0 and are dropped)
+        constexpr int MT = NB == 2 ? 2 : 1;
+        int pbase[MT];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const int q = (wave + 4 * m) * 16 + (lane & 15);
+        for (int m = 0; m < MT; ++m) {
+            const int q = (mg + 4 * m) * 16 + (lane & 15);
             pbase[m] = q < 100 ? (q / 10) * 12 + q % 10 : 0;
         }
-        floatx4 acc[2][NBA];
-        conv_lds<NBA, 2, 12>(acc, xs, xstride, cin, wsa, kpada, pbase, lane);
+        floatx4 acc[MT];
+        conv_chunks<CINA, MT, 12>(acc, xs, cin, wsa + nb * 16 * (ka + 8), ka, pbase, lane);
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int nb = 0; nb < NBA; ++nb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q = (wave + 4 * m) * 16 + 4 * (lane >> 4) + r;
-                    const int ch = nb * 16 + (lane & 15);
-                    if (q >= 100 || ch >= cya) continue;
-                    const int yy = ty0 - 1 + q / 10, xx = tx0 - 1 + q % 10;
-                    float v = acc[m][nb][r];
-                    if (relua) v = fmaxf(v, 0.f);
-                    ism[q * istride + ch] =
-                        (yy >= 0 && yy < H && xx >= 0 && xx < W) ? to_bf16(v) : (u16)0;
-                }
+            for (int r = 0; r < 4; ++r) {
+                const int q = (mg + 4 * m) * 16 + 4 * (lane >> 4) + r;
+                if (q >= 100 || ch >= cya) continue;
+                const int yy = ty0 - 1 + q / 10, xx = tx0 - 1 + q % 10;
+                float v = acc[m][r];
+                if (relua) v = fmaxf(v, 0.f);
+                ism[q * istride + ch] =
+                    (yy >= 0 && yy < H && xx >= 0 && xx < W) ? to_bf16(v) : (u16)0;
+            }
     }
     __syncthreads();
     if (!wb_early) {
-        stage_weights(wsb, wb, NBB * 16, kpadb);
+        WeightLoad<NT, UB, KPB> lb;
+        for (int f = 0; f < NB * 2 * kb; f += UB * NT) {
+            lb.load(wb, NB * 16, kb, f);
+            lb.store(wsb, NB * 16, kb, f);
+        }
         __syncthreads();
     }
-    // conv b on the 8x8 tile: lane's A pixel tile row 2*wave + (l%16)/8,
-    // column (l%16)%8, i.e. region pixel (row + 1, column + 1) whose 3x3
-    // neighbourhood starts at region index row*10 + column
-    const int ar = 2 * wave + ((lane & 15) >> 3), ac = lane & 7;
+    if (mg >= 4) return;  // conv b has four M-tiles
+    // lane's A pixel: tile row 2*mg + (l%16)/8, column (l%16)%8, i.e. region pixel
+    // (row + 1, column + 1) whose 3x3 neighbourhood starts at index row*10 + column
+    const int ar = 2 * mg + ((lane & 15) >> 3), ac = lane & 7;
     const int pbase[1] = {ar * 10 + ac};
-    floatx4 acc[1][NBB];
-    conv_lds<NBB, 1, 10>(acc, ism, istride, cya, wsb, kpadb, pbase, lane);
+    floatx4 acc[1];
+    conv_chunks<CINB, 1, 10>(acc, ism, cb, wsb + nb * 16 * (kb + 8), kb, pbase, lane);
 #pragma unroll
-    for (int nb = 0; nb < NBB; ++nb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 4 * (lane >> 4) + r;
-            const int yy = ty0 + 2 * wave + (row >> 3), xx = tx0 + (row & 7);
-            const int ch = nb * 16 + (lane & 15);
-            if (yy >= H || xx >= W || ch >= cyb) continue;
-            const long long p = ((long long)b * H + yy) * W + xx;
-            float v = acc[0][nb][r];
-            if (relub) v = fmaxf(v, 0.f);
-            ybf[p * cyb + ch] = to_bf16(v);
-        }
+    for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (lane >> 4) + r;
+        const int yy = ty0 + 2 * mg + (row >> 3), xx = tx0 + (row & 7);
+        if (yy >= H || xx >= W || ch >= cyb) continue;
+        const long long p = ((long long)b * H + yy) * W + xx;
+        float v = acc[0][r];
+        if (relub) v = fmaxf(v, 0.f);
+        ybf[p * cyb + ch] = to_bf16(v);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1173,8 +1362,15 @@ size_t tiled_lds_limit(cd_context* c) {
                          reinterpret_cast<const void*>(&k_conv3x3_tile<1, 1>),
                          reinterpret_cast<const void*>(&k_conv3x3_tile<1, 2, 1>),
                          reinterpret_cast<const void*>(&k_conv3x3_tile<2, 2, 1>),
-                         reinterpret_cast<const void*>(&k_conv_pair_tile<1, 1>),
-                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 2>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<1, 8, 16, false>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<1, 48, 16, false>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 16, 32, true>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 32, 32, true>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 64, 32, false>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<1, 0, 0, true>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<1, 0, 0, false>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 0, 0, true>),
+                         reinterpret_cast<const void*>(&k_conv_pair_tile<2, 0, 0, false>),
                          reinterpret_cast<const void*>(&k_head_smooth<6>)};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
@@ -1491,9 +1687,19 @@ bool launch_conv_pair(cd_net* n, const NetConv& a, const NetConv& b, int B, int 
     u16* y = n->t[b.out].act.as<u16>();
     const dim3 grid(div_up(W, CT), div_up(H, CT), B);
     hipStream_t s = n->ctx->stream;
-#define PAIR(NB) hipLaunchKernelGGL((k_conv_pair_tile<NB, NB>), grid, dim3(256), lds, s, x1, x2, a.c1, a.c2, wta, a.kpad, a.coutA, a.relu, wtb, b.kpad, b.coutA, b.relu, y, H, W, mode1, early)
-    if (nba == 1) PAIR(1);
-    else PAIR(2);
+    const int cina = a.c1 + a.c2, cinb = a.coutA;
+    const bool pool = mode1 == 2;
+#define PAIR(NB, CA, CB, POOL) hipLaunchKernelGGL((k_conv_pair_tile<NB, CA, CB, POOL>), grid, dim3(kPairThreads), lds, s, x1, x2, a.c1, a.c2, wta, a.kpad, a.coutA, a.relu, wtb, b.kpad, b.coutA, b.relu, y, H, W, mode1, early)
+    // 16 and 32 channels per level, as in the shipped networks
+    if (nba == 1 && !pool && cina == 8 && cinb == 16) PAIR(1, 8, 16, false);
+    else if (nba == 1 && !pool && cina == 48 && cinb == 16) PAIR(1, 48, 16, false);
+    else if (nba == 2 && pool && cina == 16 && cinb == 32) PAIR(2, 16, 32, true);
+    else if (nba == 2 && pool && cina == 32 && cinb == 32) PAIR(2, 32, 32, true);
+    else if (nba == 2 && !pool && cina == 64 && cinb == 32) PAIR(2, 64, 32, false);
+    else if (nba == 1 && pool) PAIR(1, 0, 0, true);
+    else if (nba == 1) PAIR(1, 0, 0, false);
+    else if (pool) PAIR(2, 0, 0, true);
+    else PAIR(2, 0, 0, false);
 #undef PAIR
     return true;
 }
