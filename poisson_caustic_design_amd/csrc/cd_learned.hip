@@ -1143,17 +1143,30 @@ __global__ __launch_bounds__(256) void k_smooth_tiled(const float* __restrict__ 
 // patch in LDS with the A/B fragments and K order of k_conv3x3_tile, so its
 // values are those k_conv3x3_tile<1, 1> stores; outside the image the region
 // holds 0, as k_smooth_tiled loads it; then the K steps as k_smooth_tiled
-// takes them.  The output is bit-identical to the two launches.  grid
-// (ceil(W/8), ceil(H/8), B); LDS (bytes): 2 P^2 (C + 8) + 2*16 (kpad + 8)
+// takes them, one cell per thread: the cells outside the image stay 0, so that
+// adding them changes no sum and a cell's count of neighbours is the only
+// condition left.  The output is bit-identical to the two launches.
+//
+// Bound by latency, as k_conv_pair_tile, and built like it (loads first, CIN > 0
+// unrolled for that many channels, 8 waves).  On a 128 x 128 level, 16 channels:
+// 11.2 us with 256 threads, a serial staging and bounds tested in every smoothing
+// step, 5.5 us now.
+// grid (ceil(W/8), ceil(H/8), B); LDS (bytes): 2 P^2 (C + 8) + 2*16 (kpad + 8)
 // + 8 R^2, P = R + 2, R = 8 + 2K.
-template <int K>
-__global__ __launch_bounds__(256) void k_head_smooth(const u16* __restrict__ x, int C,
-                                                     const u16* __restrict__ wt, int kpad, int H,
+template <int K, int CIN>
+__global__ __launch_bounds__(512) void k_head_smooth(const u16* __restrict__ x, int channels,
+                                                     const u16* __restrict__ wt, int kpad0, int H,
                                                      int W, float* __restrict__ out) {
+    constexpr int NT = 512;
     constexpr int R = kSmoothTile + 2 * K, P = R + 2, NQ = R * R;
-    constexpr int MT = (NQ + 63) / 64;  // M-tiles of 16 region pixels per wave
+    constexpr int MT = (NQ + NT / 4 - 1) / (NT / 4);  // M-tiles of 16 region pixels per wave
+    constexpr int KP = CIN > 0 ? conv_kpad(CIN) : 0;
+    constexpr int UP = CIN > 0 ? (P * P * (CIN / 8) + NT - 1) / NT : 2;
+    constexpr int UW = CIN > 0 ? (2 * KP + NT - 1) / NT : 1;
     static_assert(kSmoothTile == CT, "the head region is centred on the conv tile");
+    static_assert(NQ <= NT, "one region cell per thread");
     extern __shared__ uint4 tile_lds[];
+    const int C = fixed_or<CIN>(channels), kpad = fixed_or<KP>(kpad0);
     const int xstride = C + 8;
     u16* xs = reinterpret_cast<u16*>(tile_lds);
     u16* ws = xs + P * P * xstride;
@@ -1162,33 +1175,71 @@ __global__ __launch_bounds__(256) void k_head_smooth(const u16* __restrict__ x, 
     const int b = blockIdx.z;
     const int tx0 = blockIdx.x * CT, ty0 = blockIdx.y * CT;
     const int X0 = tx0 - K, Y0 = ty0 - K;  // region origin
-    // (x2 = x with no channels: never read; a null x2 here crashed the compiler)
-    stage_patch<P>(xs, xstride, x, x, C, 0, H, W, b, Y0 - 1, X0 - 1, 0);
-    stage_weights(ws, wt, 16, kpad);
+    {
+        // (x2 = x with no channels: never read)
+        PatchLoad<P, NT, UP, false, CIN> pl;
+        WeightLoad<NT, UW, KP> wl;
+        pl.load(x, x, C, 0, H, W, b, Y0 - 1, X0 - 1, 0, 0);
+        wl.load(wt, 16, kpad, 0);
+        pl.store(xs, xstride, H, W, Y0 - 1, X0 - 1);
+        wl.store(ws, 16, kpad, 0);
+        for (int f = UP * NT; CIN == 0 && f < P * P * (C / 8); f += UP * NT) {
+            pl.load(x, x, C, 0, H, W, b, Y0 - 1, X0 - 1, 0, f);
+            pl.store(xs, xstride, H, W, Y0 - 1, X0 - 1);
+        }
+        for (int f = UW * NT; CIN == 0 && f < 2 * kpad; f += UW * NT) {
+            wl.load(wt, 16, kpad, f);
+            wl.store(ws, 16, kpad, f);
+        }
+    }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int pbase[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int q = (wave + 4 * m) * 16 + (lane & 15);
+        const int q = (wave + 8 * m) * 16 + (lane & 15);
         pbase[m] = q < NQ ? (q / R) * P + q % R : 0;
     }
-    floatx4 acc[MT][1];
-    conv_lds<1, MT, P>(acc, xs, xstride, C, ws, kpad, pbase, lane);
+    floatx4 acc[MT];
+    conv_chunks<CIN, MT, P>(acc, xs, C, ws, kpad, pbase, lane);
     if ((lane & 15) == 0) {  // output channel 0
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int q = (wave + 4 * m) * 16 + 4 * (lane >> 4) + r;
+                const int q = (wave + 8 * m) * 16 + 4 * (lane >> 4) + r;
                 if (q >= NQ) continue;
                 const int gy = Y0 + q / R, gx = X0 + q % R;
-                a[q] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? acc[m][0][r] : 0.f;
+                a[q] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? acc[m][r] : 0.f;
             }
     }
     __syncthreads();
-    const float* res = smooth_lds(a, b2, R, K, X0, Y0, H, W);
-    smooth_store(res, R, K, X0, Y0, H, W, (long long)b * H * W, out);
+    const int q = min((int)threadIdx.x, NQ - 1), ry = q / R, rx = q - ry * R;
+    const int gy = Y0 + ry, gx = X0 + rx;
+    const bool inside = gx >= 0 && gx < W && gy >= 0 && gy < H;
+    // steps that update this cell: those below its distance to the region's edge
+    const int depth = inside ? min(min(rx, R - 1 - rx), min(ry, R - 1 - ry)) : 0;
+    const float cnt = (float)((gx > 0) + (gx < W - 1) + (gy > 0) + (gy < H - 1));
+    const int ql = max(q - 1, 0), qr = min(q + 1, NQ - 1), qu = max(q - R, 0),
+              qd = min(q + R, NQ - 1);
+    float c = a[q];
+#pragma unroll
+    for (int st = 1; st <= K; ++st) {
+        const float* src = st & 1 ? a : b2;
+        float sum = 0.f;
+        sum += src[ql];
+        sum += src[qr];
+        sum += src[qu];
+        sum += src[qd];
+        c = st <= depth ? c + 0.125f * (sum - cnt * c) : c;
+        if (st < K) {
+            (st & 1 ? b2 : a)[q] = c;  // (threads past the region: the last cell's value)
+            __syncthreads();
+        }
+    }
+    if (depth >= K && threadIdx.x < NQ)
+        out[((long long)b * H + gy) * W + gx] = c;
 }
 
 // operator residual u = cs * Lc y - x
@@ -1371,7 +1422,8 @@ size_t tiled_lds_limit(cd_context* c) {
                          reinterpret_cast<const void*>(&k_conv_pair_tile<1, 0, 0, false>),
                          reinterpret_cast<const void*>(&k_conv_pair_tile<2, 0, 0, true>),
                          reinterpret_cast<const void*>(&k_conv_pair_tile<2, 0, 0, false>),
-                         reinterpret_cast<const void*>(&k_head_smooth<6>)};
+                         reinterpret_cast<const void*>(&k_head_smooth<6, 0>),
+                         reinterpret_cast<const void*>(&k_head_smooth<6, 16>)};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
             hipSuccess) {
@@ -1847,9 +1899,14 @@ int finish_output(cd_net* n, int B, int H, int W, float* dst = nullptr) {
         const size_t lds = sizeof(u16) * ((size_t)P * P * (hd.c1 + 8) + 16 * (size_t)(hd.kpad + 8)) +
                            sizeof(float) * 2 * R * R;
         const dim3 grid(div_up(W, CT), div_up(H, CT), B);
-        hipLaunchKernelGGL(k_head_smooth<kHeadSmoothK>, grid, dim3(256), lds, n->ctx->stream,
-                           n->t[hd.in1].act.as<u16>(), hd.c1, n->wbf.as<u16>() + hd.woff, hd.kpad,
-                           H, W, y);
+        const u16* x = n->t[hd.in1].act.as<u16>();
+        const u16* wt = n->wbf.as<u16>() + hd.woff;
+        if (hd.c1 == 16)  // as in the shipped networks
+            hipLaunchKernelGGL((k_head_smooth<kHeadSmoothK, 16>), grid, dim3(512), lds,
+                               n->ctx->stream, x, hd.c1, wt, hd.kpad, H, W, y);
+        else
+            hipLaunchKernelGGL((k_head_smooth<kHeadSmoothK, 0>), grid, dim3(512), lds,
+                               n->ctx->stream, x, hd.c1, wt, hd.kpad, H, W, y);
         CD_CHECK_LAUNCH(n->ctx);
         return CD_OK;
     }
