@@ -440,20 +440,22 @@ __device__ __forceinline__ void nat_half(T (&ev)[2][NAT_R], const T (&rv)[2][NAT
     }
 }
 
-// Everything between the loads and the stores of a region: nsweeps sweeps.
-// edge_up / edge_down: the wave's first / last row has no row beyond it.
+// Everything between the loads and the stores of a region: nsweeps sweeps, of
+// which the wave takes part in the first `live`.  edge_up / edge_down: the wave's
+// first / last row has no row beyond it.
 template <typename T, int KIND, bool TRACK>
 __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
                                         const NatCells<T>& cl, T (*xch)[NAT_NW][2][64], T oc4,
                                         bool edge_up, bool edge_down, int wave, int lane,
-                                        int nsweeps, float (*smax)[NAT_NW][64], bool track0,
-                                        bool track1) {
+                                        int nsweeps, int live, float (*smax)[NAT_NW][64],
+                                        bool track0, bool track1) {
     const int wu = max(wave - 1, 0), wd = min(wave + 1, NAT_NW - 1);
     auto publish = [&](int c) {
         xch[c][wave][0][lane] = ev[c][0];
         xch[c][wave][1][lane] = ev[c][NAT_R - 1];
     };
-    for (int j = 0; j < nsweeps; ++j) {
+    const int mine = min(nsweeps, live);
+    for (int j = 0; j < mine; ++j) {
         T mx[2] = {(T)0, (T)0};
         T up, down;
         publish(1);
@@ -477,6 +479,11 @@ __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_
         if (TRACK) {
             smax[j][wave][lane] = fmaxf(track0 ? (float)mx[0] : 0.f, track1 ? (float)mx[1] : 0.f);
         }
+    }
+    for (int j = mine; j < nsweeps; ++j) {  // (no row of the wave counts for the maxima)
+        __syncthreads();
+        __syncthreads();
+        if (TRACK) smax[j][wave][lane] = 0.f;
     }
 }
 
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
         const TrackPlan plan =
             track_decide<NAT_NW>(track, st, tiles.ntiles, nsweeps, words, red);
         if (plan.nsweeps == 0) return;
-        nsweeps = plan.nsweeps;
+        nsweeps = __builtin_amdgcn_readfirstlane(plan.nsweeps);
         if (plan.redo) {
             const T* in = eout;
             eout = const_cast<T*>(ein);
@@ -560,15 +567,16 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     const bool rows_ok = (g.top || dy0 >= hl) && (g.bottom || dy0 + NAT_R <= NAT_RY - hl);
     auto col_ok = [&](int dx) { return rows_ok && (g.left || dx >= hl) && (g.right || dx < SW_RX - hl); };
     const bool t0 = TRACK && col_ok(2 * lane), t1 = TRACK && col_ok(2 * lane + 1);
+    const int live = live_sweeps<NAT_R, NAT_NW>(g, wave);
     const bool up0 = g.top && wave == 0, down0 = g.bottom && wave == NAT_NW - 1;
     if (mask)
-        nat_run<T, NAT_MASK, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, smax,
+        nat_run<T, NAT_MASK, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, live, smax,
                                     t0, t1);
     else if (general)
-        nat_run<T, NAT_EDGE, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, smax,
+        nat_run<T, NAT_EDGE, TRACK>(ev, rv, cl, xch, oc4, up0, down0, wave, lane, nsweeps, live, smax,
                                     t0, t1);
     else
-        nat_run<T, NAT_INNER, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, smax,
+        nat_run<T, NAT_INNER, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, live, smax,
                                      t0, t1);
 #pragma unroll
     for (int k = 0; k < NAT_R; ++k) {
@@ -605,12 +613,18 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 // and the update oc (S - cnt v - r) is formed explicitly, as the stop test
 // tracks it; a neighbour outside the grid contributes the cell's own value.
 //
-// What bounds it: dispatch, loads and stores take 4.3 us (R = 4) to 6.6 us
+// What bounds it: dispatch, loads and stores take about 5 us (R = 4) to 7 us
 // (R = 8) of a launch whatever its sweeps; a half-sweep of one region per CU
-// 0.19 to 0.28 us (0.13 / 0.27 us of it VALU issue, the rest the exchange's
-// latency), a further region per CU 2.9 us (R = 4, 5 sweeps) to 5.6 us (R = 8, 8
-// sweeps), where VALU issue and memory phases of two resident workgroups
-// overlap.  Taller regions lose less of their work to the halo, shorter ones
+// 0.14 to 0.27 us (0.13 / 0.27 us of it VALU issue of 16 full waves), a further
+// region per CU 3.0 us (R = 4, 5 sweeps) to 5.6 us (R = 8, 8 sweeps), where VALU
+// issue and memory phases of two resident workgroups overlap.  Two things cut
+// the VALU work: waves whose rows have all become inexact sit out the rest of a
+// launch (live_sweeps; a sixth of the work at R = 8, 16 sweeps), and border
+// tiles, which every barrier waits for, have a code path per kind of border
+// instead of selects per row.  Together 9.4 us for a launch of 14 sweeps at 400 x
+// 400 (10.2 before), 18.3 for 15 tracked sweeps at 768 x 768 (21.1 before).
+//
+// Taller regions lose less of their work to the halo, shorter ones
 // have the faster half-sweep, more sweeps per launch spread the fixed part over
 // a wider halo: blocked_plan weighs these.  Registers: 64 VGPRs (R = 8) keep two
 // workgroups per CU; row and column kinds per wave instead of a factor per cell
@@ -625,10 +639,14 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 constexpr int BK_NW = 16;  // waves per workgroup
 constexpr int BK_THREADS = 64 * BK_NW;
 
-// What a wave's rows meet: nothing but cells with four neighbours; also the
-// left or right grid border; also rows at or beyond the top or bottom border
-// (or, under the max-update rule, an odd width's right border).
-enum { BK_INNER = 0, BK_SIDE = 1, BK_ENDS = 2 };
+// What a wave's cells meet of the grid border, fixed per wave.  Columns: nothing;
+// the left border in lane 0 or the right one in lane 63 (odd cell), or neither;
+// a right border anywhere.  Rows: nothing; the wave's first row is the grid's
+// first; its last row is the grid's last; its last row lies below the grid's
+// last (odd heights); any.  The named rows cost nothing per sweep, a border
+// anywhere a select per cell and row.
+enum { COLS_IN = 0, COLS_LANES = 1, COLS_ANY = 2 };
+enum { ROWS_IN = 0, ROWS_TOP = 1, ROWS_BOTTOM = 2, ROWS_BELOW = 3, ROWS_ANY = 4 };
 
 // Per-lane facts of a region.  Index p: the lane's cell of column parity p.
 struct BlockCells {
@@ -649,49 +667,57 @@ struct BlockCells {
 // distance >= s are exact, and those read cells at distance >= s-1 only: the
 // stale values never reach the stored cells (distance >= halo) and stay finite
 // (each update is a bounded combination of finite values).
-template <int C, int KIND, bool TRACK, int R, int K0, int K1>
+template <int C, int COLS, int ROWS, bool TRACK, int R, int K0, int K1>
 __device__ __forceinline__ void blocked_half(float (&ev)[2][R], const float (&rv)[2][R],
                                              const BlockCells& g, unsigned end_rows,
                                              unsigned out_rows, float up_row, float down_row,
                                              float (&mx)[2]) {
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
+        if (ROWS == ROWS_BELOW && k == R - 1) continue;  // below the grid: stays 0
         const int p = (k + C) & 1;  // column parity of colour-C cells in row k (R even)
         const float o = ev[1 - C][k];
-        float up = k > 0 ? ev[1 - C][k - 1] : up_row;
-        float down = k < R - 1 ? ev[1 - C][k + 1] : down_row;
-        float left = p ? o : lane_prev(o);
-        float right = p ? lane_next(o) : o;
         const float v = ev[C][k];
-        float oc = KIND == BK_INNER ? g.om4 : g.oc[p];
-        if (KIND == BK_ENDS) {
+        const bool first = ROWS == ROWS_TOP && k == 0;
+        const bool last = (ROWS == ROWS_BOTTOM && k == R - 1) || (ROWS == ROWS_BELOW && k == R - 2);
+        // a neighbour row outside the grid
+        float up = first ? (TRACK ? v : 0.f) : k > 0 ? ev[1 - C][k - 1] : up_row;
+        float down = last ? (TRACK ? v : 0.f) : k < R - 1 ? ev[1 - C][k + 1] : down_row;
+        float oc = first || last ? g.oc_end[p] : COLS == COLS_IN ? g.om4 : g.oc[p];
+        if (ROWS == ROWS_ANY) {
             oc = (end_rows >> k) & 1u ? g.oc_end[p] : oc;
             oc = (out_rows >> k) & 1u ? 0.f : oc;
         }
         if (TRACK) {
-            if (KIND != BK_INNER) {
-                if (p == 0) left = g.miss_l ? v : left;
-                // (cell 0 has no right neighbour only where the width is odd)
-                if (p == 1 || KIND == BK_ENDS) right = g.miss_r[p] ? v : right;
-            }
-            if (KIND == BK_ENDS) {
+            if (ROWS == ROWS_ANY) {
                 if (k == 0) up = g.first ? v : up;
                 // (row k is the last in the grid where row k + 1 is not in it)
                 const bool below = k < R - 1 ? ((out_rows >> (k + 1)) & 1u) != 0 : g.last;
                 down = below ? v : down;
             }
-            const float t = __builtin_fmaf(-4.f, v, left + up + right + down) - rv[C][k];
+            float s;  // left + up + right
+            if (COLS == COLS_IN) {
+                s = (p ? o : lane_prev(o)) + up + (p ? lane_next(o) : o);
+            } else if (p == 0) {
+                s = add_prev(o, up, v) + (COLS == COLS_ANY && g.miss_r[0] ? v : o);
+            } else if (COLS == COLS_LANES) {
+                s = add_next(o, o + up, v);
+            } else {
+                const float right = lane_next(o);  // (in every lane, before the select)
+                s = o + up + (g.miss_r[1] ? v : right);
+            }
+            const float t = __builtin_fmaf(-4.f, v, s + down) - rv[C][k];
             const float dl = oc * t;
             ev[C][k] = v + dl;
             mx[p] = fmaxf(mx[p], fabsf(dl));  // (0, or a NaN that fmaxf drops, where oc = 0)
         } else {
-            const float sum = left + up + right + down;
+            const float sum = (p ? o : lane_prev(o)) + up + (p ? lane_next(o) : o) + down;
             ev[C][k] = __builtin_fmaf(oc, sum, __builtin_fmaf(g.c1, v, rv[C][k]));
         }
     }
 }
 
-template <int C, int KIND, bool TRACK, int R>
+template <int C, int COLS, int ROWS, bool TRACK, int R>
 __device__ __forceinline__ void blocked_step(float (&ev)[2][R], const float (&rv)[2][R],
                                              float (*xch)[BK_NW][2][64], const BlockCells& g,
                                              int wave, int lane, float (&mx)[2]) {
@@ -700,40 +726,65 @@ __device__ __forceinline__ void blocked_step(float (&ev)[2][R], const float (&rv
     xch[1 - C][wave][1][lane] = ev[1 - C][R - 1];
     // the row kinds are re-read each half-sweep, so that the factors derived
     // from them are not kept in registers per row
-    unsigned er = __builtin_amdgcn_readfirstlane(g.end_rows);
-    unsigned ou = __builtin_amdgcn_readfirstlane(g.out_rows);
-    if (KIND == BK_ENDS) asm volatile("" : "+s"(er), "+s"(ou));
+    unsigned er = 0, ou = 0;
+    if (ROWS == ROWS_ANY) {
+        er = __builtin_amdgcn_readfirstlane(g.end_rows);
+        ou = __builtin_amdgcn_readfirstlane(g.out_rows);
+        asm volatile("" : "+s"(er), "+s"(ou));
+    }
     // the inner rows need only this wave's registers: update them while the
     // other waves reach the barrier (the order of the updates of one colour
     // does not matter: they read only the other colour)
-    blocked_half<C, KIND, TRACK, R, 1, R - 1>(ev, rv, g, er, ou, 0.f, 0.f, mx);
+    blocked_half<C, COLS, ROWS, TRACK, R, 1, R - 1>(ev, rv, g, er, ou, 0.f, 0.f, mx);
     __syncthreads();
     float up_row = xch[1 - C][wave > 0 ? wave - 1 : 0][1][lane];
     float down_row = xch[1 - C][wave < BK_NW - 1 ? wave + 1 : BK_NW - 1][0][lane];
-    if (KIND == BK_ENDS && !TRACK) {
+    if (ROWS == ROWS_ANY && !TRACK) {
         up_row = g.first ? 0.f : up_row;
         down_row = g.last ? 0.f : down_row;
     }
-    blocked_half<C, KIND, TRACK, R, 0, 1>(ev, rv, g, er, ou, up_row, down_row, mx);
-    blocked_half<C, KIND, TRACK, R, R - 1, R>(ev, rv, g, er, ou, up_row, down_row, mx);
+    blocked_half<C, COLS, ROWS, TRACK, R, 0, 1>(ev, rv, g, er, ou, up_row, down_row, mx);
+    blocked_half<C, COLS, ROWS, TRACK, R, R - 1, R>(ev, rv, g, er, ou, up_row, down_row, mx);
 }
 
-// nsweeps sweeps of a region.  The waves of a workgroup may take this with
-// different KINDs (a choice uniform over the wave): each executes the same
-// number of barriers.
-template <int KIND, bool TRACK, int R>
+// nsweeps sweeps of a region, of which the wave takes part in the first `live`.
+// The waves of a workgroup may take this with different kinds of columns and
+// rows: each executes the same number of barriers.
+template <int COLS, int ROWS, bool TRACK, int R>
 __device__ __forceinline__ void blocked_run(float (&ev)[2][R], const float (&rv)[2][R],
                                             float (*xch)[BK_NW][2][64], const BlockCells& g,
-                                            int wave, int lane, int nsweeps,
+                                            int wave, int lane, int nsweeps, int live,
                                             float (*smax)[BK_NW][64], bool track0, bool track1) {
-    for (int j = 0; j < nsweeps; ++j) {
+    const int mine = min(nsweeps, live);
+    for (int j = 0; j < mine; ++j) {
         float mx[2] = {0.f, 0.f};
-        blocked_step<0, KIND, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
-        blocked_step<1, KIND, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
+        blocked_step<0, COLS, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
+        blocked_step<1, COLS, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, mx);
         if (TRACK) {
             smax[j][wave][lane] = fmaxf(track0 ? mx[0] : 0.f, track1 ? mx[1] : 0.f);
         }
     }
+    for (int j = mine; j < nsweeps; ++j) {  // (no row of the wave counts for the maxima)
+        __syncthreads();
+        __syncthreads();
+        if (TRACK) smax[j][wave][lane] = 0.f;
+    }
+}
+
+// The wave's kinds (uniform) for its R rows from Yw on and the region's columns
+// from X0 on.  Without tracking the columns beyond a border hold zeros wherever
+// it lies.
+template <int R, bool TRACK>
+__device__ __forceinline__ int cols_kind(bool left, bool right, int X0, int w) {
+    if (!left && !right) return COLS_IN;
+    return !TRACK || !right || X0 + SW_RX == w ? COLS_LANES : COLS_ANY;
+}
+template <int R>
+__device__ __forceinline__ int rows_kind(int Yw, int h) {
+    if (Yw > 0 && Yw + R < h) return ROWS_IN;
+    if (Yw + R < h) return ROWS_TOP;
+    if (Yw > 0 && Yw + R == h) return ROWS_BOTTOM;
+    return Yw > 0 && Yw + R == h + 1 ? ROWS_BELOW : ROWS_ANY;
 }
 
 // The intermediate-grid correction em (bricked, wm x hm, fm x fm fine cells
@@ -858,7 +909,7 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         const TrackPlan plan =
             track_decide<BK_NW>(track, st, tiles.ntiles, nsweeps, words, red);
         if (plan.nsweeps == 0) return;
-        nsweeps = plan.nsweeps;
+        nsweeps = __builtin_amdgcn_readfirstlane(plan.nsweeps);
         if (plan.redo) {
             out_index ^= 1;
             region_load<R, PROLONG>(ev, rr, eout_rs, r_rs, bk, mid, patch, rg.X0, rg.Y0, w, h,
@@ -890,9 +941,8 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         g.oc[p] = in ? (side ? om3 : om4) : 0.f;
         g.oc_end[p] = in ? (side ? om2 : om3) : 0.f;
     }
-    // (uniform over the wave)
-    const int kind = (g.first || g.last || (TRACK && rg.right && (w & 1))) ? BK_ENDS
-                     : (rg.left || rg.right) ? BK_SIDE : BK_INNER;
+    const int cols = cols_kind<R, TRACK>(rg.left, rg.right, rg.X0, w), rows = rows_kind<R>(Yw, h);
+    const bool inner = cols == COLS_IN && rows == ROWS_IN;
 #pragma unroll
     for (int k = 0; k < R; ++k)
 #pragma unroll
@@ -900,7 +950,7 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
             const int p = (k + c) & 1;
             const float rc = rhs_to_f32(rr[c][k]);
             float oc = g.om4;
-            if (kind != BK_INNER) {
+            if (!inner) {
                 const bool out = (g.out_rows >> k) & 1u;
                 oc = out ? 0.f : (g.end_rows >> k) & 1u ? g.oc_end[p] : g.oc[p];
                 const bool in = !out && x0 + p < w;
@@ -923,12 +973,15 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         t0 = col_ok(2 * lane);
         t1 = col_ok(2 * lane + 1);
     }
-    if (kind == BK_INNER)
-        blocked_run<BK_INNER, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
-    else if (kind == BK_SIDE)
-        blocked_run<BK_SIDE, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
-    else
-        blocked_run<BK_ENDS, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, smax, t0, t1);
+    const int live = live_sweeps<R, BK_NW>(rg, wave);
+#define RUN(COLS, ROWS) blocked_run<COLS, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, live, smax, t0, t1)
+    if (inner) RUN(COLS_IN, ROWS_IN);
+    else if (cols == COLS_ANY || rows == ROWS_ANY) RUN(COLS_ANY, ROWS_ANY);
+    else if (rows == ROWS_IN) RUN(COLS_LANES, ROWS_IN);
+    else if (rows == ROWS_TOP) RUN(COLS_LANES, ROWS_TOP);
+    else if (rows == ROWS_BOTTOM) RUN(COLS_LANES, ROWS_BOTTOM);
+    else RUN(COLS_LANES, ROWS_BELOW);
+#undef RUN
     // store
     const unsigned col = brick_col(min(rg.X0 / 2 + lane, (w + 1) / 2 - 1));
 #pragma unroll
@@ -1062,7 +1115,7 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
         g.oc[p] = in ? (side ? a.om3 : a.om4) : 0.f;
         g.oc_end[p] = in ? (side ? a.om2 : a.om3) : 0.f;
     }
-    const bool ends = g.first || g.last || (TRACK && (w & 1));  // (uniform over the wave)
+    const int rows = rows_kind<R>(Yw, h);  // (uniform over the wave)
 
     double ph[2][R];
     float ev[2][R], rv[2][R];
@@ -1134,8 +1187,12 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
     };
     auto sweep = [&](int n) {
         n = __builtin_amdgcn_readfirstlane(n);  // (the same in every thread)
-        if (ends) blocked_run<BK_ENDS, TRACK, R>(ev, rv, xch, g, wave, lane, n, smax, true, true);
-        else blocked_run<BK_SIDE, TRACK, R>(ev, rv, xch, g, wave, lane, n, smax, true, true);
+#define RUN(ROWS) blocked_run<COLS_ANY, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, n, INT_MAX, smax, true, true)
+        if (rows == ROWS_IN) RUN(ROWS_IN);
+        else if (rows == ROWS_TOP) RUN(ROWS_TOP);
+        else if (rows == ROWS_BOTTOM) RUN(ROWS_BOTTOM);
+        else RUN(ROWS_ANY);
+#undef RUN
     };
     // the first of n <= kStopGroup sweeps whose largest update is below tol
     double last_max = a.resume ? st->last_max_update : INFINITY;
@@ -1304,15 +1361,16 @@ struct BlockedPlan {
 
 // Time of a launch of `sweeps` sweeps over ntiles regions of 16 waves x `rows`
 // rows, in us: a first region per CU, then every further one.  Fitted to
-// launches of 5 to 16 sweeps on grids of 128 to 4096 squared (rows 4: 6.2 us for
-// 5 sweeps of up to 256 regions, 9.7 for 14; rows 8: 11.2 for 8, 16.1 with two
-// regions per CU, 50.3 with eight).  Tracking launches have about twice the VALU
+// launches of 4 to 19 sweeps on grids of 300 to 4096 squared, to 3 % (rows 4: 6.5
+// us for 5 sweeps of up to 256 regions, 9.4 for 14; rows 8: 11.2 for 8, 15.7 with
+// two regions per CU, 49.9 with eight); a half costs less than a launch's first
+// ones because waves at the inner borders sit out the later ones.  Tracking launches have about twice the VALU
 // work per sweep and, at 8 rows, one workgroup per CU.
 double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
     struct Cost { double first, first_half, next, next_half; };
     static constexpr Cost cost[2][3] = {
-        {{4.3, 0.194, 2.45, 0.042}, {5.2, 0.234, 3.2, 0.093}, {6.6, 0.283, 3.9, 0.125}},
-        {{5.7, 0.345, 3.0, 0.135}, {7.4, 0.45, 4.2, 0.17}, {8.8, 0.525, 8.0, 0.36}}};
+        {{5.4, 0.133, 2.9, 0.013}, {6.0, 0.207, 3.6, 0.042}, {6.8, 0.269, 4.5, 0.068}},
+        {{7.5, 0.222, 3.8, 0.060}, {8.1, 0.322, 4.6, 0.116}, {8.9, 0.457, 7.5, 0.336}}};
     const Cost& c = cost[track][(rows - 4) / 2];
     const int halves = 2 * sweeps;
     return c.first + c.first_half * halves +
@@ -1320,9 +1378,9 @@ double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
 }
 
 // The cut of a batch of `batch` sweeps on a w x h grid that blocked_launch_us
-// finds cheapest.  Per sweep, measured: 2048 x 2048 1.87 us (8 rows, 9 sweeps;
-// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 1.01 (8, 16; 1.31), 400 x 400 0.74
-// (4, 14; 1.29).  Tracking launches take whole groups, a halo of whole waves,
+// finds cheapest.  Per sweep, measured: 2048 x 2048 1.82 us (8 rows, 9 sweeps;
+// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 0.95 (8, 17; 1.29), 400 x 400 0.67
+// (4, 14; 1.28); tracked, 400 x 400 1.18 (6, 15; 1.92 with 4 rows, 5 sweeps).  Tracking launches take whole groups, a halo of whole waves,
 // and need room for two TrackOut in track_room bytes.
 BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room) {
     BlockedPlan best{4, kStopGroup, sweep_tiles(w, h, BK_NW * 4, 2 * kStopGroup)};
@@ -1330,7 +1388,7 @@ BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room)
     batch = std::max(batch, 1);
     for (int rows = 4; rows <= 8; rows += 2) {
         const int ry = BK_NW * rows, unit = track ? kStopGroup : 1;
-        const int most = track ? kTrackSweeps / unit * unit : 16;
+        const int most = track ? kTrackSweeps / unit * unit : 19;
         for (int sweeps = unit; sweeps <= most; sweeps += unit) {
             const int halo = track ? div_up(2 * sweeps, rows) * rows : 2 * sweeps;
             if (ry - 2 * halo < 8) break;

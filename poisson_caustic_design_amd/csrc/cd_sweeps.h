@@ -74,6 +74,18 @@ __device__ __forceinline__ Region region_of(const SweepTiles& t, int tile) {
     return g;
 }
 
+// Sweeps (from the first) that wave `wave` of a region takes part in.  After
+// half-sweep s only rows at distance >= s from an inner border are exact, and
+// only those are read by exact ones later, so a wave whose rows all lie nearer
+// need not update them: of the (wave + 1) R rows up to its last (counted from the
+// inner border), the last is still exact after (wave + 1) R - 1 half-sweeps, and
+// read by the next.  After that the wave only meets the barriers.
+template <int R, int NW>
+__device__ __forceinline__ int live_sweeps(const Region& g, int wave) {
+    static_assert(R % 2 == 0, "whole sweeps");
+    return min(g.top ? INT_MAX : (wave + 1) * R / 2, g.bottom ? INT_MAX : (NW - wave) * R / 2);
+}
+
 // XCD-aware tile order: gridDim.x is a multiple of 8 and consecutive workgroups
 // go round-robin to the 8 XCDs; each XCD gets a contiguous band of tiles so
 // that halo re-reads hit its own L2.  May return a tile >= ntiles.
@@ -98,6 +110,22 @@ __device__ __forceinline__ double lane_next(double v) {
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true);
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
+}
+
+// lane_prev(v) + b, and in lane 0 own + b; lane_next(v) + b, and in lane 63
+// own + b: an add with a wave shift does not write the lane without a source.
+// (DPP reads a register two wait states after it was written, at the earliest.)
+__device__ __forceinline__ float add_prev(float v, float b, float own) {
+    float s = own + b;
+    asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %2 wave_shr:1 row_mask:0xf bank_mask:0xf"
+        : "+v"(s) : "v"(v), "v"(b));
+    return s;
+}
+__device__ __forceinline__ float add_next(float v, float b, float own) {
+    float s = own + b;
+    asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %2 wave_shl:1 row_mask:0xf bank_mask:0xf"
+        : "+v"(s) : "v"(v), "v"(b));
+    return s;
 }
 
 // ---------------------------------------------------------------------------

@@ -111,7 +111,7 @@ def residual_rule_sweeps(b, p0, k, omega):
     return p0 + e.astype(np.float64)
 
 
-# regions of 64, 96 and 128 rows; launches of 5 to 16 sweeps
+# regions of 64, 96 and 128 rows; launches of up to 19 sweeps
 BLOCKED = SIZES + [(128, 96), (129, 97), (128, 128), (127, 129), (640, 1030), (1024, 700)]
 
 
@@ -143,6 +143,15 @@ def test_blocked_sweeps_max_update_rule(ctx, oracle, rng, w, h, k):
     assert st.sweeps == k
     scale = np.abs(ref - p0).max()
     assert np.abs(g - ref).max() <= 8 * k * 2.0 ** -24 * scale, (w, h)
+
+
+# odd and even sides over several regions: border cells in a region's last lane
+# or before it, a wave's last row on, above or below the grid's last row, waves
+# that sit out a launch's later sweeps on one side and on both
+@pytest.mark.parametrize("w,h", [(255, 301), (254, 302), (400, 257), (129, 999), (300, 130)])
+def test_blocked_sweeps_borders(ctx, oracle, rng, w, h):
+    test_blocked_sweeps_residual_rule(ctx, rng, w, h, 45)
+    test_blocked_sweeps_max_update_rule(ctx, oracle, rng, w, h, 45)
 
 
 @pytest.mark.parametrize("w,h", [(61, 40), (128, 64), (200, 136), (333, 129), (640, 520)])
