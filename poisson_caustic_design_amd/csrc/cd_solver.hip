@@ -495,7 +495,7 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     __shared__ T xch[2][NAT_NW][2][64];
     __shared__ float smax[TRACK ? kTrackSweeps : 1][NAT_NW][64];
     __shared__ unsigned red[TRACK ? NAT_NW : 1];
-    const int tile = tile_of_block();
+    const int tile = tile_of_block(tiles.ntiles);
     if (tile >= tiles.ntiles) return;
     const Region g = region_of(tiles, tile);
     const int w = tiles.w, h = tiles.h;
@@ -613,16 +613,20 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 // and the update oc (S - cnt v - r) is formed explicitly, as the stop test
 // tracks it; a neighbour outside the grid contributes the cell's own value.
 //
-// What bounds it: dispatch, loads and stores take about 5 us (R = 4) to 7 us
+// What bounds it: dispatch, loads and stores take 4.7 us (R = 4) to 5.6 us
 // (R = 8) of a launch whatever its sweeps; a half-sweep of one region per CU
 // 0.14 to 0.27 us (0.13 / 0.27 us of it VALU issue of 16 full waves), a further
-// region per CU 3.0 us (R = 4, 5 sweeps) to 5.6 us (R = 8, 8 sweeps), where VALU
+// region per CU 2.0 us (R = 4, 5 sweeps) to 6 us (R = 8, 8 sweeps), where VALU
 // issue and memory phases of two resident workgroups overlap.  Two things cut
 // the VALU work: waves whose rows have all become inexact sit out the rest of a
 // launch (live_sweeps; a sixth of the work at R = 8, 16 sweeps), and border
 // tiles, which every barrier waits for, have a code path per kind of border
 // instead of selects per row.  Together 9.4 us for a launch of 14 sweeps at 400 x
-// 400 (10.2 before), 18.3 for 15 tracked sweeps at 768 x 768 (21.1 before).
+// 400 (10.2 before), 18.3 for 15 tracked sweeps at 768 x 768 (21.1 before).  And
+// what surrounds the sweeps was more scalar work than it looks: row addresses
+// from the two bricks a wave's rows touch, one branch for all cells between inner
+// and border tiles, stores grouped by column, no division, arguments read in one
+// go (8.6 us, 17.2; 2048 x 2048 16.6 -> 15.3 for 9 sweeps).
 //
 // Taller regions lose less of their work to the halo, shorter ones
 // have the faster half-sweep, more sweeps per launch spread the fixed part over
@@ -796,9 +800,27 @@ struct MidGrid {
     int wm, hm, fm;
 };
 
+// Plane offsets (elements) of R <= 8 consecutive rows from Y on: they lie in at
+// most two bricks, so that one select per row and a constant give each.  Rows
+// beyond the plane's last brick get the offset of some row in it.
+struct BrickRows {
+    unsigned a, b;  // offset of row k less 64 k, before and from the brick border on
+    int split;
+    __device__ __forceinline__ unsigned at(int k) const { return (k < split ? a : b) + 64u * k; }
+};
+__device__ __forceinline__ BrickRows brick_rows(const Brick& bk, int Y, int h) {
+    const int nby = (h + 7) >> 3, by = min(Y >> 3, nby - 1);
+    const unsigned brow = (unsigned)bk.nbx * 512u;
+    BrickRows r;
+    r.a = (unsigned)by * brow + (unsigned)(Y & 7) * 64u;
+    r.b = r.a - 512u + (by + 1 < nby ? brow : 0u);
+    r.split = 8 - (Y & 7);
+    return r;
+}
+
 // Loads of one region: packed column `lane` of the wave's R rows, both colours,
-// from the correction and the right-hand side.  Rows and columns are clamped
-// into the grid.
+// from the correction and the right-hand side.  Columns are clamped into the
+// grid; what rows outside it load is not used.
 // PROLONG: the correction is the intermediate-grid correction interpolated
 // bilinearly at the cell centres (u, v) = ((x, y) + 0.5) / fm - 0.5, not ein;
 // the workgroup first stages the intermediate cells its region needs in
@@ -807,14 +829,18 @@ struct MidGrid {
 template <int R>
 constexpr int kPatchMax = (SW_RX / 2 + 2) * (BK_NW * R / 2 + 2);  // fm >= 2
 template <int R, bool PROLONG, typename RT>
-__device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R],
-                                            __amdgpu_buffer_rsrc_t ein_rs,
-                                            __amdgpu_buffer_rsrc_t r_rs, const Brick& bk,
-                                            const MidGrid& mid, float* patch, int X0, int Y0,
-                                            int w, int h, int wave, int lane) {
+__device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R], const float* ein,
+                                            const RT* rhs, const Brick& bk, const MidGrid& mid,
+                                            float* patch, int X0, int Y0, int w, int h, int wave,
+                                            int lane) {
     const int Yw = Y0 + R * wave;
     const int j = min(X0 / 2 + lane, (w + 1) / 2 - 1);
     const unsigned col = brick_col(j);
+    const BrickRows br = brick_rows(bk, Yw, h);
+    const __amdgpu_buffer_rsrc_t e_rs[2] = {plane_rsrc(ein, bk.plane * sizeof(float)),
+                                            plane_rsrc(ein + bk.plane, bk.plane * sizeof(float))};
+    const __amdgpu_buffer_rsrc_t r_rs[2] = {plane_rsrc(rhs, bk.plane * sizeof(RT)),
+                                            plane_rsrc(rhs + bk.plane, bk.plane * sizeof(RT))};
     int pi0[2] = {0, 0}, pj0 = 0, pw = 0;
     float ptu[2] = {0.f, 0.f};
     const float inv = PROLONG ? 1.f / mid.fm : 0.f;
@@ -846,18 +872,18 @@ __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R],
     }
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-        const int Yc = min(Yw + k, h - 1);
         int r0 = 0;
         float tv = 0.f;
+        const int Yc = min(Yw + k, h - 1);
         if (PROLONG) {
             const float v = (Yc + 0.5f) * inv - 0.5f;
             const int j0 = (int)floorf(v);
             tv = v - j0;
             r0 = (j0 - pj0) * pw;
         }
+        const unsigned row = br.at(k) - 64u * k;  // (64 k goes into the instruction)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const unsigned row = (unsigned)brick_row(bk, c, Yc);
             if (PROLONG) {
                 const int t = (c + Yc) & 1;
                 const float tu = ptu[t];
@@ -865,9 +891,10 @@ __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R],
                 const float a = pp[0], b = pp[1], cc = pp[pw], d = pp[pw + 1];
                 ev[c][k] = (a * (1.f - tu) + b * tu) * (1.f - tv) + (cc * (1.f - tu) + d * tu) * tv;
             } else {
-                ev[c][k] = buf_load<float>(ein_rs, col * 4u, row * 4u);
+                ev[c][k] = buf_load<float>(e_rs[c], (col + 64u * k) * 4u, row * 4u);
             }
-            rr[c][k] = buf_load<RT>(r_rs, col * (unsigned)sizeof(RT), row * (unsigned)sizeof(RT));
+            rr[c][k] = buf_load<RT>(r_rs[c], (col + 64u * k) * (unsigned)sizeof(RT),
+                                    row * (unsigned)sizeof(RT));
         }
     }
 }
@@ -887,21 +914,26 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
     __shared__ float smax[TRACK ? kTrackSweeps : 1][BK_NW][64];
     __shared__ unsigned red[TRACK ? BK_NW : 1];
     __shared__ float patch[PROLONG ? kPatchMax<R> : 1];
-    const int tile = tile_of_block();
+    // What the loads' addresses need is read in one go, and nothing else comes
+    // before them (400 x 400: 8.9 -> 8.6 us a launch); not where that spills
+    // scalars into the few vector registers left (3 % slower there).
+    constexpr bool kLoadsFirst = !TRACK || R > 6;
+    if (kLoadsFirst)
+        asm volatile("" ::"s"(ein), "s"(rhs), "s"(rmean), "s"(bk.nbx), "s"(bk.plane),
+                     "s"(tiles.ntiles), "s"(tiles.inv_x), "s"(tiles.ix));
+    const int tile = tile_of_block(tiles.ntiles);
     if (tile >= tiles.ntiles) return;
     const Region rg = region_of(tiles, tile);
     const int w = tiles.w, h = tiles.h;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     using RT = typename std::conditional<TRACK, float, unsigned short>::type;
-    const size_t npk = 2 * bk.plane;
-    const __amdgpu_buffer_rsrc_t ein_rs = plane_rsrc(ein, npk * sizeof(float));
-    const __amdgpu_buffer_rsrc_t r_rs = plane_rsrc(rhs, npk * sizeof(RT));
-    __amdgpu_buffer_rsrc_t eout_rs = plane_rsrc(eout, npk * sizeof(float));
+    const RT* r = static_cast<const RT*>(rhs);
     float ev[2][R], rv[2][R];
     RT rr[2][R];
     const unsigned words = TRACK ? track_load<BK_NW>(track, tiles.ntiles) : 0u;
-    region_load<R, PROLONG>(ev, rr, ein_rs, r_rs, bk, mid, patch, rg.X0, rg.Y0, w, h, wave, lane);
+    region_load<R, PROLONG>(ev, rr, ein, r, bk, mid, patch, rg.X0, rg.Y0, w, h, wave, lane);
+    if (kLoadsFirst) __builtin_amdgcn_sched_barrier(0);
     // Max-update rule: the solve can have stopped in an earlier launch of the
     // batch, and then leaves the buffers untouched.  Residual rule: only a check
     // stops it, and no sweeps are enqueued after that.
@@ -912,9 +944,9 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         nsweeps = __builtin_amdgcn_readfirstlane(plan.nsweeps);
         if (plan.redo) {
             out_index ^= 1;
-            region_load<R, PROLONG>(ev, rr, eout_rs, r_rs, bk, mid, patch, rg.X0, rg.Y0, w, h,
-                                    wave, lane);
-            eout_rs = ein_rs;
+            region_load<R, PROLONG>(ev, rr, eout, r, bk, mid, patch, rg.X0, rg.Y0, w, h, wave,
+                                    lane);
+            eout = const_cast<float*>(ein);
         }
     }
     const float rm = *rmean;
@@ -942,25 +974,6 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         g.oc_end[p] = in ? (side ? om2 : om3) : 0.f;
     }
     const int cols = cols_kind<R, TRACK>(rg.left, rg.right, rg.X0, w), rows = rows_kind<R>(Yw, h);
-    const bool inner = cols == COLS_IN && rows == ROWS_IN;
-#pragma unroll
-    for (int k = 0; k < R; ++k)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int p = (k + c) & 1;
-            const float rc = rhs_to_f32(rr[c][k]);
-            float oc = g.om4;
-            if (!inner) {
-                const bool out = (g.out_rows >> k) & 1u;
-                oc = out ? 0.f : (g.end_rows >> k) & 1u ? g.oc_end[p] : g.oc[p];
-                const bool in = !out && x0 + p < w;
-                ev[c][k] = in ? ev[c][k] : 0.f;
-                if (TRACK) rv[c][k] = in ? rc - rm : 0.f;
-                else rv[c][k] = (rm - rc) * oc;
-            } else {
-                rv[c][k] = TRACK ? rc - rm : (rm - rc) * oc;
-            }
-        }
     // the cells whose updates count for the stop rule: those at distance >= halo
     // from the region's inner borders (all exact; two tiles may count one)
     bool t0 = false, t1 = false;
@@ -973,28 +986,68 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         t0 = col_ok(2 * lane);
         t1 = col_ok(2 * lane + 1);
     }
-    const int live = live_sweeps<R, BK_NW>(rg, wave);
-#define RUN(COLS, ROWS) blocked_run<COLS, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, live, smax, t0, t1)
-    if (inner) RUN(COLS_IN, ROWS_IN);
-    else if (cols == COLS_ANY || rows == ROWS_ANY) RUN(COLS_ANY, ROWS_ANY);
-    else if (rows == ROWS_IN) RUN(COLS_LANES, ROWS_IN);
-    else if (rows == ROWS_TOP) RUN(COLS_LANES, ROWS_TOP);
-    else if (rows == ROWS_BOTTOM) RUN(COLS_LANES, ROWS_BOTTOM);
-    else RUN(COLS_LANES, ROWS_BELOW);
-#undef RUN
-    // store
-    const unsigned col = brick_col(min(rg.X0 / 2 + lane, (w + 1) / 2 - 1));
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int Y = Yw + k;
-        if (Y < rg.ys0 || Y >= rg.ys1) continue;  // uniform
+    for (int k = 0; k < R; ++k)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const int x = x0 + ((k + c) & 1);
-            if (x >= rg.xs0 && x < rg.xs1)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ev[c][k]), eout_rs, col * 4u,
-                                                      (unsigned)brick_row(bk, c, Y) * 4u,
-                                                      CD_BK_STORE_POLICY);
+            const float rc = rhs_to_f32(rr[c][k]);
+            rv[c][k] = TRACK ? rc - rm : rm - rc;
+        }
+    int kind = cols == COLS_IN && rows == ROWS_IN ? -1
+               : cols == COLS_ANY ? (int)ROWS_ANY : rows;
+    // (one branch for all cells, kept apart from the choice of the sweeps' path)
+    if (kind >= 0) {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int p = (k + c) & 1;
+                const bool out = (g.out_rows >> k) & 1u;
+                const float oc = out ? 0.f : (g.end_rows >> k) & 1u ? g.oc_end[p] : g.oc[p];
+                const bool in = !out && x0 + p < w;
+                ev[c][k] = in ? ev[c][k] : 0.f;
+                rv[c][k] = !TRACK ? rv[c][k] * oc : in ? rv[c][k] : 0.f;
+            }
+    } else if (!TRACK) {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) rv[c][k] *= g.om4;
+    }
+    kind = __builtin_amdgcn_readfirstlane(kind);
+    asm volatile("" : "+s"(kind));
+    const int live = live_sweeps<R, BK_NW>(rg, wave);
+#define RUN(COLS, ROWS) blocked_run<COLS, ROWS, TRACK, R>(ev, rv, xch, g, wave, lane, nsweeps, live, smax, t0, t1)
+    if (kind < 0) RUN(COLS_IN, ROWS_IN);
+    else if (kind == ROWS_IN) RUN(COLS_LANES, ROWS_IN);
+    else if (kind == ROWS_TOP) RUN(COLS_LANES, ROWS_TOP);
+    else if (kind == ROWS_BOTTOM) RUN(COLS_LANES, ROWS_BOTTOM);
+    else if (kind == ROWS_BELOW) RUN(COLS_LANES, ROWS_BELOW);
+    else RUN(COLS_ANY, ROWS_ANY);
+#undef RUN
+    // store: the lane's two columns, each with the wave's rows of the region
+    const unsigned col = brick_col(min(rg.X0 / 2 + lane, (w + 1) / 2 - 1));
+    const BrickRows br = brick_rows(bk, Yw, h);
+    const __amdgpu_buffer_rsrc_t out_rs[2] = {plane_rsrc(eout, bk.plane * sizeof(float)),
+                                              plane_rsrc(eout + bk.plane, bk.plane * sizeof(float))};
+    const bool all_rows = Yw >= rg.ys0 && Yw + R <= rg.ys1;
+    if (Yw + R > rg.ys0 && Yw < rg.ys1) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (x0 + p < rg.xs0 || x0 + p >= rg.xs1) continue;
+            auto store = [&](int k) {
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    __float_as_uint(ev[(k + p) & 1][k]), out_rs[(k + p) & 1], (col + 64u * k) * 4u,
+                    (br.at(k) - 64u * k) * 4u, CD_BK_STORE_POLICY);
+            };
+            if (all_rows) {
+#pragma unroll
+                for (int k = 0; k < R; ++k) store(k);
+            } else {
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    if (Yw + k >= rg.ys0 && Yw + k < rg.ys1) store(k);
+            }
         }
     }
     if (TRACK) track_store<BK_NW>(track, smax, red, tile, nsweeps, wave, lane);
@@ -1360,27 +1413,31 @@ struct BlockedPlan {
 };
 
 // Time of a launch of `sweeps` sweeps over ntiles regions of 16 waves x `rows`
-// rows, in us: a first region per CU, then every further one.  Fitted to
-// launches of 4 to 19 sweeps on grids of 300 to 4096 squared, to 3 % (rows 4: 6.5
-// us for 5 sweeps of up to 256 regions, 9.4 for 14; rows 8: 11.2 for 8, 15.7 with
-// two regions per CU, 49.9 with eight); a half costs less than a launch's first
-// ones because waves at the inner borders sit out the later ones.  Tracking launches have about twice the VALU
-// work per sweep and, at 8 rows, one workgroup per CU.
+// rows, in us: a first region per CU, a second (resident beside it, except
+// tracked at 8 rows), then every further one.  Fitted to launches of 4 to 19
+// sweeps on grids of 300 to 4096 squared, to 1 to 3 % (rows 4: 6.1 us for 5
+// sweeps of up to 256 regions, 8.6 for 14; rows 8: 10.0 for 8, 14.0 with two
+// regions per CU, 44.4 with nine); a half costs less than a launch's first ones
+// because waves at the inner borders sit out the later ones.
 double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
-    struct Cost { double first, first_half, next, next_half; };
-    static constexpr Cost cost[2][3] = {
-        {{5.4, 0.133, 2.9, 0.013}, {6.0, 0.207, 3.6, 0.042}, {6.8, 0.269, 4.5, 0.068}},
-        {{7.5, 0.222, 3.8, 0.060}, {8.1, 0.322, 4.6, 0.116}, {8.9, 0.457, 7.5, 0.336}}};
+    struct Cost { double first, first_half, second, second_half, next, next_half; };
+    static constexpr Cost cost[2][3] = {{{4.7, 0.142, 1.9, 0.005, 2.5, 0.023},
+                                         {5.1, 0.205, 1.7, 0.063, 4.0, 0.025},
+                                         {5.6, 0.268, 2.4, 0.100, 5.3, 0.042}},
+                                        {{6.9, 0.246, 3.2, 0.045, 3.5, 0.080},
+                                         {7.1, 0.332, 3.1, 0.137, 4.0, 0.134},
+                                         {7.4, 0.440, 8.0, 0.287, 6.4, 0.352}}};
     const Cost& c = cost[track][(rows - 4) / 2];
-    const int halves = 2 * sweeps;
-    return c.first + c.first_half * halves +
-           (c.next + c.next_half * halves) * (div_up(ntiles, 256) - 1);
+    const int halves = 2 * sweeps, rounds = div_up(ntiles, 256);
+    return c.first + c.first_half * halves + (rounds > 1 ? c.second + c.second_half * halves : 0.0) +
+           (c.next + c.next_half * halves) * std::max(rounds - 2, 0);
 }
 
 // The cut of a batch of `batch` sweeps on a w x h grid that blocked_launch_us
-// finds cheapest.  Per sweep, measured: 2048 x 2048 1.82 us (8 rows, 9 sweeps;
-// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 0.95 (8, 17; 1.29), 400 x 400 0.67
-// (4, 14; 1.28); tracked, 400 x 400 1.18 (6, 15; 1.92 with 4 rows, 5 sweeps).  Tracking launches take whole groups, a halo of whole waves,
+// finds cheapest.  Per sweep, measured: 2048 x 2048 1.70 us (8 rows, 9 sweeps;
+// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 0.87 (8, 17; 1.29), 400 x 400 0.62
+// (4, 14; 1.28); tracked, 400 x 400 1.12 (6, 15; 1.85 with 4 rows, 5 sweeps).
+// Tracking launches take whole groups, a halo of whole waves,
 // and need room for two TrackOut in track_room bytes.
 BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room) {
     BlockedPlan best{4, kStopGroup, sweep_tiles(w, h, BK_NW * 4, 2 * kStopGroup)};

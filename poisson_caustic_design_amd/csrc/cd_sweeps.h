@@ -29,6 +29,7 @@ struct SweepTiles {
     int w, h, we, he;
     int ry, halo, ix, iy;
     int tiles_x, tiles_y, ntiles;
+    unsigned inv_x;  // floor((2^32 - 1) / tiles_x): tile * inv_x >> 32 is tile / tiles_x or one less
 };
 
 inline SweepTiles sweep_tiles(int w, int h, int ry, int halo) {
@@ -44,10 +45,11 @@ inline SweepTiles sweep_tiles(int w, int h, int ry, int halo) {
     t.tiles_x = t.we <= SW_RX ? 1 : 1 + (t.we - SW_RX + t.ix - 1) / t.ix;
     t.tiles_y = t.he <= ry ? 1 : 1 + (t.he - ry + t.iy - 1) / t.iy;
     t.ntiles = t.tiles_x * t.tiles_y;
+    t.inv_x = UINT_MAX / (unsigned)t.tiles_x;
     return t;
 }
 
-// workgroups of a launch over ntiles tiles: a multiple of 8 (see tile_of)
+// workgroups of a launch over ntiles tiles: a multiple of 8 (see tile_of_block)
 inline int sweep_grid(int ntiles) { return (ntiles + 7) / 8 * 8; }
 
 // One region: its origin, the half-open range of cells it stores, and which of
@@ -60,7 +62,10 @@ struct Region {
 
 __device__ __forceinline__ Region region_of(const SweepTiles& t, int tile) {
     Region g;
-    const int ty = tile / t.tiles_x, tx = tile - ty * t.tiles_x;
+    // (no division and no branch: the loads that follow wait for this)
+    const int q = (int)__umulhi((unsigned)tile, t.inv_x), rem = tile - q * t.tiles_x;
+    const bool more = rem >= t.tiles_x;
+    const int ty = more ? q + 1 : q, tx = more ? rem - t.tiles_x : rem;
     g.X0 = max(min(tx * t.ix, t.we - SW_RX), 0);
     g.Y0 = max(min(ty * t.iy, t.he - t.ry), 0);
     g.left = tx == 0;
@@ -89,9 +94,9 @@ __device__ __forceinline__ int live_sweeps(const Region& g, int wave) {
 // XCD-aware tile order: gridDim.x is a multiple of 8 and consecutive workgroups
 // go round-robin to the 8 XCDs; each XCD gets a contiguous band of tiles so
 // that halo re-reads hit its own L2.  May return a tile >= ntiles.
-__device__ __forceinline__ int tile_of_block() {
-    const int per = gridDim.x >> 3;
-    return (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+__device__ __forceinline__ int tile_of_block(int ntiles) {
+    const int per = (ntiles + 7) >> 3;  // gridDim.x / 8
+    return (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
 }
 
 // value of lane l-1 (0 in lane 0) / lane l+1 (0 in lane 63): DPP wave shifts
