@@ -397,13 +397,16 @@ __global__ void k_check(const double* __restrict__ partials, int nblocks, SolveD
 // constants elsewhere.
 //
 // A half-sweep per launch was bound by its launches: two of 3.8 us (plus gaps)
-// per sweep on a 512 x 512 grid, where 8 sweeps in one launch take about 11 us.
+// per sweep on a 512 x 512 grid, where 12 sweeps in one launch take 12.9 us, of
+// which border tiles set the pace: their omega / cnt are chosen from four values
+// (a division per cell before: 13.6 us), and a missing row is read from a row of
+// zeros instead of being selected in every half-sweep.
 // ---------------------------------------------------------------------------
 constexpr int NAT_R = 4;    // rows per wave
 constexpr int NAT_NW = 16;  // waves per workgroup
 constexpr int NAT_RY = NAT_R * NAT_NW;
 
-// Per-cell constants of a tile at the grid border or with a mask.
+// Per-cell constants of a wave at the grid border or with a mask.
 template <typename T>
 struct NatCells {
     T oc[2][NAT_R], cnt[2][NAT_R];
@@ -440,16 +443,28 @@ __device__ __forceinline__ void nat_half(T (&ev)[2][NAT_R], const T (&rv)[2][NAT
     }
 }
 
+// omega over 1, 2, 3 and 4 neighbours
+template <typename T>
+struct NatOmega {
+    T o1, o2, o3, o4;
+};
+
 // Everything between the loads and the stores of a region: nsweeps sweeps, of
 // which the wave takes part in the first `live`.  edge_up / edge_down: the wave's
-// first / last row has no row beyond it.
+// first / last row has no row beyond it (it reads the row of zeros in xch[2]).
 template <typename T, int KIND, bool TRACK>
 __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_R],
                                         const NatCells<T>& cl, T (*xch)[NAT_NW][2][64], T oc4,
                                         bool edge_up, bool edge_down, int wave, int lane,
                                         int nsweeps, int live, float (*smax)[NAT_NW][64],
                                         bool track0, bool track1) {
-    const int wu = max(wave - 1, 0), wd = min(wave + 1, NAT_NW - 1);
+    const T* above[2];
+    const T* below[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        above[c] = KIND && edge_up ? xch[2][0][0] : xch[c][max(wave - 1, 0)][1];
+        below[c] = KIND && edge_down ? xch[2][0][0] : xch[c][min(wave + 1, NAT_NW - 1)][0];
+    }
     auto publish = [&](int c) {
         xch[c][wave][0][lane] = ev[c][0];
         xch[c][wave][1][lane] = ev[c][NAT_R - 1];
@@ -461,19 +476,15 @@ __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_
         publish(1);
         nat_half<T, 0, KIND, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
         __syncthreads();
-        up = xch[1][wu][1][lane];
-        down = xch[1][wd][0][lane];
-        if (KIND && edge_up) up = (T)0;
-        if (KIND && edge_down) down = (T)0;
+        up = above[1][lane];
+        down = below[1][lane];
         nat_half<T, 0, KIND, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
         nat_half<T, 0, KIND, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
         publish(0);
         nat_half<T, 1, KIND, TRACK, 1, NAT_R - 1>(ev, rv, cl, oc4, (T)0, (T)0, mx);
         __syncthreads();
-        up = xch[0][wu][1][lane];
-        down = xch[0][wd][0][lane];
-        if (KIND && edge_up) up = (T)0;
-        if (KIND && edge_down) down = (T)0;
+        up = above[0][lane];
+        down = below[0][lane];
         nat_half<T, 1, KIND, TRACK, 0, 1>(ev, rv, cl, oc4, up, down, mx);
         nat_half<T, 1, KIND, TRACK, NAT_R - 1, NAT_R>(ev, rv, cl, oc4, up, down, mx);
         if (TRACK) {
@@ -490,11 +501,13 @@ __device__ __forceinline__ void nat_run(T (&ev)[2][NAT_R], const T (&rv)[2][NAT_
 template <typename T, bool TRACK>
 __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     const T* ein, T* eout, const T* __restrict__ r, const uint8_t* __restrict__ mask,
-    SweepTiles tiles, int nsweeps, T omega, const T* __restrict__ rmean, SolveDev* st,
+    SweepTiles tiles, int nsweeps, NatOmega<T> om, const T* __restrict__ rmean, SolveDev* st,
     int out_index, TrackArgs track) {
-    __shared__ T xch[2][NAT_NW][2][64];
+    __shared__ T xch[3][NAT_NW][2][64];  // the third: one row of zeros
     __shared__ float smax[TRACK ? kTrackSweeps : 1][NAT_NW][64];
     __shared__ unsigned red[TRACK ? NAT_NW : 1];
+    // (what the loads' addresses need is read in one go)
+    asm volatile("" ::"s"(ein), "s"(r), "s"(mask), "s"(rmean), "s"(tiles.w), "s"(tiles.ntiles));
     const int tile = tile_of_block(tiles.ntiles);
     if (tile >= tiles.ntiles) return;
     const Region g = region_of(tiles, tile);
@@ -502,24 +515,28 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x0 = g.X0 + 2 * lane, Yw = g.Y0 + wave * NAT_R;
-    const T rm = *rmean;
     T ev[2][NAT_R], rv[2][NAT_R];
     NatCells<T> cl;
     uint8_t mk[2][NAT_R];
     // branch-free loads from clamped addresses: all in flight together
-    auto cell = [&](int c, int k) {
-        return (size_t)min(Yw + k, h - 1) * w + min(x0 + ((k + c) & 1), w - 1);
-    };
+    const unsigned col[2] = {(unsigned)min(x0, w - 1), (unsigned)min(x0 + 1, w - 1)};
+    auto row = [&](int k) { return (size_t)min(Yw + k, h - 1) * w; };
     const unsigned words = TRACK ? track_load<NAT_NW>(track, tiles.ntiles) : 0u;
 #pragma unroll
     for (int k = 0; k < NAT_R; ++k)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const size_t i = cell(c, k);
-            ev[c][k] = ein[i];
-            rv[c][k] = r[i];
-            mk[c][k] = mask ? mask[i] : (uint8_t)0;
+            ev[c][k] = (ein + row(k))[col[(k + c) & 1]];
+            rv[c][k] = (r + row(k))[col[(k + c) & 1]];
+            mk[c][k] = 0;
         }
+    if (mask) {
+#pragma unroll
+        for (int k = 0; k < NAT_R; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) mk[c][k] = (mask + row(k))[col[(k + c) & 1]];
+    }
+    const T rm = *rmean;
     if (TRACK) {
         const TrackPlan plan =
             track_decide<NAT_NW>(track, st, tiles.ntiles, nsweeps, words, red);
@@ -532,13 +549,14 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 #pragma unroll
             for (int k = 0; k < NAT_R; ++k)
 #pragma unroll
-                for (int c = 0; c < 2; ++c) ev[c][k] = in[cell(c, k)];
+                for (int c = 0; c < 2; ++c) ev[c][k] = (in + row(k))[col[(k + c) & 1]];
         }
     }
     const bool general = mask || g.left || g.right || g.top || g.bottom;
-    const T oc4 = omega / (T)4;
+    const T oc4 = om.o4;
     if (general) {
         cl.live = 0u;
+        if (wave == 0) xch[2][0][0][lane] = (T)0;  // (the sweeps' first barrier follows)
 #pragma unroll
         for (int k = 0; k < NAT_R; ++k)
 #pragma unroll
@@ -551,7 +569,12 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
                 if (live) cl.live |= 1u << (c * NAT_R + k);
                 else ev[c][k] = (T)0;
                 cl.cnt[c][k] = (T)n;
-                cl.oc[c][k] = live ? omega / (T)n : (T)0;
+                T oc = om.o4;  // (selects, no branches)
+                oc = n == 3 ? om.o3 : oc;
+                oc = n == 2 ? om.o2 : oc;
+                oc = n == 1 ? om.o1 : oc;
+                oc = n == 0 ? (T)INFINITY : oc;
+                cl.oc[c][k] = live ? oc : (T)0;
                 rv[c][k] = live ? rv[c][k] - rm : (T)0;
             }
     } else {
@@ -578,14 +601,22 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
     else
         nat_run<T, NAT_INNER, TRACK>(ev, rv, cl, xch, oc4, false, false, wave, lane, nsweeps, live, smax,
                                      t0, t1);
+    if (Yw + NAT_R > g.ys0 && Yw < g.ys1) {
+        const bool all_rows = Yw >= g.ys0 && Yw + NAT_R <= g.ys1;
 #pragma unroll
-    for (int k = 0; k < NAT_R; ++k) {
-        const int y = Yw + k;
-        if (y < g.ys0 || y >= g.ys1) continue;
+        for (int p = 0; p < 2; ++p) {
+            if (x0 + p < g.xs0 || x0 + p >= g.xs1) continue;
+            auto store = [&](int k) {
+                (eout + (size_t)(Yw + k) * w)[(unsigned)(x0 + p)] = ev[(k + p) & 1][k];
+            };
+            if (all_rows) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int x = x0 + ((k + c) & 1);
-            if (x >= g.xs0 && x < g.xs1) eout[(size_t)y * w + x] = ev[c][k];
+                for (int k = 0; k < NAT_R; ++k) store(k);
+            } else {
+#pragma unroll
+                for (int k = 0; k < NAT_R; ++k)
+                    if (Yw + k >= g.ys0 && Yw + k < g.ys1) store(k);
+            }
         }
     }
     if (TRACK) track_store<NAT_NW>(track, smax, red, tile, nsweeps, wave, lane);
@@ -2371,6 +2402,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                                            cd_partials_bytes(nred));
         const int most = t.ntiles == 1 ? (track ? kTrackSweeps : count_sweeps) : t.halo / 2;
         const dim3 grid(sweep_grid(t.ntiles)), blk(64 * NAT_NW);
+        const NatOmega<T> oms{om, om / 2, om / 3, om / 4};
         int cur = mixed ? 0 : ctx->host_status->cur;
         TrackArgs tr{};
         tr.group = 1;
@@ -2385,13 +2417,13 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                 tr.lid = ++track_lid;
                 tr.out = track_out(partials, t.ntiles, launches & 1);
                 hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, in, out, rhs, mask, t,
-                                   nsw, om, mean, sd, 1 - cur, tr);
+                                   nsw, oms, mean, sd, 1 - cur, tr);
                 tr.prev = tr.out;
                 tr.nprev = nsw;
                 tr.first_prev = first + done_sw;
             } else {
                 hipLaunchKernelGGL((k_rb_natural<T, false>), grid, blk, 0, s, in, out, rhs, mask, t,
-                                   nsw, om, mean, sd, 1 - cur, tr);
+                                   nsw, oms, mean, sd, 1 - cur, tr);
             }
             cur = 1 - cur;
             done_sw += nsw;
@@ -2400,7 +2432,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             tr.lid = ++track_lid;
             tr.check_only = 1;
             hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, cur ? b1 : b0,
-                               cur ? b0 : b1, rhs, mask, t, 0, om, mean, sd, 1 - cur, tr);
+                               cur ? b0 : b1, rhs, mask, t, 0, oms, mean, sd, 1 - cur, tr);
             ++launches;
         }
         CD_CHECK_LAUNCH(ctx);
