@@ -1089,11 +1089,12 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
 // A whole mixed-precision solve of a grid of one region (up to 128 x 128 cells)
 // in one launch of one workgroup: the iterate phi, the correction and the
 // right-hand side stay in registers; sweeps, checks and the choice of the next
-// batch are those of cd_solve_device_internal's loop, with the same operations
-// per cell (the reductions sum in another order).  Such a solve was bound by its
-// checks, each three launches and a round trip to the host for 10 us of sweeps:
-// 64 x 64 to 1e-6 took 665 us (490 with launches of a whole batch), 13 checks of
-// about 35 us.  Now 0.32 us a sweep, 5 us a check and 35 us for the launch.
+// batch are those of cd_solve_device_internal's loop, with the same operations and
+// reductions.  Such a solve was bound by its checks, each three launches and a
+// round trip to the host for 10 us of sweeps: 64 x 64 to 1e-6 took 665 us (490
+// with launches of a whole batch), 13 checks of about 35 us.  Now 0.36 us a
+// sweep, 5.5 us a check (4.8 with sums in an order of its own) and 43 us for the
+// launch with its first and last check.
 //
 // The kernel leaves phi alone and reports `holes` when b holds a NaN, and
 // returns at a check after kRegionSweeps sweeps (the host launches it again).
@@ -1107,24 +1108,79 @@ struct RegionArgs {
     double tol, margin;
 };
 
-// Sums of N doubles over the workgroup of 16 waves, in every thread.
-template <int N>
-__device__ __forceinline__ void region_sum(double (&v)[N], double (*red)[BK_NW], int wave, int lane) {
+// Sums over the grid in the order of the launches that a larger grid's solve
+// takes (k_rhs_moments and k_residual with k_rhs_finish and k_check): a tree over
+// the 64 cells of a row of a 64 x 4 tile, the tile's rows as (0 + 2) + (1 + 3), a
+// tree over the up to 64 tiles.  So the sums, and the solve, have the bits of
+// that route.  A lane holds two neighbouring cells of a row, so the tree's steps
+// over columns 32, 16, ... 2 apart are steps over lanes 16, 8, ... 1 apart and the
+// last one joins the lane's two cells.
+//
+// fold: M sums at once, M a power of two: at each step a lane passes on the sums
+// it will not finish, so that M sums take M - 1 exchanges.  Takes the steps from
+// lane distance O on down, log2(M) of them; lane bit O >> j then says which half
+// of the sums' index bit j was kept.
+template <int O, int M>
+__device__ __forceinline__ double fold(const double (&a)[M], int lane) {
+    if constexpr (M == 1) {
+        return a[0];
+    } else {
+        double h[M / 2];
+        const bool upper = (lane & O) != 0;
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = cd_wave_sum(v[i]);
-    __syncthreads();  // red has been read
-    if (lane == 0)
-#pragma unroll
-        for (int i = 0; i < N; ++i) red[i][wave] = v[i];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        double t = red[i][lane & (BK_NW - 1)];
-#pragma unroll
-        for (int o = BK_NW / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-        v[i] = t;
+        for (int i = 0; i < M / 2; ++i) {
+            const double keep = upper ? a[2 * i + 1] : a[2 * i];
+            const double pass = upper ? a[2 * i] : a[2 * i + 1];
+            h[i] = keep + __shfl_xor(pass, O, 64);
+        }
+        return fold<O / 2, M / 2>(h, lane);
     }
 }
+constexpr int log2_of(int n) { return n > 1 ? 1 + log2_of(n / 2) : 0; }
+
+// N grid sums of R rows per wave: take(), with each pair of rows, then finish().
+// rows: LDS for the row sums of both column halves.
+template <int R, int N>
+struct GridSum {
+    static constexpr int kFirst = log2_of(4 * N);       // steps of take
+    static constexpr int kPairs = log2_of(R / 2);       // steps over the pairs
+    double g[R / 2];
+    // v[r][p][i]: value i of the cell of column parity p in row 2 pair + r
+    __device__ __forceinline__ void take(int pair, const double (&v)[2][2][N], int lane) {
+        double a[4 * N];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int i = 0; i < N; ++i) a[r + 2 * i + 2 * N * p] = v[r][p][i];
+        g[pair] = fold<16>(a, lane);
+    }
+    __device__ __forceinline__ void finish(double (&out)[N], double (*rows)[2][R * BK_NW], int w,
+                                           int h, int wave, int lane) {
+        double t = fold<(16 >> kFirst)>(g, lane);
+#pragma unroll
+        for (int o = 16 >> (kFirst + kPairs); o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        t += __shfl_xor(t, 16 >> (kFirst - 1), 64);  // the two cells of a lane
+        // this lane's sum: index bits from lane bits 16, 8, ...
+        auto bit = [&](int j) { return (lane >> (4 - j)) & 1; };
+        int pair = 0;
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j) pair |= bit(kFirst + j) << j;
+        const int i = N > 1 ? bit(1) : 0;
+        __syncthreads();  // rows has been read
+        rows[i][lane >> 5][R * wave + 2 * pair + bit(0)] = t;
+        __syncthreads();
+        const int nbx = w > 64 ? 2 : 1, bx = lane & (nbx - 1), y = 4 * (lane / nbx);
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            double q = 0.0;
+            if (y < h && y < R * BK_NW)
+                q = (rows[n][bx][y] + rows[n][bx][y + 2]) + (rows[n][bx][y + 1] + rows[n][bx][y + 3]);
+            out[n] = cd_wave_sum(q);
+        }
+    }
+};
 
 template <int R, bool TRACK>
 __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __restrict__ b,
@@ -1133,7 +1189,7 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
                                                              SolveDev* host_st) {
     __shared__ float xch[2][BK_NW][2][64];
     __shared__ double xphi[BK_NW][2][2][64];
-    __shared__ double red[2][BK_NW];
+    __shared__ double rowsum[2][2][R * BK_NW];
     __shared__ float smax[TRACK ? kStopGroup : 1][BK_NW][64];
     __shared__ float redm[kStopGroup];
     const int w = a.w, h = a.h;
@@ -1149,32 +1205,45 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
     // right-hand side statistics (k_rhs_moments)
     double bmean, bnorm, holes;
     {
-        double bv[2][R], s[2] = {0.0, 0.0};
+        double bv[2][R], s[2], q[1];
 #pragma unroll
         for (int k = 0; k < R; ++k)
 #pragma unroll
             for (int c = 0; c < 2; ++c) bv[c][k] = (b + row(k))[col[(k + c) & 1]];
+        GridSum<R, 2> sums;
+        GridSum<R, 1> squares;
 #pragma unroll
-        for (int k = 0; k < R; ++k)
+        for (int k = 0; k < R; k += 2) {
+            double v[2][2][2];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                if (!in_grid(c, k)) continue;
-                if (isnan(bv[c][k])) s[1] += 1.0;
-                else s[0] += bv[c][k];
-            }
-        region_sum(s, red, wave, lane);
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const int c = (k + r + p) & 1;
+                    const double x = bv[c][k + r];
+                    const bool hole = in_grid(c, k + r) && isnan(x);
+                    v[r][p][0] = in_grid(c, k + r) && !hole ? x : 0.0;
+                    v[r][p][1] = hole ? 1.0 : 0.0;
+                }
+            sums.take(k / 2, v, lane);
+        }
+        sums.finish(s, rowsum, w, h, wave, lane);
         bmean = s[0] / count;
         holes = s[1];
-        double q[1] = {0.0};
 #pragma unroll
-        for (int k = 0; k < R; ++k)
+        for (int k = 0; k < R; k += 2) {
+            double v[2][2][1];
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
-                if (in_grid(c, k) && !isnan(bv[c][k])) {
-                    const double d = bv[c][k] - bmean;
-                    q[0] += d * d;
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const int c = (k + r + p) & 1;
+                    const double d = bv[c][k + r] - bmean;
+                    v[r][p][0] = in_grid(c, k + r) && !isnan(bv[c][k + r]) ? d * d : 0.0;
                 }
-        region_sum(q, red, wave, lane);
+            squares.take(k / 2, v, lane);
+        }
+        squares.finish(q, rowsum, w, h, wave, lane);
         bnorm = sqrt(q[0]);
     }
 
@@ -1230,11 +1299,14 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
             xphi[wave][c][1][lane] = ph[c][R - 1];
         }
         __syncthreads();
-        double s[2] = {0.0, 0.0};
+        double s[2];
+        GridSum<R, 2> sums;
 #pragma unroll
-        for (int k = 0; k < R; ++k)
+        for (int kp = 0; kp < R; kp += 2) {
+            double vv[2][2][2];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int rc = 0; rc < 4; ++rc) {
+                const int k = kp + (rc >> 1), c = rc & 1;
                 const int p = (k + c) & 1, x = x0 + p, y = Yw + k;
                 const double o = ph[1 - c][k];
                 double up = k > 0 ? ph[1 - c][k > 0 ? k - 1 : 0]
@@ -1248,11 +1320,13 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
                 double v = ((b + row(k))[col[p]] - bmean) -
                            ((left + up + right + down) - cnt * ph[c][k]);
                 if (!in_grid(c, k)) v = 0.0;
-                s[0] += v;
-                s[1] += v * v;
+                vv[rc >> 1][p][0] = v;
+                vv[rc >> 1][p][1] = v * v;
                 rv[c][k] = TRACK ? (float)v : bf16_to_f32(f32_to_bf16((float)v));
             }
-        region_sum(s, red, wave, lane);
+            sums.take(kp / 2, vv, lane);
+        }
+        sums.finish(s, rowsum, w, h, wave, lane);
         const double mean = s[0] / count, rn2 = s[1] - count * mean * mean;
         rsum = s[0];
         rnorm = rn2 > 0.0 ? sqrt(rn2) : (rn2 == rn2 ? 0.0 : rn2);

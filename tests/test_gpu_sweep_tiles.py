@@ -7,6 +7,7 @@ max-update stop inside a launch ends at the sweep at which the oracle stops, or
 at the iterate of the same number of sweeps taken without a stop."""
 import numpy as np
 import pytest
+import torch
 
 from oracle.bind import RED_BLACK
 from poisson_caustic_design_amd import capi
@@ -202,6 +203,31 @@ def test_one_region_solves_match_larger_route(ctx, rng, w, h):
     assert st.checks >= 2 and st.initial_rel_residual > tol
     d = (g - g.mean()) - (ref - ref.mean())
     assert np.abs(d).max() <= 2 * 420 * tol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("w,h", REGION + [(128, 3), (3, 128), (65, 5), (64, 64), (96, 97)])
+@pytest.mark.parametrize("stop,tol", [(capi.STOP_RESIDUAL, 1e-7), (capi.STOP_MAX_UPDATE, 1e-5)])
+def test_one_region_solves_equal_the_launches(ctx, rng, w, h, stop, tol):
+    """Sweeps, checks, statistics and result of the one-launch solve are those of
+    separate launches, bit for bit (which a context with a training-pair capture
+    of another geometry takes)."""
+    b, _, p0 = make(rng, w, h, False)
+    runs = []
+    for every, cap in ((0, 100000), (13, 1000)):
+        o = capi.default_opts(tol=tol, stop=stop, check_every=every, max_sweeps=cap)
+        runs.append(ctx.poisson_solve(b, p0, o))
+    x = torch.zeros(16, device="cuda:0")
+    ctx.set_capture(x.data_ptr(), x.data_ptr(), 1, 4, 4, 64, 1)
+    try:
+        for (every, cap), (g, st) in zip(((0, 100000), (13, 1000)), runs):
+            o = capi.default_opts(tol=tol, stop=stop, check_every=every, max_sweeps=cap)
+            f, sf = ctx.poisson_solve(b, p0, o)
+            assert np.array_equal(f, g)
+            for k in ("status", "sweeps", "checks", "rel_residual", "initial_rel_residual",
+                      "last_max_update"):
+                assert getattr(sf, k) == getattr(st, k), k
+    finally:
+        ctx.clear_capture()
 
 
 def test_one_region_solve_statuses(ctx, rng):
