@@ -849,9 +849,22 @@ __device__ __forceinline__ BrickRows brick_rows(const Brick& bk, int Y, int h) {
     return r;
 }
 
+// The ends of a batch under the residual rule: its first launch starts from a
+// zero correction (zero), its last one adds the correction to the iterate phi
+// instead of storing it. A pass of its own that added the correction and
+// cleared both buffers took 4.2 us and a launch gap at 400 x 400 (16.7 us at 2048 x
+// 2048) before every check; 1.48 -> 1.45 ms for the 16 checks of a solve.
+struct BatchEnds {
+    double* phi;
+    int zero;
+};
+// (an instantiation of its own: as run-time choices in every launch they cost the
+// others 4 to 10 %)
+enum { FORM_PLAIN = 0, FORM_PROLONG = 1, FORM_ENDS = 2 };
+
 // Loads of one region: packed column `lane` of the wave's R rows, both colours,
-// from the correction and the right-hand side.  Columns are clamped into the
-// grid; what rows outside it load is not used.
+// from the correction (or zero) and the right-hand side.  Columns are clamped
+// into the grid; what rows outside it load is not used.
 // PROLONG: the correction is the intermediate-grid correction interpolated
 // bilinearly at the cell centres (u, v) = ((x, y) + 0.5) / fm - 0.5, not ein;
 // the workgroup first stages the intermediate cells its region needs in
@@ -863,7 +876,7 @@ template <int R, bool PROLONG, typename RT>
 __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R], const float* ein,
                                             const RT* rhs, const Brick& bk, const MidGrid& mid,
                                             float* patch, int X0, int Y0, int w, int h, int wave,
-                                            int lane) {
+                                            int lane, bool zero) {
     const int Yw = Y0 + R * wave;
     const int j = min(X0 / 2 + lane, (w + 1) / 2 - 1);
     const unsigned col = brick_col(j);
@@ -922,7 +935,8 @@ __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R], c
                 const float a = pp[0], b = pp[1], cc = pp[pw], d = pp[pw + 1];
                 ev[c][k] = (a * (1.f - tu) + b * tu) * (1.f - tv) + (cc * (1.f - tu) + d * tu) * tv;
             } else {
-                ev[c][k] = buf_load<float>(e_rs[c], (col + 64u * k) * 4u, row * 4u);
+                ev[c][k] = 0.f;
+                if (!zero) ev[c][k] = buf_load<float>(e_rs[c], (col + 64u * k) * 4u, row * 4u);
             }
             rr[c][k] = buf_load<RT>(r_rs[c], (col + 64u * k) * (unsigned)sizeof(RT),
                                     row * (unsigned)sizeof(RT));
@@ -933,14 +947,16 @@ __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R], c
 // The right-hand side is BF16 under the residual rule (every FP64 check
 // re-rounds the current residual, so the rounding never reaches the result)
 // and FP32 under the max-update rule (TRACK), which cannot see the smooth
-// error a rounded right-hand side leaves behind.  PROLONG: the sweeps start
-// from `mid` interpolated at the cells instead of from ein.
-template <int R, bool TRACK, bool PROLONG>
-__global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) ? 4 : 8) void k_rb_blocked(
+// error a rounded right-hand side leaves behind.  FORM_PROLONG: the
+// sweeps start from `mid` interpolated at the cells instead of from ein;
+// FORM_ENDS: as `ends` says.
+template <int R, bool TRACK, int FORM>
+__global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (FORM == FORM_PROLONG && R > 4) ? 4 : 8) void k_rb_blocked(
     const float* ein, float* eout, const void* __restrict__ rhs, Brick bk, SweepTiles tiles,
     int nsweeps, float om2, float om3, float om4, const float* __restrict__ rmean, SolveDev* st,
-    int out_index, MidGrid mid, TrackArgs track) {
+    int out_index, MidGrid mid, TrackArgs track, BatchEnds ends) {
     static_assert(R % 2 == 0, "colours alternate by row");
+    constexpr bool PROLONG = FORM == FORM_PROLONG, ENDS = FORM == FORM_ENDS;
     __shared__ float xch[2][BK_NW][2][64];
     __shared__ float smax[TRACK ? kTrackSweeps : 1][BK_NW][64];
     __shared__ unsigned red[TRACK ? BK_NW : 1];
@@ -963,7 +979,8 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
     float ev[2][R], rv[2][R];
     RT rr[2][R];
     const unsigned words = TRACK ? track_load<BK_NW>(track, tiles.ntiles) : 0u;
-    region_load<R, PROLONG>(ev, rr, ein, r, bk, mid, patch, rg.X0, rg.Y0, w, h, wave, lane);
+    region_load<R, PROLONG>(ev, rr, ein, r, bk, mid, patch, rg.X0, rg.Y0, w, h, wave, lane,
+                            ENDS && ends.zero);
     if (kLoadsFirst) __builtin_amdgcn_sched_barrier(0);
     // Max-update rule: the solve can have stopped in an earlier launch of the
     // batch, and then leaves the buffers untouched.  Residual rule: only a check
@@ -976,7 +993,7 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
         if (plan.redo) {
             out_index ^= 1;
             region_load<R, PROLONG>(ev, rr, eout, r, bk, mid, patch, rg.X0, rg.Y0, w, h, wave,
-                                    lane);
+                                    lane, false);
             eout = const_cast<float*>(ein);
         }
     }
@@ -1062,7 +1079,27 @@ __global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (PROLONG && R > 4) 
     const __amdgpu_buffer_rsrc_t out_rs[2] = {plane_rsrc(eout, bk.plane * sizeof(float)),
                                               plane_rsrc(eout + bk.plane, bk.plane * sizeof(float))};
     const bool all_rows = Yw >= rg.ys0 && Yw + R <= rg.ys1;
-    if (Yw + R > rg.ys0 && Yw < rg.ys1) {
+    if (ENDS && ends.phi && Yw + R > rg.ys0 && Yw < rg.ys1) {
+        // the end of a batch: phi += e (all loads first, from clamped addresses)
+        double ph[2][R];
+        const unsigned xc[2] = {(unsigned)min(max(x0, rg.xs0), rg.xs1 - 1),
+                                (unsigned)min(max(x0 + 1, rg.xs0), rg.xs1 - 1)};
+        auto prow = [&](int k) {
+            return ends.phi + (size_t)min(max(Yw + k, rg.ys0), rg.ys1 - 1) * w;
+        };
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) ph[p][k] = prow(k)[xc[p]];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (x0 + p < rg.xs0 || x0 + p >= rg.xs1) continue;
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                if (Yw + k >= rg.ys0 && Yw + k < rg.ys1)
+                    prow(k)[xc[p]] = ph[p][k] + (double)ev[(k + p) & 1][k];
+        }
+    } else if (Yw + R > rg.ys0 && Yw < rg.ys1) {
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             if (x0 + p < rg.xs0 || x0 + p >= rg.xs1) continue;
@@ -1574,30 +1611,34 @@ template <int R>
 void launch_blocked_rows(bool track, const MidGrid* pro, dim3 grid, hipStream_t s,
                          const float* ein, float* eout, const void* rhs, const Brick& bk,
                          const SweepTiles& t, int nsweeps, float om2, float om3, float om4,
-                         const float* rmean, SolveDev* st, int out_index, const TrackArgs& tr) {
+                         const float* rmean, SolveDev* st, int out_index, const TrackArgs& tr,
+                         const BatchEnds& ends) {
     const dim3 blk(BK_THREADS);
     const MidGrid mid = pro ? *pro : MidGrid{};
     if (track)
-        hipLaunchKernelGGL((k_rb_blocked<R, true, false>), grid, blk, 0, s, ein, eout, rhs, bk, t,
-                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+        hipLaunchKernelGGL((k_rb_blocked<R, true, FORM_PLAIN>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr, ends);
     else if (pro)
-        hipLaunchKernelGGL((k_rb_blocked<R, false, true>), grid, blk, 0, s, ein, eout, rhs, bk, t,
-                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+        hipLaunchKernelGGL((k_rb_blocked<R, false, FORM_PROLONG>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr, ends);
+    else if (ends.phi || ends.zero)
+        hipLaunchKernelGGL((k_rb_blocked<R, false, FORM_ENDS>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr, ends);
     else
-        hipLaunchKernelGGL((k_rb_blocked<R, false, false>), grid, blk, 0, s, ein, eout, rhs, bk, t,
-                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr);
+        hipLaunchKernelGGL((k_rb_blocked<R, false, FORM_PLAIN>), grid, blk, 0, s, ein, eout, rhs, bk, t,
+                           nsweeps, om2, om3, om4, rmean, st, out_index, mid, tr, ends);
 }
 
 // one launch of nsweeps sweeps from ein to eout
 void launch_blocked(const BlockedPlan& pl, bool track, const MidGrid* pro, hipStream_t s,
                     const float* ein, float* eout, const void* rhs, const Brick& bk, int nsweeps,
                     float om2, float om3, float om4, const float* rmean, SolveDev* st,
-                    int out_index, const TrackArgs& tr) {
+                    int out_index, const TrackArgs& tr, const BatchEnds& ends = BatchEnds{}) {
     const dim3 grid(sweep_grid(pl.t.ntiles));
     switch (pl.rows) {
-    case 4: launch_blocked_rows<4>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
-    case 6: launch_blocked_rows<6>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
-    default: launch_blocked_rows<8>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr); break;
+    case 4: launch_blocked_rows<4>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr, ends); break;
+    case 6: launch_blocked_rows<6>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr, ends); break;
+    default: launch_blocked_rows<8>(track, pro, grid, s, ein, eout, rhs, bk, pl.t, nsweeps, om2, om3, om4, rmean, st, out_index, tr, ends); break;
     }
 }
 
@@ -2373,8 +2414,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const int kResidualRows = nred >= 16384 ? 8 : nred >= 8192 ? 4 : nred >= 4096 ? 2 : 1;
     const dim3 cgrid(div_up(w, RED_BX), div_up(h, RED_BY * kResidualRows));
     const int ncheck = cgrid.x * cgrid.y;  // <= nred
-    // flush: fold the current FP32 correction into phi64 first (the learned
-    // iterations add theirs to phi64 themselves)
+    // flush: fold the current FP32 correction into phi64 first (the last launch of
+    // a batch under the blocked residual rule has done that, and so have learned
+    // iterations)
     // the end of every check: k_check on the residual pass's partials, then the
     // host's wait for the status (the residual pass's timer is open)
     // (wait false: the caller enqueues the work that follows and waits itself)
@@ -2425,10 +2467,12 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     int track_lid = 0;  // tracking launches of this solve
     // count_sweeps sweeps in launches between e32 and e32b, the first reading
     // e32; pro: it starts from this intermediate-grid correction, interpolated
-    // at the cells, instead.  ahead: sweeps of them that one launch has already
-    // taken (residual rule)
+    // at the cells, instead.  ends.zero: it starts from zero instead; ends.phi: the
+    // last launch adds the correction to it.  ahead: sweeps of them that one launch
+    // has already taken
     auto enqueue_blocked_om = [&](int first, int count_sweeps, float om2, float om3, float om4,
-                                  const MidGrid* pro = nullptr, int ahead = 0) -> int {
+                                  const MidGrid* pro = nullptr, int ahead = 0,
+                                  BatchEnds ends = BatchEnds{}) -> int {
         CD_TRY(timer_begin());
         const BlockedPlan pl = blocked_plan(w, h, count_sweeps - ahead, track != 0,
                                             cd_partials_bytes(nred));
@@ -2446,7 +2490,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             tr.lid = ++track_lid;
             tr.out = track_out(partials, pl.t.ntiles, launches & 1);
             launch_blocked(pl, track != 0, launches == 0 ? pro : nullptr, s, ein, eout, rhs, bk,
-                           nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr);
+                           nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr,
+                           BatchEnds{done_sw + nsw == count_sweeps ? ends.phi : nullptr,
+                                     launches == 0 ? ends.zero : 0});
             tr.prev = tr.out;
             tr.nprev = nsw;
             tr.first_prev = first + done_sw;
@@ -2513,9 +2559,13 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         return timer_end(CD_KERNEL_SOR_SWEEP, launches,
                          (mixed ? 12.0 : 24.0) * (double)n * count_sweeps);
     };
-    auto enqueue_sweeps = [&](int first, int count_sweeps, int ahead = 0) -> int {
+    // a batch of sweeps, of which `ahead` are already enqueued; fold: phi takes the
+    // correction (blocked residual rule; else the check's flush does that)
+    auto enqueue_sweeps = [&](int first, int count_sweeps, int ahead = 0, bool fold = true) -> int {
         if (blocked)
-            return enqueue_blocked_om(first, count_sweeps, om2, om3, om4, nullptr, ahead);
+            return enqueue_blocked_om(first, count_sweeps, om2, om3, om4, nullptr, ahead,
+                                      track ? BatchEnds{}
+                                            : BatchEnds{fold ? phi : nullptr, 1});
         if (mixed)
             return enqueue_natural(e32, e32b, r32, (float)omega, &sd->rmean32, first, count_sweeps);
         return enqueue_natural(phi, phi2, b, omega, &sd->bmean, first, count_sweeps);
@@ -2671,7 +2721,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
 
     int check_id = 0;
     int cum = 0;
-    CD_TRY(enqueue_check(check_id));
+    CD_TRY(enqueue_check(check_id, !blocked));  // (no correction yet)
     if (capture && !ctx->host_status->done) CD_TRY(capture_pair());
     double prev_rel = ctx->host_status->rel;
     int k = kmax;
@@ -2853,12 +2903,6 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         fk = 0;
         phi_cur = phi;
     }
-    // plain sweeps after learned iterations start from a zero correction (the
-    // iterations left their FP32 work in both ping-pong buffers)
-    if (fcg_iter > 0 && !done) {
-        CD_TRY(cd_fill_f32(ctx, e32, npk, 0.f));
-        CD_TRY(cd_fill_f32(ctx, e32b, npk, 0.f));
-    }
     // Max-update rule in mixed precision: the sweeps see the right-hand side
     // rounded (BF16 / FP32) at the last check, which perturbs every update by
     // up to omega/4 times that rounding of the check's residual.  A stop is
@@ -2872,8 +2916,8 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     bool confirming = false;
     // Residual rule on the blocked layout: a full batch (not one sized to end the
     // solve) is expected to be followed by another, whose first launch goes out
-    // before the host has the check's status.  It only writes the correction,
-    // which the next check folds in: if the solve stops here, nothing reads it.
+    // before the host has the check's status.  It only writes the correction:
+    // if the solve stops here, nothing reads it.
     // (A batch has at least 8 sweeps.)  400 x 400: 1.87 -> 1.76 ms to 1e-6.
     constexpr int kAhead = 8;
     const bool look_ahead = blocked && !track && !ctx->profiling && !capture;
@@ -2883,11 +2927,12 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         CD_TRY(enqueue_sweeps(cum, nsw, ahead));
         cum += nsw;
         ++check_id;
-        CD_TRY(enqueue_check(check_id, true, false));
+        // (a batch that one early launch took whole has not reached phi yet)
+        CD_TRY(enqueue_check(check_id, !blocked || track || ahead == nsw, false));
         ahead = 0;
         if (look_ahead && nsw == kmax && kmax >= kAhead && o->max_sweeps - cum >= kAhead) {
             ahead = std::min(kAhead, blocked_plan(w, h, kAhead, false, 0).sweeps);
-            CD_TRY(enqueue_sweeps(cum, ahead));
+            CD_TRY(enqueue_sweeps(cum, ahead, 0, false));
         }
         CD_TRY(wait_check());
         const SolveDev& hs = *ctx->host_status;
