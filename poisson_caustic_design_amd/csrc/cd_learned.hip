@@ -380,60 +380,6 @@ __device__ __forceinline__ void conv_lds(floatx4 (&acc)[MT][NB], const u16* __re
     }
 }
 
-template <int NB, int OUT, int IN = 0>
-__global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1,
-                                                      const u16* __restrict__ x2, int c1, int c2,
-                                                      const u16* __restrict__ wt, int kpad, int H,
-                                                      int W, int cblocks, u16* __restrict__ ybf,
-                                                      float* __restrict__ yf, int cy, int relu,
-                                                      int mode1,
-                                                      const float* __restrict__ g = nullptr,
-                                                      const u16* __restrict__ mask = nullptr,
-                                                      float* __restrict__ y2 = nullptr,
-                                                      int cy2 = 0) {
-    extern __shared__ uint4 tile_lds[];
-    u16* xs = reinterpret_cast<u16*>(tile_lds);
-    const int cin = c1 + c2;
-    const int xstride = cin + 8;                      // u16 per tile pixel
-    u16* ws = xs + 100 * xstride;                     // 16-byte aligned: xstride % 8 == 0
-    const int cblk = blockIdx.z % cblocks, b = blockIdx.z / cblocks;
-    const int tx0 = blockIdx.x * CT, ty0 = blockIdx.y * CT;
-    if (IN == 0)
-        stage_patch<10>(xs, xstride, x1, x2, c1, c2, H, W, b, ty0 - 1, tx0 - 1, mode1);
-    else
-        stage_grad<10>(xs, xstride, g, mask, c1, H, W, b, ty0 - 1, tx0 - 1);
-    stage_weights(ws, wt + (size_t)cblk * NB * 16 * kpad, NB * 16, kpad);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // this lane's A pixel: tile row 2*wave + (l%16)/8, column (l%16)%8
-    const int ar = 2 * wave + ((lane & 15) >> 3), ac = lane & 7;
-    const int pbase[1] = {ar * 10 + ac};
-    floatx4 acc2[1][NB];
-    conv_lds<NB, 1, 10>(acc2, xs, xstride, cin, ws, kpad, pbase, lane);
-    floatx4(&acc)[NB] = acc2[0];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            // D row 4*(l/16) + r is tile pixel (2*wave + row/8, row % 8)
-            const int row = 4 * (lane >> 4) + r;
-            const int yy = ty0 + 2 * wave + (row >> 3), xx = tx0 + (row & 7);
-            const int ch = (cblk * NB + nb) * 16 + (lane & 15);
-            if (yy >= H || xx >= W || ch >= cy + (OUT == 2 ? cy2 : 0)) continue;
-            const long long p = ((long long)b * H + yy) * W + xx;
-            float v = acc[nb][r];
-            if (OUT == 0) {
-                if (relu) v = fmaxf(v, 0.f);
-                ybf[p * cy + ch] = to_bf16(v);
-            } else if (OUT == 1 || ch < cy) {
-                yf[p * cy + ch] = v;
-            } else {
-                y2[p * cy2 + ch - cy] = v;
-            }
-        }
-    }
-}
-
 // A compile-time value, or (0) the runtime one: sizes that are constants in the
 // instantiations for the shipped channel counts.
 template <int N>
@@ -501,6 +447,48 @@ struct PatchLoad {
     }
 };
 
+// The same for an FP32 gradient g of CIN channels, rounded to BF16 and zeroed where
+// mask (NULL: none) is not positive, as stage_grad reads it.
+template <int P, int NT, int U, int CIN>
+struct GradLoad {
+    float4 v0[U], v1[U];
+    V8 m[U];
+    int px[U], gi[U];
+    __device__ __forceinline__ void load(const float* __restrict__ g, const u16* __restrict__ mask,
+                                         int H, int W, int b, int oy, int ox) {
+        constexpr int ng = CIN / 8;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int it = min((int)threadIdx.x + NT * u, P * P * ng - 1);
+            px[u] = it / ng;
+            gi[u] = it - px[u] * ng;
+            const int yc = min(max(oy + px[u] / P, 0), H - 1);
+            const int xc = min(max(ox + px[u] % P, 0), W - 1);
+            const long long q = (((long long)b * H + yc) * W + xc) * CIN + gi[u] * 8;
+            v0[u] = *reinterpret_cast<const float4*>(g + q);
+            v1[u] = *reinterpret_cast<const float4*>(g + q + 4);
+            if (mask) m[u].u = *reinterpret_cast<const uint4*>(mask + q);
+        }
+    }
+    __device__ __forceinline__ void store(u16* __restrict__ xs, int H, int W, int oy, int ox,
+                                          bool masked) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int yy = oy + px[u] / P, xx = ox + px[u] % P;
+            const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+            const float gv[8] = {v0[u].x, v0[u].y, v0[u].z, v0[u].w,
+                                 v1[u].x, v1[u].y, v1[u].z, v1[u].w};
+            V8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool on = in && !(masked && !(from_bf16(m[u].h[e]) > 0.f));
+                o.h[e] = on ? to_bf16(gv[e]) : (u16)0;
+            }
+            *reinterpret_cast<uint4*>(xs + px[u] * (CIN + 8) + gi[u] * 8) = o.u;
+        }
+    }
+};
+
 // The same for `rows` weight rows of kpad (LDS row stride kpad + 8; KPAD: 0 any).
 template <int NT, int U, int KPAD>
 struct WeightLoad {
@@ -527,25 +515,24 @@ struct WeightLoad {
 // K of a 3x3 convolution over cin channels, padded to whole chunks
 constexpr int conv_kpad(int cin) { return (9 * cin + 31) / 32 * 32; }
 
-// The K loop of conv_lds for one block of 16 output channels (weight rows from
+// The K loop of conv_lds for NB blocks of 16 output channels (weight rows from
 // ws) and MT M-tiles, on a patch of side P.  CIN > 0: unrolled, all offsets
 // constants but for the lane's quarter of a chunk, so that the chunks' LDS reads
 // and MFMAs have no address chain between them.  CIN 0: conv_lds.  Same chunk
 // order, same bits.
-template <int CIN, int MT, int P>
-__device__ __forceinline__ void conv_chunks(floatx4 (&acc)[MT], const u16* __restrict__ xs,
+template <int CIN, int NB, int MT, int P>
+__device__ __forceinline__ void conv_chunks(floatx4 (&acc)[MT][NB], const u16* __restrict__ xs,
                                             int cin, const u16* __restrict__ ws, int kpad,
                                             const int (&pbase)[MT], int lane) {
     if (CIN == 0) {
-        floatx4 a2[MT][1];
-        conv_lds<1, MT, P>(a2, xs, cin + 8, cin, ws, kpad, pbase, lane);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = a2[m][0];
+        conv_lds<NB, MT, P>(acc, xs, cin + 8, cin, ws, kpad, pbase, lane);
         return;
     }
     constexpr int C = CIN > 0 ? CIN : 8, XS = C + 8, KP = conv_kpad(C);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[m][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int qd = lane >> 4;
     const u16* wrow = ws + (lane & 15) * (KP + 8) + 8 * qd;
     const u16* xm[MT];
@@ -566,8 +553,10 @@ __device__ __forceinline__ void conv_chunks(floatx4 (&acc)[MT], const u16* __res
             off = qd == 0 ? offset(kc) : qd == 1 ? offset(kc + 8)
                 : qd == 2 ? offset(kc + 16) : offset(kc + 24);
         }
-        V8 bw;
-        bw.u = *reinterpret_cast<const uint4*>(wrow + kc);
+        V8 bw[NB];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            bw[nb].u = *reinterpret_cast<const uint4*>(wrow + nb * 16 * (KP + 8) + kc);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             V8 a;
@@ -576,7 +565,87 @@ __device__ __forceinline__ void conv_chunks(floatx4 (&acc)[MT], const u16* __res
                 const bool in = kc + 8 * qd < 9 * C;
                 a.u = make_uint4(in ? a.u.x : 0, in ? a.u.y : 0, in ? a.u.z : 0, in ? a.u.w : 0);
             }
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, bw.v, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                acc[m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, bw[nb].v, acc[m][nb],
+                                                                     0, 0, 0);
+        }
+    }
+}
+
+// CIN > 0 (mode1 0 or 1): that many input channels; all of the patch's and the
+// weights' loads are issued before the first store, the K loop is unrolled.
+// At 8 x 128 x 128: 3.1 to 7.1 us a convolution (5.0 to 8.4 staged one after the
+// other with a chunk's addresses computed in the K loop).
+template <int NB, int OUT, int IN = 0, int CIN = 0>
+__global__ __launch_bounds__(256) void k_conv3x3_tile(const u16* __restrict__ x1,
+                                                      const u16* __restrict__ x2, int c1, int c2,
+                                                      const u16* __restrict__ wt, int kpad, int H,
+                                                      int W, int cblocks, u16* __restrict__ ybf,
+                                                      float* __restrict__ yf, int cy, int relu,
+                                                      int mode1,
+                                                      const float* __restrict__ g = nullptr,
+                                                      const u16* __restrict__ mask = nullptr,
+                                                      float* __restrict__ y2 = nullptr,
+                                                      int cy2 = 0) {
+    extern __shared__ uint4 tile_lds[];
+    u16* xs = reinterpret_cast<u16*>(tile_lds);
+    constexpr int KP = CIN > 0 ? conv_kpad(CIN) : 0;
+    const int cin = fixed_or<CIN>(c1 + c2);
+    const int xstride = cin + 8;                      // u16 per tile pixel
+    u16* ws = xs + 100 * xstride;                     // 16-byte aligned: xstride % 8 == 0
+    const int cblk = blockIdx.z % cblocks, b = blockIdx.z / cblocks;
+    const int tx0 = blockIdx.x * CT, ty0 = blockIdx.y * CT;
+    const u16* wb = wt + (size_t)cblk * NB * 16 * kpad;
+    if constexpr (CIN > 0) {
+        constexpr int UP = (100 * (CIN / 8) + 255) / 256, UW = (NB * 2 * KP + 255) / 256;
+        WeightLoad<256, UW, KP> wl;
+        if constexpr (IN == 0) {
+            PatchLoad<10, 256, UP, false, CIN> pl;
+            pl.load(x1, x2, c1, c2, H, W, b, ty0 - 1, tx0 - 1, mode1, 0);
+            wl.load(wb, NB * 16, KP, 0);
+            pl.store(xs, xstride, H, W, ty0 - 1, tx0 - 1);
+        } else {
+            GradLoad<10, 256, UP, CIN> gl;
+            gl.load(g, mask, H, W, b, ty0 - 1, tx0 - 1);
+            wl.load(wb, NB * 16, KP, 0);
+            gl.store(xs, H, W, ty0 - 1, tx0 - 1, mask != nullptr);
+        }
+        wl.store(ws, NB * 16, KP, 0);
+    } else {
+        if (IN == 0)
+            stage_patch<10>(xs, xstride, x1, x2, c1, c2, H, W, b, ty0 - 1, tx0 - 1, mode1);
+        else
+            stage_grad<10>(xs, xstride, g, mask, c1, H, W, b, ty0 - 1, tx0 - 1);
+        stage_weights(ws, wb, NB * 16, kpad);
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // this lane's A pixel: tile row 2*wave + (l%16)/8, column (l%16)%8
+    const int ar = 2 * wave + ((lane & 15) >> 3), ac = lane & 7;
+    const int pbase[1] = {ar * 10 + ac};
+    floatx4 acc2[1][NB];
+    conv_chunks<CIN, NB, 1, 10>(acc2, xs, cin, ws, kpad, pbase, lane);
+    floatx4(&acc)[NB] = acc2[0];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            // D row 4*(l/16) + r is tile pixel (2*wave + row/8, row % 8)
+            const int row = 4 * (lane >> 4) + r;
+            const int yy = ty0 + 2 * wave + (row >> 3), xx = tx0 + (row & 7);
+            const int ch = (cblk * NB + nb) * 16 + (lane & 15);
+            if (yy >= H || xx >= W || ch >= cy + (OUT == 2 ? cy2 : 0)) continue;
+            const long long p = ((long long)b * H + yy) * W + xx;
+            float v = acc[nb][r];
+            if (OUT == 0) {
+                if (relu) v = fmaxf(v, 0.f);
+                ybf[p * cy + ch] = to_bf16(v);
+            } else if (OUT == 1 || ch < cy) {
+                yf[p * cy + ch] = v;
+            } else {
+                y2[p * cy2 + ch - cy] = v;
+            }
         }
     }
 }
@@ -669,8 +738,8 @@ __global__ __launch_bounds__(kPairThreads) void k_conv_pair_tile(
             const int q = (mg + 4 * m) * 16 + (lane & 15);
             pbase[m] = q < 100 ? (q / 10) * 12 + q % 10 : 0;
         }
-        floatx4 acc[MT];
-        conv_chunks<CINA, MT, 12>(acc, xs, cin, wsa + nb * 16 * (ka + 8), ka, pbase, lane);
+        floatx4 acc[MT][1];
+        conv_chunks<CINA, 1, MT, 12>(acc, xs, cin, wsa + nb * 16 * (ka + 8), ka, pbase, lane);
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -678,7 +747,7 @@ __global__ __launch_bounds__(kPairThreads) void k_conv_pair_tile(
                 const int q = (mg + 4 * m) * 16 + 4 * (lane >> 4) + r;
                 if (q >= 100 || ch >= cya) continue;
                 const int yy = ty0 - 1 + q / 10, xx = tx0 - 1 + q % 10;
-                float v = acc[m][r];
+                float v = acc[m][0][r];
                 if (relua) v = fmaxf(v, 0.f);
                 ism[q * istride + ch] =
                     (yy >= 0 && yy < H && xx >= 0 && xx < W) ? to_bf16(v) : (u16)0;
@@ -698,15 +767,15 @@ __global__ __launch_bounds__(kPairThreads) void k_conv_pair_tile(
     // (row + 1, column + 1) whose 3x3 neighbourhood starts at index row*10 + column
     const int ar = 2 * mg + ((lane & 15) >> 3), ac = lane & 7;
     const int pbase[1] = {ar * 10 + ac};
-    floatx4 acc[1];
-    conv_chunks<CINB, 1, 10>(acc, ism, cb, wsb + nb * 16 * (kb + 8), kb, pbase, lane);
+    floatx4 acc[1][1];
+    conv_chunks<CINB, 1, 1, 10>(acc, ism, cb, wsb + nb * 16 * (kb + 8), kb, pbase, lane);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int row = 4 * (lane >> 4) + r;
         const int yy = ty0 + 2 * mg + (row >> 3), xx = tx0 + (row & 7);
         if (yy >= H || xx >= W || ch >= cyb) continue;
         const long long p = ((long long)b * H + yy) * W + xx;
-        float v = acc[0][r];
+        float v = acc[0][0][r];
         if (relub) v = fmaxf(v, 0.f);
         ybf[p * cyb + ch] = to_bf16(v);
     }
@@ -1201,8 +1270,8 @@ __global__ __launch_bounds__(512) void k_head_smooth(const u16* __restrict__ x, 
         const int q = (wave + 8 * m) * 16 + (lane & 15);
         pbase[m] = q < NQ ? (q / R) * P + q % R : 0;
     }
-    floatx4 acc[MT];
-    conv_chunks<CIN, MT, P>(acc, xs, C, ws, kpad, pbase, lane);
+    floatx4 acc[MT][1];
+    conv_chunks<CIN, 1, MT, P>(acc, xs, C, ws, kpad, pbase, lane);
     if ((lane & 15) == 0) {  // output channel 0
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -1211,7 +1280,7 @@ __global__ __launch_bounds__(512) void k_head_smooth(const u16* __restrict__ x, 
                 const int q = (wave + 8 * m) * 16 + 4 * (lane >> 4) + r;
                 if (q >= NQ) continue;
                 const int gy = Y0 + q / R, gx = X0 + q % R;
-                a[q] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? acc[m][r] : 0.f;
+                a[q] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? acc[m][0][r] : 0.f;
             }
     }
     __syncthreads();
@@ -1479,22 +1548,31 @@ int launch_conv(cd_net* n, const NetConv& cv, int B, int H, int W, bool grad_inp
         const int cblocks = nb / nbw;
         const size_t lds = lds_t;
         const dim3 grid(div_up(W, CT), div_up(H, CT), B * cblocks);
-        if (cv.out < 0) {  // head: FP32 output [npix][8]
-            if (nbw != 1 || cblocks != 1) return CD_ERR_BAD_ARG;
-            hipLaunchKernelGGL((k_conv3x3_tile<1, 1>), grid, dim3(256), lds, s, x1, x2, cv.c1,
-                               cv.c2, wt, cv.kpad, H, W, cblocks, (u16*)nullptr,
-                               n->head.as<float>(), 8, 0, mode1);
+        const bool head = cv.out < 0;  // FP32 output [npix][8]
+        if (head && (nbw != 1 || cblocks != 1)) return CD_ERR_BAD_ARG;
+        u16* y = head ? nullptr : n->t[cv.out].act.as<u16>();
+        float* yf = head ? n->head.as<float>() : nullptr;
+        const int cy = head ? 8 : cv.coutA, relu = head ? 0 : cv.relu;
+        // input channels of the shipped networks unrolled
+        const int cin = mode1 == 2 ? 0 : cv.c1 + cv.c2;
+#define TILE(NB, OUT, CIN) hipLaunchKernelGGL((k_conv3x3_tile<NB, OUT, 0, CIN>), grid, dim3(256), lds, s, x1, x2, cv.c1, cv.c2, wt, cv.kpad, H, W, cblocks, y, yf, cy, relu, mode1)
+        if (head) {
+            if (cin == 16) TILE(1, 1, 16);
+            else TILE(1, 1, 0);
+        } else if (nbw == 2) {
+            if (cin == 16) TILE(2, 0, 16);
+            else if (cin == 32) TILE(2, 0, 32);
+            else if (cin == 64) TILE(2, 0, 64);
+            else TILE(2, 0, 0);
         } else {
-            u16* y = n->t[cv.out].act.as<u16>();
-            if (nbw == 2)
-                hipLaunchKernelGGL((k_conv3x3_tile<2, 0>), grid, dim3(256), lds, s, x1, x2,
-                                   cv.c1, cv.c2, wt, cv.kpad, H, W, cblocks, y, (float*)nullptr,
-                                   cv.coutA, cv.relu, mode1);
-            else
-                hipLaunchKernelGGL((k_conv3x3_tile<1, 0>), grid, dim3(256), lds, s, x1, x2,
-                                   cv.c1, cv.c2, wt, cv.kpad, H, W, cblocks, y, (float*)nullptr,
-                                   cv.coutA, cv.relu, mode1);
+            if (cin == 8) TILE(1, 0, 8);
+            else if (cin == 16) TILE(1, 0, 16);
+            else if (cin == 32) TILE(1, 0, 32);
+            else if (cin == 48) TILE(1, 0, 48);
+            else if (cin == 64) TILE(1, 0, 64);
+            else TILE(1, 0, 0);
         }
+#undef TILE
     } else if (!grad_input) {
         const u16* x1 = mode1 ? x1src
                               : (cv.in1 < 0 ? n->x8.as<u16>() : n->t[cv.in1].act.as<u16>());
@@ -1537,6 +1615,12 @@ int launch_conv(cd_net* n, const NetConv& cv, int B, int H, int W, bool grad_inp
             const int cblocks = nb / nbg;
             const dim3 grid(div_up(W, CT), div_up(H, CT), B * cblocks);
             auto kernel = nbg == 2 ? k_conv3x3_tile<2, 2, 1> : k_conv3x3_tile<1, 2, 1>;
+            if (cv.coutA == 8)  // gradient channels of the shipped networks unrolled
+                kernel = nbg == 2 ? k_conv3x3_tile<2, 2, 1, 8> : k_conv3x3_tile<1, 2, 1, 8>;
+            else if (cv.coutA == 16)
+                kernel = nbg == 2 ? k_conv3x3_tile<2, 2, 1, 16> : k_conv3x3_tile<1, 2, 1, 16>;
+            else if (cv.coutA == 32)
+                kernel = nbg == 2 ? k_conv3x3_tile<2, 2, 1, 32> : k_conv3x3_tile<1, 2, 1, 32>;
             hipLaunchKernelGGL(kernel, grid, dim3(256), lds_g, s, (const u16*)nullptr,
                                (const u16*)nullptr, cv.coutA, 0, wt, cv.kpadT, H, W, cblocks,
                                (u16*)nullptr, d1, cv.c1, 0, 0, g, mask, d2, cv.c2);
