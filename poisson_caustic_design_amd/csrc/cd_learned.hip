@@ -794,13 +794,16 @@ __global__ __launch_bounds__(kPairThreads) void k_conv_pair_tile(
 // fragments of all three dx (dx = 2 is the same words one dword on, dx = 1 a
 // 16-bit funnel shift).  Wave w takes 16 input channels (w % NCI), all 9 taps and
 // all NCO blocks, and every (4 / NCI)-th group of 4 x 8 pixels.  The waves'
-// sums meet in LDS and go out with FP32 atomics, one set per workgroup, after
-// as many tiles as the grid leaves it.
+// sums meet in LDS, each wave sums a share of the entries over them, and go out
+// with FP32 atomics, one set per workgroup, after as many tiles as the grid leaves
+// it.
 //
 // Bound by the staging's LDS stores and loads (each input pixel is read once
 // per 32 output channels).  Gathering each fragment from global memory, element
 // by element with a division per pixel, took 97 us per convolution at 8 x 128 x
-// 128 (18 of them, 1.75 of the 2.16 ms of a training gradient); 16 us now.
+// 128 (18 of them, 1.75 of the 2.16 ms of a training gradient); 8 to 18 us
+// now (with one wave summing and adding for all, and branches around the loads, 9
+// to 21).
 // grid: (workgroups over the tiles, ceil(cin / (16 NCI)), ceil(cg / (16 NCO))).
 // ---------------------------------------------------------------------------
 constexpr int WG_TR = 8, WG_TC = 32;             // tile rows, columns
@@ -819,8 +822,8 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
     constexpr int KP = 4 / NCI;    // waves sharing 16 input channels
     constexpr int XG = 2 * NCI;    // groups of 8 input channels
     constexpr int XDW = NCI * 16 * WG_XCH + XG * 4, GDW = NCO * 16 * WG_GCH;
-    static_assert(NCI * 64 * 36 * NCO <= XDW + GDW, "the waves' sums fit the staging buffer");
-    __shared__ __align__(16) unsigned lds[XDW + GDW];
+    constexpr int RDW = 4 * 36 * 64;  // the waves' sums of 16 output channels
+    __shared__ __align__(16) unsigned lds[XDW + GDW > RDW ? XDW + GDW : RDW];
     unsigned* xs = lds;
     unsigned* gs = lds + XDW;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -850,33 +853,29 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
             const int it = threadIdx.x + 256 * u;
             const int gi = it % XG, t = it / XG;
             const int pair = t % (WG_TC / 2 + 1), row = t / (WG_TC / 2 + 1);
-            const int ci = ci0 + gi * 8, yy = yo + row - 1, xx = xo + 2 * pair - 1;
-            const u16* src = ci < c1 ? x1 + ci : x2 + (ci - c1);
-            const int cs = ci < c1 ? c1 : c2;
-            const bool rok = it < XN && ci < cin && yy >= 0 && yy < H;
+            // (clamped addresses, no branches: channels past cin read the last ones)
+            const int ci = min(ci0 + gi * 8, cin - 8), yy = yo + row - 1, xx = xo + 2 * pair - 1;
+            const bool use2 = ci >= c1;
+            const u16* src = use2 ? x2 + (ci - c1) : x1 + ci;
+            const int cs = use2 ? c2 : c1;
+            const long long r0 = img + (long long)min(max(yy, 0), H - 1) * W;
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                xv[u][e].u = make_uint4(0, 0, 0, 0);
-                if (rok && xx + e >= 0 && xx + e < W)
-                    xv[u][e].u = *reinterpret_cast<const uint4*>(
-                        src + (img + (long long)yy * W + xx + e) * cs);
-            }
+            for (int e = 0; e < 2; ++e)
+                xv[u][e].u = *reinterpret_cast<const uint4*>(
+                    src + (r0 + min(max(xx + e, 0), W - 1)) * cs);
         }
 #pragma unroll
         for (int u = 0; u < GIT; ++u) {
             const int it = threadIdx.x + 256 * u;
             const int q = it % (4 * NCO), t = it / (4 * NCO);
             const int pair = t % (WG_TC / 2), row = t / (WG_TC / 2);
-            const int co = co0 + 4 * q, yy = yo + row, xx = xo + 2 * pair;
+            const int co = min(co0 + 4 * q, cg - 4), yy = min(yo + row, H - 1), xx = xo + 2 * pair;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                gv[u][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+                const long long p = (img + (long long)yy * W + min(xx + e, W - 1)) * cg + co;
+                gv[u][e] = *reinterpret_cast<const float4*>(g + p);
                 mv[u][e] = make_ushort4(0x3f80, 0x3f80, 0x3f80, 0x3f80);  // 1.0: not masked
-                if (co < cg && yy < H && xx + e < W) {
-                    const long long p = (img + (long long)yy * W + xx + e) * cg + co;
-                    gv[u][e] = *reinterpret_cast<const float4*>(g + p);
-                    if (mask) mv[u][e] = *reinterpret_cast<const ushort4*>(mask + p);
-                }
+                if (mask) mv[u][e] = *reinterpret_cast<const ushort4*>(mask + p);
             }
         }
 #pragma unroll
@@ -885,10 +884,14 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
             const int gi = it % XG, t = it / XG;
             const int pair = t % (WG_TC / 2 + 1), row = t / (WG_TC / 2 + 1);
             if (it >= XN) continue;
+            const int yy = yo + row - 1, xx = xo + 2 * pair - 1;
+            const bool rok = ci0 + gi * 8 < cin && yy >= 0 && yy < H;
+            const unsigned lo = rok && xx >= 0 && xx < W ? 0xffffu : 0u;
+            const unsigned hi = rok && xx + 1 >= 0 && xx + 1 < W ? 0xffff0000u : 0u;
             unsigned* dst = xs + gi * (8 * WG_XCH + 4) + row * WG_XROW + pair;
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                dst[e * WG_XCH] = (unsigned)xv[u][0].h[e] | ((unsigned)xv[u][1].h[e] << 16);
+                dst[e * WG_XCH] = ((unsigned)xv[u][0].h[e] & lo) | (((unsigned)xv[u][1].h[e] << 16) & hi);
         }
 #pragma unroll
         for (int u = 0; u < GIT; ++u) {
@@ -898,11 +901,12 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
             unsigned o[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
+                const bool in = co0 + 4 * q < cg && yo + row < H && xo + 2 * pair + e < W;
                 const float f[4] = {gv[u][e].x, gv[u][e].y, gv[u][e].z, gv[u][e].w};
                 const u16 m[4] = {mv[u][e].x, mv[u][e].y, mv[u][e].z, mv[u][e].w};
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (from_bf16(m[k]) > 0.f) o[k] |= (unsigned)to_bf16(f[k]) << (16 * e);
+                    o[k] |= in && from_bf16(m[k]) > 0.f ? (unsigned)to_bf16(f[k]) << (16 * e) : 0u;
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) gs[(4 * q + k) * WG_GCH + row * (WG_TC / 2) + pair] = o[k];
@@ -939,39 +943,25 @@ __global__ __launch_bounds__(256) void k_wgrad(const u16* __restrict__ x1,
             }
         }
     }
-    // sum over the waves of an input block, one after the other
-    float* red = reinterpret_cast<float*>(lds) + (cb * 64 + lane);
-    for (int k = 1; k < KP; ++k) {
-        __syncthreads();
-        if (kpart == k)
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-#pragma unroll
-                for (int m = 0; m < NCO; ++m)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        red[((t * NCO + m) * 4 + r) * NCI * 64] = acc[t][m][r];
-        __syncthreads();
-        if (kpart == 0)
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-#pragma unroll
-                for (int m = 0; m < NCO; ++m)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        acc[t][m][r] += red[((t * NCO + m) * 4 + r) * NCI * 64];
-    }
+    // sum over the waves of an input block: all waves leave theirs, each then
+    // sums and adds its share of the entries
     const int ci = ci0 + cb * 16 + (lane & 15);
-    if (kpart != 0 || ci >= cin) return;
+    float* red = reinterpret_cast<float*>(lds) + lane;
 #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    for (int m = 0; m < NCO; ++m) {
+        __syncthreads();
 #pragma unroll
-        for (int m = 0; m < NCO; ++m)
+        for (int e = 0; e < 36; ++e) red[(wave * 36 + e) * 64] = acc[e / 4][m][e % 4];
+        __syncthreads();
+        for (int i = 0; i < 36 / KP; ++i) {
+            const int e = kpart * (36 / KP) + i;
+            float v = red[(cb * 36 + e) * 64];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int co = co0 + m * 16 + 4 * (lane >> 4) + r;  // output channel row of D
-                if (co < cg) atomicAdd(dw + (size_t)co * kpad + t * cin + ci, acc[t][m][r]);
-            }
+            for (int k = 1; k < KP; ++k) v += red[((cb + NCI * k) * 36 + e) * 64];
+            const int co = co0 + m * 16 + 4 * (lane >> 4) + e % 4;  // output channel row of D
+            if (ci < cin && co < cg) atomicAdd(dw + (size_t)co * kpad + (e / 4) * cin + ci, v);
+        }
+    }
 }
 
 // ---- elementwise / pooling ---------------------------------------------------
@@ -1106,104 +1096,71 @@ __global__ __launch_bounds__(256) void k_smooth_step(const float* __restrict__ i
     out[p] = in[p] + 0.125f * lap_field(in, 1, p, xx, yy, H, W);
 }
 
-// k smoothing steps in one launch: a 16x16 output tile with a k-cell halo
-// lives in LDS (two buffers); step s updates the cells at distance >= s from
-// the halo border, so the tile interior equals k global steps.  Same
-// arithmetic and summation order as k_smooth_step (bit-identical).  The input
-// has element stride `istride` (8: head channel 0).
-// 8x8 tiles (256 workgroups at 128x128, halo regions of (8 + 2k)^2 cells):
-// 6.2 us for k = 6 against 10.2 us with 16x16 tiles (64 workgroups), whose
-// waves carry three to four cells each through the steps
-#ifndef CD_SMOOTH_TILE
-#define CD_SMOOTH_TILE 8
-#endif
-constexpr int kSmoothTile = CD_SMOOTH_TILE;
-constexpr int kSmoothMaxK = 12;  // halo <= 12: 2 (tile + 2k)^2 floats of LDS
-// cells of a region per thread, at most
-constexpr int kSmoothCells =
-    ((kSmoothTile + 2 * kSmoothMaxK) * (kSmoothTile + 2 * kSmoothMaxK) + 255) / 256;
-// The k smoothing steps on an R x R region (R = kSmoothTile + 2k, image origin
-// (X0, Y0)) held in LDS at a (b: scratch of the same size); returns the buffer
-// holding the result.  Each thread keeps the region coordinates of its (at
-// most kSmoothCells) cells for every step.
-__device__ __forceinline__ float* smooth_lds(float* a, float* b, int R, int k, int X0, int Y0,
-                                             int H, int W) {
-    const int RR = R * R;
-    int rxs[kSmoothCells], rys[kSmoothCells];
+// k smoothing steps in one launch: an 8x8 output tile with a k-cell halo, the
+// (8 + 2k)^2 region, lives in LDS (two buffers), one cell per thread; step st
+// updates the cells at distance >= st from the region's border, so the tile
+// equals k global steps.  Cells outside the image stay 0, so that adding them
+// changes no sum and a cell's count of neighbours is the only condition left.
+// Same arithmetic and summation order as k_smooth_step (bit-identical).
+// 8x8 tiles: 256 workgroups at 128x128 (16x16 tiles took 1.6 times as long).
+constexpr int kSmoothTile = 8;
+constexpr int kSmoothMaxK = 12;  // (8 + 2k)^2 <= 1024 threads
+// K: the number of steps (0: k).  a holds the region of image origin (X0, Y0), b is
+// scratch of the same size; the calls of all threads of the workgroup meet.
+// Returns whether this thread's cell (gx, gy) is one of the tile, with its value.
+template <int K>
+__device__ __forceinline__ bool smooth_region(float* a, float* b, int k, int X0, int Y0, int H,
+                                              int W, int& gx, int& gy, float& c) {
+    const int steps = K > 0 ? K : k, R = kSmoothTile + 2 * steps, NQ = R * R;
+    const int q = min((int)threadIdx.x, NQ - 1), ry = q / R, rx = q - ry * R;
+    gy = Y0 + ry;
+    gx = X0 + rx;
+    const bool inside = gx >= 0 && gx < W && gy >= 0 && gy < H;
+    // steps that update this cell: those below its distance to the region's edge
+    const int depth = inside ? min(min(rx, R - 1 - rx), min(ry, R - 1 - ry)) : 0;
+    const float cnt = (float)((gx > 0) + (gx < W - 1) + (gy > 0) + (gy < H - 1));
+    const int ql = max(q - 1, 0), qr = min(q + 1, NQ - 1), qu = max(q - R, 0),
+              qd = min(q + R, NQ - 1);
+    c = a[q];
 #pragma unroll
-    for (int u = 0; u < kSmoothCells; ++u) {
-        const int idx = threadIdx.x + 256 * u;
-        rys[u] = idx / R;
-        rxs[u] = idx - rys[u] * R;
-    }
-    for (int st = 1; st <= k; ++st) {
-#pragma unroll
-        for (int u = 0; u < kSmoothCells; ++u) {
-            const int idx = threadIdx.x + 256 * u;
-            if (256 * u >= RR) break;  // no thread has cells from here on
-            if (idx >= RR) continue;
-            const int rx = rxs[u], ry = rys[u];
-            const int gx = X0 + rx, gy = Y0 + ry;
-            float c = a[idx];
-            if (rx >= st && rx < R - st && ry >= st && ry < R - st && gx >= 0 && gx < W &&
-                gy >= 0 && gy < H) {
-                float sum = 0.f, cnt = 0.f;
-                if (gx > 0) { sum += a[idx - 1]; cnt += 1.f; }
-                if (gx < W - 1) { sum += a[idx + 1]; cnt += 1.f; }
-                if (gy > 0) { sum += a[idx - R]; cnt += 1.f; }
-                if (gy < H - 1) { sum += a[idx + R]; cnt += 1.f; }
-                c = c + 0.125f * (sum - cnt * c);
-            }
-            b[idx] = c;
+    for (int st = 1; st <= steps; ++st) {
+        const float* src = st & 1 ? a : b;
+        float sum = 0.f;
+        sum += src[ql];
+        sum += src[qr];
+        sum += src[qu];
+        sum += src[qd];
+        c = st <= depth ? c + 0.125f * (sum - cnt * c) : c;
+        if (st < steps) {
+            (st & 1 ? b : a)[q] = c;  // (threads past the region: the last cell's value)
+            __syncthreads();
         }
-        __syncthreads();
-        float* t = a;
-        a = b;
-        b = t;
     }
-    return a;
-}
-
-// the tile's interior of the smoothed region to out [B][H][W]
-__device__ __forceinline__ void smooth_store(const float* a, int R, int k, int X0, int Y0,
-                                             int H, int W, long long base,
-                                             float* __restrict__ out) {
-    for (int idx = threadIdx.x; idx < kSmoothTile * kSmoothTile; idx += blockDim.x) {
-        const int ty = idx / kSmoothTile, tx = idx - ty * kSmoothTile;
-        const int gx = X0 + k + tx, gy = Y0 + k + ty;
-        if (gx < W && gy < H) out[base + (long long)gy * W + gx] = a[(ty + k) * R + tx + k];
-    }
+    return inside && depth >= steps && (int)threadIdx.x < NQ;
 }
 
 // k smoothing steps of a field read with element stride istride (8: head
-// channel 0), one tile plus its k-cell halo per workgroup; the loads of all of
-// a thread's cells are issued before the first LDS store
-__global__ __launch_bounds__(256) void k_smooth_tiled(const float* __restrict__ in, int istride,
-                                                      float* __restrict__ out, int B, int H,
-                                                      int W, int k) {
+// channel 0), one tile plus its k-cell halo per workgroup of (8 + 2k)^2 threads
+// (rounded up to whole waves).  At 8 x 128 x 128, k = 6: 11.3 us with two cells a
+// thread and the image's bounds tested in every step, 7.7 us now.
+__global__ __launch_bounds__(1024) void k_smooth_tiled(const float* __restrict__ in, int istride,
+                                                       float* __restrict__ out, int B, int H,
+                                                       int W, int k) {
     extern __shared__ float lds[];
     const int R = kSmoothTile + 2 * k, RR = R * R;
-    float* a = lds;
-    float* b = lds + RR;
     const int bz = blockIdx.z;
     const int X0 = blockIdx.x * kSmoothTile - k, Y0 = blockIdx.y * kSmoothTile - k;
     const long long base = (long long)bz * H * W;
-    float v[kSmoothCells];
-#pragma unroll
-    for (int u = 0; u < kSmoothCells; ++u) {
-        const int idx = threadIdx.x + 256 * u;
-        const int ry = idx / R, rx = idx - ry * R;
-        const int gx = X0 + rx, gy = Y0 + ry;
-        v[u] = (idx < RR && gx >= 0 && gx < W && gy >= 0 && gy < H)
-                   ? in[(base + (long long)gy * W + gx) * istride]
-                   : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < kSmoothCells; ++u)
-        if (threadIdx.x + 256 * u < RR) a[threadIdx.x + 256 * u] = v[u];
+    const int q = min((int)threadIdx.x, RR - 1);
+    const int gx0 = X0 + q % R, gy0 = Y0 + q / R;
+    const float v = in[(base + (long long)min(max(gy0, 0), H - 1) * W + min(max(gx0, 0), W - 1)) *
+                       istride];
+    lds[q] = gx0 >= 0 && gx0 < W && gy0 >= 0 && gy0 < H ? v : 0.f;
     __syncthreads();
-    a = smooth_lds(a, b, R, k, X0, Y0, H, W);
-    smooth_store(a, R, k, X0, Y0, H, W, base, out);
+    int gx, gy;
+    float c;
+    if (smooth_region<0>(lds, lds + RR, k, X0, Y0, H, W, gx, gy, c))
+        out[base + (long long)gy * W + gx] = c;
 }
 
 // Head convolution and output smoothing in one launch (inference, K steps):
@@ -1212,9 +1169,7 @@ __global__ __launch_bounds__(256) void k_smooth_tiled(const float* __restrict__ 
 // patch in LDS with the A/B fragments and K order of k_conv3x3_tile, so its
 // values are those k_conv3x3_tile<1, 1> stores; outside the image the region
 // holds 0, as k_smooth_tiled loads it; then the K steps as k_smooth_tiled
-// takes them, one cell per thread: the cells outside the image stay 0, so that
-// adding them changes no sum and a cell's count of neighbours is the only
-// condition left.  The output is bit-identical to the two launches.
+// takes them.  The output is bit-identical to the two launches.
 //
 // Bound by latency, as k_conv_pair_tile, and built like it (loads first, CIN > 0
 // unrolled for that many channels, 8 waves).  On a 128 x 128 level, 16 channels:
@@ -1284,30 +1239,9 @@ __global__ __launch_bounds__(512) void k_head_smooth(const u16* __restrict__ x, 
             }
     }
     __syncthreads();
-    const int q = min((int)threadIdx.x, NQ - 1), ry = q / R, rx = q - ry * R;
-    const int gy = Y0 + ry, gx = X0 + rx;
-    const bool inside = gx >= 0 && gx < W && gy >= 0 && gy < H;
-    // steps that update this cell: those below its distance to the region's edge
-    const int depth = inside ? min(min(rx, R - 1 - rx), min(ry, R - 1 - ry)) : 0;
-    const float cnt = (float)((gx > 0) + (gx < W - 1) + (gy > 0) + (gy < H - 1));
-    const int ql = max(q - 1, 0), qr = min(q + 1, NQ - 1), qu = max(q - R, 0),
-              qd = min(q + R, NQ - 1);
-    float c = a[q];
-#pragma unroll
-    for (int st = 1; st <= K; ++st) {
-        const float* src = st & 1 ? a : b2;
-        float sum = 0.f;
-        sum += src[ql];
-        sum += src[qr];
-        sum += src[qu];
-        sum += src[qd];
-        c = st <= depth ? c + 0.125f * (sum - cnt * c) : c;
-        if (st < K) {
-            (st & 1 ? b2 : a)[q] = c;  // (threads past the region: the last cell's value)
-            __syncthreads();
-        }
-    }
-    if (depth >= K && threadIdx.x < NQ)
+    int gx, gy;
+    float c;
+    if (smooth_region<K>(a, b2, K, X0, Y0, H, W, gx, gy, c))
         out[((long long)b * H + gy) * W + gx] = c;
 }
 
@@ -1653,10 +1587,11 @@ int launch_wgrad(cd_net* n, const NetConv& cv, int B, int H, int W) {
     const int nci = div_up(cin, 16) % 2 == 0 ? 2 : 1, nco = cv.coutA > 16 ? 2 : 1;
     const int tx = div_up(W, WG_TC), ty = div_up(H, WG_TR);
     const int gy = div_up(cin, 16 * nci), gz = div_up(cv.coutA, 16 * nco);
-    // up to 1.5 workgroups per CU, each over several tiles where the image has
-    // more: fewer atomics (768 to 3072 workgroups 20 us against 16 at 8 x 128 x
-    // 128, 48 to 16 channels)
-    const int gx = std::min(tx * ty * B, std::max(1, 384 / (gy * gz)));
+    // up to 1.5 workgroups per CU, each over the same number of tiles (a training
+    // gradient at 8 x 128 x 128 takes 524 us; 528 with up to 256 workgroups, 543
+    // with 512, 547 with 768: more atomics)
+    const int gmax = std::max(1, 384 / (gy * gz));
+    const int gx = div_up(tx * ty * B, div_up(tx * ty * B, gmax));
 #define WGRAD(CI, CO) hipLaunchKernelGGL((k_wgrad<CI, CO>), dim3(gx, gy, gz), dim3(256), 0, c->stream, x1, x2, cv.c1, cv.c2, g, mask, cv.coutA, B, H, W, n->gw.as<float>() + cv.woff, cv.kpad, tx, ty)
     if (nci == 1 && nco == 1) WGRAD(1, 1);
     else if (nci == 1) WGRAD(1, 2);
@@ -1955,7 +1890,7 @@ int smooth_steps(cd_net* n, DevBuf& a, DevBuf& b, int k, int B, int H, int W) {
     if (k <= kSmoothMaxK) {
         const int R = kSmoothTile + 2 * k;
         const dim3 grid(div_up(W, kSmoothTile), div_up(H, kSmoothTile), B);
-        hipLaunchKernelGGL(k_smooth_tiled, grid, dim3(256), sizeof(float) * 2 * R * R,
+        hipLaunchKernelGGL(k_smooth_tiled, grid, dim3(div_up(R * R, 64) * 64), sizeof(float) * 2 * R * R,
                            n->ctx->stream, a.as<float>(), 1, b.as<float>(), B, H, W, k);
         std::swap(a.ptr, b.ptr);
         std::swap(a.bytes, b.bytes);
@@ -1998,7 +1933,7 @@ int finish_output(cd_net* n, int B, int H, int W, float* dst = nullptr) {
         // head channel 0 -> k steps -> y in one launch
         const int R = kSmoothTile + 2 * k;
         const dim3 grid(div_up(W, kSmoothTile), div_up(H, kSmoothTile), B);
-        hipLaunchKernelGGL(k_smooth_tiled, grid, dim3(256), sizeof(float) * 2 * R * R,
+        hipLaunchKernelGGL(k_smooth_tiled, grid, dim3(div_up(R * R, 64) * 64), sizeof(float) * 2 * R * R,
                            n->ctx->stream, n->head.as<float>(), 8, y, B, H, W, k);
         CD_CHECK_LAUNCH(n->ctx);
         return CD_OK;
