@@ -37,3 +37,36 @@ def test_paired_convolutions_equal_separate_ones(ctx, channels, linear, batch, h
     net.close()
     assert np.abs(ys[0]).max() > 0
     assert np.array_equal(ys[0], ys[1])
+
+
+def test_resampling_of_more_rows_than_a_grid_holds(ctx):
+    """2060 images of 64 rows: every resampling kernel goes round its rows.  The
+    materialised forward equals the fused one, and the gradient of the mean loss
+    is the mean of the quarters' gradients (whose output gradients differ by the
+    exact factor 4, so every rounding to BF16 is the same) up to the order of the
+    FP32 sums over 10^6 pixels: sqrt(10^6) 2^-24 = 6e-5."""
+    b, h, w = 2060, 64, 8
+    arch = capi.default_arch(levels=3, channels=[8, 16, 8, 0, 0, 0], linear=1, out_smooth=0)
+    net = capi.Net(ctx, arch)
+    net.set_params(NetRef(3, (8, 16, 8), linear=True).random_params(3))
+    rng = np.random.default_rng(8)
+    x, t = (torch.tensor(rng.standard_normal((b, h, w)), dtype=torch.float32, device="cuda:0")
+            for _ in range(2))
+    ys = []
+    for fused in (True, False):
+        net.set_fused_forward(fused)
+        y = torch.zeros_like(x)
+        torch.cuda.synchronize()
+        net.forward(x.data_ptr(), y.data_ptr(), b, h, w)
+        ys.append(y.cpu().numpy())
+    assert np.array_equal(ys[0], ys[1])
+    _, g = net.loss_grad(x.data_ptr(), t.data_ptr(), b, h, w)
+    parts = []
+    for q in range(4):
+        i = slice(q * b // 4, (q + 1) * b // 4)
+        xq, tq = x[i].contiguous(), t[i].contiguous()
+        torch.cuda.synchronize()
+        parts.append(net.loss_grad(xq.data_ptr(), tq.data_ptr(), b // 4, h, w)[1])
+    net.close()
+    mean = np.mean(parts, axis=0)
+    assert np.linalg.norm(g - mean) <= 6e-5 * np.linalg.norm(mean)
