@@ -2025,10 +2025,14 @@ __global__ void k_fcg_coef(const double* __restrict__ partials, int nblocks, Fcg
 // The learned iteration's FCG step folded into its convergence check:
 // p = z + beta p_old (z: the smoothed correction, packed), phi_out = phi_in +
 // alpha p, and the FP64 residual of phi_out with its BF16 copy and partial
-// norms (as k_residual<2>).  phi and p are ping-pong pairs: the stencil reads
-// phi_in and p_old at the four neighbours and forms their new values itself
-// (the same FP32 and FP64 operations as at the centre, so every cell's new
-// value is one number).  fd->pprev is pointed at p_new for the next iteration.
+// norms (as k_residual<2>).  phi and p are ping-pong pairs.  A wave takes ROWS rows
+// of 64 columns one below the other: a row's new values serve as the next row's
+// upper and the previous row's lower neighbours, the lanes beside as left and
+// right ones; only the rows and columns around the wave's are formed once more
+// (with the same FP32 and FP64 operations, so every cell's new value is one
+// number).  Bound by memory: reading all five points of three fields per cell took
+// 14.9 us at 1024 x 1024 (12.3 now; an iteration at 2048 x 2048 159 -> 147 us).
+// fd->pprev is pointed at p_new for the next iteration.
 // x8 (may be NULL): the workgroup also writes the next iteration's network
 // input, the lf x lf block means of the new residual (BF16, channel 0 of 8 of
 // a coarse grid lwc wide).  The host passes x8 only when the workgroups tile
@@ -2036,9 +2040,9 @@ __global__ void k_fcg_coef(const double* __restrict__ partials, int nblocks, Fcg
 // 4*ROWS rows of a workgroup are one or two coarse rows.  The FP64 residual is
 // mean-free to rounding, so its block means need no projection.
 // rows whose loads a thread issues together, and the most rows a thread takes
-// (2 / 8 measured as fast as 4 / 8 and 2 / 4 at 1024^2 and 2048^2)
+// (2 / 8 measured as fast at 1024^2, 1 % of an iteration slower at 2048^2)
 #ifndef CD_STEP_G
-#define CD_STEP_G 2
+#define CD_STEP_G 4
 #endif
 #ifndef CD_STEP_ROWS
 #define CD_STEP_ROWS 8
@@ -2059,19 +2063,21 @@ __global__ __launch_bounds__(256) void k_residual_step(const double* __restrict_
     constexpr int G = ROWS < CD_STEP_G ? ROWS : CD_STEP_G;  // rows whose loads are in flight together
     __shared__ double smem[32];
     __shared__ float csum[2][4][64];  // (coarse row, thread row, column) partial block sums
-    float cpart0 = 0.f, cpart1 = 0.f;  // this thread's sums per coarse row
+    __shared__ double rvs[4 * ROWS][64];
     const double bmean = st->bmean;
     const float alpha = (float)fd->alpha, beta = (float)fd->beta;
     const int ob = xcd_order();
     const int bx = ob % gridDim.x, by = ob / gridDim.x;
-    const int x0 = bx * blockDim.x + threadIdx.x;
-    const int y0 = by * blockDim.y * ROWS + threadIdx.y;
+    const int lane = threadIdx.x;
+    const int x0 = bx * 64 + lane;
+    const int ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int Y0 = by * 4 * ROWS + ty * ROWS;  // the wave's first row
     const int x = min(x0, w - 1);
-    const int xl = max(x - 1, 0), xr = min(x + 1, w - 1);
-    // bricked offsets (a plane pair holds < 2^29 elements in blocked mode): the
-    // column parts of this cell and of its left / right neighbours are the same
-    // on every row; their planes alternate with the row
-    const unsigned cj = brick_col(x >> 1), cjl = brick_col(xl >> 1), cjr = brick_col(xr >> 1);
+    // lanes 0 and 63: the column beyond the wave's
+    const bool edge = lane == 0 || lane == 63;
+    const int xe = lane == 0 ? max(x - 1, 0) : min(x + 1, w - 1);
+    // bricked offsets (a plane pair holds < 2^29 elements in blocked mode)
+    const unsigned cj = brick_col(x >> 1), cje = brick_col(xe >> 1);
     // (24-bit multiplies, full rate: row and brick indices are < 2^24)
     const unsigned plane = (unsigned)bk.plane, brow = (unsigned)bk.nbx * 512u;
     auto rowo = [&](int c, int y) -> unsigned {
@@ -2090,69 +2096,76 @@ __global__ __launch_bounds__(256) void k_residual_step(const double* __restrict_
     auto ld64 = [](__amdgpu_buffer_rsrc_t rs, unsigned off) {
         return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
     };
-    // new direction and iterate at (xx, yy) from the loaded phi_in, z, p_old
-    auto pnew = [&](float zv, float pv) { return zv + beta * pv; };
-    auto phinew = [&](double ph, float pn) { return ph + (double)(alpha * pn); };
-    double rs = 0.0, rq = 0.0;
+    // a cell of phi_in, z and p_old; its new direction and iterate
+    struct Cell {
+        double ph;
+        float z, p;
+    };
+    auto load = [&](int col, unsigned cjc, int y) {
+        Cell c;
+        const int yc = min(max(y, 0), h - 1);
+        const unsigned bi = (rowo((col + yc) & 1, yc) + cjc) * 4u;
+        c.ph = ld64(phi_rs, (__umul24((unsigned)yc, (unsigned)w) + (unsigned)col) * 8u);
+        c.z = buf_load<float>(z_rs, bi, 0);
+        c.p = buf_load<float>(p_rs, bi, 0);
+        return c;
+    };
+    auto pnew = [&](const Cell& c) { return c.z + beta * c.p; };
+    auto phinew = [&](const Cell& c) { return c.ph + (double)(alpha * pnew(c)); };
+    Cell mid = load(x, cj, Y0);
+    double up = phinew(load(x, cj, Y0 - 1)), cur = phinew(mid);
 #pragma unroll
     for (int g = 0; g < ROWS; g += G) {
-        double ph[G][5], bb[G];
-        float zv[G][5], pv[G][5];
+        Cell next[G], side[G];
+        double bb[G];
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int y = min(y0 + (g + k) * (int)blockDim.y, h - 1);
-            const int yu = max(y - 1, 0), yd = min(y + 1, h - 1);
-            const int c = (x + y) & 1, o = 1 - c;
-            // centre, left, up, right, down (a clamped neighbour at the border
-            // is some valid cell: its value is not used)
-            const unsigned ro = rowo(o, y);
-            const unsigned bis[5] = {rowo(c, y) + cj, ro + cjl, rowo(o, yu) + cj, ro + cjr,
-                                     rowo(o, yd) + cj};
-            // byte offsets of the natural-layout cells: centre, left, up, right,
-            // down (the clamped ones at the border are valid cells, unused)
-            const unsigned co = (__umul24((unsigned)y, (unsigned)w) + (unsigned)x) * 8u;
-            const unsigned ws8 = (unsigned)w * 8u;
-            const unsigned pos[5] = {co, co - (unsigned)(x - xl) * 8u, co - (unsigned)(y - yu) * ws8,
-                                     co + (unsigned)(xr - x) * 8u, co + (unsigned)(yd - y) * ws8};
-#pragma unroll
-            for (int t = 0; t < 5; ++t) {
-                ph[k][t] = ld64(phi_rs, pos[t]);
-                zv[k][t] = buf_load<float>(z_rs, bis[t] * 4u, 0);
-                pv[k][t] = buf_load<float>(p_rs, bis[t] * 4u, 0);
-            }
-            bb[k] = ld64(b_rs, co);
+            next[k] = load(x, cj, Y0 + g + k + 1);
+            side[k] = Cell{0.0, 0.f, 0.f};
+            if (edge) side[k] = load(xe, cje, Y0 + g + k);
+            bb[k] = ld64(b_rs, (__umul24((unsigned)min(Y0 + g + k, h - 1), (unsigned)w) + (unsigned)x) * 8u);
         }
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int y = y0 + (g + k) * (int)blockDim.y;
-            if (x0 >= w || y >= h) break;
-            double nv[5];
-            float pc = 0.f;
-#pragma unroll
-            for (int t = 0; t < 5; ++t) {
-                const float pn = pnew(zv[k][t], pv[k][t]);
-                if (t == 0) pc = pn;
-                nv[t] = phinew(ph[k][t], pn);
-            }
+            const int y = Y0 + g + k;
+            const double down = phinew(next[k]), beyond = phinew(side[k]);
+            double left = lane_prev(cur), right = lane_next(cur);
+            left = lane == 0 ? beyond : left;
+            right = lane == 63 ? beyond : right;
             // neighbours in the order left, up, right, down
             double s = 0.0, cnt = 0.0;
-            if (x > 0) { cnt += 1.0; s += nv[1]; }
-            if (y > 0) { cnt += 1.0; s += nv[2]; }
-            if (x < w - 1) { cnt += 1.0; s += nv[3]; }
-            if (y < h - 1) { cnt += 1.0; s += nv[4]; }
-            const double rv = (bb[k] - bmean) - (s - cnt * nv[0]);
-            rs += rv;
-            rq += rv * rv;
-            if (x8) {
-                if ((int)threadIdx.y + 4 * (g + k) >= lf) cpart1 += (float)rv;
-                else cpart0 += (float)rv;
+            if (x > 0) { cnt += 1.0; s += left; }
+            if (y > 0) { cnt += 1.0; s += up; }
+            if (x < w - 1) { cnt += 1.0; s += right; }
+            if (y < h - 1) { cnt += 1.0; s += down; }
+            const double rv = (bb[k] - bmean) - (s - cnt * cur);
+            const bool in = x0 < w && y < h;
+            rvs[ty * ROWS + g + k][lane] = in ? rv : 0.0;
+            if (in) {
+                const unsigned bi = rowo((x + y) & 1, y) + cj;
+                __builtin_amdgcn_raw_buffer_store_b64(
+                    __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, cur), phio_rs,
+                    (__umul24((unsigned)y, (unsigned)w) + (unsigned)x) * 8u, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pnew(mid)), pn_rs, bi * 4u, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16((float)rv), r16_rs, bi * 2u, 0, 0);
             }
-            const unsigned bi = rowo((x + y) & 1, y) + cj;
-            __builtin_amdgcn_raw_buffer_store_b64(
-                __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, nv[0]), phio_rs,
-                (__umul24((unsigned)y, (unsigned)w) + (unsigned)x) * 8u, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pc), pn_rs, bi * 4u, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16((float)rv), r16_rs, bi * 2u, 0, 0);
+            up = cur;
+            cur = down;
+            mid = next[k];
+        }
+    }
+    // the sums take the rows ty, ty + 4, ... (the order of k_residual)
+    __syncthreads();
+    double rs = 0.0, rq = 0.0;
+    float cpart0 = 0.f, cpart1 = 0.f;  // this thread's sums per coarse row
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k) {
+        const double rv = rvs[ty + 4 * k][lane];
+        rs += rv;
+        rq += rv * rv;
+        if (x8) {
+            if (ty + 4 * k >= lf) cpart1 += (float)rv;
+            else cpart0 += (float)rv;
         }
     }
     double aq[2] = {rs, rq};
