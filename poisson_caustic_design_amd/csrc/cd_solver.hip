@@ -950,8 +950,11 @@ __device__ __forceinline__ void region_load(float (&ev)[2][R], RT (&rr)[2][R], c
 // error a rounded right-hand side leaves behind.  FORM_PROLONG: the
 // sweeps start from `mid` interpolated at the cells instead of from ein;
 // FORM_ENDS: as `ends` says.
+// (Registers for two workgroups per CU, but for tracking at 8 rows, which would
+// spill; an interpolating launch at 8 rows spills two and still takes a learned
+// iteration at 2048 x 2048 from 148 to 145 us.)
 template <int R, bool TRACK, int FORM>
-__global__ __launch_bounds__(BK_THREADS, (TRACK && R > 6) || (FORM == FORM_PROLONG && R > 4) ? 4 : 8) void k_rb_blocked(
+__global__ __launch_bounds__(BK_THREADS, TRACK && R > 6 ? 4 : 8) void k_rb_blocked(
     const float* ein, float* eout, const void* __restrict__ rhs, Brick bk, SweepTiles tiles,
     int nsweeps, float om2, float om3, float om4, const float* __restrict__ rmean, SolveDev* st,
     int out_index, MidGrid mid, TrackArgs track, BatchEnds ends) {
