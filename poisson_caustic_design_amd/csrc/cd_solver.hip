@@ -1892,8 +1892,15 @@ struct FcgDev {
 };
 
 // start of the learned iterations of a solve; p0: the zeroed first direction
-__global__ void k_fcg_init(FcgDev* fd, const float* p0) {
+// derived (NULL: none): (mean, rms) of an unnormalised input, (0, 1); zero (NULL:
+// none): the mean that the intermediate sweeps subtract
+__global__ void k_fcg_init(FcgDev* fd, const float* p0, double* derived, float* zero) {
     if (threadIdx.x != 0) return;
+    if (derived) {
+        derived[0] = 0.0;
+        derived[1] = 1.0;
+    }
+    if (zero) zero[0] = 0.f;
     fd->beta = 0.0;
     fd->alpha = 0.0;
     fd->pq = 0.0;
@@ -2421,8 +2428,11 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     hipLaunchKernelGGL(k_rhs_moments, rgrid, rblk, 0, s, b, w, h, sd, 1, partials);
     hipLaunchKernelGGL(k_rhs_finish, dim3(1), dim3(1024), 0, s, partials, nred, sd, 1, count);
     CD_CHECK_LAUNCH(ctx);
-    if (mixed) CD_TRY(cd_fill_f32(ctx, e32, blocked ? npk : n, 0.f));
-    if (blocked) CD_TRY(cd_fill_f32(ctx, e32b, npk, 0.f));
+    // (under the blocked residual rule every batch starts from zero by itself, and
+    // learned iterations write their corrections before they read them: what the
+    // buffers hold outside the grid is loaded, but not used)
+    if (mixed && (track || !blocked)) CD_TRY(cd_fill_f32(ctx, e32, blocked ? npk : n, 0.f));
+    if (blocked && track) CD_TRY(cd_fill_f32(ctx, e32b, npk, 0.f));
 
     const int fblocks = std::min(div_up((long long)n, CD_BLOCK), 65536);
     // residual launch of a check: kResidualRows rows per thread, fewer on
@@ -2627,11 +2637,8 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         CD_TRY(ctx->ensure(ctx->fcg_emb, sizeof(float) * npm));
         CD_TRY(ctx->ensure(ctx->fcg_rm, sizeof(unsigned short) * npm));
         CD_TRY(ctx->ensure(ctx->fcg_zero, sizeof(float) * 4));
-        // padding cells stay finite; the intermediate sweeps subtract a zero mean
-        CD_TRY(cd_fill_f32(ctx, ctx->fcg_em.as<float>(), npm, 0.f));
-        CD_TRY(cd_fill_f32(ctx, ctx->fcg_emb.as<float>(), npm, 0.f));
+        // the right-hand side's padding stays finite
         CD_TRY(cd_fill_f32(ctx, ctx->fcg_rm.as<float>(), npm / 2, 0.f));
-        CD_TRY(cd_fill_f32(ctx, ctx->fcg_zero.as<float>(), 4, 0.f));
     }
     if (learned || capture)
         CD_TRY(ctx->ensure(ctx->lc_stats, sizeof(double) * 2 * (kMaxPairsPerSolve + 2)));
@@ -2750,15 +2757,11 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const double start_rel = ctx->host_status->rel;
     if (learned && !done) {
         CD_TRY(cd_fill_f32(ctx, ctx->fcg_p.as<float>(), npk, 0.f));
-        CD_TRY(cd_fill_f32(ctx, ctx->fcg_q.as<float>(), npk, 0.f));
         hipLaunchKernelGGL(k_fcg_init, dim3(1), dim3(64), 0, s, ctx->fcg_dev.as<FcgDev>(),
-                           ctx->fcg_p.as<float>());
+                           ctx->fcg_p.as<float>(),
+                           direct_input ? ctx->lc_stats.as<double>() + 2 : nullptr,
+                           mid ? ctx->fcg_zero.as<float>() : nullptr);
         CD_CHECK_LAUNCH(ctx);
-        if (direct_input) {  // (mean, rms) of the unnormalised input: (0, 1)
-            double* derived = ctx->lc_stats.as<double>() + 2;
-            CD_TRY(cd_fill_f64(ctx, derived, 1, 0.0));
-            CD_TRY(cd_fill_f64(ctx, derived + 1, 1, 1.0));
-        }
         CD_TRY(ctx->ensure(ctx->phi_start, sizeof(double) * n));
         CD_HIP(ctx, hipMemcpyAsync(ctx->phi_start.ptr, phi, sizeof(double) * n,
                                    hipMemcpyDeviceToDevice, s));
