@@ -141,18 +141,21 @@ __global__ __launch_bounds__(256) void k_mesh_init(double* __restrict__ txy,
 }
 
 // image integral over quad slot k of vertex v (polygon_utils.cpp:311-366):
-// one thread per (vertex, adjacent-triangle slot)
-// One thread per (vertex, adjacent-quad slot), 64 threads per workgroup; the
-// clipping work polygons live in LDS (one column per lane) instead of
-// per-thread scratch memory.
+// one thread per (vertex, adjacent-triangle slot), 64 threads per workgroup.  The
+// clipping work polygons live in LDS (one column per lane) instead of per-thread
+// scratch memory.  Bound by the chain load - compare - divide - store of each
+// vertex at few waves per SIMD: fewer operations alone (comparisons for the cross
+// products) gave 3 %; 20 instead of 24 KiB of LDS (8 workgroups per CU instead of
+// 6), the first side from registers and the last without stores: 1165 -> 786 us at
+// a 512^2 mesh on 2048^2 pixels.
 constexpr int kQuadBlock = 64;
 __global__ __launch_bounds__(kQuadBlock) void k_quad_integrals(const double* __restrict__ pixels,
                                                                int nx, int ny, double W,
                                                                const double* __restrict__ xy,
                                                                int mx, int my,
                                                                double* __restrict__ quadacc) {
-    __shared__ double clipbuf[4 * CLIP_MAX * kQuadBlock];
-    double* buf = clipbuf + threadIdx.x;
+    __shared__ Pt clipbuf[2 * CLIP_MAX * kQuadBlock];
+    Pt* poly = clipbuf + threadIdx.x;
     const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long V = (long long)mx * my;
     if (gid >= 6 * V) return;
@@ -175,7 +178,8 @@ __global__ __launch_bounds__(kQuadBlock) void k_quad_integrals(const double* __r
         for (int py = (int)ylo; py < yhi; ++py)
             for (int pxi = (int)xlo; pxi < xhi; ++pxi) {
                 const double cx = ((double)pxi + 0.5) * px, cy = ((double)py + 0.5) * px;
-                acc += quad_pixel_area_s<kQuadBlock>(q, cx, cy, px, buf) *
+                acc += quad_pixel_area<kQuadBlock>(q, cx, cy, px, poly,
+                                                   poly + CLIP_MAX * kQuadBlock) *
                        pixels[(size_t)py * nx + pxi];
             }
     }

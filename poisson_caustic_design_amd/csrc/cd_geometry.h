@@ -104,112 +104,91 @@ __device__ __forceinline__ double bilinear(F at, int w, int h, double x, double 
 }
 
 // ---- convex clipping (Sutherland-Hodgman) ---------------------------------
-// Side of c relative to the directed line a->b: sign of (b-a) x (c-b)
-// (polygon_utils.cpp:33-41).  A subject vertex is kept unless strictly on the
-// outer side; a crossing is emitted only for strictly opposite consecutive
-// vertices with crossing parameter strictly inside (0,1)
-// (polygon_utils.cpp:43-60, 94-116).
-__device__ __forceinline__ int side_of(double ax, double ay, double bx, double by, double cx,
-                                       double cy) {
-    const double x = (bx - ax) * (cy - by) - (by - ay) * (cx - bx);
-    return x < 0 ? -1 : (x > 0 ? 1 : 0);
-}
+// A subject vertex is kept unless strictly on the outer side of the clip edge;
+// a crossing is emitted only for strictly opposite consecutive vertices with
+// crossing parameter strictly inside (0,1) (polygon_utils.cpp:43-60, 94-116).
+// A side adds at most one vertex to a convex polygon, so three leave 7; 10 has room
+// for a further pair, where rounding puts a crossing beyond its segment's end and
+// the next side lies between the two.
+constexpr int CLIP_MAX = 10;
 
-__device__ __forceinline__ bool crossing(double ax, double ay, double bx, double by, double sx,
-                                         double sy, double ex, double ey, double& ox, double& oy) {
-    const double cex = bx - ax, cey = by - ay;
-    const double dsx = ex - sx, dsy = ey - sy;
-    const double dx = ax - sx, dy = ay - sy;
-    const double den = dsx * cey - dsy * cex;
-    if (den == 0.0) return false;
-    const double t = (dx * cey - dy * cex) / den;
-    if (t <= 0 || t >= 1) return false;
-    ox = sx + t * dsx;
-    oy = sy + t * dsy;
-    return true;
-}
+struct Pt {
+    double x, y;
+};
 
-constexpr int CLIP_MAX = 12;
-
-// Clip polygon (px,py; n vertices) against the directed edge a->b keeping the
-// side `dir`; output into (qx,qy); returns the output count.  Vertex i of a
-// polygon is stored at index i * S (S = 1: a private array; S = 64: one
-// column per lane of a 64-wide LDS block, bank-conflict free).
-template <int S>
-__device__ __forceinline__ int clip_edge_s(const double* px, const double* py, int n, double ax,
-                                           double ay, double bx, double by, int dir, double* qx,
-                                           double* qy) {
-    int m = 0;
-    if (n == 0) return 0;
-    double sx = px[(n - 1) * S], sy = py[(n - 1) * S];
-    int ss = side_of(ax, ay, bx, by, sx, sy);
-    for (int i = 0; i < n; ++i) {
-        const double ex = px[i * S], ey = py[i * S];
-        const int se = side_of(ax, ay, bx, by, ex, ey);
-        if (ss != -dir && m < CLIP_MAX) { qx[m * S] = sx; qy[m * S] = sy; ++m; }
-        if (ss + se == 0 && ss != 0 && m < CLIP_MAX) {
-            double ox, oy;
-            if (crossing(ax, ay, bx, by, sx, sy, ex, ey, ox, oy)) {
-                qx[m * S] = ox;
-                qy[m * S] = oy;
-                ++m;
-            }
-        }
-        sx = ex; sy = ey; ss = se;
+// The clip edges are the sides of a pixel square, so the side of a vertex, the
+// sign of a cross product with one zero term (polygon_utils.cpp:33-41), is one
+// comparison of its coordinate with c, and numerator and denominator of the
+// crossing parameter keep one product each, with the square's extent w along the
+// edge: bit-equal to the full products.
+// Segment s->e of a polygon against one side: AXIS 0: x against c, 1: y; LOW: kept
+// at or above c, else at or below.  m vertices were emitted before; returns how many
+// were after.
+template <int AXIS, bool LOW, typename Emit>
+__device__ __forceinline__ int clip_segment(const Pt& s, const Pt& e, double c, double w, int m,
+                                            Emit emit) {
+    const double su = AXIS ? s.y : s.x, eu = AXIS ? e.y : e.x;
+    if (!(LOW ? su < c : su > c) && m < CLIP_MAX) emit(m++, s);
+    if (((su < c && eu > c) || (su > c && eu < c)) && m < CLIP_MAX) {
+        const double dx = e.x - s.x, dy = e.y - s.y;
+        const double den = (AXIS ? dy : dx) * w;
+        const double t = ((c - su) * w) / den;
+        if (den != 0.0 && t > 0 && t < 1) emit(m++, Pt{s.x + t * dx, s.y + t * dy});
     }
     return m;
 }
 
-template <int S>
-__device__ __forceinline__ double shoelace_s(const double* x, const double* y, int n) {
-    if (n < 3) return 0.0;
-    double s = 0.0;
+// the polygon of n vertices that load(i) gives; the next vertex's load is issued
+// before the current segment is worked on
+template <int AXIS, bool LOW, typename Load, typename Emit>
+__device__ __forceinline__ int clip_side(int n, double c, double w, Load load, Emit emit) {
+    int m = 0;
+    Pt s = load(n - 1), next = load(0);
+#pragma unroll 1
     for (int i = 0; i < n; ++i) {
-        const int k = (i + 1 == n) ? 0 : i + 1;
-        s += x[i * S] * y[k * S] - x[k * S] * y[i * S];
+        const Pt e = next;
+        next = load(i + 1 < n ? i + 1 : i);
+        m = clip_segment<AXIS, LOW>(s, e, c, w, m, emit);
+        s = e;
     }
-    return 0.5 * s;
+    return m;
 }
 
-__device__ __forceinline__ int clip_edge(const double* px, const double* py, int n, double ax,
-                                         double ay, double bx, double by, int dir, double* qx,
-                                         double* qy) {
-    return clip_edge_s<1>(px, py, n, ax, ay, bx, by, dir, qx, qy);
-}
-
-__device__ __forceinline__ double shoelace_n(const double* x, const double* y, int n) {
-    return shoelace_s<1>(x, y, n);
-}
-
-// Signed area of quad q (4 vertices) intersected with the pixel square of
-// side px centred at (cx, cy), square vertices ordered as
-// polygon_utils.cpp:336-346.  buf holds the four work polygons (ax, ay, bx,
-// by; CLIP_MAX vertices each, stride S).
+// Signed area of quad q (4 vertices) intersected with the pixel square of side
+// px centred at (cx, cy), its sides taken in the order of
+// polygon_utils.cpp:336-346.  Vertex i of the two work polygons is a[i * S] and
+// b[i * S] (CLIP_MAX vertices each; S = 64: one column per lane of a wave).  The
+// first side takes the quad from registers, and the last side's polygon is not
+// stored: its area is summed as its vertices come.
 template <int S>
-__device__ __forceinline__ double quad_pixel_area_s(const double* q, double cx, double cy,
-                                                    double px, double* buf) {
-    const double sx[4] = {cx - px / 2.0, cx - px / 2.0, cx + px / 2.0, cx + px / 2.0};
-    const double sy[4] = {cy - px / 2.0, cy + px / 2.0, cy + px / 2.0, cy - px / 2.0};
-    const int dir = side_of(sx[0], sy[0], sx[1], sy[1], sx[2], sy[2]);
-    double* ax = buf;
-    double* ay = buf + CLIP_MAX * S;
-    double* bx = buf + 2 * CLIP_MAX * S;
-    double* by = buf + 3 * CLIP_MAX * S;
-    for (int i = 0; i < 4; ++i) { ax[i * S] = q[2 * i]; ay[i * S] = q[2 * i + 1]; }
-    int n = clip_edge_s<S>(ax, ay, 4, sx[3], sy[3], sx[0], sy[0], dir, bx, by);
+__device__ __forceinline__ double quad_pixel_area(const double* q, double cx, double cy, double px,
+                                                  Pt* a, Pt* b) {
+    const double l = cx - px / 2.0, r = cx + px / 2.0, lo = cy - px / 2.0, hi = cy + px / 2.0;
+    const double w = r - l, h = hi - lo;
+    auto to = [](Pt* p) { return [p](int m, Pt v) { p[m * S] = v; }; };
+    auto from = [](const Pt* p) { return [p](int i) { return p[i * S]; }; };
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int k = (i + 3) & 3;
+        n = clip_segment<1, true>(Pt{q[2 * k], q[2 * k + 1]}, Pt{q[2 * i], q[2 * i + 1]}, lo, w, n,
+                                  to(b));
+    }
     if (n == 0) return 0.0;
-    n = clip_edge_s<S>(bx, by, n, sx[0], sy[0], sx[1], sy[1], dir, ax, ay);
+    n = clip_side<0, true>(n, l, h, from(b), to(a));
     if (n == 0) return 0.0;
-    n = clip_edge_s<S>(ax, ay, n, sx[1], sy[1], sx[2], sy[2], dir, bx, by);
+    n = clip_side<1, false>(n, hi, w, from(a), to(b));
     if (n == 0) return 0.0;
-    n = clip_edge_s<S>(bx, by, n, sx[2], sy[2], sx[3], sy[3], dir, ax, ay);
-    return shoelace_s<S>(ax, ay, n);
-}
-
-__device__ __forceinline__ double quad_pixel_area(const double* q, double cx, double cy,
-                                                  double px) {
-    double buf[4 * CLIP_MAX];
-    return quad_pixel_area_s<1>(q, cx, cy, px, buf);
+    Pt first = {0.0, 0.0}, prev = {0.0, 0.0};
+    double sum = 0.0;
+    n = clip_side<0, false>(n, r, h, from(b), [&](int m, Pt v) {
+        if (m == 0) first = v;
+        else sum += prev.x * v.y - v.x * prev.y;
+        prev = v;
+    });
+    if (n < 3) return 0.0;
+    sum += prev.x * first.y - first.x * prev.y;
+    return 0.5 * sum;
 }
 
 }  // namespace cdgeo
