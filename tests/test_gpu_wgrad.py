@@ -3,7 +3,7 @@ pixel tiles against images that are smaller, larger and no multiple of them,
 input channels of one to eight blocks of 16 with and without a remainder, output
 channels of half a block to four, linear and with ReLU masks, batches.
 
-The checker's activations are rounded to BF16 as the kernels store them; its
+The reference's activations are rounded to BF16 as the kernels store them; its
 gradients are not, so each of the up to 13 layers a gradient passes adds one
 2^-9 rounding per element: 2^-9 sqrt(13) = 0.7 % if independent, 2 % allowed
 over the whole gradient and 6 % (a block may have passed few independent
