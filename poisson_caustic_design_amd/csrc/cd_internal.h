@@ -246,10 +246,6 @@ struct SolveWork {
     double* phi2 = nullptr;
 };
 
-// Bytes of the reduction partials: four doubles for each of nred workgroups,
-// and room for the per-tile maxima of the max-update rule on small grids.
-constexpr size_t cd_partials_bytes(size_t nred) { return sizeof(double) * 4 * nred + 32768; }
-
 // Poisson solve on device-resident data.  b is the right-hand side (not
 // modified), phi the warm start/result (FP64).  mask: optional per-cell
 // neighbour-validity bits (NULL: no holes).  work: NULL takes the context's

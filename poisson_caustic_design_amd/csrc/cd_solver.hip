@@ -34,9 +34,6 @@
 
 namespace {
 
-constexpr int RED_BX = 64;
-constexpr int RED_BY = 4;
-
 // mask bits: neighbour validity (left, up, right, down) and "cell is a hole"
 constexpr uint8_t M_L = 1, M_U = 2, M_R = 4, M_D = 8, M_HOLE = 0x80;
 
@@ -127,26 +124,6 @@ __global__ __launch_bounds__(256) void k_flush(double* __restrict__ phi, float* 
         phi[i] += (double)ev;
         ea[i] = 0.f;
     }
-}
-
-// Bricked checkerboard layout of the blocked sweeps.  Colour c = (x+y)&1 and
-// packed column j = x>>1 split the grid into two planes of h x wp cells
-// (wp = (w+1)/2); each plane is stored in bricks of 8 rows x 64 packed columns
-// (2 KiB of FP32), bricks row-major.  A wave of the blocked kernel reads
-// 8 consecutive rows of one brick as one contiguous 2 KiB stream.
-struct Brick {
-    int wpb;       // packed columns rounded up to 64
-    int nbx;       // bricks per row of bricks
-    size_t plane;  // elements per colour plane (rows rounded up to 8)
-};
-
-inline Brick make_brick(int w, int h) {
-    Brick b;
-    const int wp = (w + 1) / 2;
-    b.wpb = (wp + 63) / 64 * 64;
-    b.nbx = b.wpb / 64;
-    b.plane = (size_t)((h + 7) / 8 * 8) * b.wpb;
-    return b;
 }
 
 __device__ __forceinline__ size_t brick_row(const Brick& b, int c, int Y) {
@@ -402,10 +379,6 @@ __global__ void k_check(const double* __restrict__ partials, int nblocks, SolveD
 // (a division per cell before: 13.6 us), and a missing row is read from a row of
 // zeros instead of being selected in every half-sweep.
 // ---------------------------------------------------------------------------
-constexpr int NAT_R = 4;    // rows per wave
-constexpr int NAT_NW = 16;  // waves per workgroup
-constexpr int NAT_RY = NAT_R * NAT_NW;
-
 // Per-cell constants of a wave at the grid border or with a mask.
 template <typename T>
 struct NatCells {
@@ -671,9 +644,6 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 #ifndef CD_BK_STORE_POLICY
 #define CD_BK_STORE_POLICY 16  // sc1: written through, not left dirty in L2
 #endif
-constexpr int BK_NW = 16;  // waves per workgroup
-constexpr int BK_THREADS = 64 * BK_NW;
-
 // What a wave's cells meet of the grid border, fixed per wave.  Columns: nothing;
 // the left border in lane 0 or the right one in lane 63 (odd cell), or neither;
 // a right border anywhere.  Rows: nothing; the wave's first row is the grid's
@@ -830,24 +800,6 @@ struct MidGrid {
     Brick bkm;
     int wm, hm, fm;
 };
-
-// Plane offsets (elements) of R <= 8 consecutive rows from Y on: they lie in at
-// most two bricks, so that one select per row and a constant give each.  Rows
-// beyond the plane's last brick get the offset of some row in it.
-struct BrickRows {
-    unsigned a, b;  // offset of row k less 64 k, before and from the brick border on
-    int split;
-    __device__ __forceinline__ unsigned at(int k) const { return (k < split ? a : b) + 64u * k; }
-};
-__device__ __forceinline__ BrickRows brick_rows(const Brick& bk, int Y, int h) {
-    const int nby = (h + 7) >> 3, by = min(Y >> 3, nby - 1);
-    const unsigned brow = (unsigned)bk.nbx * 512u;
-    BrickRows r;
-    r.a = (unsigned)by * brow + (unsigned)(Y & 7) * 64u;
-    r.b = r.a - 512u + (by + 1 < nby ? brow : 0u);
-    r.split = 8 - (Y & 7);
-    return r;
-}
 
 // The ends of a batch under the residual rule: its first launch starts from a
 // zero correction (zero), its last one adds the correction to the iterate phi
@@ -1139,8 +1091,6 @@ __global__ __launch_bounds__(BK_THREADS, TRACK && R > 6 ? 4 : 8) void k_rb_block
 // The kernel leaves phi alone and reports `holes` when b holds a NaN, and
 // returns at a check after kRegionSweeps sweeps (the host launches it again).
 // ---------------------------------------------------------------------------
-constexpr int kRegionSweeps = 16384;
-
 struct RegionArgs {
     int w, h, max_sweeps, kmax, adaptive, check_holes, resume;
     unsigned seq;
@@ -1523,91 +1473,6 @@ __global__ void k_set_holes_nan(double* __restrict__ phi, const uint8_t* __restr
                                 size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n && (mask[i] & M_HOLE)) phi[i] = NAN;
-}
-
-inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
-
-// Tiles of the natural-layout sweeps: the halo (twice the sweeps of a launch)
-// that is cheapest per sweep by what launches measured: about 5 us of dispatch,
-// loads and stores, and 0.43 us (FP64) or 0.28 us (FP32) per half-sweep and
-// round of one workgroup per CU.  At 400 x 400 in FP64 halos of 8 / 16 / 24 / 28
-// take 2.18 / 1.49 / 1.29 / 1.25 us per sweep; at 700 x 700 the 369 tiles of halo
-// 24 need a second round and take 2.12, halo 20 1.41.  track_room: bytes for a
-// tracking launch's two TrackOut.
-SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t track_room) {
-    const double half_us = fp64 ? 0.43 : 0.28, fixed_us = 5.0;
-    SweepTiles best = sweep_tiles(w, h, NAT_RY, 4);
-    double best_cost = INFINITY;
-    for (int halo = 4; halo <= 28; halo += 4) {
-        const SweepTiles t = sweep_tiles(w, h, NAT_RY, halo);
-        if (track && track_bytes(t.ntiles) > track_room) continue;
-        const int sweeps = std::min(halo / 2, std::max(batch, 1));
-        const double cost = (fixed_us + 2 * sweeps * half_us * div_up(t.ntiles, 256)) / sweeps;
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = t;
-        }
-    }
-    return best;
-}
-
-// How a batch of sweeps is cut into launches: sweeps per launch, rows per wave.
-struct BlockedPlan {
-    int rows, sweeps;
-    SweepTiles t;
-};
-
-// Time of a launch of `sweeps` sweeps over ntiles regions of 16 waves x `rows`
-// rows, in us: a first region per CU, a second (resident beside it, except
-// tracked at 8 rows), then every further one.  Fitted to launches of 4 to 19
-// sweeps on grids of 300 to 4096 squared, to 1 to 3 % (rows 4: 6.1 us for 5
-// sweeps of up to 256 regions, 8.6 for 14; rows 8: 10.0 for 8, 14.0 with two
-// regions per CU, 44.4 with nine); a half costs less than a launch's first ones
-// because waves at the inner borders sit out the later ones.
-double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
-    struct Cost { double first, first_half, second, second_half, next, next_half; };
-    static constexpr Cost cost[2][3] = {{{4.7, 0.142, 1.9, 0.005, 2.5, 0.023},
-                                         {5.1, 0.205, 1.7, 0.063, 4.0, 0.025},
-                                         {5.6, 0.268, 2.4, 0.100, 5.3, 0.042}},
-                                        {{6.9, 0.246, 3.2, 0.045, 3.5, 0.080},
-                                         {7.1, 0.332, 3.1, 0.137, 4.0, 0.134},
-                                         {7.4, 0.440, 8.0, 0.287, 6.4, 0.352}}};
-    const Cost& c = cost[track][(rows - 4) / 2];
-    const int halves = 2 * sweeps, rounds = div_up(ntiles, 256);
-    return c.first + c.first_half * halves + (rounds > 1 ? c.second + c.second_half * halves : 0.0) +
-           (c.next + c.next_half * halves) * std::max(rounds - 2, 0);
-}
-
-// The cut of a batch of `batch` sweeps on a w x h grid that blocked_launch_us
-// finds cheapest.  Per sweep, measured: 2048 x 2048 1.70 us (8 rows, 9 sweeps;
-// 2.78 with 4 rows, 5 sweeps), 1024 x 1024 0.87 (8, 17; 1.29), 400 x 400 0.62
-// (4, 14; 1.28); tracked, 400 x 400 1.12 (6, 15; 1.85 with 4 rows, 5 sweeps).
-// Tracking launches take whole groups, a halo of whole waves,
-// and need room for two TrackOut in track_room bytes.
-BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room) {
-    BlockedPlan best{4, kStopGroup, sweep_tiles(w, h, BK_NW * 4, 2 * kStopGroup)};
-    double best_us = INFINITY;
-    batch = std::max(batch, 1);
-    for (int rows = 4; rows <= 8; rows += 2) {
-        const int ry = BK_NW * rows, unit = track ? kStopGroup : 1;
-        const int most = track ? kTrackSweeps / unit * unit : 19;
-        for (int sweeps = unit; sweeps <= most; sweeps += unit) {
-            const int halo = track ? div_up(2 * sweeps, rows) * rows : 2 * sweeps;
-            if (ry - 2 * halo < 8) break;
-            SweepTiles t = sweep_tiles(w, h, ry, halo);
-            if (track && track_bytes(t.ntiles) > track_room) continue;
-            // a grid of one region takes any number of sweeps
-            const int per = t.ntiles > 1 ? sweeps : track ? most : batch;
-            const int full = batch / per, rest = batch % per;
-            const double us = full * blocked_launch_us(rows, per, t.ntiles, track) +
-                              (rest ? blocked_launch_us(rows, rest, t.ntiles, track) : 0.0);
-            if (us < best_us) {
-                best_us = us;
-                best = BlockedPlan{rows, per, t};
-            }
-        }
-    }
-    return best;
 }
 
 template <int R>

@@ -11,46 +11,10 @@
 // one region takes any number of sweeps in one launch.
 #pragma once
 
-#include <algorithm>
-#include <climits>
-
 #include "cd_internal.h"
+#include "cd_plan.h"
 
 namespace {
-
-constexpr int SW_RX = 128;  // region columns (64 lanes, two cells each)
-
-// Tiling of a w x h grid by regions of SW_RX x ry cells with `halo` overlap.
-// Region (tx, ty) starts at (min(tx*ix, we - SW_RX), min(ty*iy, he - ry)), never
-// below 0; we, he are w, h rounded up to even, so that a cell's colour is its
-// lane slot's on every region.  It stores columns [tx*ix + halo, (tx+1)*ix +
-// halo) (from 0 for the first region, to w for the last), and rows alike.
-struct SweepTiles {
-    int w, h, we, he;
-    int ry, halo, ix, iy;
-    int tiles_x, tiles_y, ntiles;
-    unsigned inv_x;  // floor((2^32 - 1) / tiles_x): tile * inv_x >> 32 is tile / tiles_x or one less
-};
-
-inline SweepTiles sweep_tiles(int w, int h, int ry, int halo) {
-    SweepTiles t;
-    t.w = w;
-    t.h = h;
-    t.we = (w + 1) / 2 * 2;
-    t.he = (h + 1) / 2 * 2;
-    t.ry = ry;
-    t.halo = halo;
-    t.ix = SW_RX - 2 * halo;
-    t.iy = ry - 2 * halo;
-    t.tiles_x = t.we <= SW_RX ? 1 : 1 + (t.we - SW_RX + t.ix - 1) / t.ix;
-    t.tiles_y = t.he <= ry ? 1 : 1 + (t.he - ry + t.iy - 1) / t.iy;
-    t.ntiles = t.tiles_x * t.tiles_y;
-    t.inv_x = UINT_MAX / (unsigned)t.tiles_x;
-    return t;
-}
-
-// workgroups of a launch over ntiles tiles: a multiple of 8 (see tile_of_block)
-inline int sweep_grid(int ntiles) { return (ntiles + 7) / 8 * 8; }
 
 // One region: its origin, the half-open range of cells it stores, and which of
 // its sides lie on the grid border.
@@ -150,35 +114,6 @@ __device__ __forceinline__ float add_next(float v, float b, float own) {
 // region's loads, which the decision would otherwise hold back; a word shared
 // by all tiles (atomicOr) cost 0.6 us of a launch at 50 tiles and 9 us at 1000.
 // ---------------------------------------------------------------------------
-// A max-update stop of the blocked sweeps falls at the end of a group of this
-// many sweeps, counted from the last check.
-constexpr int kStopGroup = 5;
-
-constexpr int kTrackSlots = 16;   // floats of maxima per tile
-constexpr int kTrackSweeps = 15;  // most sweeps of a tracking launch
-
-struct TrackOut {
-    unsigned* bits;  // [ntiles]
-    float* maxima;   // [ntiles][kTrackSlots]
-};
-// bytes of two TrackOut for ntiles tiles, and their placement in `base`
-inline size_t track_bytes(int ntiles) { return 2 * (size_t)ntiles * 4 * (1 + kTrackSlots); }
-inline TrackOut track_out(void* base, int ntiles, int which) {
-    unsigned* u = static_cast<unsigned*>(base) + (size_t)which * ntiles * (1 + kTrackSlots);
-    return {u, reinterpret_cast<float*>(u + ntiles)};
-}
-
-struct TrackArgs {
-    TrackOut out;    // this launch's
-    TrackOut prev;   // the previous launch's, null for a batch's first
-    int nprev;       // sweeps of the previous launch
-    int first_prev;  // sweeps of the solve before it
-    int group;       // sweeps the stop is rounded up to
-    int lid;         // launch number within the solve
-    int check_only;  // after a batch's last launch: decide, at most repeat it
-    double tol;
-};
-
 // The decision of a tracking launch, the same in every workgroup.
 struct TrackPlan {
     int nsweeps;  // sweeps to take (0: nothing to do)
