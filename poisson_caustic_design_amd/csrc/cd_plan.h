@@ -48,7 +48,9 @@ inline Brick make_brick(int w, int h) {
 
 // Plane offsets (elements) of R <= 8 consecutive rows from Y on: they lie in at
 // most two bricks, so that one select per row and a constant give each.  Rows
-// beyond the plane's last brick get the offset of some row in it.
+// beyond the plane's last brick get the offset of some row in it.  a and b are
+// offsets in the plane by themselves: a kernel passes them as scalar offsets, to
+// which the hardware adds the rest without wrapping.
 struct BrickRows {
     unsigned a, b;  // offset of row k less 64 k, before and from the brick border on
     int split;
@@ -59,7 +61,7 @@ CD_HD BrickRows brick_rows(const Brick& bk, int Y, int h) {
     const unsigned brow = (unsigned)bk.nbx * 512u;
     BrickRows r;
     r.a = (unsigned)by * brow + (unsigned)(Y & 7) * 64u;
-    r.b = r.a - 512u + (by + 1 < nby ? brow : 0u);
+    r.b = by + 1 < nby ? r.a + brow - 512u : (unsigned)by * brow;
     r.split = 8 - (Y & 7);
     return r;
 }
