@@ -116,23 +116,24 @@ constexpr int kRegionSweeps = 16384;
 // many sweeps, counted from the last check.
 constexpr int kStopGroup = 5;
 
-constexpr int kTrackSlots = 16;   // floats of maxima per tile
 constexpr int kTrackSweeps = 15;  // most sweeps of a tracking launch
 
+// slots: the most sweeps of a launch of the batch
 struct TrackOut {
     unsigned* bits;  // [ntiles]
-    float* maxima;   // [ntiles][kTrackSlots]
+    float* maxima;   // [ntiles][slots]
 };
 // bytes of two TrackOut for ntiles tiles, and their placement in `base`
-inline size_t track_bytes(int ntiles) { return 2 * (size_t)ntiles * 4 * (1 + kTrackSlots); }
-inline TrackOut track_out(void* base, int ntiles, int which) {
-    unsigned* u = static_cast<unsigned*>(base) + (size_t)which * ntiles * (1 + kTrackSlots);
+inline size_t track_bytes(int ntiles, int slots) { return 2 * (size_t)ntiles * 4 * (1 + slots); }
+inline TrackOut track_out(void* base, int ntiles, int slots, int which) {
+    unsigned* u = static_cast<unsigned*>(base) + (size_t)which * ntiles * (1 + slots);
     return {u, reinterpret_cast<float*>(u + ntiles)};
 }
 
 struct TrackArgs {
     TrackOut out;    // this launch's
     TrackOut prev;   // the previous launch's, null for a batch's first
+    int slots;       // floats of maxima per tile
     int nprev;       // sweeps of the previous launch
     int first_prev;  // sweeps of the solve before it
     int group;       // sweeps the stop is rounded up to
@@ -141,20 +142,27 @@ struct TrackArgs {
     double tol;
 };
 
+// Sweeps of a launch of the natural-layout sweeps: a grid of one region takes any
+// number.
+inline int natural_sweeps(const SweepTiles& t, int batch, bool track) {
+    return t.ntiles > 1 ? t.halo / 2 : track ? kTrackSweeps : batch;
+}
+
 // Tiles of the natural-layout sweeps: the halo (twice the sweeps of a launch)
 // that is cheapest per sweep by what launches measured: about 5 us of dispatch,
 // loads and stores, and 0.43 us (FP64) or 0.28 us (FP32) per half-sweep and
 // round of one workgroup per CU.  At 400 x 400 in FP64 halos of 8 / 16 / 24 / 28
 // take 2.18 / 1.49 / 1.29 / 1.25 us per sweep; at 700 x 700 the 369 tiles of halo
 // 24 need a second round and take 2.12, halo 20 1.41.  track_room: bytes for a
-// tracking launch's two TrackOut.
+// tracking launch's two TrackOut; cd_partials_bytes has room for those of the
+// smallest halo on every shape.
 SweepTiles natural_tiles(int w, int h, bool fp64, int batch, bool track, size_t track_room) {
     const double half_us = fp64 ? 0.43 : 0.28, fixed_us = 5.0;
     SweepTiles best = sweep_tiles(w, h, NAT_RY, 4);
     double best_cost = INFINITY;
     for (int halo = 4; halo <= 28; halo += 4) {
         const SweepTiles t = sweep_tiles(w, h, NAT_RY, halo);
-        if (track && track_bytes(t.ntiles) > track_room) continue;
+        if (track && track_bytes(t.ntiles, natural_sweeps(t, batch, true)) > track_room) continue;
         const int sweeps = std::min(halo / 2, std::max(batch, 1));
         const double cost = (fixed_us + 2 * sweeps * half_us * div_up(t.ntiles, 256)) / sweeps;
         if (cost < best_cost) {
@@ -197,9 +205,11 @@ double blocked_launch_us(int rows, int sweeps, int ntiles, bool track) {
 // 2.78 with 4 rows, 5 sweeps), 1024 x 1024 0.87 (8, 17; 1.29), 400 x 400 0.62
 // (4, 14; 1.28); tracked, 400 x 400 1.12 (6, 15; 1.85 with 4 rows, 5 sweeps).
 // Tracking launches take whole groups, a halo of whole waves,
-// and need room for two TrackOut in track_room bytes.
+// and need room for two TrackOut in track_room bytes; cd_partials_bytes has room
+// for those of 4 rows and one group on every shape (48 bytes a region of 104
+// columns, where the partials of up to 4 rows have 32 per 64).
 BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room) {
-    BlockedPlan best{4, kStopGroup, sweep_tiles(w, h, BK_NW * 4, 2 * kStopGroup)};
+    BlockedPlan best{};
     double best_us = INFINITY;
     batch = std::max(batch, 1);
     for (int rows = 4; rows <= 8; rows += 2) {
@@ -209,9 +219,9 @@ BlockedPlan blocked_plan(int w, int h, int batch, bool track, size_t track_room)
             const int halo = track ? div_up(2 * sweeps, rows) * rows : 2 * sweeps;
             if (ry - 2 * halo < 8) break;
             SweepTiles t = sweep_tiles(w, h, ry, halo);
-            if (track && track_bytes(t.ntiles) > track_room) continue;
             // a grid of one region takes any number of sweeps
             const int per = t.ntiles > 1 ? sweeps : track ? most : batch;
+            if (track && track_bytes(t.ntiles, per) > track_room) continue;
             const int full = batch / per, rest = batch % per;
             const double us = full * blocked_launch_us(rows, per, t.ntiles, track) +
                               (rest ? blocked_launch_us(rows, rest, t.ntiles, track) : 0.0);

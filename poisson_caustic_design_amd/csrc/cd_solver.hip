@@ -2369,6 +2369,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
                                             cd_partials_bytes(nred));
         TrackArgs tr{};
         tr.group = kStopGroup;
+        tr.slots = pl.sweeps;
         tr.tol = o->tol;
         const int skipped = ahead > 0 ? 1 : 0;
         int launches = skipped;
@@ -2379,7 +2380,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             float* ein = bufs[launches & 1];
             float* eout = bufs[1 - (launches & 1)];
             tr.lid = ++track_lid;
-            tr.out = track_out(partials, pl.t.ntiles, launches & 1);
+            tr.out = track_out(partials, pl.t.ntiles, tr.slots, launches & 1);
             launch_blocked(pl, track != 0, launches == 0 ? pro : nullptr, s, ein, eout, rhs, bk,
                            nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr,
                            BatchEnds{done_sw + nsw == count_sweeps ? ends.phi : nullptr,
@@ -2411,12 +2412,13 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         using T = std::remove_pointer_t<decltype(b0)>;
         const SweepTiles t = natural_tiles(w, h, sizeof(T) == 8, count_sweeps, track != 0,
                                            cd_partials_bytes(nred));
-        const int most = t.ntiles == 1 ? (track ? kTrackSweeps : count_sweeps) : t.halo / 2;
+        const int most = natural_sweeps(t, count_sweeps, track != 0);
         const dim3 grid(sweep_grid(t.ntiles)), blk(64 * NAT_NW);
         const NatOmega<T> oms{om, om / 2, om / 3, om / 4};
         int cur = mixed ? 0 : ctx->host_status->cur;
         TrackArgs tr{};
         tr.group = 1;
+        tr.slots = most;
         tr.tol = o->tol;
         CD_TRY(timer_begin());
         int launches = 0;
@@ -2426,7 +2428,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             T* out = cur ? b0 : b1;
             if (track) {
                 tr.lid = ++track_lid;
-                tr.out = track_out(partials, t.ntiles, launches & 1);
+                tr.out = track_out(partials, t.ntiles, tr.slots, launches & 1);
                 hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, in, out, rhs, mask, t,
                                    nsw, oms, mean, sd, 1 - cur, tr);
                 tr.prev = tr.out;

@@ -41,11 +41,35 @@ void rows_in_plane() {
         }
 }
 
+// Every tracking plan's words and maxima fit behind the partials' other use, on
+// any shape, and its halo is whole waves (the cells that count are whole waves').
+void tracking_room() {
+    for (int h : {2, 3, 4, 5, 8, 60, 64, 65, 97, 300, 4000})
+        for (double wd = 2; wd * h < 5e8; wd *= 1.07) {
+            const int w = (int)wd;
+            const size_t room = cd_partials_bytes((size_t)div_up(w, RED_BX) * div_up(h, RED_BY));
+            for (int batch : {1, 4, 5, 7, 15, 92, 1000}) {
+                const BlockedPlan p = blocked_plan(w, h, batch, true, room);
+                CHECK(p.t.ntiles >= 1 && track_bytes(p.t.ntiles, p.sweeps) <= room,
+                      "%d x %d, batch %d, blocked", w, h, batch);
+                CHECK(p.t.ntiles == 1 || (p.t.halo % p.rows == 0 && p.t.halo >= 2 * p.sweeps),
+                      "%d x %d, batch %d: halo %d, %d rows, %d sweeps", w, h, batch, p.t.halo,
+                      p.rows, p.sweeps);
+                for (bool fp64 : {false, true}) {
+                    const SweepTiles t = natural_tiles(w, h, fp64, batch, true, room);
+                    CHECK(track_bytes(t.ntiles, natural_sweeps(t, batch, true)) <= room,
+                          "%d x %d, batch %d, natural", w, h, batch);
+                }
+            }
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const struct { const char* name; void (*fn)(); } checks[] = {
         {"rows_in_plane", rows_in_plane},
+        {"tracking_room", tracking_room},
     };
     for (const auto& c : checks)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {

@@ -23,3 +23,7 @@ def plan_check(tmp_path_factory):
 
 def test_region_rows_lie_in_the_plane(plan_check):
     plan_check("rows_in_plane")
+
+
+def test_tracking_words_fit_on_every_shape(plan_check):
+    plan_check("tracking_room")
