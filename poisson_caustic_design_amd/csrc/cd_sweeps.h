@@ -8,7 +8,7 @@
 // region border equal n global half-sweeps, and those are stored.  Regions at
 // the grid border end there (no halo on that side): what lies beyond reads as
 // zero, so a border cell's neighbour sum needs no weights, and a grid that fits
-// one region takes any number of sweeps in one launch.
+// one region takes up to kRegionSweeps sweeps in one launch.
 #pragma once
 
 #include "cd_internal.h"

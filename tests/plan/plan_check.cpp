@@ -64,12 +64,27 @@ void tracking_room() {
         }
 }
 
+// No plan puts more sweeps into a launch than a solve in one workgroup takes.
+void launch_length() {
+    for (int w : {2, 40, 128, 129, 500})
+        for (int h : {2, 40, 64, 128, 129, 500})
+            for (int batch : {1, 100, 16384, 16385, 100000, INT_MAX})
+                for (bool track : {false, true}) {
+                    const BlockedPlan p = blocked_plan(w, h, batch, track, 1u << 20);
+                    CHECK(p.sweeps <= kRegionSweeps, "%d x %d, batch %d: %d", w, h, batch, p.sweeps);
+                    const int n =
+                        natural_sweeps(natural_tiles(w, h, true, batch, track, 1u << 20), batch, track);
+                    CHECK(n <= kRegionSweeps, "%d x %d, batch %d: %d", w, h, batch, n);
+                }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const struct { const char* name; void (*fn)(); } checks[] = {
         {"rows_in_plane", rows_in_plane},
         {"tracking_room", tracking_room},
+        {"launch_length", launch_length},
     };
     for (const auto& c : checks)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {

@@ -27,3 +27,7 @@ def test_region_rows_lie_in_the_plane(plan_check):
 
 def test_tracking_words_fit_on_every_shape(plan_check):
     plan_check("tracking_room")
+
+
+def test_launches_are_bounded(plan_check):
+    plan_check("launch_length")
