@@ -143,6 +143,39 @@ struct TrackArgs {
     double tol;
 };
 
+// The tracking launches of a batch: each reads the words of the one before and
+// leaves its own in the other TrackOut, the one that only checks too (it may repeat
+// a launch and leave words, while workgroups that start later still read).
+struct TrackBatch {
+    void* base;  // both TrackOut
+    int ntiles;
+    TrackArgs a;
+    int launches;
+    // the next launch: nsweeps sweeps after the solve's first `first`
+    TrackArgs launch(int lid, int nsweeps, int first) {
+        a.lid = lid;
+        a.out = track_out(base, ntiles, a.slots, launches++ & 1);
+        const TrackArgs now = a;
+        a.prev = a.out;
+        a.nprev = nsweeps;
+        a.first_prev = first;
+        return now;
+    }
+    // after the last one
+    TrackArgs check(int lid) {
+        TrackArgs now = launch(lid, 0, 0);
+        now.check_only = 1;
+        return now;
+    }
+};
+inline TrackBatch track_batch(void* base, int ntiles, int slots, int group, double tol) {
+    TrackBatch t{base, ntiles, {}, 0};
+    t.a.slots = slots;
+    t.a.group = group;
+    t.a.tol = tol;
+    return t;
+}
+
 // Sweeps of a launch of the natural-layout sweeps: a grid of one region takes any
 // number up to kRegionSweeps.
 inline int natural_sweeps(const SweepTiles& t, int batch, bool track) {

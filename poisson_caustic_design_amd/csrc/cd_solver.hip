@@ -2367,10 +2367,7 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         CD_TRY(timer_begin());
         const BlockedPlan pl = blocked_plan(w, h, count_sweeps - ahead, track != 0,
                                             cd_partials_bytes(nred));
-        TrackArgs tr{};
-        tr.group = kStopGroup;
-        tr.slots = pl.sweeps;
-        tr.tol = o->tol;
+        TrackBatch words = track_batch(partials, pl.t.ntiles, pl.sweeps, kStopGroup, o->tol);
         const int skipped = ahead > 0 ? 1 : 0;
         int launches = skipped;
         float* bufs[2] = {e32, e32b};
@@ -2379,22 +2376,17 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
             const int nsw = std::min(pl.sweeps, count_sweeps - done_sw);
             float* ein = bufs[launches & 1];
             float* eout = bufs[1 - (launches & 1)];
-            tr.lid = ++track_lid;
-            tr.out = track_out(partials, pl.t.ntiles, tr.slots, launches & 1);
             launch_blocked(pl, track != 0, launches == 0 ? pro : nullptr, s, ein, eout, rhs, bk,
-                           nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr,
+                           nsw, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1),
+                           words.launch(++track_lid, nsw, first + done_sw),
                            BatchEnds{done_sw + nsw == count_sweeps ? ends.phi : nullptr,
                                      launches == 0 ? ends.zero : 0});
-            tr.prev = tr.out;
-            tr.nprev = nsw;
-            tr.first_prev = first + done_sw;
             done_sw += nsw;
         }
         if (track) {  // the last launch's own decision
-            tr.lid = ++track_lid;
-            tr.check_only = 1;
             launch_blocked(pl, true, nullptr, s, bufs[launches & 1], bufs[1 - (launches & 1)], rhs,
-                           bk, 0, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1), tr);
+                           bk, 0, om2, om3, om4, &sd->rmean32, sd, 1 - (launches & 1),
+                           words.check(++track_lid));
             ++launches;
         }
         CD_CHECK_LAUNCH(ctx);
@@ -2416,34 +2408,25 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         const dim3 grid(sweep_grid(t.ntiles)), blk(64 * NAT_NW);
         const NatOmega<T> oms{om, om / 2, om / 3, om / 4};
         int cur = mixed ? 0 : ctx->host_status->cur;
-        TrackArgs tr{};
-        tr.group = 1;
-        tr.slots = most;
-        tr.tol = o->tol;
+        TrackBatch words = track_batch(partials, t.ntiles, most, 1, o->tol);
         CD_TRY(timer_begin());
         int launches = 0;
         for (int done_sw = 0; done_sw < count_sweeps; ++launches) {
             const int nsw = std::min(most, count_sweeps - done_sw);
             T* in = cur ? b1 : b0;
             T* out = cur ? b0 : b1;
-            if (track) {
-                tr.lid = ++track_lid;
-                tr.out = track_out(partials, t.ntiles, tr.slots, launches & 1);
+            const TrackArgs tr = words.launch(++track_lid, nsw, first + done_sw);
+            if (track)
                 hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, in, out, rhs, mask, t,
                                    nsw, oms, mean, sd, 1 - cur, tr);
-                tr.prev = tr.out;
-                tr.nprev = nsw;
-                tr.first_prev = first + done_sw;
-            } else {
+            else
                 hipLaunchKernelGGL((k_rb_natural<T, false>), grid, blk, 0, s, in, out, rhs, mask, t,
                                    nsw, oms, mean, sd, 1 - cur, tr);
-            }
             cur = 1 - cur;
             done_sw += nsw;
         }
         if (track) {  // the last launch's own decision
-            tr.lid = ++track_lid;
-            tr.check_only = 1;
+            const TrackArgs tr = words.check(++track_lid);
             hipLaunchKernelGGL((k_rb_natural<T, true>), grid, blk, 0, s, cur ? b1 : b0,
                                cur ? b0 : b1, rhs, mask, t, 0, oms, mean, sd, 1 - cur, tr);
             ++launches;

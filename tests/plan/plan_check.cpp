@@ -2,6 +2,8 @@
 // One check per argument; prints what fails and exits with 1.
 #include <cstdio>
 #include <cstring>
+#include <utility>
+#include <vector>
 
 #include "cd_plan.h"
 
@@ -78,6 +80,39 @@ void launch_length() {
                 }
 }
 
+// No tracking launch writes what it reads, and each reads what the one before wrote.
+void track_words() {
+    for (int ntiles : {1, 7, 600})
+        for (int slots : {2, 5, 15})
+            for (int launches = 1; launches < 6; ++launches) {
+                std::vector<unsigned> buf(track_bytes(ntiles, slots) / 4);
+                TrackBatch b = track_batch(buf.data(), ntiles, slots, 5, 1.0);
+                auto range = [&](const TrackOut& t) {  // [first, last) word of a TrackOut
+                    const long lo = t.bits - buf.data();
+                    const long hi = reinterpret_cast<unsigned*>(t.maxima) - buf.data() +
+                                    (long)ntiles * slots;
+                    return std::pair<long, long>(lo, hi);
+                };
+                unsigned* last = nullptr;
+                for (int i = 0; i <= launches; ++i) {
+                    const TrackArgs a = i < launches ? b.launch(i + 1, slots, slots * i)
+                                                     : b.check(i + 1);
+                    CHECK(a.prev.bits == last, "launch %d of %d", i, launches);
+                    CHECK(a.check_only == (i == launches), "launch %d of %d", i, launches);
+                    CHECK(i == 0 || (a.nprev == slots && a.first_prev == slots * (i - 1)),
+                          "launch %d of %d", i, launches);
+                    const auto out = range(a.out);
+                    CHECK(out.first >= 0 && out.second <= (long)buf.size(), "launch %d", i);
+                    if (last) {
+                        const auto prev = range(a.prev);
+                        CHECK(out.second <= prev.first || prev.second <= out.first,
+                              "launch %d of %d writes what it reads", i, launches);
+                    }
+                    last = a.out.bits;
+                }
+            }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -85,6 +120,7 @@ int main(int argc, char** argv) {
         {"rows_in_plane", rows_in_plane},
         {"tracking_room", tracking_room},
         {"launch_length", launch_length},
+        {"track_words", track_words},
     };
     for (const auto& c : checks)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {

@@ -31,3 +31,7 @@ def test_tracking_words_fit_on_every_shape(plan_check):
 
 def test_launches_are_bounded(plan_check):
     plan_check("launch_length")
+
+
+def test_tracking_launches_do_not_write_what_they_read(plan_check):
+    plan_check("track_words")
