@@ -17,9 +17,9 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <exception>
 #include <limits>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -110,7 +110,9 @@ struct OrderBuilder {
     // entry is the one its ancestors' splits put there: a value of the call,
     // which lets the halves go in parallel.  Past the array's end (undefined in
     // the reference) it is NaN, not below any split value.
-    void node(int start, int end, int level, const double next[2]) {
+    // (Nothing in here throws: a thread that cannot be had, for whatever reason, only
+    // leaves its half to this one.)
+    void node(int start, int end, int level, const double next[2]) noexcept {
         const double inf = std::numeric_limits<double>::infinity();
         double mn[2] = {inf, inf}, mx_[2] = {-inf, -inf};
         if (end - start <= kLeafSize || level >= kMaxDepth) return;
@@ -131,7 +133,7 @@ struct OrderBuilder {
             std::thread first;
             try {
                 first = std::thread([&] { node(start, m, level + 1, mid); });
-            } catch (const std::system_error&) {  // no thread to be had: one after the other
+            } catch (const std::exception&) {  // no thread or memory: one after the other
             }
             if (first.joinable()) {
                 node(m, end, level + 1, next);
