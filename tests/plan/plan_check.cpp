@@ -113,6 +113,17 @@ void track_words() {
             }
 }
 
+// The launch that goes out ahead of a batch is one launch, so that the batch goes on
+// from its output.
+void early_launch() {
+    for (int w = 2; w <= 6000; w += w < 700 ? 1 : 37)
+        for (int h = 2; h <= 6000; h += h < 300 ? 3 : 53) {
+            const int ahead = std::min(8, blocked_plan(w, h, 8, false, 0).sweeps);
+            const int per = blocked_plan(w, h, ahead, false, 0).sweeps;
+            CHECK(per >= ahead, "%d x %d: %d sweeps in launches of %d", w, h, ahead, per);
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -121,6 +132,7 @@ int main(int argc, char** argv) {
         {"tracking_room", tracking_room},
         {"launch_length", launch_length},
         {"track_words", track_words},
+        {"early_launch", early_launch},
     };
     for (const auto& c : checks)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {

@@ -35,3 +35,7 @@ def test_launches_are_bounded(plan_check):
 
 def test_tracking_launches_do_not_write_what_they_read(plan_check):
     plan_check("track_words")
+
+
+def test_the_early_launch_is_one_launch(plan_check):
+    plan_check("early_launch")
