@@ -14,8 +14,12 @@
 //     `check_every` sweeps e is folded into the FP64 base (defect correction)
 //     and the FP64 relative residual is evaluated on the device.
 //   * CD_PREC_FP64: the same sweeps in FP64 directly on phi.
-//   * stop rules are evaluated by device kernels that set a `done` flag; later
-//     sweep launches of the same batch see the flag and exit immediately.
+//   * stop rules are evaluated on the device.  Residual rule: a check sets the
+//     `done` flag, and the host, which waits for it, enqueues no more sweeps (a
+//     launch that went out early only writes the correction).  Max-update rule:
+//     every launch decides from the words of the one before whether the solve
+//     stopped in it; then it repeats that launch up to the stop and records its
+//     number in `stop_lid`, and the launches after it return at once.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -637,13 +641,15 @@ __global__ __launch_bounds__(64 * NAT_NW) void k_rb_natural(
 // a wider halo: blocked_plan weighs these.  Registers: 64 VGPRs (R = 8) keep two
 // workgroups per CU; row and column kinds per wave instead of a factor per cell
 // made room for that (102 VGPRs before, one workgroup per CU, 21.9 us for 8
-// sweeps at 2048 x 2048 against 16.1).  Measured and not taken: 8 waves of 16
-// rows 19.1 us, 12 of 8 18.1, 8 of 8 18.6, 4 of 16 23.6, 16 of 10 24.9.
+// sweeps at 2048 x 2048 against 16.1).  Against those 16.1, when all waves still took
+// every sweep and the set-up was longer, and not measured since: 8 waves of 16 rows
+// 19.1 us, 12 of 8 18.1, 8 of 8 18.6, 4 of 16 23.6, 16 of 10 24.9.
 // ---------------------------------------------------------------------------
 // cache policy bits of the blocked kernel's stores
 #ifndef CD_BK_STORE_POLICY
 #define CD_BK_STORE_POLICY 16  // sc1: written through, not left dirty in L2
 #endif
+
 // What a wave's cells meet of the grid border, fixed per wave.  Columns: nothing;
 // the left border in lane 0 or the right one in lane 63 (odd cell), or neither;
 // a right border anywhere.  Rows: nothing; the wave's first row is the grid's
@@ -657,7 +663,6 @@ enum { ROWS_IN = 0, ROWS_TOP = 1, ROWS_BOTTOM = 2, ROWS_BELOW = 3, ROWS_ANY = 4 
 struct BlockCells {
     float om4, c1;             // omega / 4, 1 - omega
     float oc[2], oc_end[2];    // omega / cnt in a row with both neighbour rows, with one
-    bool miss_l;               // cell 0 has no left neighbour
     bool miss_r[2];            // the cell has no right neighbour
     unsigned end_rows;         // bit k: row k of the wave has one neighbour row
     unsigned out_rows;         // bit k: row k lies outside the grid
@@ -967,7 +972,6 @@ __global__ __launch_bounds__(BK_THREADS, TRACK && R > 6 ? 4 : 8) void k_rb_block
         if (Yw + k == 0 || Yw + k == h - 1) g.end_rows |= 1u << k;
         if (Yw + k >= h) g.out_rows |= 1u << k;
     }
-    g.miss_l = x0 == 0;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const bool in = x0 + p < w;
@@ -1249,7 +1253,6 @@ __global__ __launch_bounds__(BK_THREADS) void k_solve_region(const double* __res
         if (Yw + k == 0 || Yw + k == h - 1) g.end_rows |= 1u << k;
         if (Yw + k >= h) g.out_rows |= 1u << k;
     }
-    g.miss_l = x0 == 0;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const bool in = x0 + p < w;
@@ -2236,9 +2239,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const dim3 rblk(RED_BX, RED_BY);
     const dim3 rgrid(div_up(w, RED_BX), div_up(h, RED_BY));
     const int nred = rgrid.x * rgrid.y;
-    // FP32 sweeps without holes take the temporally blocked kernel on the
-    // packed layout; FP64 sweeps and hole masks take the per-half-sweep kernel.
-    // (the blocked kernel addresses a plane pair through 32-bit byte offsets)
+    // FP32 sweeps without holes take k_rb_blocked on the bricked layout; FP64
+    // sweeps and hole masks take k_rb_natural, blocked in time as well.
+    // (the bricked layout's kernels address a plane pair through 32-bit byte offsets)
     const Brick bk = make_brick(w, h);
     const bool blocked = mixed && mask == nullptr && 2 * bk.plane * sizeof(float) < (1ull << 31);
     const size_t npk = 2 * bk.plane;
@@ -2305,9 +2308,6 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
     const int kResidualRows = nred >= 16384 ? 8 : nred >= 8192 ? 4 : nred >= 4096 ? 2 : 1;
     const dim3 cgrid(div_up(w, RED_BX), div_up(h, RED_BY * kResidualRows));
     const int ncheck = cgrid.x * cgrid.y;  // <= nred
-    // flush: fold the current FP32 correction into phi64 first (the last launch of
-    // a batch under the blocked residual rule has done that, and so have learned
-    // iterations)
     // the end of every check: k_check on the residual pass's partials, then the
     // host's wait for the status (the residual pass's timer is open)
     // (wait false: the caller enqueues the work that follows and waits itself)
@@ -2329,6 +2329,9 @@ int cd_solve_device_internal(cd_context* ctx, const double* b, double* phi, cons
         }
         return CD_OK;
     };
+    // flush: fold the current FP32 correction into phi64 first (the last launch of
+    // a batch under the blocked residual rule has done that, and so have learned
+    // iterations)
     auto enqueue_check = [&](int check_id, bool flush = true, bool wait = true) -> int {
         CD_TRY(timer_begin());
         if (blocked) {
