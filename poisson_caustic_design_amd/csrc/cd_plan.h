@@ -61,7 +61,8 @@ CD_HD BrickRows brick_rows(const Brick& bk, int Y, int h) {
     const unsigned brow = (unsigned)bk.nbx * 512u;
     BrickRows r;
     r.a = (unsigned)by * brow + (unsigned)(Y & 7) * 64u;
-    r.b = by + 1 < nby ? r.a + brow - 512u : (unsigned)by * brow;
+    const int b = (int)(r.a + (by + 1 < nby ? brow : 0u)) - 512;
+    r.b = (unsigned)(b > 0 ? b : 0);  // (below 0 on a single row of bricks)
     r.split = 8 - (Y & 7);
     return r;
 }
@@ -119,12 +120,15 @@ constexpr int kStopGroup = 5;
 
 constexpr int kTrackSweeps = 15;  // most sweeps of a tracking launch
 
-// slots: the most sweeps of a launch of the batch
+// A launch's words.  The maxima are as many a tile as the launch has sweeps, which
+// writer and reader hold anyway (a stride of its own in the arguments spilled 5 more
+// scalars at 6 rows).
 struct TrackOut {
     unsigned* bits;  // [ntiles]
-    float* maxima;   // [ntiles][slots]
+    float* maxima;   // [ntiles][sweeps of the launch]
 };
-// bytes of two TrackOut for ntiles tiles, and their placement in `base`
+// bytes of two TrackOut for ntiles tiles and launches of up to `slots` sweeps, and
+// their placement in `base`
 inline size_t track_bytes(int ntiles, int slots) { return 2 * (size_t)ntiles * 4 * (1 + slots); }
 inline TrackOut track_out(void* base, int ntiles, int slots, int which) {
     unsigned* u = static_cast<unsigned*>(base) + (size_t)which * ntiles * (1 + slots);
@@ -134,7 +138,6 @@ inline TrackOut track_out(void* base, int ntiles, int slots, int which) {
 struct TrackArgs {
     TrackOut out;    // this launch's
     TrackOut prev;   // the previous launch's, null for a batch's first
-    int slots;       // floats of maxima per tile
     int nprev;       // sweeps of the previous launch
     int first_prev;  // sweeps of the solve before it
     int group;       // sweeps the stop is rounded up to
@@ -148,13 +151,13 @@ struct TrackArgs {
 // a launch and leave words, while workgroups that start later still read).
 struct TrackBatch {
     void* base;  // both TrackOut
-    int ntiles;
+    int ntiles, slots;
     TrackArgs a;
     int launches;
     // the next launch: nsweeps sweeps after the solve's first `first`
     TrackArgs launch(int lid, int nsweeps, int first) {
         a.lid = lid;
-        a.out = track_out(base, ntiles, a.slots, launches++ & 1);
+        a.out = track_out(base, ntiles, slots, launches++ & 1);
         const TrackArgs now = a;
         a.prev = a.out;
         a.nprev = nsweeps;
@@ -169,8 +172,7 @@ struct TrackBatch {
     }
 };
 inline TrackBatch track_batch(void* base, int ntiles, int slots, int group, double tol) {
-    TrackBatch t{base, ntiles, {}, 0};
-    t.a.slots = slots;
+    TrackBatch t{base, ntiles, slots, {}, 0};
     t.a.group = group;
     t.a.tol = tol;
     return t;

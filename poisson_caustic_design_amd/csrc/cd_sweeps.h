@@ -179,7 +179,7 @@ __device__ __forceinline__ TrackPlan track_decide(const TrackArgs& a, SolveDev* 
         const int j = stop >= 0 ? stop : a.nprev - 1;
         float m = 0.f;
         for (int i = threadIdx.x; i < ntiles; i += 64 * NW)
-            m = fmaxf(m, a.prev.maxima[(size_t)i * a.slots + j]);
+            m = fmaxf(m, a.prev.maxima[(size_t)i * a.nprev + j]);
         m = wave_max_pos(m);
         __syncthreads();  // red has been read
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = __float_as_uint(m);
@@ -210,7 +210,7 @@ __device__ __forceinline__ void track_store(const TrackArgs& a, const float (*sm
         float m = smax[j][0][lane];
         for (int v = 1; v < NW; ++v) m = fmaxf(m, smax[j][v][lane]);
         m = wave_max_pos(m);
-        if (lane == 0) a.out.maxima[(size_t)tile * a.slots + j] = m;
+        if (lane == 0) a.out.maxima[(size_t)tile * nsweeps + j] = m;
         if (!((double)m < a.tol)) over |= 1u << j;
     }
     if (lane == 0) red[wave] = over;
