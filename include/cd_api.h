@@ -92,7 +92,9 @@ int cd_get_api_version(void);
 /* Kernel timing over HIP events on the context stream (off by default).
  * kernel ids: cd_kernel_id */
 typedef enum {
-    CD_KERNEL_SOR_SWEEP = 0,    /* the red-black SOR sweep kernel(s)                 */
+    CD_KERNEL_SOR_SWEEP = 0,    /* the red-black SOR sweep kernel(s); a solve in one
+                                 * launch (mixed precision, up to 128 x 128 cells)
+                                 * counts here with its checks                       */
     CD_KERNEL_RESIDUAL = 1,     /* FP64 residual + correction flush                  */
     CD_KERNEL_RASTER = 2,       /* mesh rasterization                                */
     CD_KERNEL_VERTEX = 3,       /* per-vertex kernels                                */
